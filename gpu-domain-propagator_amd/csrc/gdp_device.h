@@ -97,6 +97,7 @@ constexpr int kStatusApply = 2;    // split-row segments queued for the apply ph
 // Words of the problem-wide status block (separate from the ring).
 constexpr int kGlobalError = 0;    // a bounded device wait timed out
 constexpr int kGlobalSteps = 1;    // steps run by the persistent kernel
+constexpr int kGlobalTicket = 2;   // workgroups of unpack_rounds_kernel that are done
 constexpr int kGlobalWords = 8;
 
 // State of one unit (int32 words, read as 64-bit pairs).  A step's changes
@@ -112,7 +113,8 @@ struct UnitState {
     int envelope;     // input bounds outside the storage-class envelope
     int changed[2];   // last step of each parity in which the unit moved a bound
     int mark_limit;   // accepted candidates of a step from which all rows are processed
-    int pad[7];
+    int error;        // a bounded device wait timed out (host copy of the outcome)
+    int pad[6];
 };
 
 // Accepted candidates counted per unit and step (ring of kMoveSlots steps,
@@ -212,6 +214,39 @@ struct DevState {
     int n_active;
     int n_lds;             // binary columns read from LDS (persistent launch of one unit; else 0)
     unsigned *SB;          // 2-bit codes of the binary columns (sb_words per unit)
+};
+
+// ---- double-buffered rounds (one bound vector) ----
+// Two blocks of bound records take turns: round s reads the bounds S_{s-1}
+// from block (s - 1) & 1 and folds its candidates into block s & 1, which
+// still holds S_{s-2}; the columns that round s - 1 moved are folded into it
+// in the same phase (maximum and minimum commute), so that at the end of the
+// round it holds S_s.  A round is then one phase, with one kernel boundary or
+// one grid barrier, in place of sweep, apply and publish.  Every round
+// processes every row: no marks.  Crossed bounds of round s - 1 are found
+// while its moved columns are folded in round s, whose own candidates are
+// then dropped with their block.
+// Records: int32 pairs for the integer columns, then FP64 pairs from byte
+// snap_offF (the DevMatrix of these kernels has n16 = 0, snap_off32 = 0).
+constexpr int kPlanBins = 9;          // tree widths 2^8 .. 2^0
+constexpr int kMaxGatherBlocks = 512; // workgroups of the persistent launch
+constexpr int kRoundsOver = 0x40000000;  // host word: no further round runs
+struct RoundPlan {
+    int n_items;                      // segments of split rows, then group items
+    int n_segs;
+    int item0[kPlanBins + 1];         // first item of the bin of width 2^(8 - q)
+    int row0[kPlanBins + 1];          // first layout row of the bin
+    int rows_per_item[kPlanBins];
+    int logg[kPlanBins];              // lanes per row (log2)
+    int logk[kPlanBins];              // entries per lane (log2)
+    char *block[2];
+    double2 *AX[2];                   // exact integer values beyond int32, per block
+    unsigned *bm[2];                  // columns moved in a round, by parity
+    unsigned long long *slots;        // arrivals of the persistent launch's barrier, two sets
+    double *lbs, *ubs;                // the caller's vectors
+    int mark_limit, max_rounds;
+    int *host_word;                   // pinned: progress of the launches (see round_kernel)
+    UnitState *host_state;            // pinned: the outcome
 };
 
 // State arrays of unit u (replicas mode); the shared arrays are unchanged.

@@ -45,6 +45,12 @@ __global__ void apply_split_kernel(DevMatrix M, DevState D, int step, int guard,
 __global__ void publish_kernel(DevMatrix M, DevState D, int step, int guard, int first_step, int n_units);
 template <int kThreads, bool kLds>
 __global__ void mega_kernel(DevMatrix M, DevState D, int first_step, int max_steps, int n_units);
+__global__ void reset_rounds_kernel(DevState D, RoundPlan R);
+__global__ void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin);
+__global__ void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
+__global__ void round_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
+__global__ void rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
+__global__ void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status);
 __global__ void load_kernel(DevMatrix M, DevState D, int n_list, const int *list, const double *const *lbp,
                             const double *const *ubp);
@@ -272,6 +278,46 @@ void upload(T *dst, const T *src, size_t count, hipStream_t s) {
         check(hipMemcpyAsync(dst, src, count * sizeof(T), hipMemcpyHostToDevice, s), "H2D");
 }
 
+// Words of pinned host memory that kernels write a run's progress and outcome
+// to: 256 bytes per problem out of slabs of 64 KiB, which stay for the next
+// problems (one slab per 256 problems alive at a time).
+struct HostSlot {
+    UnitState state;
+    int word;
+};
+
+class HostSlots {
+  public:
+    HostSlot *take() {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (free_.empty()) {
+            char *slab = nullptr;
+            check(hipHostMalloc(reinterpret_cast<void **>(&slab), kSlots * kSlotBytes,
+                                hipHostMallocPortable | hipHostMallocMapped),
+                  "hipHostMalloc");
+            for (size_t k = 0; k < kSlots; k++) free_.push_back(slab + (kSlots - 1 - k) * kSlotBytes);
+        }
+        char *p = free_.back();
+        free_.pop_back();
+        return reinterpret_cast<HostSlot *>(p);
+    }
+    void give(HostSlot *p) {
+        std::lock_guard<std::mutex> lk(mu_);
+        free_.push_back(reinterpret_cast<char *>(p));
+    }
+
+  private:
+    static constexpr size_t kSlotBytes = 256, kSlots = 256;
+    std::mutex mu_;
+    std::vector<char *> free_;
+};
+static_assert(sizeof(HostSlot) <= 256, "a host slot holds the outcome and the progress word");
+
+HostSlots &host_slots() {
+    static HostSlots *h = new HostSlots();  // outlives every problem
+    return *h;
+}
+
 // Phase times of a problem's creation, printed to stderr when the
 // environment variable GDP_TRACE_CREATE is set (a diagnostic of where the
 // creation time goes: host ordering, allocations, copies, device layout).
@@ -409,6 +455,13 @@ struct Problem {
     std::vector<int> graph_last;
     long long graph_key = -1;
     std::mutex run_mutex;
+    // double-buffered rounds (one bound vector; gdp_device.h, RoundPlan)
+    bool rounds_ok = false;           // the problem's single runs take them
+    DevMatrix Mr{};                   // the matrix with the rounds' record layout
+    RoundPlan R{};
+    bool rounds_state = false;        // R's arrays are in the current run state
+    int rounds_grid = 0, rounds_threads = 0;  // persistent launch
+    HostSlot *host = nullptr;
     int servers = 0;                  // servers attached (they own the unit slots)
     bool graphs_enabled = true;       // GPU_LOOP may capture graphs of the current run state
     bool staging_held = false;
@@ -429,6 +482,7 @@ struct Problem {
         if (state_buf) (void)cached_free(state_buf);
         for (void *p : hint_owned) (void)cached_free(p);
         for (void *p : owned) (void)cached_free(p);
+        if (host) host_slots().give(host);
         if (staging_held) staging().release();
     }
 };
@@ -484,10 +538,31 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
     return off;
 }
 
-// Points the problem's run state at `base` (cap units, see carve_state).
-void bind_state(Problem *P, char *base, int cap) {
+// The arrays of the double-buffered rounds (one bound vector), after those
+// of carve_state.  Returns the bytes needed.
+size_t carve_rounds(const DevMatrix &Mr, char *base, RoundPlan &R) {
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        char *p = base ? base + off : nullptr;
+        off += (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+        return p;
+    };
+    for (int k = 0; k < 2; k++) {
+        R.block[k] = take(static_cast<size_t>(Mr.snap_stride));
+        R.AX[k] = reinterpret_cast<double2 *>(take(Mr.n_int * sizeof(double2)));
+        R.bm[k] = reinterpret_cast<unsigned *>(take(Mr.nwords * sizeof(unsigned)));
+    }
+    R.slots = reinterpret_cast<unsigned long long *>(take(2 * kMaxGatherBlocks * sizeof(unsigned long long)));
+    return off;
+}
+
+// Points the problem's run state at `base` (cap units, see carve_state);
+// with `rounds`, the arrays of the double-buffered rounds follow.
+void bind_state(Problem *P, char *base, int cap, bool rounds) {
     UnitTables T;
-    carve_state(P->M, P->replicas, P->n_inst, cap, base, P->D, T);
+    const size_t off = carve_state(P->M, P->replicas, P->n_inst, cap, base, P->D, T);
+    if (rounds) carve_rounds(P->Mr, base + off, P->R);
+    P->rounds_state = rounds;
     P->d_list = T.list;
     P->d_params = T.params;
     P->d_lbp = T.lbp;
@@ -508,9 +583,11 @@ void alloc_units(Problem *P, int cap) {
     P->n_units = 0;
     DevState D{};
     UnitTables T;
-    const size_t bytes = carve_state(P->M, P->replicas, P->n_inst, cap, nullptr, D, T);
+    size_t bytes = carve_state(P->M, P->replicas, P->n_inst, cap, nullptr, D, T);
+    RoundPlan R;
+    if (P->rounds_ok) bytes += carve_rounds(P->Mr, nullptr, R);
     check(cached_malloc(&P->state_buf, bytes), "hipMalloc run state");
-    bind_state(P, static_cast<char *>(P->state_buf), cap);
+    bind_state(P, static_cast<char *>(P->state_buf), cap, P->rounds_ok);
     const size_t k = P->replicas ? static_cast<size_t>(cap) : 1;
     const DevMatrix &M = P->M;
     check(hipMemsetAsync(P->D.units, 0, sizeof(UnitState) * P->n_units, P->stream), "memset units");
@@ -739,6 +816,69 @@ RowOrder device_row_order(const std::vector<InstanceView> &inst, const std::vect
     }
     if (prev >= 0) R.count[prev] = R.mp - R.start[prev];
     return R;
+}
+
+// The plan of the double-buffered rounds of a single problem with default
+// tuning: start / count hold the first layout row and the rows of each bin
+// key (10 - log2 of the tree width).
+void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
+    const Tuning def;
+    const Tuning &T = P->tuning;
+    // Every round processes every row, which costs about 8.5 ps per entry; the
+    // three-phase rounds of larger problems skip the rows whose columns did not
+    // move.  200,000 rows, 2.2M nonzeros, 32 rounds: 0.80 ms a call (three
+    // phases: 1.3 persistent, 2.4 in the host loop).  3.1M nonzeros over 500,000
+    // columns, 65 rounds: 2.4 ms (2.4 / 5.9).  19.3M nonzeros: 4.8 ms (3.1).
+    constexpr int kMaxRoundEntries = 4 << 20;
+    if (!P->replicas || P->n_inst != 1 || n_padded > kMaxRoundEntries) return;
+    if (T.item_nnz != def.item_nnz || T.mega_blocks_per_cu != def.mega_blocks_per_cu ||
+        T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
+        !std::equal(T.group_log, T.group_log + 10, def.group_log))
+        return;
+    RoundPlan &R = P->R;
+    R.n_segs = P->M.n_seg_parts;
+    // Entries per lane: few while the passes (256 lane entries of K each) still
+    // find a free SIMD, because a pass is a chain of dependent loads, a butterfly
+    // and divisions that grows with K.  Per persistent round with 1 / 2 / 4:
+    // 33K entry slots 7.3 / 7.5 / 8.8 us, 115K 8.5 / 8.1 / 8.9 us, 330K 12.5 /
+    // 10.3 / 10.4 us.
+    const int logk_want = n_padded <= (64 << 10) ? 0 : (n_padded <= (512 << 10) ? 1 : 2);
+    int at = R.n_segs;
+    for (int q = 0; q < kPlanBins; q++) {
+        const int b = kPlanBins - 1 - q, key = 10 - b;
+        const int logk = std::max(std::min(logk_want, b), b - 6);
+        const int logg = b - logk;
+        R.logk[q] = logk;
+        R.logg[q] = logg;
+        R.rows_per_item[q] = 64 >> logg;
+        R.item0[q] = at;
+        R.row0[q] = start[key];
+        at += (count[key] + R.rows_per_item[q] - 1) / R.rows_per_item[q];
+    }
+    R.item0[kPlanBins] = at;
+    R.row0[kPlanBins] = P->M.m;
+    // bins without rows have no start of their own
+    for (int q = kPlanBins - 1; q >= 0; q--)
+        if (count[2 + q] == 0) R.row0[q] = R.row0[q + 1];
+    R.n_items = at;
+    DevMatrix &M = P->Mr;
+    M = P->M;
+    M.n16 = 0;
+    M.snap_off32 = 0;
+    M.snap_offF = (M.n_int * 8 + 15) / 16 * 16;
+    M.snap_stride = M.snap_offF + 16LL * (M.n - M.n_int) + 16;
+    P->host = host_slots().take();
+    int per_cu = 0;
+    // at most 256 workgroups while the items allow it: the barrier grows with
+    // them (1.2 us for 16, 3 us for 256, 4.3 us for 512), and a workgroup of 256
+    // threads spreads few items over more compute units
+    P->rounds_threads = R.n_items <= 1024 ? 256 : (R.n_items <= 2048 ? 512 : 1024);
+    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(rounds_kernel),
+                                                       P->rounds_threads, 0),
+          "occupancy");
+    const int waves = P->rounds_threads / 64;
+    P->rounds_grid = std::max(1, std::min({per_cu * P->cu_count, kMaxGatherBlocks, (R.n_items + waves - 1) / waves}));
+    P->rounds_ok = true;
 }
 
 Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tuning *tuning) {
@@ -1038,6 +1178,8 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
             P->stats.n_units = replicas ? 0 : NI;
         }
 
+        plan_rounds(P, R.start.data(), R.count.data(), n_padded);
+
         P->mega_threads = T.mega_threads == 256 || T.mega_threads == 1024 ? T.mega_threads : 512;
         P->mega_fn = P->mega_threads == 256    ? reinterpret_cast<const void *>(mega_kernel<256, false>)
                      : P->mega_threads == 1024 ? reinterpret_cast<const void *>(mega_kernel<1024, false>)
@@ -1278,11 +1420,124 @@ UnitState read_unit(Problem *P, int u) {
     return st;
 }
 
+// ---- double-buffered rounds of one bound vector ----
+
+// Waits until the launches have started round `step` or are over; returns
+// the progress word.
+int wait_round(Problem *P, int step) {
+    const int *word = &P->host->word;
+    for (unsigned spins = 1;; spins++) {
+        const int w = __atomic_load_n(word, __ATOMIC_RELAXED);
+        if (w >= step) return w;
+        __builtin_ia32_pause();
+        if (spins % 8192 == 0) {
+            // an idle stream whose launches never got there, or a failed one
+            const hipError_t e = hipStreamQuery(P->stream);
+            if (e == hipErrorNotReady) continue;
+            check(e, "round launches");
+            const int end = __atomic_load_n(word, __ATOMIC_RELAXED);
+            if (end >= step) return end;
+            throw std::runtime_error("the round launches ended early");
+        }
+    }
+}
+
+// Issues round `step`.
+void launch_round(Problem *P, int step) {
+    const int grid = std::max(1, std::min(8 * P->cu_count, grid_for(P->R.n_items)));
+    hipLaunchKernelGGL(round_kernel, dim3(grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+    if (P->Mr.n_seg_parts > 0)
+        hipLaunchKernelGGL(round_apply_kernel, dim3(std::max(1, std::min(1024, grid_for(P->Mr.n_seg_parts)))),
+                           dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+}
+
+// Rounds 1 .. max_rounds, each one launch (two with split rows) that stops
+// itself on the device once the run is over; `first` .. `last` of them as one
+// captured graph.
+void launch_round_graph(Problem *P, int ci, int first, int last) {
+    hipStream_t s = P->stream;
+    if (static_cast<int>(P->graphs.size()) <= ci) {
+        P->graphs.resize(ci + 1, nullptr);
+        P->graph_last.resize(ci + 1, 0);
+    }
+    if (!P->graphs[ci]) {
+        hipGraph_t graph;
+        check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture");
+        for (int step = first; step <= last; step++) launch_round(P, step);
+        check(hipStreamEndCapture(s, &graph), "end capture");
+        hipGraphExec_t exec;
+        check(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "instantiate");
+        (void)hipGraphDestroy(graph);
+        P->graphs[ci] = exec;
+        P->graph_last[ci] = last;
+    }
+    check(hipGraphLaunch(P->graphs[ci], s), "graph launch");
+}
+
+RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds) {
+    hipStream_t s = P->stream;
+    RoundPlan &R = P->R;
+    const DevMatrix &M = P->Mr;
+    R.lbs = d_lbs;
+    R.ubs = d_ubs;
+    R.max_rounds = max_rounds;
+    R.mark_limit = P->mark_limit[0];
+    R.host_word = &P->host->word;
+    R.host_state = &P->host->state;
+    __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
+    const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
+    hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R);
+    hipLaunchKernelGGL(load_rounds_kernel, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
+    check(hipGetLastError(), "load launch");
+    check(hipEventRecord(P->ev0, s), "event");
+    if (sync_type == MEGAKERNEL_ID) {
+        void *args[] = {const_cast<DevMatrix *>(&M), &P->D, &R};
+        check(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(rounds_kernel), dim3(P->rounds_grid),
+                                         dim3(P->rounds_threads), args, 0, s),
+              "rounds_kernel launch");
+    } else if (sync_type == GPU_LOOP_ID && P->graphs_enabled) {
+        // the next chunk is launched while the last rounds of the previous
+        // one run
+        const int chunk = std::max(1, P->tuning.graph_rounds);
+        const long long key = (1LL << 40) + max_rounds;
+        if (key != P->graph_key) {
+            P->drop_graphs();
+            P->graph_key = key;
+        }
+        for (int first = 1, ci = 0; first <= max_rounds; first += chunk, ci++) {
+            const int last = std::min(max_rounds, first + chunk - 1);
+            launch_round_graph(P, ci, first, last);
+            if (last < max_rounds && wait_round(P, std::max(first, last - 1)) == kRoundsOver) break;
+        }
+    } else {
+        // launches run ahead of the host's look at the progress by kAhead
+        // rounds, so that the device never waits for it
+        constexpr int kAhead = 2;
+        for (int step = 1; step <= max_rounds; step++) {
+            launch_round(P, step);
+            if (step > kAhead && wait_round(P, step - kAhead) == kRoundsOver) break;
+        }
+        check(hipGetLastError(), "round launch");
+    }
+    check(hipEventRecord(P->ev1, s), "event");
+    hipLaunchKernelGGL(unpack_rounds_kernel, dim3(std::min(gx, 256)), dim3(256), 0, s, M, P->D, R);
+    check(hipGetLastError(), "unpack launch");
+    check(hipStreamSynchronize(s), "rounds sync");
+    const UnitState st = P->host->state;
+    if (st.error) throw std::runtime_error("device wait timed out");
+    RunResult r = outcome(st);
+    float ms = 0.f;
+    if (!st.crossed) check(hipEventElapsedTime(&ms, P->ev0, P->ev1), "elapsed");
+    r.kernel_ms = ms;
+    return r;
+}
+
 // A complete run of one bound vector (device pointers) as unit 0, from
 // round 1.  Host buffers stay on the stack.
 RunResult run_single(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds) {
     if (sync_type < CPU_LOOP_ID || sync_type > MEGAKERNEL_ID) throw std::runtime_error("Unknown sync type");
     if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
+    if (P->rounds_state) return run_rounds(P, d_lbs, d_ubs, sync_type, max_rounds);
     const int list[1] = {0};
     const int caps[1] = {max_rounds};
     P->D.n_active = 1;
@@ -1677,8 +1932,14 @@ class BorrowedState {
   public:
     BorrowedState(Problem *P, char *base)
         : P_(P), D_(P->D), list_(P->d_list), params_(P->d_params), lbp_(P->d_lbp), ubp_(P->d_ubp),
-          hint_ptr_(P->d_hint_ptr), capacity_(P->capacity), n_units_(P->n_units), graphs_(P->graphs_enabled) {
-        bind_state(P, base, 1);
+          hint_ptr_(P->d_hint_ptr), capacity_(P->capacity), n_units_(P->n_units), graphs_(P->graphs_enabled),
+          R_(P->R), rounds_state_(P->rounds_state) {
+        // the double-buffered rounds where their arrays fit too
+        DevState D{};
+        UnitTables T;
+        RoundPlan R;
+        const size_t need = carve_state(P->M, P->replicas, P->n_inst, 1, nullptr, D, T);
+        bind_state(P, base, 1, P->rounds_ok && need + carve_rounds(P->Mr, nullptr, R) <= kScratchBytes);
         P->graphs_enabled = false;
     }
     ~BorrowedState() {
@@ -1691,6 +1952,8 @@ class BorrowedState {
         P_->capacity = capacity_;
         P_->n_units = n_units_;
         P_->graphs_enabled = graphs_;
+        P_->R = R_;
+        P_->rounds_state = rounds_state_;
     }
     BorrowedState(const BorrowedState &) = delete;
     BorrowedState &operator=(const BorrowedState &) = delete;
@@ -1704,6 +1967,8 @@ class BorrowedState {
     int *hint_ptr_;
     int capacity_, n_units_;
     bool graphs_;
+    RoundPlan R_;
+    bool rounds_state_;
 };
 }  // namespace
 

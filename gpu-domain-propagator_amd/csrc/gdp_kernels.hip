@@ -133,8 +133,20 @@ __device__ __forceinline__ void lds_binary_bounds(int id, double &l, double &u) 
     u = (code & 2u) ? 0.0 : 1.0;
 }
 
-__device__ __forceinline__ uint4 load_chunk(const DevState &D, unsigned off) {
-    return *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(D.S16) + (off & ~15u));
+// kCoherent: a device-coherent load (sc1: past the L1, coherent across the
+// XCDs' L2s) for a launch in which other workgroups wrote the snapshot, with
+// no cache invalidation between the rounds.  A buffer load, since atomic
+// loads end at 8 bytes; its offset is checked against the block's size.
+template <bool kCoherent>
+__device__ __forceinline__ uint4 load_chunk(const DevMatrix &M, const DevState &D, unsigned off) {
+    if constexpr (kCoherent) {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(D.S16, 0, static_cast<int>(M.snap_stride), 0x00020000);
+        constexpr int kSc1 = 16;
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(off & ~15u), 0, kSc1);
+        return make_uint4(v[0], v[1], v[2], v[3]);
+    } else {
+        return *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(D.S16) + (off & ~15u));
+    }
 }
 
 // Bounds of `id` from the chunk at its record offset `off`.
@@ -159,12 +171,13 @@ __device__ __forceinline__ void decode_bounds(const DevMatrix &M, int id, unsign
 }
 
 // Bounds of internal column `id` at the start of the round.
+template <bool kCoherent>
 __device__ __forceinline__ void load_bounds(const DevMatrix &M, const DevState &D, int id, double &l, double &u) {
     if (id < D.n_lds) {
         lds_binary_bounds(id, l, u);
     } else {
         const unsigned off = record_offset(M, id);
-        decode_bounds(M, id, off, load_chunk(D, off), l, u);
+        decode_bounds(M, id, off, load_chunk<kCoherent>(M, D, off), l, u);
     }
 }
 
@@ -334,7 +347,7 @@ __device__ __forceinline__ double seq_eps_max(const DevMatrix &M, const DevState
     double run = 0.0;
     for (int e = 0; e < len; e++) {
         double l, u;
-        load_bounds(M, D, M.col[start + e] & kIdMask, l, u);
+        load_bounds<false>(M, D, M.col[start + e] & kIdMask, l, u);
         run = eps_max_step(run, fabs(M.val[start + e]) * (u - l));
     }
     return run;
@@ -375,7 +388,7 @@ __device__ __forceinline__ void row_extent(const DevMatrix &M, int r, int &start
 
 // K consecutive entries of one lane: loads, contributions, pairwise tree of
 // the K contributions in natural order, and the cross-lane reduction.
-template <int K>
+template <int K, bool kCoherent = false>
 struct LaneEntries {
     int jp[K];
     double a[K], l[K], u[K];
@@ -429,7 +442,7 @@ struct LaneEntries {
             }
             off[k] = record_offset(M, jp[k] & kIdMask);
             chunk[k] = make_uint4(0u, 0u, 0u, 0u);
-            if ((jp[k] & kIdMask) >= D.n_lds) chunk[k] = load_chunk(D, off[k]);
+            if ((jp[k] & kIdMask) >= D.n_lds) chunk[k] = load_chunk<kCoherent>(M, D, off[k]);
         }
 #pragma unroll
         for (int k = 0; k < K; k++) {
@@ -598,7 +611,7 @@ __device__ __forceinline__ Sink make_sink(const DevState &V) {
 // Rows [first, first + nrows) of one tree-width bin: groups of 2^logg lanes,
 // K consecutive entries per lane.  Rows not marked for this step are
 // skipped (a pass with no marked row loads nothing).
-template <int K>
+template <int K, bool kCoherent>
 __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int first, int nrows, int logg,
                                           int step, bool all_rows) {
     const DevState &V = S.V;
@@ -620,7 +633,7 @@ __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int
             lhs = sd.x;
             rhs = sd.y;
         }
-        LaneEntries<K> E;
+        LaneEntries<K, kCoherent> E;
         E.load(M, V, start, gl * K, len);
         E.reduce(g);
         const double minact = 0.0 + E.tmin;
@@ -664,7 +677,7 @@ __device__ __forceinline__ int long_item(const DevMatrix &M, const Sink &S, int 
         for (int e = lane; e < len; e += 64) {
             const int jp = M.col[start + e];
             double l, u;
-            load_bounds(M, V, jp & kIdMask, l, u);
+            load_bounds<false>(M, V, jp & kIdMask, l, u);
             moved += apply_entry(M, S, jp, M.val[start + e], l, u, sd.x, sd.y, acc_min, acc_max, mininf, maxinf);
         }
     }
@@ -675,6 +688,7 @@ __device__ __forceinline__ int long_item(const DevMatrix &M, const Sink &S, int 
 // wave.  A segment whose exact maximum Ms satisfies !(Ms - run > eps) cannot
 // replace the running value (floating-point subtraction is monotone), so it
 // is skipped; the others are scanned entry by entry in order.
+template <bool kCoherent>
 __device__ __forceinline__ double split_eps_scan(const DevMatrix &M, const DevState &V, const int4 info, int start, int len) {
     constexpr int K = kSegLen / 64;
     const int lane = threadIdx.x & 63;
@@ -687,7 +701,7 @@ __device__ __forceinline__ double split_eps_scan(const DevMatrix &M, const DevSt
             const double mt = __shfl(ms, t, 64);
             if (!eps_gt(mt, run)) continue;
             const int s0 = (b + t) * kSegLen;
-            LaneEntries<K> E;
+            LaneEntries<K, kCoherent> E;
             E.load(M, V, start + s0, lane * K, len - s0);
             run = E.eps_scan(64, run);
         }
@@ -697,7 +711,8 @@ __device__ __forceinline__ double split_eps_scan(const DevMatrix &M, const DevSt
 
 // Stores the activity partial of segment `part` and the step that computed
 // it (lane 0 of the wave).
-__device__ __forceinline__ void store_part(const DevState &V, int part, const LaneEntries<kSegLen / 64> &E,
+template <bool kCoherent>
+__device__ __forceinline__ void store_part(const DevState &V, int part, const LaneEntries<kSegLen / 64, kCoherent> &E,
                                            int step) {
     SegPart *p = &V.seg_parts[part];
     coherent_store_d(&p->smin, E.tmin);
@@ -712,6 +727,7 @@ __device__ __forceinline__ void store_part(const DevState &V, int part, const La
 // completes the row's count adds the partials in segment order and decides
 // the row gate; when it passes, the row's activity is stored and its
 // segments are queued for the apply phase that follows the sweep.
+template <bool kCoherent>
 __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, const DevState &V, int u, int lr, int s, int cnt,
                          int *st, int step, bool all_rows, int unit_start) {
     constexpr int K = kSegLen / 64;
@@ -739,7 +755,7 @@ __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, 
         const int part = info.y + s + q;
         if (!all_rows && ((keep >> q) & 1ull)) continue;
         const int s0 = (s + q) * kSegLen;
-        LaneEntries<K> E;
+        LaneEntries<K, kCoherent> E;
         E.load(M, V, start + s0, lane * K, len - s0);
         E.reduce(64);
         if (lane == 0) store_part(V, part, E, step);
@@ -786,7 +802,7 @@ __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, 
     const double2 sd = M.sides[r];
     const GateBounds gb = gate_bounds(am, ax, ni, xi, sd.x, sd.y, dm);
     bool gate = gb.hi;
-    if (!gb.decided()) gate = row_gate(am, ax, ni, xi, sd.x, sd.y, split_eps_scan(M, V, info, start, len));
+    if (!gb.decided()) gate = row_gate(am, ax, ni, xi, sd.x, sd.y, split_eps_scan<kCoherent>(M, V, info, start, len));
     int pos = 0;
     if (lane == 0) {
         coherent_store(&V.seg_count[lr], 0u);
@@ -836,7 +852,7 @@ __device__ __forceinline__ void sweep_item(const DevMatrix &M, const DevState &D
     int moved = 0;
     if (kind == kItemSeg) {
         const int r = M.seg_rows[d.y].x;
-        if (us.all_rows || V.marks[r] == step) seg_item(M, D, V, u, d.y, d.z, d.w, st, step, us.all_rows, us.start);
+        if (us.all_rows || V.marks[r] == step) seg_item<false>(M, D, V, u, d.y, d.z, d.w, st, step, us.all_rows, us.start);
         return;
     }
     if (kind == kItemLong) {
@@ -845,21 +861,23 @@ __device__ __forceinline__ void sweep_item(const DevMatrix &M, const DevState &D
         const int logg = (d.x >> 4) & 15;
         const int logk = (d.x >> 8) & 15;
         switch (logk) {
-            case 0: moved = group_item<1>(M, S, d.y, d.z, logg, step, us.all_rows); break;
-            case 1: moved = group_item<2>(M, S, d.y, d.z, logg, step, us.all_rows); break;
-            default: moved = group_item<4>(M, S, d.y, d.z, logg, step, us.all_rows); break;
+            case 0: moved = group_item<1, false>(M, S, d.y, d.z, logg, step, us.all_rows); break;
+            case 1: moved = group_item<2, false>(M, S, d.y, d.z, logg, step, us.all_rows); break;
+            default: moved = group_item<4, false>(M, S, d.y, d.z, logg, step, us.all_rows); break;
         }
     }
     note_change(D, u, step, moved);
 }
 
 // Applies the candidates of queued task `task` = unit * n_seg_parts + segment
-// (one wave; the row's activity is read back from its SegState).
-__device__ __forceinline__ void apply_split_task(const DevMatrix &M, const DevState &D, int task, int step, int *st) {
+// (one wave; the row's activity is read back from its SegState).  Returns the
+// lane's accepted candidates; u: the task's unit.
+template <bool kCoherent>
+__device__ __forceinline__ int apply_split_task(const DevMatrix &M, const DevState &D, int task, int &u) {
     constexpr int K = kSegLen / 64;
     const int lane = threadIdx.x & 63;
     task = uniform(task);
-    const int u = task / M.n_seg_parts;
+    u = task / M.n_seg_parts;
     const int part = task - u * M.n_seg_parts;
     const DevState V = unit_view(M, D, u);
     const Sink S = make_sink(V);
@@ -882,18 +900,22 @@ __device__ __forceinline__ void apply_split_task(const DevMatrix &M, const DevSt
         if (e < len) {
             const int jp = M.col[start + e];
             double l, uu;
-            load_bounds(M, V, jp & kIdMask, l, uu);
+            load_bounds<kCoherent>(M, V, jp & kIdMask, l, uu);
             moved += apply_entry(M, S, jp, M.val[start + e], l, uu, sd.x, sd.y, minact, maxact, ni, xi);
         }
     }
-    note_change(D, u, step, moved);
+    return moved;
 }
 
 // The apply phase: the waves of the grid take the queued segments in turn.
 __device__ __forceinline__ void apply_phase(const DevMatrix &M, const DevState &D, int step, int wave, int nwaves) {
     int *st = status_row(D, step);
     const int count = coherent_load(&st[kStatusApply]);
-    for (int t = wave; t < count; t += nwaves) apply_split_task(M, D, coherent_load(&D.apply_tasks[t]), step, st);
+    for (int t = wave; t < count; t += nwaves) {
+        int u;
+        const int moved = apply_split_task<false>(M, D, coherent_load(&D.apply_tasks[t]), u);
+        note_change(D, u, step, moved);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1394,6 +1416,373 @@ template __global__ void mega_kernel<1024, false>(DevMatrix, DevState, int, int,
 template __global__ void mega_kernel<256, true>(DevMatrix, DevState, int, int, int);
 template __global__ void mega_kernel<512, true>(DevMatrix, DevState, int, int, int);
 template __global__ void mega_kernel<1024, true>(DevMatrix, DevState, int, int, int);
+
+// ---------------------------------------------------------------------------
+// double-buffered rounds of one bound vector (gdp_device.h, RoundPlan)
+// ---------------------------------------------------------------------------
+
+// The state of round `step`: records read from block (step - 1) & 1,
+// candidates and moved-column bits into the other parity's arrays.
+__device__ __forceinline__ DevState round_view(const DevMatrix &M, const DevState &D, const RoundPlan &R, int step) {
+    const bool odd = step & 1;
+    char *nxt = odd ? R.block[1] : R.block[0];
+    DevState V = D;
+    V.S16 = reinterpret_cast<unsigned *>(odd ? R.block[0] : R.block[1]);
+    V.AI = reinterpret_cast<int2 *>(nxt);
+    V.AF = reinterpret_cast<double2 *>(nxt + M.snap_offF);
+    V.AX = odd ? R.AX[1] : R.AX[0];
+    V.bm = odd ? R.bm[1] : R.bm[0];
+    V.n_lds = 0;
+    return V;
+}
+
+// The accumulator view of a parity (as read after its round).
+__device__ __forceinline__ DevState block_view(const DevMatrix &M, const DevState &D, const RoundPlan &R, int parity) {
+    char *block = parity ? R.block[1] : R.block[0];
+    DevState V = D;
+    V.AI = reinterpret_cast<int2 *>(block);
+    V.AF = reinterpret_cast<double2 *>(block + M.snap_offF);
+    V.AX = parity ? R.AX[1] : R.AX[0];
+    V.bm = parity ? R.bm[1] : R.bm[0];
+    return V;
+}
+
+// Folds the columns that round step - 1 moved into the block of round `step`
+// and clears their bits.  Returns whether one of the lane's columns is
+// crossed.  Each wave takes `chunk` words of the bitmap at a time (one lane
+// each) and works through the nonzero ones two at a time, a half-wave per
+// word.
+__device__ __forceinline__ bool carry_moved(const DevMatrix &M, const DevState &D, const RoundPlan &R, int step,
+                                            int wave, int nwaves) {
+    const DevState C = block_view(M, D, R, (step - 1) & 1);
+    const DevState N = block_view(M, D, R, step & 1);
+    const int lane = threadIdx.x & 63;
+    const int half = lane >> 5, b = lane & 31;
+    int chunk = (M.nwords + nwaves - 1) / nwaves;
+    chunk = chunk < 2 ? 2 : (chunk > 64 ? 64 : chunk);
+    bool crossed = false;
+    for (int w0 = (nwaves - 1 - wave) * chunk; w0 < M.nwords; w0 += nwaves * chunk) {
+        const int w = w0 + lane;
+        const unsigned bits = lane < chunk && w < M.nwords ? coherent_load(&C.bm[w]) : 0u;
+        if (bits) coherent_store(&C.bm[w], 0u);
+        unsigned long long pending = __ballot(bits != 0u);
+        while (pending) {
+            const int t0 = __ffsll(static_cast<long long>(pending)) - 1;
+            pending &= pending - 1;
+            int t1 = -1;
+            if (pending) {
+                t1 = __ffsll(static_cast<long long>(pending)) - 1;
+                pending &= pending - 1;
+            }
+            const int t = half ? t1 : t0;
+            const unsigned wb = __shfl(bits, t < 0 ? 0 : t, 64);
+            if (t < 0 || !((wb >> b) & 1u)) continue;
+            const int id = (w0 + t) * 32 + b;
+            const AccRaw raw = acc_load(M, C, id);
+            double l, u;
+            acc_resolve(M, C, id, raw, l, u);
+            crossed |= eps_gt(l, u);
+            if (id < M.n_int) {
+                atomic_max_i(&N.AI[id].x, static_cast<int>(static_cast<unsigned long long>(raw.w) & 0xffffffffull));
+                atomic_min_i(&N.AI[id].y, static_cast<int>(static_cast<unsigned long long>(raw.w) >> 32));
+            } else {
+                atomic_max_d(&N.AF[id - M.n_int].x, raw.fl);
+                atomic_min_d(&N.AF[id - M.n_int].y, raw.fu);
+            }
+        }
+    }
+    return crossed;
+}
+
+// Item `it` of a round: a segment of a split row, or the rows of one pass
+// (or a few) of a bin.  The bins' item ranges are kernel arguments, so an
+// item costs no load.  Returns the lane's accepted candidates.
+template <bool kCoherent>
+__device__ __forceinline__ int round_item(const DevMatrix &M, const DevState &V, const RoundPlan &R, int it, int step,
+                                          int *st) {
+    it = uniform(it);
+    if (it < R.n_segs) {
+        const int lr = uniform(M.part_row[it]);
+        seg_item<kCoherent>(M, V, V, 0, lr, it - uniform(M.seg_rows[lr].y), 1, st, step, true, 1);
+        return 0;
+    }
+    int first = 0, nrows = 0, logg = 0, logk = 0;
+#pragma unroll
+    for (int q = 0; q < kPlanBins; q++)
+        if (it >= R.item0[q] && it < R.item0[q + 1]) {
+            first = R.row0[q] + (it - R.item0[q]) * R.rows_per_item[q];
+            nrows = R.row0[q + 1] - first;
+            nrows = nrows < R.rows_per_item[q] ? nrows : R.rows_per_item[q];
+            logg = R.logg[q];
+            logk = R.logk[q];
+        }
+    const Sink S = make_sink(V);
+    switch (logk) {
+        case 0: return group_item<1, kCoherent>(M, S, first, nrows, logg, step, true);
+        case 1: return group_item<2, kCoherent>(M, S, first, nrows, logg, step, true);
+        default: return group_item<4, kCoherent>(M, S, first, nrows, logg, step, true);
+    }
+}
+
+// Resets the state words, the status ring, the global words and the
+// barrier's arrival slots for a run (one workgroup).
+__global__ __launch_bounds__(256) void reset_rounds_kernel(DevState D, RoundPlan R) {
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        UnitState s = {};
+        s.start = 1;
+        s.markall = 1;
+        s.max_rounds = R.max_rounds;
+        s.mark_limit = R.mark_limit;
+        D.units[0] = s;
+    }
+    for (int k = tid; k < kStatusRows * kStatusWords; k += 256) D.status[k] = 0;
+    for (int k = tid; k < kGlobalWords; k += 256) D.global[k] = 0;
+    for (int k = tid; k < 2 * kMoveLanes; k += 256) D.moved[moved_index(0, k & 1, k >> 1)] = 0;
+    for (int k = tid; k < 2 * kMaxGatherBlocks; k += 256) R.slots[k] = 0ull;
+}
+
+// Loads the caller's vectors into both blocks and flags crossed bounds and
+// bounds outside a column's storage class (the storage classes of the
+// original matrix: n16, n_bin of the arguments).
+__global__ __launch_bounds__(256) void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin) {
+    const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+    const int stride = gridDim.x * blockDim.x;
+    const DevState A = block_view(M, D, R, 0), B = block_view(M, D, R, 1);
+    for (int id = tid; id < M.n; id += stride) {
+        const int j = M.perm[id];
+        const double l = R.lbs[j], u = R.ubs[j];
+        if (eps_gt(l, u)) atomic_or_i(&D.units[0].crossed, 1);
+        if (id < M.n_int) {
+            const double lim = id < n16 ? 32767.0 : 2147483647.0;
+            const double lo_lim = id < n_bin ? 0.0 : -lim, hi_lim = id < n_bin ? 1.0 : lim;
+            const bool fits = l >= lo_lim && l <= hi_lim && u >= lo_lim && u <= hi_lim && floor(l) == l &&
+                              floor(u) == u;
+            if (!fits && !eps_gt(l, u)) atomic_or_i(&D.units[0].envelope, 1);
+            const int2 v = make_int2(fits ? static_cast<int>(l) : 0, fits ? static_cast<int>(u) : 0);
+            A.AI[id] = v;
+            B.AI[id] = v;
+            A.AX[id] = make_double2(-INFINITY, INFINITY);
+            B.AX[id] = make_double2(-INFINITY, INFINITY);
+        } else {
+            A.AF[id - M.n_int] = make_double2(l, u);
+            B.AF[id - M.n_int] = make_double2(l, u);
+        }
+    }
+    for (int w = tid; w < M.nwords; w += stride) {
+        A.bm[w] = 0u;
+        B.bm[w] = 0u;
+    }
+    for (int q = tid; q < M.n_seg_rows; q += stride) D.seg_count[q] = 0u;
+}
+
+// Whether a round moved a bound, for the launches: the round's number in any
+// of kMoveLanes words, each on its own line, by parity (the last rounds of
+// each parity, so that no round has to clear them).  Writers look first: a
+// store that every workgroup sends to one line costs about 50 ns each.
+__device__ __forceinline__ void note_round_moved(const DevState &D, int step) {
+    int *w = &D.moved[moved_index(0, step & 1, blockIdx.x % kMoveLanes)];
+    if (coherent_load(w) != step) coherent_store(w, step);
+}
+__device__ __forceinline__ bool round_moved(const DevState &D, int step) {
+    const int lane = threadIdx.x & 63;
+    const int w = lane < kMoveLanes ? coherent_load(&D.moved[moved_index(0, step & 1, lane)]) : 0;
+    return __any(w == step);
+}
+
+// One round as one launch.  The launch first checks on the device whether
+// the run goes on (input usable, not infeasible, the previous round moved a
+// bound); the first workgroup tells the host: its word becomes `step` when
+// the round runs, else kRoundsOver.
+__global__ __launch_bounds__(256) void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+    __shared__ int any_moved;
+    const long long *p = reinterpret_cast<const long long *>(&D.units[0]);
+    const long long w0 = coherent_load(p), w2 = coherent_load(p + 2);
+    const bool runs = (w0 >> 32) == 0 && w2 == 0 && (step == 1 || round_moved(D, step - 1));
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(R.host_word, runs ? step : kRoundsOver, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (!runs) return;
+    if (threadIdx.x == 0) any_moved = 0;
+    __syncthreads();
+    const int waves = blockDim.x >> 6;
+    const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));
+    const int nwaves = gridDim.x * waves;
+    int *st = status_row(D, step);
+    const DevState V = round_view(M, D, R, step);
+    if (step > 1 && carry_moved(M, D, R, step, wave, nwaves)) atomic_max_i(&D.units[0].infeasible, step - 1);
+    int moved = 0;
+    for (int it = wave; it < R.n_items; it += nwaves) moved |= round_item<false>(M, V, R, it, step, st);
+    if (__any(moved != 0) && (threadIdx.x & 63) == 0) any_moved = 1;
+    __syncthreads();
+    if (threadIdx.x == 0 && any_moved) note_round_moved(D, step);
+}
+
+// The candidates of the split rows whose gate passed in the round.
+__global__ __launch_bounds__(256) void round_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+    const int count = coherent_load(&status_row(D, step)[kStatusApply]);
+    const int waves = blockDim.x >> 6;
+    const DevState V = round_view(M, D, R, step);
+    int moved = 0, u;
+    for (int t = blockIdx.x * waves + (threadIdx.x >> 6); t < count; t += gridDim.x * waves)
+        moved |= apply_split_task<false>(M, V, coherent_load(&D.apply_tasks[t]), u);
+    if (__any(moved != 0) && (threadIdx.x & 63) == 0) note_round_moved(D, step);
+}
+
+// Grid barrier by gathering: every workgroup stores its arrival (sequence
+// number and flags) into a slot of its own, and the first wave of every
+// workgroup polls all slots, so that a barrier is one store and one load
+// deep and hands every workgroup the union of all flags.  Two sets of slots
+// take turns: a set is written again only after everybody has left the
+// barrier between.  Waiting is bounded as in grid_barrier.
+// wg_flags (LDS, zero at first): the workgroup's flags, two words in turn.
+__device__ __forceinline__ bool gather_barrier(const DevState &D, const RoundPlan &R, unsigned seq, unsigned flags,
+                                               unsigned *wg_flags, unsigned &all_flags) {
+    __shared__ unsigned result[2];
+    mem_wait();
+    if (flags) atomicOr(&wg_flags[seq & 1], flags);
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        unsigned long long *slots = R.slots + (seq & 1) * kMaxGatherBlocks;
+        const int nb = gridDim.x;
+        if (threadIdx.x == 0)
+            coherent_store(&slots[blockIdx.x], (static_cast<unsigned long long>(seq) << 32) | wg_flags[seq & 1]);
+        unsigned got = 0u;
+        bool ok = true;
+        const long long t0 = wall_clock64();
+        for (int base = 0; base < nb && ok; base += 64) {
+            const int k = base + static_cast<int>(threadIdx.x);
+            while (true) {
+                const unsigned long long v =
+                    k < nb ? coherent_load(&slots[k]) : (static_cast<unsigned long long>(seq) << 32);
+                if (!__any(static_cast<unsigned>(v >> 32) != seq)) {
+                    got |= static_cast<unsigned>(v);
+                    break;
+                }
+                if (wall_clock64() - t0 > kWaitTimeoutTicks || coherent_load(&D.global[kGlobalError])) {
+                    ok = false;
+                    break;
+                }
+            }
+        }
+#pragma unroll
+        for (int h = 1; h < 64; h <<= 1) got |= static_cast<unsigned>(__shfl_xor(static_cast<int>(got), h, 64));
+        if (threadIdx.x == 0) {
+            if (!ok) atomic_or_i(&D.global[kGlobalError], 1);
+            wg_flags[(seq + 1) & 1] = 0u;
+            result[0] = got;
+            result[1] = ok ? 1u : 0u;
+        }
+    }
+    __syncthreads();
+    all_flags = result[0];
+    return result[1] != 0u;
+}
+
+// Rounds 1 .. max_rounds in one persistent launch.  Bounds are gathered with
+// device-coherent loads (nothing is invalidated between the rounds, so the
+// matrix stays in the caches); one barrier per round, and a second one in
+// rounds in which a split row passed its gate.
+__global__ __launch_bounds__(1024) void rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
+    constexpr unsigned kMoved = 1u, kCrossed = 2u;
+    const long long w2 = coherent_load(reinterpret_cast<const long long *>(&D.units[0]) + 2);
+    if (w2 != 0) return;  // crossed or outside the envelope
+    const int waves = blockDim.x >> 6;
+    const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));
+    const int nwaves = gridDim.x * waves;
+    __shared__ unsigned wg_flags[2];
+    if (threadIdx.x < 2) wg_flags[threadIdx.x] = 0u;
+    __syncthreads();
+    unsigned seq = 0, all = 0;
+    int last = 0, infeasible = 0;
+    bool ok = true;
+    for (int step = 1; ok && step <= R.max_rounds; step++) {
+        int *st = status_row(D, step);
+        const DevState V = round_view(M, D, R, step);
+        unsigned flags = 0u;
+        if (step > 1 && carry_moved(M, D, R, step, wave, nwaves)) flags |= kCrossed;
+        for (int it = wave; it < R.n_items; it += nwaves)
+            if (round_item<true>(M, V, R, it, step, st)) flags |= kMoved;
+        ok = gather_barrier(D, R, ++seq, flags, wg_flags, all);
+        unsigned seen = all;
+        if (ok && M.n_seg_parts > 0) {
+            const int count = coherent_load(&st[kStatusApply]);
+            if (count > 0) {
+                flags = 0u;
+                int u;
+                for (int t = wave; t < count; t += nwaves)
+                    if (apply_split_task<true>(M, V, coherent_load(&D.apply_tasks[t]), u)) flags |= kMoved;
+                ok = gather_barrier(D, R, ++seq, flags, wg_flags, all);
+                seen |= all;
+            }
+        }
+        if (!ok) break;
+        if (seen & kCrossed) {
+            infeasible = step - 1;
+            break;
+        }
+        if (!(seen & kMoved)) break;
+        last = step;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        D.units[0].infeasible = infeasible;
+        D.moved[moved_index(0, last & 1, 0)] = last;
+    }
+}
+
+// Writes the final bounds to the caller's vectors (not when the input was
+// outside the envelope), finds crossed bounds of the last round, and the last
+// workgroup to finish writes the outcome to pinned host memory.
+__global__ __launch_bounds__(256) void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
+    const long long *p = reinterpret_cast<const long long *>(&D.units[0]);
+    const int infeasible = static_cast<int>(coherent_load(p) >> 32);
+    const long long w2 = coherent_load(p + 2);
+    // the last round that moved a bound
+    const int lane = threadIdx.x & 63;
+    int last = lane < 2 * kMoveLanes ? coherent_load(&D.moved[moved_index(0, lane & 1, lane >> 1)]) : 0;
+#pragma unroll
+    for (int h = 1; h < 64; h <<= 1) {
+        const int o = __shfl_xor(last, h, 64);
+        last = o > last ? o : last;
+    }
+    last = uniform(infeasible ? infeasible : last);
+    const DevState V = block_view(M, D, R, last & 1);
+    if ((w2 >> 32) == 0) {
+        const int stride = gridDim.x * blockDim.x;
+        bool crossed = false;
+        for (int id = blockIdx.x * blockDim.x + threadIdx.x; id < M.n; id += stride) {
+            const int j = M.perm[id];
+            double l, u;
+            if (id < M.n_int) {
+                const int2 a = V.AI[id];
+                l = static_cast<double>(a.x);
+                u = static_cast<double>(a.y);
+                if (a.x == kAiHigh || a.y == kAiLow) {
+                    const double2 x = V.AX[id];
+                    l = x.x > l ? x.x : l;
+                    u = x.y < u ? x.y : u;
+                }
+            } else {
+                const double2 a = V.AF[id - M.n_int];
+                l = a.x;
+                u = a.y;
+            }
+            crossed |= eps_gt(l, u);
+            R.lbs[j] = l;
+            R.ubs[j] = u;
+        }
+        if (last > 0 && __any(crossed) && (threadIdx.x & 63) == 0) atomic_max_i(&D.units[0].infeasible, last);
+    }
+    mem_wait();
+    __syncthreads();
+    if (threadIdx.x == 0 &&
+        atomic_add_i(&D.global[kGlobalTicket], 1) == static_cast<int>(gridDim.x) - 1) {
+        UnitState s = D.units[0];
+        s.infeasible = coherent_load(&D.units[0].infeasible);
+        s.changed[last & 1] = last;
+        s.error = coherent_load(&D.global[kGlobalError]);
+        *R.host_state = s;
+    }
+}
 
 // ---------------------------------------------------------------------------
 // loading and reading bound vectors
