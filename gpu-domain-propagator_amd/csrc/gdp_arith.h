@@ -35,8 +35,10 @@ GDP_HD bool eps_le(double x, double y) { return (x - y) <= kEps; }
 GDP_HD bool eps_lt(double x, double y) { return (x - y) < -kEps; }
 GDP_HD bool eps_ge(double x, double y) { return (x - y) >= -kEps; }
 GDP_HD bool eps_gt(double x, double y) { return (x - y) > kEps; }
-GDP_HD bool is_pos_inf(double x) { return eps_ge(x, kInf); }
-GDP_HD bool is_neg_inf(double x) { return eps_le(x, -kInf); }
+// eps_ge(x, kInf) and eps_le(x, -kInf): doubles next to 1e20 lie 16384 apart,
+// so the tolerance never decides and one comparison gives the same answer.
+GDP_HD bool is_pos_inf(double x) { return x >= kInf; }
+GDP_HD bool is_neg_inf(double x) { return x <= -kInf; }
 
 // Integer rounding of a candidate bound (propagation_methods.cuh:40-52).
 GDP_HD double round_upper(bool is_cont, double ub) { return is_cont ? ub : floor(ub + kEps); }
@@ -52,7 +54,7 @@ struct Contribution {
 
 GDP_HD Contribution contribution(double a, double l, double u) {
     Contribution c;
-    const bool pos = eps_gt(a, 0.0);
+    const bool pos = a > kEps;  // eps_gt(a, 0)
     c.min_inf = pos ? is_neg_inf(l) : is_pos_inf(u);
     c.max_inf = pos ? is_pos_inf(u) : is_neg_inf(l);
     c.min_part = c.min_inf ? 0.0 : (a > 0 ? a * l : a * u);
@@ -78,61 +80,62 @@ GDP_HD bool row_gate(double minact, double maxact, int min_inf, int max_inf,
 // (propagation_methods.cuh:198-201).
 GDP_HD double eps_max_step(double running, double d) { return eps_gt(d, running) ? d : running; }
 
-// New upper bound from one row (propagation_methods.cuh:78-106).  `num_inf`
-// is the infinity count of the activity the bound is derived from.
-GDP_HD bool tighten_upper(double a, double slack, double surplus, int num_inf,
-                          double l, double u, bool is_cont, double &nb) {
-    double v;
+// Candidate bound of one variable from one side of a row
+// (propagation_methods.cuh:78-134): an upper bound v + l or a lower bound
+// v + u, v the side's slack or surplus over the coefficient; `num_inf` is the
+// infinity count of the activity it is derived from, and the other bound
+// drops out when it is the one infinite contribution.  Lower bounds are
+// computed mirrored (ceil(v - eps) = -floor(-v + eps), exactly), so that both
+// kinds share their instructions in a wave.  Returns whether it tightens.
+GDP_HD bool candidate(bool upper, double v, int num_inf, double l, double u, bool is_cont, double &nb) {
     if (num_inf == 0) {
-        v = a > 0 ? slack / a : surplus / a;
-        v += l;
-    } else if (num_inf == 1 && is_neg_inf(l)) {
-        v = a > 0 ? slack / a : surplus / a;
-    } else {
+        v += upper ? l : u;
+    } else if (num_inf != 1 || !(upper ? is_neg_inf(l) : is_pos_inf(u))) {
         return false;
     }
-    v = round_upper(is_cont, v);
-    if (eps_lt(v, u)) { nb = v; return true; }
-    return false;
+    const double x = upper ? v : -v;
+    const double w = round_upper(is_cont, x);
+    if (!eps_lt(w, upper ? u : -l)) return false;
+    nb = upper ? w : -w;
+    return true;
 }
 
-// New lower bound from one row (propagation_methods.cuh:108-134).
+// New upper / lower bound from one row, `num_inf` the infinity count of the
+// activity it is derived from.
+GDP_HD bool tighten_upper(double a, double slack, double surplus, int num_inf,
+                          double l, double u, bool is_cont, double &nb) {
+    return candidate(true, (a > 0 ? slack : surplus) / a, num_inf, l, u, is_cont, nb);
+}
 GDP_HD bool tighten_lower(double a, double slack, double surplus, int num_inf,
                           double l, double u, bool is_cont, double &nb) {
-    double v;
-    if (num_inf == 0) {
-        v = a > 0 ? surplus / a : slack / a;
-        v += u;
-    } else if (num_inf == 1 && is_pos_inf(u)) {
-        v = a > 0 ? surplus / a : slack / a;
-    } else {
-        return false;
-    }
-    v = round_lower(is_cont, v);
-    if (eps_gt(v, l)) { nb = v; return true; }
-    return false;
+    return candidate(false, (a > 0 ? surplus : slack) / a, num_inf, l, u, is_cont, nb);
 }
 
 // Both candidate bounds of one variable from one row, with the
 // per-variable gates of propagation_methods.cuh:223-276.  Both candidates
-// are computed from the same (l, u).  Returns bit 0 = lower tightened,
+// are computed from the same (l, u).  The right side bounds a positive
+// coefficient's variable from above and any other's from below, the left
+// side the other way round.  Returns bit 0 = lower tightened,
 // bit 1 = upper tightened.
 GDP_HD int tighten_variable(double a, double lhs, double rhs, double minact, double maxact,
                             int min_inf, int max_inf, bool is_cont, double l, double u,
                             double &nl, double &nu) {
+    const bool pos = a > 0.0;
+    const double width = pos ? a * (u - l) : a * (l - u);
     const double slack = rhs - minact;
-    const double surplus = lhs - maxact;
+    double nb;
     int r = 0;
-    if (a > 0.0) {
-        if (eps_gt(a * (u - l), rhs - minact) && !is_pos_inf(rhs) && !is_neg_inf(minact))
-            r |= tighten_upper(a, slack, surplus, min_inf, l, u, is_cont, nu) ? 2 : 0;
-        if (eps_gt(a * (u - l), maxact - lhs) && !is_neg_inf(lhs) && !is_pos_inf(maxact))
-            r |= tighten_lower(a, slack, surplus, max_inf, l, u, is_cont, nl) ? 1 : 0;
-    } else {
-        if (eps_gt(a * (l - u), rhs - minact) && !is_pos_inf(rhs) && !is_neg_inf(minact))
-            r |= tighten_lower(a, slack, surplus, min_inf, l, u, is_cont, nl) ? 1 : 0;
-        if (eps_gt(a * (l - u), maxact - lhs) && !is_neg_inf(lhs) && !is_pos_inf(maxact))
-            r |= tighten_upper(a, slack, surplus, max_inf, l, u, is_cont, nu) ? 2 : 0;
+    if (eps_gt(width, slack) && !is_pos_inf(rhs) && !is_neg_inf(minact) &&
+        candidate(pos, slack / a, min_inf, l, u, is_cont, nb)) {
+        if (pos) nu = nb;
+        else nl = nb;
+        r = pos ? 2 : 1;
+    }
+    if (eps_gt(width, maxact - lhs) && !is_neg_inf(lhs) && !is_pos_inf(maxact) &&
+        candidate(!pos, (lhs - maxact) / a, max_inf, l, u, is_cont, nb)) {
+        if (pos) nl = nb;
+        else nu = nb;
+        r |= pos ? 1 : 2;
     }
     return r;
 }

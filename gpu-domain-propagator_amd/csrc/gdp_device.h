@@ -82,8 +82,11 @@ constexpr int kFilterLdsBytes = (kMaxFilterUnits / 32) * 4 * 2 + kMaxFilterUnits
 // their records.  At most kMaxLdsBinBytes of LDS per workgroup.
 constexpr int kMaxLdsBinBytes = 64 * 1024;
 
-// Rows start at multiples of kRowAlign entries (padding entries hold column
-// 0 and coefficient 0 and are never used); the low bits of row_ptr[r] hold
+// Rows start at multiples of kRowAlign entries (padding entries hold the
+// column id n, whose record at the end of a snapshot block has bounds (0, 0),
+// and coefficient 0: they add nothing to an activity and are never
+// tightened; four of them follow the last row, for the lanes past a row's
+// end); the low bits of row_ptr[r] hold
 // the number of padding entries after row r.  Aligned starts let a lane load
 // its 4 consecutive entries with one 16-byte column load and two 16-byte
 // coefficient loads.
@@ -187,6 +190,7 @@ struct DevMatrix {
     long long snap_stride; // bytes between the snapshot blocks of two units
     int n_bin;             // binary columns: internal ids [0, n_bin) (replicas mode; blocks: 0)
     int sb_words;          // words of a unit's binary codes: ceil(n_bin / 64) * 4
+    int n_padded;          // entries of the padded rows (four padding entries follow)
 };
 
 struct DevState {
@@ -231,14 +235,18 @@ struct DevState {
 constexpr int kPlanBins = 9;          // tree widths 2^8 .. 2^0
 constexpr int kMaxGatherBlocks = 512; // workgroups of the persistent launch
 constexpr int kRoundsOver = 0x40000000;  // host word: no further round runs
-struct RoundPlan {
-    int n_items;                      // segments of split rows, then group items
+// Where each tree-width bin's rows and items start (building the item list).
+struct RoundBins {
     int n_segs;
     int item0[kPlanBins + 1];         // first item of the bin of width 2^(8 - q)
     int row0[kPlanBins + 1];          // first layout row of the bin
     int rows_per_item[kPlanBins];
     int logg[kPlanBins];              // lanes per row (log2)
     int logk[kPlanBins];              // entries per lane (log2)
+};
+struct RoundPlan {
+    int n_items;
+    const int4 *items;                // as DevMatrix's: one segment of a split row, or one pass of rows
     char *block[2];
     double2 *AX[2];                   // exact integer values beyond int32, per block
     unsigned *bm[2];                  // columns moved in a round, by parity

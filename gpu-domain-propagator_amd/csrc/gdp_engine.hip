@@ -45,6 +45,7 @@ __global__ void apply_split_kernel(DevMatrix M, DevState D, int step, int guard,
 __global__ void publish_kernel(DevMatrix M, DevState D, int step, int guard, int first_step, int n_units);
 template <int kThreads, bool kLds>
 __global__ void mega_kernel(DevMatrix M, DevState D, int first_step, int max_steps, int n_units);
+__global__ void plan_rounds_kernel(DevMatrix M, RoundBins B, int4 *items);
 __global__ void reset_rounds_kernel(DevState D, RoundPlan R);
 __global__ void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin);
 __global__ void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
@@ -684,8 +685,9 @@ void device_layout_build(CsrUpload &csr, const std::vector<int> &col_off, int mp
         int *t_coff = dev_alloc<int>(NI + 1, tmp);
         int *t_cnt = dev_alloc<int>(n_ids + 2, tmp);  // counts (n_ids + 1: the scan's total), the out-of-range flag
         upload(t_coff, col_off.data(), NI + 1, s);
-        check(hipMemsetAsync(d_col, 0, sizeof(int) * n_padded, s), "memset layout");
-        check(hipMemsetAsync(d_val, 0, sizeof(double) * n_padded, s), "memset layout");
+        check(hipMemsetD32Async(d_col, n_ids, static_cast<size_t>(n_padded) + kRowAlign, s), "memset layout");
+        check(hipMemsetAsync(d_val, 0, sizeof(double) * (static_cast<size_t>(n_padded) + kRowAlign), s),
+              "memset layout");
         check(hipMemsetAsync(t_cnt, 0, sizeof(int) * (n_ids + 2), s), "memset counts");
         csr.finish();
         trace.mark("wait_csr");
@@ -835,32 +837,38 @@ void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
         T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
         !std::equal(T.group_log, T.group_log + 10, def.group_log))
         return;
-    RoundPlan &R = P->R;
-    R.n_segs = P->M.n_seg_parts;
+    RoundBins B;
+    B.n_segs = P->M.n_seg_parts;
     // Entries per lane: few while the passes (256 lane entries of K each) still
     // find a free SIMD, because a pass is a chain of dependent loads, a butterfly
     // and divisions that grows with K.  Per persistent round with 1 / 2 / 4:
     // 33K entry slots 7.3 / 7.5 / 8.8 us, 115K 8.5 / 8.1 / 8.9 us, 330K 12.5 /
     // 10.3 / 10.4 us.
     const int logk_want = n_padded <= (64 << 10) ? 0 : (n_padded <= (512 << 10) ? 1 : 2);
-    int at = R.n_segs;
+    int at = B.n_segs;
     for (int q = 0; q < kPlanBins; q++) {
         const int b = kPlanBins - 1 - q, key = 10 - b;
         const int logk = std::max(std::min(logk_want, b), b - 6);
         const int logg = b - logk;
-        R.logk[q] = logk;
-        R.logg[q] = logg;
-        R.rows_per_item[q] = 64 >> logg;
-        R.item0[q] = at;
-        R.row0[q] = start[key];
-        at += (count[key] + R.rows_per_item[q] - 1) / R.rows_per_item[q];
+        B.logk[q] = logk;
+        B.logg[q] = logg;
+        B.rows_per_item[q] = 64 >> logg;
+        B.item0[q] = at;
+        B.row0[q] = start[key];
+        at += (count[key] + B.rows_per_item[q] - 1) / B.rows_per_item[q];
     }
-    R.item0[kPlanBins] = at;
-    R.row0[kPlanBins] = P->M.m;
+    B.item0[kPlanBins] = at;
+    B.row0[kPlanBins] = P->M.m;
     // bins without rows have no start of their own
     for (int q = kPlanBins - 1; q >= 0; q--)
-        if (count[2 + q] == 0) R.row0[q] = R.row0[q + 1];
+        if (count[2 + q] == 0) B.row0[q] = B.row0[q + 1];
+    RoundPlan &R = P->R;
     R.n_items = at;
+    int4 *items = dev_alloc<int4>(at, P->owned);
+    R.items = items;
+    hipLaunchKernelGGL(plan_rounds_kernel, dim3(std::max(1, std::min(256, (at + 255) / 256))), dim3(256), 0, P->stream,
+                       P->M, B, items);
+    check(hipGetLastError(), "plan launch");
     DevMatrix &M = P->Mr;
     M = P->M;
     M.n16 = 0;
@@ -1110,8 +1118,8 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         M.mark_rows = T.row_marking ? 1 : 0;
         M.n_seg_rows = static_cast<int>(h_seg_rows.size());
         M.n_seg_parts = n_parts;
-        int *d_col = dev_alloc<int>(n_padded, o);
-        double *d_val = dev_alloc<double>(n_padded, o);
+        int *d_col = dev_alloc<int>(static_cast<size_t>(n_padded) + kRowAlign, o);
+        double *d_val = dev_alloc<double>(static_cast<size_t>(n_padded) + kRowAlign, o);
         int4 *d_items = dev_alloc<int4>(h_items.size(), o);
         int4 *d_seg_rows = dev_alloc<int4>(h_seg_rows.size(), o);
         int *d_part_row = dev_alloc<int>(h_part_row.size(), o);
@@ -1144,6 +1152,7 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
                             P->d_inv_perm, d_col, d_val, d_cptr, d_crows, d_cseg, d_citem, s, trace);
         M.row_ptr = d_rp;
         M.sides = d_sides;
+        M.n_padded = n_padded;
         M.col = d_col;
         M.val = d_val;
         M.items = d_items;

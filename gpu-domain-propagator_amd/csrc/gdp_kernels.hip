@@ -108,17 +108,27 @@ __device__ __forceinline__ void mem_wait() { __builtin_amdgcn_s_waitcnt(0); }
 // bounds snapshot and accumulator
 // ---------------------------------------------------------------------------
 
-// Snapshot records are read with one aligned 16-byte load of the chunk that
-// holds them, decoded without branches, so that the gathers of a lane issue
-// back to back whatever the storage classes of their columns.
+// How a kernel reads the snapshot.
+//   kRecords        int16, int32 and FP64 records (DevMatrix's three classes)
+//   kWide           int32 and FP64 records only (the double-buffered rounds)
+//   kWideCoherent   the same with device-coherent loads (sc1: past the L1,
+//                   coherent across the XCDs' L2s), for a launch in which other
+//                   workgroups wrote the records and nothing is invalidated
+constexpr int kRecords = 0, kWide = 1, kWideCoherent = 2;
+
 // Byte offset of the record of internal column `id` in the unit's block.
+template <int kMode>
 __device__ __forceinline__ unsigned record_offset(const DevMatrix &M, int id) {
     const unsigned uid = static_cast<unsigned>(id);
-    const unsigned a16 = uid * 4u;
-    const unsigned a32 = static_cast<unsigned>(M.snap_off32) + (uid - static_cast<unsigned>(M.n16)) * 8u;
-    const unsigned af = static_cast<unsigned>(M.snap_offF) + (uid - static_cast<unsigned>(M.n_int)) * 16u;
-    const unsigned a = id < M.n16 ? a16 : a32;
-    return id < M.n_int ? a : af;
+    if constexpr (kMode == kRecords) {
+        const unsigned a16 = uid * 4u;
+        const unsigned a32 = uid * 8u + (static_cast<unsigned>(M.snap_off32) - static_cast<unsigned>(M.n16) * 8u);
+        const unsigned af = uid * 16u + (static_cast<unsigned>(M.snap_offF) - static_cast<unsigned>(M.n_int) * 16u);
+        return id < M.n16 ? a16 : (id < M.n_int ? a32 : af);
+    } else {
+        const unsigned af = uid * 16u + (static_cast<unsigned>(M.snap_offF) - static_cast<unsigned>(M.n_int) * 16u);
+        return id < M.n_int ? uid * 8u : af;
+    }
 }
 
 // Dynamic LDS of the persistent kernel: the unit filter's arrays in a launch
@@ -126,59 +136,49 @@ __device__ __forceinline__ unsigned record_offset(const DevMatrix &M, int id) {
 // (other kernels run with D.n_lds = 0 and never touch it).
 extern __shared__ __align__(16) unsigned dyn_lds[];
 
-// Bounds of binary column `id` < D.n_lds from its 2-bit code in LDS.
-__device__ __forceinline__ void lds_binary_bounds(int id, double &l, double &u) {
-    const unsigned code = dyn_lds[id >> 4] >> ((id & 15) * 2);
-    l = (code & 1u) ? 1.0 : 0.0;
-    u = (code & 2u) ? 0.0 : 1.0;
+// The 16 bytes from byte `off` of the unit's snapshot block (a multiple of 4),
+// zeros from kNoRecord.  One buffer load whatever the record's class: the
+// record's own bytes come first, so nothing has to be picked out of an
+// aligned chunk, the address takes no 64-bit arithmetic, and the lanes
+// without an entry are cut off by the bounds check instead of by masks.
+constexpr unsigned kNoRecord = 0xfffffff0u;
+template <int kMode>
+__device__ __forceinline__ uint4 load_record(const DevMatrix &M, const DevState &D, unsigned off) {
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(D.S16, 0, static_cast<int>(M.snap_stride), 0x00020000);
+    constexpr int kSc1 = 16;
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(off), 0,
+                                                         kMode == kWideCoherent ? kSc1 : 0);
+    return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
-// kCoherent: a device-coherent load (sc1: past the L1, coherent across the
-// XCDs' L2s) for a launch in which other workgroups wrote the snapshot, with
-// no cache invalidation between the rounds.  A buffer load, since atomic
-// loads end at 8 bytes; its offset is checked against the block's size.
-template <bool kCoherent>
-__device__ __forceinline__ uint4 load_chunk(const DevMatrix &M, const DevState &D, unsigned off) {
-    if constexpr (kCoherent) {
-        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(D.S16, 0, static_cast<int>(M.snap_stride), 0x00020000);
-        constexpr int kSc1 = 16;
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(off & ~15u), 0, kSc1);
-        return make_uint4(v[0], v[1], v[2], v[3]);
-    } else {
-        return *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(D.S16) + (off & ~15u));
-    }
-}
-
-// Bounds of `id` from the chunk at its record offset `off`.
-__device__ __forceinline__ void decode_bounds(const DevMatrix &M, int id, unsigned off, const uint4 c, double &l,
+// Bounds of `id` from its record; of a binary column id < D.n_lds from its
+// 2-bit code in LDS instead.
+template <int kMode>
+__device__ __forceinline__ void decode_bounds(const DevMatrix &M, const DevState &D, int id, const uint4 c, double &l,
                                               double &u) {
-    const unsigned odd = (off >> 2) & 1u, upper = (off >> 3) & 1u;
-    // 4-byte record: dword (off >> 2) & 3; 8-byte record: that dword and the next
-    const unsigned x01 = odd ? c.y : c.x;
-    const unsigned x23 = odd ? c.w : c.z;
-    const unsigned lo = upper ? x23 : x01;
-    const unsigned hi = upper ? c.w : c.y;
-    const double l16 = static_cast<double>(static_cast<short>(lo & 0xffffu));
-    const double u16 = static_cast<double>(static_cast<short>(lo >> 16));
-    const double l32 = static_cast<double>(static_cast<int>(lo));
-    const double u32 = static_cast<double>(static_cast<int>(hi));
+    int il = static_cast<int>(c.x), iu = static_cast<int>(c.y);
+    if constexpr (kMode == kRecords) {
+        const bool c16 = id < M.n16;
+        il = c16 ? static_cast<short>(c.x & 0xffffu) : il;
+        iu = c16 ? static_cast<int>(c.x) >> 16 : iu;
+        if (id < D.n_lds) {
+            const unsigned code = dyn_lds[id >> 4] >> ((id & 15) * 2);
+            il = static_cast<int>(code & 1u);
+            iu = static_cast<int>(((code >> 1) & 1u) ^ 1u);
+        }
+    }
     const double lf = __hiloint2double(static_cast<int>(c.y), static_cast<int>(c.x));
     const double uf = __hiloint2double(static_cast<int>(c.w), static_cast<int>(c.z));
-    const bool c16 = id < M.n16, c32 = id < M.n_int;
-    const double li = c16 ? l16 : l32, ui = c16 ? u16 : u32;
-    l = c32 ? li : lf;
-    u = c32 ? ui : uf;
+    const bool whole = id < M.n_int;
+    l = whole ? static_cast<double>(il) : lf;
+    u = whole ? static_cast<double>(iu) : uf;
 }
 
 // Bounds of internal column `id` at the start of the round.
-template <bool kCoherent>
+template <int kMode>
 __device__ __forceinline__ void load_bounds(const DevMatrix &M, const DevState &D, int id, double &l, double &u) {
-    if (id < D.n_lds) {
-        lds_binary_bounds(id, l, u);
-    } else {
-        const unsigned off = record_offset(M, id);
-        decode_bounds(M, id, off, load_chunk<kCoherent>(M, D, off), l, u);
-    }
+    const unsigned off = id < D.n_lds ? kNoRecord : record_offset<kMode>(M, id);
+    decode_bounds<kMode>(M, D, id, load_record<kMode>(M, D, off), l, u);
 }
 
 __device__ __forceinline__ bool fits_int32(double v) { return v >= -2147483647.0 && v <= 2147483647.0; }
@@ -347,7 +347,7 @@ __device__ __forceinline__ double seq_eps_max(const DevMatrix &M, const DevState
     double run = 0.0;
     for (int e = 0; e < len; e++) {
         double l, u;
-        load_bounds<false>(M, D, M.col[start + e] & kIdMask, l, u);
+        load_bounds<kRecords>(M, D, M.col[start + e] & kIdMask, l, u);
         run = eps_max_step(run, fabs(M.val[start + e]) * (u - l));
     }
     return run;
@@ -386,84 +386,128 @@ __device__ __forceinline__ void row_extent(const DevMatrix &M, int r, int &start
     len = (b & ~(kRowAlign - 1)) - start - (a & (kRowAlign - 1));
 }
 
+// The values of a lane and of its partner in step h = 2^k of a butterfly whose
+// earlier steps ran (lanes of a group of h hold the same value): lane i ^ h,
+// or, where that is cheaper, another lane of the same partner group.  In
+// registers: DPP within 16 lanes, the row swaps of this target beyond.
+template <int h>
+__device__ __forceinline__ void partner(int v, int &a, int &b) {
+    if constexpr (h <= 8) {
+        constexpr int kCtrl = h == 1 ? 0xB1 : (h == 2 ? 0x4E : (h == 4 ? 0x141 : 0x140));
+        a = v;
+        b = __builtin_amdgcn_update_dpp(v, v, kCtrl, 0xf, 0xf, false);
+    } else if constexpr (h == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(v), static_cast<unsigned>(v), false, false);
+        a = static_cast<int>(r[0]);
+        b = static_cast<int>(r[1]);
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(v), static_cast<unsigned>(v), false, false);
+        a = static_cast<int>(r[0]);
+        b = static_cast<int>(r[1]);
+    }
+}
+template <int h>
+__device__ __forceinline__ void partner_d(double v, double &a, double &b) {
+    int al, ah, bl, bh;
+    partner<h>(__double2loint(v), al, bl);
+    partner<h>(__double2hiint(v), ah, bh);
+    a = __hiloint2double(ah, al);
+    b = __hiloint2double(bh, bl);
+}
+template <int h>
+__device__ __forceinline__ double step_add(double v) {
+    double a, b;
+    partner_d<h>(v, a, b);
+    return a + b;
+}
+template <int h>
+__device__ __forceinline__ double step_max(double v) {
+    double a, b;
+    partner_d<h>(v, a, b);
+    return fmax(a, b);
+}
+template <int h>
+__device__ __forceinline__ int step_add(int v) {
+    int a, b;
+    partner<h>(v, a, b);
+    return a + b;
+}
+
 // K consecutive entries of one lane: loads, contributions, pairwise tree of
 // the K contributions in natural order, and the cross-lane reduction.
-template <int K, bool kCoherent = false>
+// A sweep is bound by its instructions as much as by its gathers (200,000
+// rows, 2.2M nonzeros, nothing moving: 500 vector instructions per pass, 45%
+// of the 19 us), so the entries past the row's end are ordinary entries of a
+// zero column with a zero coefficient, infinite contributions are looked at
+// only where a lane of the wave has one, and their two counts share a word
+// (at most kSegLen each).
+template <int K, int kMode>
 struct LaneEntries {
     int jp[K];
     double a[K], l[K], u[K];
     double tmin, tmax, dmax;
-    int mininf, maxinf;
+    int infs;     // infinite contributions: minimum side in the low 16 bits, maximum side in the high
+    bool some;    // some lane of the wave has one
+
+    __device__ __forceinline__ int min_inf() const { return infs & 0xffff; }
+    __device__ __forceinline__ int max_inf() const { return infs >> 16; }
 
     __device__ __forceinline__ void load(const DevMatrix &M, const DevState &D, int base, int first, int len) {
-        double smin[K], smax[K];
-        mininf = 0;
-        maxinf = 0;
-        dmax = 0.0;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            jp[k] = 0;
-            a[k] = 0.0;
+        // the lane's K entries in one go (base + first is a multiple of K and
+        // the row is padded to a multiple of kRowAlign, a multiple of K), a
+        // lane past the end the padding entries behind the last row
+        const size_t e = static_cast<size_t>(first < len ? base + first : M.n_padded);
+        const int *cp = M.col + e;
+        const double *vp = M.val + e;
+        if constexpr (K == 4) {
+            const int4 c = *reinterpret_cast<const int4 *>(cp);
+            const double2 v0 = *reinterpret_cast<const double2 *>(vp);
+            const double2 v1 = *reinterpret_cast<const double2 *>(vp + 2);
+            jp[0] = c.x; jp[1] = c.y; jp[2] = c.z; jp[3] = c.w;
+            a[0] = v0.x; a[1] = v0.y; a[2] = v1.x; a[3] = v1.y;
+        } else if constexpr (K == 2) {
+            const int2 c = *reinterpret_cast<const int2 *>(cp);
+            const double2 v0 = *reinterpret_cast<const double2 *>(vp);
+            jp[0] = c.x; jp[1] = c.y;
+            a[0] = v0.x; a[1] = v0.y;
+        } else {
+            jp[0] = *cp;
+            a[0] = *vp;
         }
-        // the lane's K entries in one go: base + first is a multiple of K and
-        // the row is padded to a multiple of kRowAlign (a multiple of K)
-        if (first < len) {
-            const int *cp = M.col + base + first;
-            const double *vp = M.val + base + first;
-            if constexpr (K == 4) {
-                const int4 c = *reinterpret_cast<const int4 *>(cp);
-                const double2 v0 = *reinterpret_cast<const double2 *>(vp);
-                const double2 v1 = *reinterpret_cast<const double2 *>(vp + 2);
-                jp[0] = c.x; jp[1] = c.y; jp[2] = c.z; jp[3] = c.w;
-                a[0] = v0.x; a[1] = v0.y; a[2] = v1.x; a[3] = v1.y;
-            } else if constexpr (K == 2) {
-                const int2 c = *reinterpret_cast<const int2 *>(cp);
-                const double2 v0 = *reinterpret_cast<const double2 *>(vp);
-                jp[0] = c.x; jp[1] = c.y;
-                a[0] = v0.x; a[1] = v0.y;
-            } else {
-#pragma unroll
-                for (int k = 0; k < K; k++) {
-                    jp[k] = cp[k];
-                    a[k] = vp[k];
-                }
-            }
-        }
-        // every gather first (entries past the end read column 0's bounds and
-        // are discarded), then the decoding and the contributions; binary
+        // every gather first, then the decoding and the contributions; binary
         // columns held in LDS are read there instead
-        unsigned off[K];
-        uint4 chunk[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            if (first + k >= len) {
-                jp[k] = 0;
-                a[k] = 0.0;
-            }
-            off[k] = record_offset(M, jp[k] & kIdMask);
-            chunk[k] = make_uint4(0u, 0u, 0u, 0u);
-            if ((jp[k] & kIdMask) >= D.n_lds) chunk[k] = load_chunk<kCoherent>(M, D, off[k]);
-        }
+        uint4 rec[K];
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int id = jp[k] & kIdMask;
-            if (id < D.n_lds) lds_binary_bounds(id, l[k], u[k]);
-            else decode_bounds(M, id, off[k], chunk[k], l[k], u[k]);
+            rec[k] = load_record<kMode>(M, D, id < D.n_lds ? kNoRecord : record_offset<kMode>(M, id));
         }
+        dmax = 0.0;
+        bool any = false;
 #pragma unroll
         for (int k = 0; k < K; k++) {
-            smin[k] = 0.0;
-            smax[k] = 0.0;
-            if (first + k >= len) {
-                l[k] = 0.0;
-                u[k] = 0.0;
-            } else {
-                const Contribution q = contribution(a[k], l[k], u[k]);
-                smin[k] = q.min_part;
-                smax[k] = q.max_part;
-                mininf += q.min_inf;
-                maxinf += q.max_inf;
-                dmax = fmax(dmax, q.delta);
+            decode_bounds<kMode>(M, D, jp[k] & kIdMask, rec[k], l[k], u[k]);
+            dmax = fmax(dmax, fabs(a[k]) * (u[k] - l[k]));
+            any |= is_neg_inf(l[k]) | is_pos_inf(u[k]);
+        }
+        infs = 0;
+        some = __any(any);
+        double smin[K], smax[K];
+        if (some) {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const bool lo = is_neg_inf(l[k]), up = is_pos_inf(u[k]);
+                const bool pos = a[k] > kEps;
+                const bool mi = pos ? lo : up, xi = pos ? up : lo;
+                smin[k] = mi ? 0.0 : a[k] * (a[k] > 0.0 ? l[k] : u[k]);
+                smax[k] = xi ? 0.0 : a[k] * (a[k] > 0.0 ? u[k] : l[k]);
+                infs += (mi ? 1 : 0) + (xi ? 0x10000 : 0);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                smin[k] = a[k] * (a[k] > 0.0 ? l[k] : u[k]);
+                smax[k] = a[k] * (a[k] > 0.0 ? u[k] : l[k]);
             }
         }
 #pragma unroll
@@ -478,15 +522,23 @@ struct LaneEntries {
         tmax = smax[0];
     }
 
+    // One step of the butterfly; kMax: the largest width too.
+    template <int h, bool kMax>
+    __device__ __forceinline__ void step() {
+        tmin = step_add<h>(tmin);
+        tmax = step_add<h>(tmax);
+        if (some) infs = step_add<h>(infs);
+        if constexpr (kMax) dmax = step_max<h>(dmax);
+    }
     // xor butterfly over groups of g lanes (natural pairwise order)
+    template <bool kMax>
     __device__ __forceinline__ void reduce(int g) {
-        for (int h = 1; h < g; h <<= 1) {
-            tmin = tmin + shfl_xor_d(tmin, h);
-            tmax = tmax + shfl_xor_d(tmax, h);
-            mininf += __shfl_xor(mininf, h, 64);
-            maxinf += __shfl_xor(maxinf, h, 64);
-            dmax = fmax(dmax, shfl_xor_d(dmax, h));
-        }
+        if (g > 1) step<1, kMax>();
+        if (g > 2) step<2, kMax>();
+        if (g > 4) step<4, kMax>();
+        if (g > 8) step<8, kMax>();
+        if (g > 16) step<16, kMax>();
+        if (g > 32) step<32, kMax>();
     }
 
     // Sequential epsilon-maximum over the entries of each group of g lanes in
@@ -495,12 +547,9 @@ struct LaneEntries {
     // the row hold zeros, which never replace the running value.
     __device__ __forceinline__ double eps_scan(int g, double run) const {
         const int gbase = (threadIdx.x & 63) & ~(g - 1);
-        double d[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) d[k] = fabs(a[k]) * (u[k] - l[k]);
         for (int j = 0; j < g; j++) {
 #pragma unroll
-            for (int k = 0; k < K; k++) run = eps_max_step(run, __shfl(d[k], gbase + j, 64));
+            for (int k = 0; k < K; k++) run = eps_max_step(run, __shfl(fabs(a[k]) * (u[k] - l[k]), gbase + j, 64));
         }
         return run;
     }
@@ -511,7 +560,10 @@ struct LaneEntries {
         int moved = 0;
 #pragma unroll
         for (int k = 0; k < K; k++)
+        {
             if (first + k < len) moved += apply_entry(M, S, jp[k], a[k], l[k], u[k], lhs, rhs, minact, maxact, ni, xi);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         return moved;
     }
 };
@@ -611,7 +663,7 @@ __device__ __forceinline__ Sink make_sink(const DevState &V) {
 // Rows [first, first + nrows) of one tree-width bin: groups of 2^logg lanes,
 // K consecutive entries per lane.  Rows not marked for this step are
 // skipped (a pass with no marked row loads nothing).
-template <int K, bool kCoherent>
+template <int K, int kMode>
 __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int first, int nrows, int logg,
                                           int step, bool all_rows) {
     const DevState &V = S.V;
@@ -619,6 +671,7 @@ __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int
     const int g = 1 << logg;
     const int gl = lane & (g - 1);
     const int per_pass = 64 >> logg;
+    const unsigned long long gmask = (g == 64 ? ~0ull : (1ull << g) - 1ull) << (lane & ~(g - 1) & 63);
     const int end = first + nrows;
     int moved = 0;
     for (int base = first; base < end; base += per_pass) {
@@ -633,20 +686,26 @@ __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int
             lhs = sd.x;
             rhs = sd.y;
         }
-        LaneEntries<K, kCoherent> E;
+        LaneEntries<K, kMode> E;
         E.load(M, V, start, gl * K, len);
-        E.reduce(g);
+        E.template reduce<false>(g);
         const double minact = 0.0 + E.tmin;
         const double maxact = 0.0 + E.tmax;
-        const bool active = take && len > 0;
-        const GateBounds gb = gate_bounds(minact, maxact, E.mininf, E.maxinf, lhs, rhs, E.dmax);
-        bool gate = gb.hi;
-        const bool undecided = active && !gb.decided();
+        const int ni = E.min_inf(), xi = E.max_inf();
+        // The gate is monotone in the largest width, so a row passes it when
+        // one of its lanes does with its own largest: one ballot in place of
+        // a maximum over the lanes.
+        const GateBounds gb = gate_bounds(minact, maxact, ni, xi, lhs, rhs, E.dmax);
+        const unsigned long long hi = __ballot(gb.hi && len > 0);
+        if (hi == 0ull) continue;
+        const unsigned long long lo = __ballot(gb.lo && len > 0);
+        bool gate = (hi & gmask) != 0ull;
+        const bool undecided = gate && (lo & gmask) == 0ull;
         if (__any(undecided)) {
             const double dm = E.eps_scan(g, 0.0);
-            if (undecided) gate = row_gate(minact, maxact, E.mininf, E.maxinf, lhs, rhs, dm);
+            if (undecided) gate = row_gate(minact, maxact, ni, xi, lhs, rhs, dm);
         }
-        if (active && gate) moved += E.apply(M, S, gl * K, len, lhs, rhs, minact, maxact, E.mininf, E.maxinf);
+        if (gate) moved += E.apply(M, S, gl * K, len, lhs, rhs, minact, maxact, ni, xi);
     }
     return moved;
 }
@@ -663,13 +722,13 @@ __device__ __forceinline__ int long_item(const DevMatrix &M, const Sink &S, int 
     double acc_min = 0.0, acc_max = 0.0, dmax = 0.0;
     int mininf = 0, maxinf = 0;
     for (int s0 = 0; s0 < len; s0 += kSegLen) {
-        LaneEntries<K> E;
+        LaneEntries<K, kRecords> E;
         E.load(M, V, start + s0, lane * K, len - s0);
-        E.reduce(64);
+        E.template reduce<true>(64);
         acc_min = acc_min + E.tmin;
         acc_max = acc_max + E.tmax;
-        mininf += E.mininf;
-        maxinf += E.maxinf;
+        mininf += E.min_inf();
+        maxinf += E.max_inf();
         dmax = fmax(dmax, E.dmax);
     }
     int moved = 0;
@@ -677,7 +736,7 @@ __device__ __forceinline__ int long_item(const DevMatrix &M, const Sink &S, int 
         for (int e = lane; e < len; e += 64) {
             const int jp = M.col[start + e];
             double l, u;
-            load_bounds<false>(M, V, jp & kIdMask, l, u);
+            load_bounds<kRecords>(M, V, jp & kIdMask, l, u);
             moved += apply_entry(M, S, jp, M.val[start + e], l, u, sd.x, sd.y, acc_min, acc_max, mininf, maxinf);
         }
     }
@@ -688,7 +747,7 @@ __device__ __forceinline__ int long_item(const DevMatrix &M, const Sink &S, int 
 // wave.  A segment whose exact maximum Ms satisfies !(Ms - run > eps) cannot
 // replace the running value (floating-point subtraction is monotone), so it
 // is skipped; the others are scanned entry by entry in order.
-template <bool kCoherent>
+template <int kMode>
 __device__ __forceinline__ double split_eps_scan(const DevMatrix &M, const DevState &V, const int4 info, int start, int len) {
     constexpr int K = kSegLen / 64;
     const int lane = threadIdx.x & 63;
@@ -701,7 +760,7 @@ __device__ __forceinline__ double split_eps_scan(const DevMatrix &M, const DevSt
             const double mt = __shfl(ms, t, 64);
             if (!eps_gt(mt, run)) continue;
             const int s0 = (b + t) * kSegLen;
-            LaneEntries<K, kCoherent> E;
+            LaneEntries<K, kMode> E;
             E.load(M, V, start + s0, lane * K, len - s0);
             run = E.eps_scan(64, run);
         }
@@ -711,14 +770,14 @@ __device__ __forceinline__ double split_eps_scan(const DevMatrix &M, const DevSt
 
 // Stores the activity partial of segment `part` and the step that computed
 // it (lane 0 of the wave).
-template <bool kCoherent>
-__device__ __forceinline__ void store_part(const DevState &V, int part, const LaneEntries<kSegLen / 64, kCoherent> &E,
+template <int kMode>
+__device__ __forceinline__ void store_part(const DevState &V, int part, const LaneEntries<kSegLen / 64, kMode> &E,
                                            int step) {
     SegPart *p = &V.seg_parts[part];
     coherent_store_d(&p->smin, E.tmin);
     coherent_store_d(&p->smax, E.tmax);
     coherent_store_d(&p->dmax, E.dmax);
-    coherent_store_2i(&p->infs, E.mininf | (E.maxinf << 16), step);
+    coherent_store_2i(&p->infs, E.infs, step);
 }
 
 // Segments [s, s + cnt) of split row lr (cnt <= kSegsPerItem) for unit u.
@@ -727,7 +786,7 @@ __device__ __forceinline__ void store_part(const DevState &V, int part, const La
 // completes the row's count adds the partials in segment order and decides
 // the row gate; when it passes, the row's activity is stored and its
 // segments are queued for the apply phase that follows the sweep.
-template <bool kCoherent>
+template <int kMode>
 __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, const DevState &V, int u, int lr, int s, int cnt,
                          int *st, int step, bool all_rows, int unit_start) {
     constexpr int K = kSegLen / 64;
@@ -755,9 +814,9 @@ __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, 
         const int part = info.y + s + q;
         if (!all_rows && ((keep >> q) & 1ull)) continue;
         const int s0 = (s + q) * kSegLen;
-        LaneEntries<K, kCoherent> E;
+        LaneEntries<K, kMode> E;
         E.load(M, V, start + s0, lane * K, len - s0);
-        E.reduce(64);
+        E.template reduce<true>(64);
         if (lane == 0) store_part(V, part, E, step);
     }
     unsigned old = 0;
@@ -802,7 +861,7 @@ __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, 
     const double2 sd = M.sides[r];
     const GateBounds gb = gate_bounds(am, ax, ni, xi, sd.x, sd.y, dm);
     bool gate = gb.hi;
-    if (!gb.decided()) gate = row_gate(am, ax, ni, xi, sd.x, sd.y, split_eps_scan<kCoherent>(M, V, info, start, len));
+    if (!gb.decided()) gate = row_gate(am, ax, ni, xi, sd.x, sd.y, split_eps_scan<kMode>(M, V, info, start, len));
     int pos = 0;
     if (lane == 0) {
         coherent_store(&V.seg_count[lr], 0u);
@@ -852,7 +911,7 @@ __device__ __forceinline__ void sweep_item(const DevMatrix &M, const DevState &D
     int moved = 0;
     if (kind == kItemSeg) {
         const int r = M.seg_rows[d.y].x;
-        if (us.all_rows || V.marks[r] == step) seg_item<false>(M, D, V, u, d.y, d.z, d.w, st, step, us.all_rows, us.start);
+        if (us.all_rows || V.marks[r] == step) seg_item<kRecords>(M, D, V, u, d.y, d.z, d.w, st, step, us.all_rows, us.start);
         return;
     }
     if (kind == kItemLong) {
@@ -861,9 +920,9 @@ __device__ __forceinline__ void sweep_item(const DevMatrix &M, const DevState &D
         const int logg = (d.x >> 4) & 15;
         const int logk = (d.x >> 8) & 15;
         switch (logk) {
-            case 0: moved = group_item<1, false>(M, S, d.y, d.z, logg, step, us.all_rows); break;
-            case 1: moved = group_item<2, false>(M, S, d.y, d.z, logg, step, us.all_rows); break;
-            default: moved = group_item<4, false>(M, S, d.y, d.z, logg, step, us.all_rows); break;
+            case 0: moved = group_item<1, kRecords>(M, S, d.y, d.z, logg, step, us.all_rows); break;
+            case 1: moved = group_item<2, kRecords>(M, S, d.y, d.z, logg, step, us.all_rows); break;
+            default: moved = group_item<4, kRecords>(M, S, d.y, d.z, logg, step, us.all_rows); break;
         }
     }
     note_change(D, u, step, moved);
@@ -872,7 +931,7 @@ __device__ __forceinline__ void sweep_item(const DevMatrix &M, const DevState &D
 // Applies the candidates of queued task `task` = unit * n_seg_parts + segment
 // (one wave; the row's activity is read back from its SegState).  Returns the
 // lane's accepted candidates; u: the task's unit.
-template <bool kCoherent>
+template <int kMode>
 __device__ __forceinline__ int apply_split_task(const DevMatrix &M, const DevState &D, int task, int &u) {
     constexpr int K = kSegLen / 64;
     const int lane = threadIdx.x & 63;
@@ -900,7 +959,7 @@ __device__ __forceinline__ int apply_split_task(const DevMatrix &M, const DevSta
         if (e < len) {
             const int jp = M.col[start + e];
             double l, uu;
-            load_bounds<kCoherent>(M, V, jp & kIdMask, l, uu);
+            load_bounds<kMode>(M, V, jp & kIdMask, l, uu);
             moved += apply_entry(M, S, jp, M.val[start + e], l, uu, sd.x, sd.y, minact, maxact, ni, xi);
         }
     }
@@ -913,7 +972,7 @@ __device__ __forceinline__ void apply_phase(const DevMatrix &M, const DevState &
     const int count = coherent_load(&st[kStatusApply]);
     for (int t = wave; t < count; t += nwaves) {
         int u;
-        const int moved = apply_split_task<false>(M, D, coherent_load(&D.apply_tasks[t]), u);
+        const int moved = apply_split_task<kRecords>(M, D, coherent_load(&D.apply_tasks[t]), u);
         note_change(D, u, step, moved);
     }
 }
@@ -1294,7 +1353,7 @@ __device__ __forceinline__ bool grid_barrier(const DevState &D, unsigned nblocks
 // the sweep queued any; publish.  The number of steps run goes to the global
 // status block (-1 after a failed wait).
 template <int kThreads, bool kLds>
-__global__ __launch_bounds__(kThreads) void mega_kernel(DevMatrix M, DevState D_arg, int first_step, int max_steps,
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void mega_kernel(DevMatrix M, DevState D_arg, int first_step, int max_steps,
                                                         int n_units) {
     // kLds: a launch of one unit that reads binary columns from LDS; without
     // it n_lds is a constant 0, and the LDS reads and code updates compile out
@@ -1494,33 +1553,46 @@ __device__ __forceinline__ bool carry_moved(const DevMatrix &M, const DevState &
     return crossed;
 }
 
-// Item `it` of a round: a segment of a split row, or the rows of one pass
-// (or a few) of a bin.  The bins' item ranges are kernel arguments, so an
-// item costs no load.  Returns the lane's accepted candidates.
-template <bool kCoherent>
+// Lists the items of the rounds: the segments of the split rows, then the
+// bins' rows from wide to narrow.
+__global__ __launch_bounds__(256) void plan_rounds_kernel(DevMatrix M, RoundBins B, int4 *items) {
+    const int n = B.item0[kPlanBins];
+    for (int it = blockIdx.x * blockDim.x + threadIdx.x; it < n; it += gridDim.x * blockDim.x) {
+        int4 d = make_int4(0, 0, 0, 0);
+        if (it < B.n_segs) {
+            const int lr = M.part_row[it];
+            d = make_int4(kItemSeg, lr, it - M.seg_rows[lr].y, 1);
+        } else {
+#pragma unroll
+            for (int q = 0; q < kPlanBins; q++)
+                if (it >= B.item0[q] && it < B.item0[q + 1]) {
+                    const int first = B.row0[q] + (it - B.item0[q]) * B.rows_per_item[q];
+                    d = make_int4(kItemGroup | (B.logg[q] << 4) | (B.logk[q] << 8), first,
+                                  min(B.rows_per_item[q], B.row0[q + 1] - first), 0);
+                }
+        }
+        items[it] = d;
+    }
+}
+
+// Item `it` of a round.  Returns the lane's accepted candidates.
+template <int kMode>
 __device__ __forceinline__ int round_item(const DevMatrix &M, const DevState &V, const RoundPlan &R, int it, int step,
                                           int *st) {
-    it = uniform(it);
-    if (it < R.n_segs) {
-        const int lr = uniform(M.part_row[it]);
-        seg_item<kCoherent>(M, V, V, 0, lr, it - uniform(M.seg_rows[lr].y), 1, st, step, true, 1);
+    int4 d = R.items[uniform(it)];
+    d.x = uniform(d.x);
+    d.y = uniform(d.y);
+    d.z = uniform(d.z);
+    if ((d.x & 15) == kItemSeg) {
+        seg_item<kMode>(M, V, V, 0, d.y, d.z, 1, st, step, true, 1);
         return 0;
     }
-    int first = 0, nrows = 0, logg = 0, logk = 0;
-#pragma unroll
-    for (int q = 0; q < kPlanBins; q++)
-        if (it >= R.item0[q] && it < R.item0[q + 1]) {
-            first = R.row0[q] + (it - R.item0[q]) * R.rows_per_item[q];
-            nrows = R.row0[q + 1] - first;
-            nrows = nrows < R.rows_per_item[q] ? nrows : R.rows_per_item[q];
-            logg = R.logg[q];
-            logk = R.logk[q];
-        }
+    const int logg = (d.x >> 4) & 15;
     const Sink S = make_sink(V);
-    switch (logk) {
-        case 0: return group_item<1, kCoherent>(M, S, first, nrows, logg, step, true);
-        case 1: return group_item<2, kCoherent>(M, S, first, nrows, logg, step, true);
-        default: return group_item<4, kCoherent>(M, S, first, nrows, logg, step, true);
+    switch ((d.x >> 8) & 15) {
+        case 0: return group_item<1, kMode>(M, S, d.y, d.z, logg, step, true);
+        case 1: return group_item<2, kMode>(M, S, d.y, d.z, logg, step, true);
+        default: return group_item<4, kMode>(M, S, d.y, d.z, logg, step, true);
     }
 }
 
@@ -1569,6 +1641,7 @@ __global__ __launch_bounds__(256) void load_rounds_kernel(DevMatrix M, DevState 
             B.AF[id - M.n_int] = make_double2(l, u);
         }
     }
+    if (tid == 0) A.AF[M.n - M.n_int] = B.AF[M.n - M.n_int] = make_double2(0.0, 0.0);  // the padding entries' column
     for (int w = tid; w < M.nwords; w += stride) {
         A.bm[w] = 0u;
         B.bm[w] = 0u;
@@ -1594,7 +1667,7 @@ __device__ __forceinline__ bool round_moved(const DevState &D, int step) {
 // the run goes on (input usable, not infeasible, the previous round moved a
 // bound); the first workgroup tells the host: its word becomes `step` when
 // the round runs, else kRoundsOver.
-__global__ __launch_bounds__(256) void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
     __shared__ int any_moved;
     const long long *p = reinterpret_cast<const long long *>(&D.units[0]);
     const long long w0 = coherent_load(p), w2 = coherent_load(p + 2);
@@ -1611,7 +1684,7 @@ __global__ __launch_bounds__(256) void round_kernel(DevMatrix M, DevState D, Rou
     const DevState V = round_view(M, D, R, step);
     if (step > 1 && carry_moved(M, D, R, step, wave, nwaves)) atomic_max_i(&D.units[0].infeasible, step - 1);
     int moved = 0;
-    for (int it = wave; it < R.n_items; it += nwaves) moved |= round_item<false>(M, V, R, it, step, st);
+    for (int it = wave; it < R.n_items; it += nwaves) moved |= round_item<kWide>(M, V, R, it, step, st);
     if (__any(moved != 0) && (threadIdx.x & 63) == 0) any_moved = 1;
     __syncthreads();
     if (threadIdx.x == 0 && any_moved) note_round_moved(D, step);
@@ -1624,7 +1697,7 @@ __global__ __launch_bounds__(256) void round_apply_kernel(DevMatrix M, DevState 
     const DevState V = round_view(M, D, R, step);
     int moved = 0, u;
     for (int t = blockIdx.x * waves + (threadIdx.x >> 6); t < count; t += gridDim.x * waves)
-        moved |= apply_split_task<false>(M, V, coherent_load(&D.apply_tasks[t]), u);
+        moved |= apply_split_task<kWide>(M, V, coherent_load(&D.apply_tasks[t]), u);
     if (__any(moved != 0) && (threadIdx.x & 63) == 0) note_round_moved(D, step);
 }
 
@@ -1701,7 +1774,7 @@ __global__ __launch_bounds__(1024) void rounds_kernel(DevMatrix M, DevState D, R
         unsigned flags = 0u;
         if (step > 1 && carry_moved(M, D, R, step, wave, nwaves)) flags |= kCrossed;
         for (int it = wave; it < R.n_items; it += nwaves)
-            if (round_item<true>(M, V, R, it, step, st)) flags |= kMoved;
+            if (round_item<kWideCoherent>(M, V, R, it, step, st)) flags |= kMoved;
         ok = gather_barrier(D, R, ++seq, flags, wg_flags, all);
         unsigned seen = all;
         if (ok && M.n_seg_parts > 0) {
@@ -1710,7 +1783,7 @@ __global__ __launch_bounds__(1024) void rounds_kernel(DevMatrix M, DevState D, R
                 flags = 0u;
                 int u;
                 for (int t = wave; t < count; t += nwaves)
-                    if (apply_split_task<true>(M, V, coherent_load(&D.apply_tasks[t]), u)) flags |= kMoved;
+                    if (apply_split_task<kWideCoherent>(M, V, coherent_load(&D.apply_tasks[t]), u)) flags |= kMoved;
                 ok = gather_barrier(D, R, ++seq, flags, wg_flags, all);
                 seen |= all;
             }
@@ -1856,6 +1929,7 @@ __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int 
                 V.SF[id - M.n_int] = make_double2(l, uu);
             }
         }
+        if (tid == 0) V.SF[M.n - M.n_int] = make_double2(0.0, 0.0);  // the padding entries' column
         // 2-bit codes of the binary columns, padding words zero
         for (int w = tid; w < M.sb_words; w += stride) {
             unsigned cw = 0u;
