@@ -220,6 +220,18 @@ struct DevState {
     unsigned *SB;          // 2-bit codes of the binary columns (sb_words per unit)
 };
 
+// A vector that the units of a launch mostly agree with (the base of a
+// server's requests, the first of several node vectors): the partial
+// activities of the split rows' segments are computed for it once, and a unit
+// starts with them in place of its own wherever it has the same bounds.
+struct ReferenceView {
+    const SegPart *parts = nullptr;  // null: no reference
+    const double *lbs = nullptr, *ubs = nullptr;  // caller's column order
+    unsigned *diff = nullptr;        // per listed unit: columns that differ (nwords each)
+    int *n_diff = nullptr;           // per listed unit: words of diff that are not zero
+    int start = 0;                   // step that the copied partials are stamped with
+};
+
 // ---- double-buffered rounds (one bound vector) ----
 // Two blocks of bound records take turns: round s reads the bounds S_{s-1}
 // from block (s - 1) & 1 and folds its candidates into block s & 1, which

@@ -54,7 +54,10 @@ __global__ void rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status);
 __global__ void load_kernel(DevMatrix M, DevState D, int n_list, const int *list, const double *const *lbp,
-                            const double *const *ubp);
+                            const double *const *ubp, ReferenceView ref);
+__global__ void load_reference_kernel(DevMatrix M, DevState V, const double *lbs, const double *ubs);
+__global__ void reference_parts_kernel(DevMatrix M, DevState V, SegPart *parts);
+__global__ void drop_parts_kernel(DevMatrix M, DevState D, int n_list, const int *list, ReferenceView ref, int limit);
 __global__ void hint_kernel(DevMatrix M, DevState D, int n_list, const int *list, const int *hint_ptr,
                             const int *hints, const int *inv_perm, int start_step);
 __global__ void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list, double *const *lbp,
@@ -441,6 +444,11 @@ struct Problem {
     int *d_hint_ptr = nullptr, *d_hints = nullptr;
     size_t hints_cap = 0;
     std::vector<void *> hint_owned;
+    // reference vector of a launch of many units (gdp_device.h, ReferenceView)
+    char *ref_block = nullptr;
+    SegPart *ref_parts = nullptr;
+    char *ref_diff = nullptr;        // n_diff, then diff, of up to ref_units units
+    int ref_units = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int device = 0;
@@ -482,6 +490,8 @@ struct Problem {
         if (stream) (void)hipStreamDestroy(stream);
         if (state_buf) (void)cached_free(state_buf);
         for (void *p : hint_owned) (void)cached_free(p);
+        for (void *p : {static_cast<void *>(ref_block), static_cast<void *>(ref_parts), static_cast<void *>(ref_diff)})
+            (void)cached_free(p);
         for (void *p : owned) (void)cached_free(p);
         if (host) host_slots().give(host);
         if (staging_held) staging().release();
@@ -1239,11 +1249,53 @@ void reserve_hints(Problem *P, size_t count) {
     P->d_hints = dev_alloc<int>(P->hints_cap, P->hint_owned);
 }
 
+// Makes (d_lbs, d_ubs) the reference of the problem's next loads: its
+// snapshot and its segment partials.
+void set_reference(Problem *P, const double *d_lbs, const double *d_ubs) {
+    const DevMatrix &M = P->M;
+    if (!P->ref_block) check(cached_malloc(&P->ref_block, static_cast<size_t>(M.snap_stride)), "hipMalloc reference");
+    if (!P->ref_parts)
+        check(cached_malloc(&P->ref_parts, sizeof(SegPart) * std::max(1, M.n_seg_parts)), "hipMalloc reference");
+    DevState V{};
+    V.S16 = reinterpret_cast<unsigned *>(P->ref_block);
+    V.S32 = reinterpret_cast<int2 *>(P->ref_block + M.snap_off32);
+    V.SF = reinterpret_cast<double2 *>(P->ref_block + M.snap_offF);
+    hipLaunchKernelGGL(load_reference_kernel, dim3(std::max(1, std::min(1024, (M.n + 255) / 256))), dim3(256), 0,
+                       P->stream, M, V, d_lbs, d_ubs);
+    hipLaunchKernelGGL(reference_parts_kernel, dim3(std::max(1, std::min(2048, grid_for(M.n_seg_parts)))), dim3(256), 0,
+                       P->stream, M, V, P->ref_parts);
+    check(hipGetLastError(), "reference launch");
+}
+
+// The reference for a load of n_list units, its per-unit notes cleared.
+ReferenceView reference_view(Problem *P, int n_list, const double *d_lbs, const double *d_ubs, int start) {
+    ReferenceView ref;
+    const size_t notes = (static_cast<size_t>(n_list) * sizeof(int) + 255) / 256 * 256;
+    if (n_list > P->ref_units) {
+        check(hipStreamSynchronize(P->stream), "sync");
+        check(cached_free(P->ref_diff), "hipFree");
+        P->ref_diff = nullptr;
+        P->ref_units = 0;
+        check(cached_malloc(&P->ref_diff, notes + sizeof(unsigned) * P->M.nwords * static_cast<size_t>(n_list)),
+              "hipMalloc reference");
+        P->ref_units = n_list;
+    }
+    ref.n_diff = reinterpret_cast<int *>(P->ref_diff);
+    ref.diff = reinterpret_cast<unsigned *>(P->ref_diff + notes);
+    check(hipMemsetAsync(ref.n_diff, 0, sizeof(int) * n_list, P->stream), "memset reference");
+    ref.parts = P->ref_parts;
+    ref.lbs = d_lbs;
+    ref.ubs = d_ubs;
+    ref.start = start;
+    return ref;
+}
+
 // Loads the listed units' bound vectors for a fresh run (status ring
 // cleared, round 1 in step `start`) or for units joining a running server
 // (`fresh` false).
 void load_units(Problem *P, int n_list, const int *list, double *const *lbp, double *const *ubp,
-                const int *hint_ptr, const int *hints, const int *max_rounds, int start, bool fresh) {
+                const int *hint_ptr, const int *hints, const int *max_rounds, int start, bool fresh,
+                const double *ref_lb = nullptr, const double *ref_ub = nullptr) {
     hipStream_t s = P->stream;
     DevMatrix &M = P->M;
     DevState &D = P->D;
@@ -1267,7 +1319,16 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
                        n_list, P->d_params, start, fresh ? 1 : 0);
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
     const int gy = P->replicas ? std::max(1, std::min(n_list, 1024)) : 1;
-    hipLaunchKernelGGL(load_kernel, dim3(gx, gy), dim3(256), 0, s, M, D, n_list, P->d_list, P->d_lbp, P->d_ubp);
+    ReferenceView ref;
+    if (ref_lb) ref = reference_view(P, n_list, ref_lb, ref_ub, start);
+    hipLaunchKernelGGL(load_kernel, dim3(gx, gy), dim3(256), 0, s, M, D, n_list, P->d_list, P->d_lbp, P->d_ubp, ref);
+    if (ref_lb) {
+        // walking the columns of up to this many words costs less than an
+        // eighth of the unit's segments
+        const int limit = std::max(16, M.nwords / 64);
+        hipLaunchKernelGGL(drop_parts_kernel, dim3(std::max(1, std::min(8, (M.nwords + 255) / 256)), gy), dim3(256), 0, s,
+                           M, D, n_list, P->d_list, ref, limit);
+    }
     check(hipGetLastError(), "load launch");
     if (hint_ptr != nullptr && M.mark_rows && hint_ptr[n_list] > 0) {
         reserve_hints(P, hint_ptr[n_list]);
@@ -1575,7 +1636,13 @@ void run_units(Problem *P, int n_list, const int *list, double *const *lbp, doub
     if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
     std::vector<int> caps(n_list, max_rounds);
     P->D.n_active = P->replicas ? n_list : 0;
-    load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps.data(), 1, true);
+    // hinted vectors (children of propagated nodes) mostly agree with each
+    // other: the first one is the reference of all
+    const bool related = P->replicas && n_list > 1 && P->M.n_seg_parts > 0 && P->M.mark_rows &&
+                         hint_ptr != nullptr && hint_ptr[n_list] > 0;
+    if (related) set_reference(P, lbp[0], ubp[0]);
+    load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps.data(), 1, true, related ? lbp[0] : nullptr,
+               related ? ubp[0] : nullptr);
     // bounds outside the envelope are an error before any round
     std::vector<UnitState> st = read_units(P, n_list, list);
     bool any_active = false;
@@ -2420,6 +2487,11 @@ void server_set_base(Server *S, const double *lbs, const double *ubs) {
     S->base_lb.assign(lbs, lbs + S->n);
     S->base_ub.assign(ubs, ubs + S->n);
     S->has_base = true;
+    // requests mostly agree with the base: its segment partials are theirs
+    if (S->P->M.n_seg_parts > 0 && S->P->M.mark_rows) {
+        set_reference(S->P, S->d_base, S->d_base + S->n);
+        check(hipStreamSynchronize(S->P->stream), "reference sync");
+    }
 }
 
 namespace {
@@ -2813,7 +2885,8 @@ int step_impl(Server *S) {
     t_copies = Clock::now();
     if (!adm.empty())
         load_units(P, static_cast<int>(adm.size()), adm.data(), adm_lb.data(), adm_ub.data(), hint_ptr.data(),
-                   hints.data(), caps.data(), S->step, false);
+                   hints.data(), caps.data(), S->step, false,
+                   S->has_base && P->M.n_seg_parts > 0 && P->M.mark_rows ? S->d_base : nullptr, S->d_base + n);
     t_run = Clock::now();
     t_retire = t_run;
     // ---- every active slot advances one round ----

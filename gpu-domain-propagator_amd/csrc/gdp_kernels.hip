@@ -1892,8 +1892,11 @@ __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, in
 // snapshot and accumulator, clears their bitmaps, marks and split-row
 // counters, and flags crossed input bounds and bounds outside a column's
 // storage class.  Grid: x over internal ids, y over listed units.
+// With a reference (replicas), every unit notes the columns in which it
+// differs from it and takes over its segment partials.
 __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int n_list, const int *list,
-                                                   const double *const *lbp, const double *const *ubp) {
+                                                   const double *const *lbp, const double *const *ubp,
+                                                   ReferenceView ref) {
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     const int n_pass = M.replicas ? n_list : 1;  // blocks mode: one pass over all columns
@@ -1910,6 +1913,17 @@ __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int 
                 l = lbs[j];
                 uu = ubs[j];
                 if (eps_gt(l, uu)) atomic_or_i(&D.units[cu].crossed, 1);
+            }
+            if (ref.parts != nullptr) {
+                const bool differs = __double_as_longlong(l) != __double_as_longlong(ref.lbs[j]) ||
+                                     __double_as_longlong(uu) != __double_as_longlong(ref.ubs[j]);
+                const unsigned long long both = __ballot(differs);
+                const int lane = threadIdx.x & 63;
+                if ((lane & 31) == 0) {
+                    const unsigned w = static_cast<unsigned>(lane ? both >> 32 : both);
+                    ref.diff[static_cast<size_t>(k) * M.nwords + (id >> 5)] = w;
+                    if (w) atomic_add_i(&ref.n_diff[k], 1);
+                }
             }
             if (id < M.n_int) {
                 const double lim = id < M.n16 ? 32767.0 : 2147483647.0;
@@ -1952,8 +1966,97 @@ __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int 
             // step of this run (steps restart with every run) and make it
             // recompute segments whose columns did not move
             for (int q = tid; q < M.n_seg_parts; q += stride) {
-                V.seg_parts[q].stamp = 0;
+                if (ref.parts != nullptr) {
+                    SegPart part = ref.parts[q];
+                    part.stamp = ref.start;
+                    V.seg_parts[q] = part;
+                } else {
+                    V.seg_parts[q].stamp = 0;
+                }
                 V.seg_marks[q] = 0;
+            }
+        }
+    }
+}
+
+// The snapshot block of a reference vector (records as load_kernel writes
+// them).  Values outside a column's class leave a wrong record: a unit with
+// the same value there is refused, one with another drops the segment.
+__global__ __launch_bounds__(256) void load_reference_kernel(DevMatrix M, DevState V, const double *lbs,
+                                                             const double *ubs) {
+    for (int id = blockIdx.x * blockDim.x + threadIdx.x; id < M.n; id += gridDim.x * blockDim.x) {
+        const int j = M.perm[id];
+        const double l = lbs[j], u = ubs[j];
+        if (id < M.n_int) {
+            const bool fits = fits_int32(l) && fits_int32(u);
+            const int il = fits ? static_cast<int>(l) : 0, iu = fits ? static_cast<int>(u) : 0;
+            if (id < M.n16) V.S16[id] = pack16(il, iu);
+            else V.S32[id - M.n16] = make_int2(il, iu);
+        } else {
+            V.SF[id - M.n_int] = make_double2(l, u);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) V.SF[M.n - M.n_int] = make_double2(0.0, 0.0);
+}
+
+// The segment partials of a reference vector, one wave per segment.
+__global__ __launch_bounds__(256) void reference_parts_kernel(DevMatrix M, DevState V_arg, SegPart *parts) {
+    constexpr int K = kSegLen / 64;
+    DevState V = V_arg;
+    V.n_lds = 0;
+    const int lane = threadIdx.x & 63;
+    const int waves = gridDim.x * (blockDim.x >> 6);
+    for (int q = uniform(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)); q < M.n_seg_parts; q += waves) {
+        const int4 info = M.seg_rows[M.part_row[q]];
+        int start, len;
+        row_extent(M, info.x, start, len);
+        const int s0 = (q - info.y) * kSegLen;
+        LaneEntries<K, kRecords> E;
+        E.load(M, V, start + s0, lane * K, len - s0);
+        E.template reduce<true>(64);
+        if (lane == 0) {
+            SegPart p;
+            p.smin = E.tmin;
+            p.smax = E.tmax;
+            p.dmax = E.dmax;
+            p.infs = E.infs;
+            p.stamp = 0;
+            parts[q] = p;
+        }
+    }
+}
+
+// Drops the copied partials of the segments that hold a column in which the
+// unit differs from the reference; all of them where so many words differ
+// that walking the columns would cost more than the segments.  A wave looks
+// at 64 words, and its lanes take the entries of a differing column.
+__global__ __launch_bounds__(256) void drop_parts_kernel(DevMatrix M, DevState D, int n_list, const int *list,
+                                                         ReferenceView ref, int limit) {
+    const int lane = threadIdx.x & 63;
+    const int waves = gridDim.x * (blockDim.x >> 6);
+    const int wave = uniform(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    for (int k = blockIdx.y; k < n_list; k += gridDim.y) {
+        const DevState V = unit_view(M, D, uniform(list[k]));
+        if (ref.n_diff[k] > limit) {
+            for (int q = wave * 64 + lane; q < M.n_seg_parts; q += waves * 64) V.seg_parts[q].stamp = 0;
+            continue;
+        }
+        for (int w0 = wave * 64; w0 < M.nwords; w0 += waves * 64) {
+            const int w = w0 + lane;
+            const unsigned mine = w < M.nwords ? ref.diff[static_cast<size_t>(k) * M.nwords + w] : 0u;
+            unsigned long long pending = __ballot(mine != 0u);
+            while (pending) {
+                const int t = __ffsll(static_cast<long long>(pending)) - 1;
+                pending &= pending - 1;
+                unsigned bits = static_cast<unsigned>(__shfl(static_cast<int>(mine), t, 64));
+                while (bits) {
+                    const int id = (w0 + t) * 32 + __ffs(static_cast<int>(bits)) - 1;
+                    bits &= bits - 1;
+                    for (int q = M.col_ptr[id] + lane; q < M.col_ptr[id + 1]; q += 64) {
+                        const int part = M.col_seg[q];
+                        if (part >= 0) V.seg_parts[part].stamp = 0;
+                    }
+                }
             }
         }
     }
@@ -1965,12 +2068,15 @@ __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int 
 __global__ __launch_bounds__(256) void hint_kernel(DevMatrix M, DevState D, int n_list, const int *list,
                                                    const int *hint_ptr, const int *hints, const int *inv_perm,
                                                    int start_step) {
+    // a wave per hinted column, its lanes over the column's entries
+    const int lane = threadIdx.x & 63;
+    const int waves = gridDim.x * (blockDim.x >> 6);
+    const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     for (int k = blockIdx.y; k < n_list; k += gridDim.y) {
         const DevState V = unit_view(M, D, list[k]);
-        for (int h = hint_ptr[k] + blockIdx.x * blockDim.x + threadIdx.x; h < hint_ptr[k + 1];
-             h += gridDim.x * blockDim.x) {
+        for (int h = hint_ptr[k] + wave; h < hint_ptr[k + 1]; h += waves) {
             const int id = inv_perm[hints[h]];
-            for (int q = M.col_ptr[id]; q < M.col_ptr[id + 1]; q++) {
+            for (int q = M.col_ptr[id] + lane; q < M.col_ptr[id + 1]; q += 64) {
                 V.marks[M.col_rows[q]] = start_step;
                 if (M.col_item[q] >= 0) V.item_mark[M.col_item[q]] = start_step;
             }
