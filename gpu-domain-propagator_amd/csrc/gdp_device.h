@@ -47,13 +47,16 @@
 //                  bounds cross)
 //   bm[nwords]     uint32  columns moved in the current step (scanned by publish)
 //   marks[m']      int32   step in which the row must be processed
-//   item_mark[]    int32   per group item: step in which one of its rows must be
-//                          processed (set with the row marks), so that a
-//                          step with few marked rows visits few items
+//   lists          wl[m'], wl_seg[segments], wl_cnt: the marked rows of the
+//                          next step, listed by tree width (a row once: the
+//                          mark is exchanged and the first marker lists it),
+//                          and the segments of split rows to recompute; a step
+//                          of marked rows works through them in full passes
+//                          whatever items the rows lie in
 //   split rows     seg_parts, seg_state, seg_count, seg_marks: a marked split
 //                  row recomputes only the segments holding a column that
-//                  moved in the previous step (and segments not yet computed
-//                  in the run); the others keep their stored partials
+//                  moved in the previous step; the others keep their stored
+//                  partials
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -67,11 +70,17 @@ constexpr int kItemLong = 1;   // one row, one wave, all segments (rows not spli
 constexpr int kItemSeg = 2;    // up to kSegsPerItem consecutive segments of a split row
 constexpr int kSegsPerItem = 4;
 constexpr int kItemUnitShift = 12;  // items[].x >> 12: unit of the item (blocks mode)
-// Most units of one persistent launch whose activity its workgroups keep in LDS.
-constexpr int kMaxFilterUnits = 4096;
+// Units of a launch whose work a workgroup lays out in LDS at a time.
+constexpr int kWindowUnits = 1024;
 // Bytes of the persistent kernel's dynamic LDS in a launch of several units:
-// the working / all-rows bits and first steps of up to kMaxFilterUnits units.
-constexpr int kFilterLdsBytes = (kMaxFilterUnits / 32) * 4 * 2 + kMaxFilterUnits * 4;
+// the running sums of the units' work (one more than units) and their
+// all-rows bits.
+constexpr int kWindowLdsBytes = (kWindowUnits + 64) * 4 + (kWindowUnits / 32) * 4;
+// Lists of marked work: class 0 the segments of split rows, 1 the unsplit
+// long rows, 2 + q the rows of tree width 2^(8 - q).
+constexpr int kClasses = 11;
+constexpr int kListStride = 16;       // DevMatrix::list_at entries per unit
+constexpr int kCountWords = 8;        // 64-bit counter words per unit and step parity, two classes each
 // Binary columns (integer columns whose bound envelope lies in [0, 1]) have
 // internal ids [0, n_bin) in replicas mode, and each unit keeps their bounds
 // also as 2-bit codes, 16 columns to a 32-bit word: bit 0 = (lb >= 1), bit
@@ -178,11 +187,11 @@ struct DevMatrix {
     int n_seg_parts;
     const int *col_ptr;    // csc of the internal ids (marking)
     const int *col_rows;
-    const int *col_seg;    // per csc entry: its segment of a split row (-1: other rows)
-    const int *col_item;   // per csc entry: the group item holding its row (-1: a split or
-                           // unsplit long row, whose items test the row mark itself)
-    const int *item_row;   // per item: the row whose mark a seg / long item tests (-1: group
-                           // item, which tests its own item mark)
+    const int *col_seg;    // per csc entry: its segment of a split row, or -1 - the class of its row
+    const int *list_at;    // first place in wl (class 0: in wl_seg) of each class (blocks: of each
+                           // unit's classes, kListStride per unit)
+    const int *unit_item;  // blocks: first sweep item of each unit, and the end
+    unsigned long long class_logg, class_logk;  // lanes per row and entries per lane (log2), 4 bits a class
     const int *perm;       // internal id -> caller's column (-1: padding id)
     const int *word_unit;  // blocks mode: unit of each bitmap word
     int snap_off32;        // byte offset of S32 in a unit's snapshot block
@@ -202,11 +211,13 @@ struct DevState {
     double2 *AF;
     unsigned *bm;
     int *marks;
-    int *item_mark;        // per group item: step in which one of its rows must be processed
+    int *wl;               // marked rows of the next step, by class
+    int *wl_seg;           // segments to recompute in the next step
+    unsigned long long *wl_cnt;  // [units][2][kCountWords] listed rows per class, by step parity
     SegPart *seg_parts;
     int *seg_marks;        // step in which a split row's segment must be recomputed
     SegState *seg_state;
-    unsigned *seg_count;   // segments reduced in the current step
+    unsigned *seg_count;   // segments reduced in the current step (a step of all rows), or still to reduce
     // shared by all units
     UnitState *units;
     int *moved;            // [units][kMoveSlots][kMoveLanes] accepted candidates, kMoveStride ints apart
@@ -221,7 +232,7 @@ struct DevState {
 };
 
 // A vector that the units of a launch mostly agree with (the base of a
-// server's requests, the first of several node vectors): the partial
+// server's requests, the majority of three node vectors): the partial
 // activities of the split rows' segments are computed for it once, and a unit
 // starts with them in place of its own wherever it has the same bounds.
 struct ReferenceView {
@@ -230,6 +241,12 @@ struct ReferenceView {
     unsigned *diff = nullptr;        // per listed unit: columns that differ (nwords each)
     int *n_diff = nullptr;           // per listed unit: words of diff that are not zero
     int start = 0;                   // step that the copied partials are stamped with
+};
+
+// Up to three vectors whose bitwise majority is the reference.
+struct ReferenceVectors {
+    const double *lb[3], *ub[3];
+    int n;
 };
 
 // ---- double-buffered rounds (one bound vector) ----
@@ -283,7 +300,8 @@ __device__ __forceinline__ DevState unit_view(const DevMatrix &M, const DevState
     V.AF += k * (M.n - M.n_int);
     V.bm += k * M.nwords;
     V.marks += k * M.m;
-    V.item_mark += k * M.n_items;
+    V.wl += k * M.m;
+    V.wl_seg += k * M.n_seg_parts;
     V.seg_parts += k * M.n_seg_parts;
     V.seg_marks += k * M.n_seg_parts;
     V.seg_state += k * M.n_seg_rows;

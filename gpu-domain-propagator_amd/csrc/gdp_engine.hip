@@ -40,7 +40,7 @@
 
 namespace gdp {
 
-__global__ void sweep_kernel(DevMatrix M, DevState D, int step, int guard, int first_step);
+__global__ void sweep_kernel(DevMatrix M, DevState D, int step, int guard, int first_step, int n_units);
 __global__ void apply_split_kernel(DevMatrix M, DevState D, int step, int guard, int first_step);
 __global__ void publish_kernel(DevMatrix M, DevState D, int step, int guard, int first_step, int n_units);
 template <int kThreads, bool kLds>
@@ -55,8 +55,9 @@ __global__ void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status);
 __global__ void load_kernel(DevMatrix M, DevState D, int n_list, const int *list, const double *const *lbp,
                             const double *const *ubp, ReferenceView ref);
-__global__ void load_reference_kernel(DevMatrix M, DevState V, const double *lbs, const double *ubs);
+__global__ void load_reference_kernel(DevMatrix M, DevState V, ReferenceVectors R, double *lbs, double *ubs);
 __global__ void reference_parts_kernel(DevMatrix M, DevState V, SegPart *parts);
+__global__ void fill_parts_kernel(DevMatrix M, DevState D, int n_list, const int *list, int start_step, int chunk);
 __global__ void drop_parts_kernel(DevMatrix M, DevState D, int n_list, const int *list, ReferenceView ref, int limit);
 __global__ void hint_kernel(DevMatrix M, DevState D, int n_list, const int *list, const int *hint_ptr,
                             const int *hints, const int *inv_perm, int start_step);
@@ -74,13 +75,13 @@ __global__ void layout_rows_kernel(int mp, const long long *src_start, const int
                                    const int *internal, const int *vartype, int *col_out, double *val_out,
                                    int *col_cnt, int *bad);
 __global__ void layout_csc_kernel(int mp, const int *row_ptr_out, const int *col_out, const int *row_part,
-                                  const int *row_item, int *fill, int *col_rows, int *col_seg, int *col_item);
+                                  int *fill, int *col_rows, int *col_seg);
 __global__ void layout_rows_short_kernel(int r_begin, int mp, const long long *src_start, const int *row_inst,
                                          const int *inst_col_off, const int *col_in, const double *val_in,
                                          const int *row_ptr_out, const int *internal, const int *vartype,
                                          int *col_out, double *val_out, int *col_cnt, int *bad);
 __global__ void layout_csc_short_kernel(int r_begin, int mp, const int *row_ptr_out, const int *col_out,
-                                        const int *row_item, int *fill, int *col_rows, int *col_seg, int *col_item);
+                                        int *fill, int *col_rows, int *col_seg);
 __global__ void measure_kernel(int n, const double *lb, const double *ub, const double *wl, const double *wu,
                                const double *ll, const double *lu, double *pl, double *pu, double *fin_part,
                                int *inf_part);
@@ -446,6 +447,7 @@ struct Problem {
     std::vector<void *> hint_owned;
     // reference vector of a launch of many units (gdp_device.h, ReferenceView)
     char *ref_block = nullptr;
+    double *ref_lb = nullptr, *ref_ub = nullptr;  // in ref_block
     SegPart *ref_parts = nullptr;
     char *ref_diff = nullptr;        // n_diff, then diff, of up to ref_units units
     int ref_units = 0;
@@ -507,9 +509,10 @@ namespace {
 // counters), the problem-wide status ring, global words and barrier, and
 // the launch tables the host fills (listed units, reset parameters,
 // bound-vector pointers, hint starts).  With base null only the size is
-// computed.  Returns the bytes needed.
+// computed.  Without `lists` (the allocation-free entry point, where they do
+// not fit) every step processes all rows.  Returns the bytes needed.
 size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char *base, DevState &D,
-                   UnitTables &T) {
+                   UnitTables &T, bool lists) {
     size_t off = 0;
     auto take = [&](size_t bytes) {
         char *p = base ? base + off : nullptr;
@@ -529,7 +532,6 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
     D.bm = reinterpret_cast<unsigned *>(take(k * M.nwords * sizeof(unsigned)));
     D.SB = reinterpret_cast<unsigned *>(take(k * M.sb_words * sizeof(unsigned)));
     D.marks = reinterpret_cast<int *>(take(k * M.m * sizeof(int)));
-    D.item_mark = reinterpret_cast<int *>(take(k * M.n_items * sizeof(int)));
     D.seg_parts = reinterpret_cast<SegPart *>(take(k * M.n_seg_parts * sizeof(SegPart)));
     D.seg_marks = reinterpret_cast<int *>(take(k * M.n_seg_parts * sizeof(int)));
     D.seg_state = reinterpret_cast<SegState *>(take(k * M.n_seg_rows * sizeof(SegState)));
@@ -545,6 +547,13 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
     T.lbp = reinterpret_cast<double **>(take(units * sizeof(double *)));
     T.ubp = reinterpret_cast<double **>(take(units * sizeof(double *)));
     T.hint_ptr = reinterpret_cast<int *>(take((units + 1) * sizeof(int)));
+    D.wl = D.wl_seg = nullptr;
+    D.wl_cnt = nullptr;
+    if (lists) {
+        D.wl = reinterpret_cast<int *>(take(k * M.m * sizeof(int)));
+        D.wl_seg = reinterpret_cast<int *>(take(k * M.n_seg_parts * sizeof(int)));
+        D.wl_cnt = reinterpret_cast<unsigned long long *>(take(units * 2 * kCountWords * sizeof(unsigned long long)));
+    }
     D.active = T.list;
     return off;
 }
@@ -569,9 +578,10 @@ size_t carve_rounds(const DevMatrix &Mr, char *base, RoundPlan &R) {
 
 // Points the problem's run state at `base` (cap units, see carve_state);
 // with `rounds`, the arrays of the double-buffered rounds follow.
-void bind_state(Problem *P, char *base, int cap, bool rounds) {
+void bind_state(Problem *P, char *base, int cap, bool rounds, bool lists = true) {
     UnitTables T;
-    const size_t off = carve_state(P->M, P->replicas, P->n_inst, cap, base, P->D, T);
+    const size_t off = carve_state(P->M, P->replicas, P->n_inst, cap, base, P->D, T, lists);
+    P->M.mark_rows = lists && P->tuning.row_marking ? 1 : 0;
     if (rounds) carve_rounds(P->Mr, base + off, P->R);
     P->rounds_state = rounds;
     P->d_list = T.list;
@@ -594,7 +604,7 @@ void alloc_units(Problem *P, int cap) {
     P->n_units = 0;
     DevState D{};
     UnitTables T;
-    size_t bytes = carve_state(P->M, P->replicas, P->n_inst, cap, nullptr, D, T);
+    size_t bytes = carve_state(P->M, P->replicas, P->n_inst, cap, nullptr, D, T, true);
     RoundPlan R;
     if (P->rounds_ok) bytes += carve_rounds(P->Mr, nullptr, R);
     check(cached_malloc(&P->state_buf, bytes), "hipMalloc run state");
@@ -683,12 +693,12 @@ class CsrUpload {
 // row_inst[r], at the starts of d_rp), the columns' entries are counted, the
 // counts scanned into the column starts and the column-to-row index filled.
 // Column indices outside an instance's range are reported here.  src_start,
-// row_inst (null for one instance), row_part and row_item are device arrays
+// row_inst (null for one instance) and row_part are device arrays
 // of the mp layout rows.  Synchronous.
 void device_layout_build(CsrUpload &csr, const std::vector<int> &col_off, int mp, int n_wide, int n_ids, int n_padded,
-                         const long long *src_start, const int *row_inst, const int *row_part, const int *row_item,
+                         const long long *src_start, const int *row_inst, const int *row_part,
                          const int *d_rp, const int *d_internal, int *d_col, double *d_val, int *d_cptr,
-                         int *d_crows, int *d_cseg, int *d_citem, hipStream_t s, CreateTrace &trace) {
+                         int *d_crows, int *d_cseg, hipStream_t s, CreateTrace &trace) {
     const int NI = static_cast<int>(col_off.size()) - 1;
     std::vector<void *> tmp;
     try {
@@ -723,11 +733,11 @@ void device_layout_build(CsrUpload &csr, const std::vector<int> &col_off, int mp
         order_exclusive_sum(t_cnt, d_cptr, n_ids + 1, s);
         check(hipMemcpyAsync(t_cnt, d_cptr, sizeof(int) * n_ids, hipMemcpyDeviceToDevice, s), "fill positions");
         if (n_wide > 0)
-            hipLaunchKernelGGL(layout_csc_kernel, dim3(grid), dim3(256), 0, s, n_wide, d_rp, d_col, row_part, row_item,
-                               t_cnt, d_crows, d_cseg, d_citem);
+            hipLaunchKernelGGL(layout_csc_kernel, dim3(grid), dim3(256), 0, s, n_wide, d_rp, d_col, row_part,
+                               t_cnt, d_crows, d_cseg);
         if (mp > n_wide)
             hipLaunchKernelGGL(layout_csc_short_kernel, dim3(grid_short), dim3(256), 0, s, n_wide, mp, d_rp, d_col,
-                               row_item, t_cnt, d_crows, d_cseg, d_citem);
+                               t_cnt, d_crows, d_cseg);
         check(hipGetLastError(), "layout launch");
         check(hipStreamSynchronize(s), "layout");
         trace.mark("layout_csc");
@@ -925,11 +935,13 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         }
         if (nnz_total > 0x7fffff00LL || col_off[NI] > kIdMask) throw std::runtime_error("problem too large");
         // row marking pays while the rows it marks (about accepted candidates
-        // x mean column length) stay below a quarter of the rows
+        // x mean column length) stay below an eighth of the rows (1M rows: 2.80
+        // ms with a quarter, 2.75 with an eighth, 2.78 with a sixteenth; batches
+        // and node vectors the same with all three)
         for (int i = 0; i < NI; i++) {
             const long long lim = T.mark_limit > 0 ? T.mark_limit
                                                     : static_cast<long long>(inst[i].m) * inst[i].n /
-                                                          (4LL * std::max(1, inst[i].nnz));
+                                                          (8LL * std::max(1, inst[i].nnz));
             P->mark_limit.push_back(static_cast<int>(std::max(64LL, std::min(lim, 1LL << 30))));
         }
         if (replicas) P->mark_limit.resize(1);
@@ -1054,9 +1066,12 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         std::vector<int4> h_seg_rows;
         std::vector<int> h_part_row;
         int n_parts = 0;
+        std::vector<int> first_part(NI, 0);
+        unsigned long long class_logg = 0, class_logk = 0;
         {
             std::vector<std::pair<int, int>> giant;  // (layout row, instance)
             for (int i = 0; i < NI; i++) {
+                first_part[i] = n_parts;
                 const int st = R.start[i], cnt = R.count[i];  // key 0: the long rows
                 for (int q = 0; q < cnt; q++) {
                     const int row = st + q;
@@ -1086,6 +1101,10 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
             logg = std::max(logg, b - 2);  // at most 4 entries per lane
             logg = std::min(logg, 6);
             const int logk = b - logg;
+            if (key >= 2) {  // the class of the bin's rows
+                class_logg |= static_cast<unsigned long long>(logg) << (4 * key);
+                class_logk |= static_cast<unsigned long long>(logk) << (4 * key);
+            }
             const int per_pass = 64 >> logg;
             int rows_per_item = std::max(1, item_nnz / width);
             rows_per_item = ((rows_per_item + per_pass - 1) / per_pass) * per_pass;
@@ -1099,15 +1118,16 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         for (const auto &v : inst_items) h_items.insert(h_items.end(), v.begin(), v.end());
         if (NI >= (1 << (31 - kItemUnitShift))) throw std::runtime_error("too many instances in a batch");
 
-        // per item: the row whose mark a seg / long item tests (-1: group item)
-        std::vector<int> h_item_row(h_items.size(), -1);
-        for (size_t q = 0; q < h_items.size(); q++) {
-            const int4 it = h_items[q];
-            const int kind = it.x & 15;
-            if (kind == kItemSeg)
-                h_item_row[q] = h_seg_rows[it.y].x;
-            else if (kind == kItemLong)
-                h_item_row[q] = it.y;
+        // per unit (blocks) the first sweep item, and the first place of each
+        // class in the lists of marked rows (a bin's rows lie together, and so
+        // do their list places)
+        std::vector<int> h_unit_item(NI + 1, 0), h_list_at(static_cast<size_t>(NI) * kListStride, 0);
+        for (int i = 0; i < NI; i++) {
+            h_unit_item[i + 1] = h_unit_item[i] + static_cast<int>(inst_items[i].size());
+            int *at = &h_list_at[static_cast<size_t>(i) * kListStride];
+            at[0] = first_part[i];
+            at[1] = R.start[i];
+            for (int c = 2; c < kClasses; c++) at[c] = R.start[static_cast<size_t>(c) * NI + i];
         }
 
         P->stats.m = P->m;
@@ -1137,29 +1157,28 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         const size_t n_csc = std::max<long long>(1, nnz_total);
         int *d_crows = dev_alloc<int>(n_csc, o);
         int *d_cseg = dev_alloc<int>(n_csc, o);
-        int *d_citem = dev_alloc<int>(n_csc, o);
-        int *d_item_row = dev_alloc<int>(h_item_row.size(), o);
+        int *d_unit_item = dev_alloc<int>(h_unit_item.size(), o);
+        int *d_list_at = dev_alloc<int>(h_list_at.size(), o);
         int *d_word_unit = dev_alloc<int>(word_unit.size(), o);
-        // per layout row: first segment of a split row, group item (-1: none)
+        // per layout row: first segment of a split row (-1: none)
         int *t_row_part = dev_alloc<int>(mp, tmp);
-        int *t_row_item = dev_alloc<int>(mp, tmp);
         trace.mark("device_setup_alloc");
         upload(d_items, h_items.data(), h_items.size(), s);
-        upload(d_item_row, h_item_row.data(), h_item_row.size(), s);
+        upload(d_unit_item, h_unit_item.data(), h_unit_item.size(), s);
+        upload(d_list_at, h_list_at.data(), h_list_at.size(), s);
         upload(d_seg_rows, h_seg_rows.data(), h_seg_rows.size(), s);
         upload(d_part_row, h_part_row.data(), h_part_row.size(), s);
         upload(d_word_unit, word_unit.data(), word_unit.size(), s);
         check(hipMemsetAsync(t_row_part, 0xff, sizeof(int) * mp, s), "memset row tables");
-        check(hipMemsetAsync(t_row_item, 0xff, sizeof(int) * mp, s), "memset row tables");
-        order_row_tables(M.n_items, d_items, M.n_seg_rows, d_seg_rows, t_row_item, t_row_part, s);
+        order_row_tables(M.n_seg_rows, d_seg_rows, t_row_part, s);
         check(hipStreamSynchronize(s), "upload");
         trace.mark("upload_order");
         // rows wider than 64 entries: the long rows and the bins of widths 2^9..2^7
         int n_wide = 0;
         for (int key = 0; key < 4; key++)
             for (int i = 0; i < NI; i++) n_wide += R.count[key * NI + i];
-        device_layout_build(csr, col_off, mp, n_wide, n_ids, n_padded, R.src, R.inst, t_row_part, t_row_item, d_rp,
-                            P->d_inv_perm, d_col, d_val, d_cptr, d_crows, d_cseg, d_citem, s, trace);
+        device_layout_build(csr, col_off, mp, n_wide, n_ids, n_padded, R.src, R.inst, t_row_part, d_rp,
+                            P->d_inv_perm, d_col, d_val, d_cptr, d_crows, d_cseg, s, trace);
         M.row_ptr = d_rp;
         M.sides = d_sides;
         M.n_padded = n_padded;
@@ -1171,8 +1190,10 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         M.col_ptr = d_cptr;
         M.col_rows = d_crows;
         M.col_seg = d_cseg;
-        M.col_item = d_citem;
-        M.item_row = d_item_row;
+        M.list_at = d_list_at;
+        M.unit_item = d_unit_item;
+        M.class_logg = class_logg;
+        M.class_logk = class_logk;
         M.perm = d_perm;
         M.word_unit = d_word_unit;
 
@@ -1192,8 +1213,8 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
             UnitTables T;
             if (replicas)
                 P->stats.unit_state_bytes =
-                    static_cast<long long>(carve_state(M, true, NI, 2, nullptr, D, T) -
-                                           carve_state(M, true, NI, 1, nullptr, D, T));
+                    static_cast<long long>(carve_state(M, true, NI, 2, nullptr, D, T, true) -
+                                           carve_state(M, true, NI, 1, nullptr, D, T, true));
             P->stats.n_units = replicas ? 0 : NI;
         }
 
@@ -1213,10 +1234,10 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
             if (T.mega_blocks_per_cu > 0) per_cu = std::min(per_cu, T.mega_blocks_per_cu);
             return std::max(1, per_cu);
         };
-        // the grid with the unit filter's LDS (launches of several units);
+        // the grid with the window's LDS (launches of several units);
         // launches of one unit hold as many binary columns' codes in LDS as
         // keep that many workgroups resident
-        const int per_cu = mega_per_cu(P->mega_fn, kFilterLdsBytes);
+        const int per_cu = mega_per_cu(P->mega_fn, kWindowLdsBytes);
         P->mega_grid = per_cu * P->cu_count;
         int n_lds = std::min(n_bin, kMaxLdsBinBytes * 4) / 64 * 64;
         while (n_lds > 0 && mega_per_cu(P->mega_fn_lds, static_cast<size_t>(n_lds) / 4) < per_cu)
@@ -1249,26 +1270,38 @@ void reserve_hints(Problem *P, size_t count) {
     P->d_hints = dev_alloc<int>(P->hints_cap, P->hint_owned);
 }
 
-// Makes (d_lbs, d_ubs) the reference of the problem's next loads: its
-// snapshot and its segment partials.
-void set_reference(Problem *P, const double *d_lbs, const double *d_ubs) {
+// Makes the bitwise majority of the n_vectors (at most 3) vectors at lbp, ubp
+// (device pointers) the reference of the problem's next loads, with its
+// snapshot and its segment partials.  Children of one node differ from it in
+// columns of their own, so the majority of three is mostly the parent.
+void set_reference(Problem *P, double *const *lbp, double *const *ubp, int n_vectors) {
     const DevMatrix &M = P->M;
-    if (!P->ref_block) check(cached_malloc(&P->ref_block, static_cast<size_t>(M.snap_stride)), "hipMalloc reference");
+    const size_t block = (static_cast<size_t>(M.snap_stride) + 255) / 256 * 256;
+    const size_t n = static_cast<size_t>(P->n);
+    if (!P->ref_block) check(cached_malloc(&P->ref_block, block + 2 * n * sizeof(double)), "hipMalloc reference");
     if (!P->ref_parts)
         check(cached_malloc(&P->ref_parts, sizeof(SegPart) * std::max(1, M.n_seg_parts)), "hipMalloc reference");
+    P->ref_lb = reinterpret_cast<double *>(P->ref_block + block);
+    P->ref_ub = P->ref_lb + n;
     DevState V{};
     V.S16 = reinterpret_cast<unsigned *>(P->ref_block);
     V.S32 = reinterpret_cast<int2 *>(P->ref_block + M.snap_off32);
     V.SF = reinterpret_cast<double2 *>(P->ref_block + M.snap_offF);
+    ReferenceVectors R{};
+    R.n = std::min(3, n_vectors);
+    for (int k = 0; k < R.n; k++) {
+        R.lb[k] = lbp[k];
+        R.ub[k] = ubp[k];
+    }
     hipLaunchKernelGGL(load_reference_kernel, dim3(std::max(1, std::min(1024, (M.n + 255) / 256))), dim3(256), 0,
-                       P->stream, M, V, d_lbs, d_ubs);
+                       P->stream, M, V, R, P->ref_lb, P->ref_ub);
     hipLaunchKernelGGL(reference_parts_kernel, dim3(std::max(1, std::min(2048, grid_for(M.n_seg_parts)))), dim3(256), 0,
                        P->stream, M, V, P->ref_parts);
     check(hipGetLastError(), "reference launch");
 }
 
 // The reference for a load of n_list units, its per-unit notes cleared.
-ReferenceView reference_view(Problem *P, int n_list, const double *d_lbs, const double *d_ubs, int start) {
+ReferenceView reference_view(Problem *P, int n_list, int start) {
     ReferenceView ref;
     const size_t notes = (static_cast<size_t>(n_list) * sizeof(int) + 255) / 256 * 256;
     if (n_list > P->ref_units) {
@@ -1284,8 +1317,8 @@ ReferenceView reference_view(Problem *P, int n_list, const double *d_lbs, const 
     ref.diff = reinterpret_cast<unsigned *>(P->ref_diff + notes);
     check(hipMemsetAsync(ref.n_diff, 0, sizeof(int) * n_list, P->stream), "memset reference");
     ref.parts = P->ref_parts;
-    ref.lbs = d_lbs;
-    ref.ubs = d_ubs;
+    ref.lbs = P->ref_lb;
+    ref.ubs = P->ref_ub;
     ref.start = start;
     return ref;
 }
@@ -1295,7 +1328,7 @@ ReferenceView reference_view(Problem *P, int n_list, const double *d_lbs, const 
 // (`fresh` false).
 void load_units(Problem *P, int n_list, const int *list, double *const *lbp, double *const *ubp,
                 const int *hint_ptr, const int *hints, const int *max_rounds, int start, bool fresh,
-                const double *ref_lb = nullptr, const double *ref_ub = nullptr) {
+                bool referenced = false) {
     hipStream_t s = P->stream;
     DevMatrix &M = P->M;
     DevState &D = P->D;
@@ -1320,9 +1353,9 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
     const int gy = P->replicas ? std::max(1, std::min(n_list, 1024)) : 1;
     ReferenceView ref;
-    if (ref_lb) ref = reference_view(P, n_list, ref_lb, ref_ub, start);
+    if (referenced) ref = reference_view(P, n_list, start);
     hipLaunchKernelGGL(load_kernel, dim3(gx, gy), dim3(256), 0, s, M, D, n_list, P->d_list, P->d_lbp, P->d_ubp, ref);
-    if (ref_lb) {
+    if (referenced) {
         // walking the columns of up to this many words costs less than an
         // eighth of the unit's segments
         const int limit = std::max(16, M.nwords / 64);
@@ -1331,6 +1364,14 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
     }
     check(hipGetLastError(), "load launch");
     if (hint_ptr != nullptr && M.mark_rows && hint_ptr[n_list] > 0) {
+        if (M.n_seg_parts > 0) {
+            // segments a wave looks at: few while the units are few
+            const int chunk = std::max(1, std::min(4, n_list / 16));
+            const long long wgs = static_cast<long long>((n_list + 7) / 8) * 8 *
+                                  ((M.n_seg_parts + 4 * chunk - 1) / (4 * chunk));
+            hipLaunchKernelGGL(fill_parts_kernel, dim3(static_cast<int>(std::min<long long>(wgs, 1 << 20))), dim3(256), 0,
+                               s, M, D, n_list, P->d_list, start, chunk);
+        }
         reserve_hints(P, hint_ptr[n_list]);
         upload(P->d_hint_ptr, hint_ptr, n_list + 1, s);
         upload(P->d_hints, hints, hint_ptr[n_list], s);
@@ -1349,7 +1390,8 @@ void launch_step(Problem *P, int step, int guard, int first_step) {
     const int apply_grid = std::max(1, std::min(1024, grid_for(static_cast<long long>(M.n_seg_parts) *
                                                                  (P->replicas ? D.n_active : 1))));
     const int sweep_grid = static_cast<int>(std::min<long long>(grid_for(n_work), P->sweep_grid));
-    hipLaunchKernelGGL(sweep_kernel, dim3(sweep_grid), dim3(256), 0, s, M, D, step, guard, first_step);
+    hipLaunchKernelGGL(sweep_kernel, dim3(sweep_grid), dim3(256), 0, s, M, D, step, guard, first_step,
+                       P->n_units);
     if (M.n_seg_parts > 0)
         hipLaunchKernelGGL(apply_split_kernel, dim3(apply_grid), dim3(256), 0, s, M, D, step, guard, first_step);
     const long long pub_waves = static_cast<long long>(P->replicas ? D.n_active : 1) * ((M.nwords + 7) / 8);
@@ -1436,10 +1478,10 @@ double run_steps(Problem *P, int sync_type, int max_rounds) {
         }
     } else {
         int first = 1, steps = max_rounds, n_units = P->n_units;
-        // dynamic LDS: the unit filter's arrays for several units, else the
+        // dynamic LDS: the sweep's window for several units, else the
         // binary columns' codes
         DevState Dm = D;
-        size_t lds_bytes = kFilterLdsBytes;
+        size_t lds_bytes = kWindowLdsBytes;
         const void *fn = P->mega_fn;
         if ((P->replicas ? D.n_active : n_units) == 1) {
             lds_bytes = static_cast<size_t>(P->n_lds) / 4;
@@ -1636,13 +1678,11 @@ void run_units(Problem *P, int n_list, const int *list, double *const *lbp, doub
     if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
     std::vector<int> caps(n_list, max_rounds);
     P->D.n_active = P->replicas ? n_list : 0;
-    // hinted vectors (children of propagated nodes) mostly agree with each
-    // other: the first one is the reference of all
+    // hinted vectors (children of propagated nodes) mostly agree with each other
     const bool related = P->replicas && n_list > 1 && P->M.n_seg_parts > 0 && P->M.mark_rows &&
                          hint_ptr != nullptr && hint_ptr[n_list] > 0;
-    if (related) set_reference(P, lbp[0], ubp[0]);
-    load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps.data(), 1, true, related ? lbp[0] : nullptr,
-               related ? ubp[0] : nullptr);
+    if (related) set_reference(P, lbp, ubp, n_list);
+    load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps.data(), 1, true, related);
     // bounds outside the envelope are an error before any round
     std::vector<UnitState> st = read_units(P, n_list, list);
     bool any_active = false;
@@ -1821,7 +1861,15 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
                 }
             };
             for (int r = 0; r < M.m; r++) {
-                if (!all_rows && marks[r] != step) continue;
+                if (!all_rows) {
+                    // a split row is processed when one of its segments is marked
+                    bool marked = marks[r] == step;
+                    if (split_of[r] >= 0) {
+                        const int4 sr = seg_rows[split_of[r]];
+                        marked = std::find(&seg_marks[sr.y], &seg_marks[sr.y] + sr.z, step) != &seg_marks[sr.y] + sr.z;
+                    }
+                    if (!marked) continue;
+                }
                 const int a = rp[r], b = rp[r + 1];
                 const int start = a & ~(kRowAlign - 1);
                 const int len = (b & ~(kRowAlign - 1)) - start - (a & (kRowAlign - 1));
@@ -2010,12 +2058,14 @@ class BorrowedState {
         : P_(P), D_(P->D), list_(P->d_list), params_(P->d_params), lbp_(P->d_lbp), ubp_(P->d_ubp),
           hint_ptr_(P->d_hint_ptr), capacity_(P->capacity), n_units_(P->n_units), graphs_(P->graphs_enabled),
           R_(P->R), rounds_state_(P->rounds_state) {
-        // the double-buffered rounds where their arrays fit too
+        // the lists of marked rows and the double-buffered rounds where their
+        // arrays fit too
         DevState D{};
         UnitTables T;
         RoundPlan R;
-        const size_t need = carve_state(P->M, P->replicas, P->n_inst, 1, nullptr, D, T);
-        bind_state(P, base, 1, P->rounds_ok && need + carve_rounds(P->Mr, nullptr, R) <= kScratchBytes);
+        const size_t need = carve_state(P->M, P->replicas, P->n_inst, 1, nullptr, D, T, true);
+        bind_state(P, base, 1, P->rounds_ok && need + carve_rounds(P->Mr, nullptr, R) <= kScratchBytes,
+                   need <= kScratchBytes);
         P->graphs_enabled = false;
     }
     ~BorrowedState() {
@@ -2028,6 +2078,7 @@ class BorrowedState {
         P_->capacity = capacity_;
         P_->n_units = n_units_;
         P_->graphs_enabled = graphs_;
+        P_->M.mark_rows = P_->tuning.row_marking ? 1 : 0;
         P_->R = R_;
         P_->rounds_state = rounds_state_;
     }
@@ -2051,7 +2102,7 @@ class BorrowedState {
 size_t problem_run_state_bytes(const Problem *P) {
     DevState D{};
     UnitTables T;
-    return carve_state(P->M, P->replicas, P->n_inst, 1, nullptr, D, T);
+    return carve_state(P->M, P->replicas, P->n_inst, 1, nullptr, D, T, false);
 }
 
 RunResult problem_propagate_no_alloc(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds) {
@@ -2161,7 +2212,7 @@ Tuning autotune(const std::vector<InstanceView> &instances, const double *lbs, c
             // the full-sweep threshold: the default and larger ones (marks
             // pushed in more rounds)
             const auto &v = instances[0];
-            const long long def = std::max(64LL, static_cast<long long>(v.m) * v.n / (4LL * std::max(1, v.nnz)));
+            const long long def = std::max(64LL, static_cast<long long>(v.m) * v.n / (8LL * std::max(1, v.nnz)));
             for (long long f : {4LL, 16LL}) {
                 Tuning t = best;
                 t.mark_limit = static_cast<int>(std::min(def * f, 1LL << 30));
@@ -2489,7 +2540,8 @@ void server_set_base(Server *S, const double *lbs, const double *ubs) {
     S->has_base = true;
     // requests mostly agree with the base: its segment partials are theirs
     if (S->P->M.n_seg_parts > 0 && S->P->M.mark_rows) {
-        set_reference(S->P, S->d_base, S->d_base + S->n);
+        double *lb = S->d_base, *ub = S->d_base + S->n;
+        set_reference(S->P, &lb, &ub, 1);
         check(hipStreamSynchronize(S->P->stream), "reference sync");
     }
 }
@@ -2886,7 +2938,7 @@ int step_impl(Server *S) {
     if (!adm.empty())
         load_units(P, static_cast<int>(adm.size()), adm.data(), adm_lb.data(), adm_ub.data(), hint_ptr.data(),
                    hints.data(), caps.data(), S->step, false,
-                   S->has_base && P->M.n_seg_parts > 0 && P->M.mark_rows ? S->d_base : nullptr, S->d_base + n);
+                   S->has_base && P->M.n_seg_parts > 0 && P->M.mark_rows);
     t_run = Clock::now();
     t_retire = t_run;
     // ---- every active slot advances one round ----

@@ -116,22 +116,24 @@ __device__ __forceinline__ void mem_wait() { __builtin_amdgcn_s_waitcnt(0); }
 //                   workgroups wrote the records and nothing is invalidated
 constexpr int kRecords = 0, kWide = 1, kWideCoherent = 2;
 
-// Byte offset of the record of internal column `id` in the unit's block.
+// Byte offset of the record of internal column `id` in the unit's block: the
+// record's size and the class's base picked by class, then one shift and add
+// (picking among the three finished offsets becomes branches).
 template <int kMode>
 __device__ __forceinline__ unsigned record_offset(const DevMatrix &M, int id) {
     const unsigned uid = static_cast<unsigned>(id);
+    const unsigned base32 = static_cast<unsigned>(M.snap_off32) - static_cast<unsigned>(M.n16) * 8u;
+    const unsigned baseF = static_cast<unsigned>(M.snap_offF) - static_cast<unsigned>(M.n_int) * 16u;
+    unsigned shift = id < M.n_int ? 3u : 4u;
+    unsigned base = id < M.n_int ? (kMode == kRecords ? base32 : 0u) : baseF;
     if constexpr (kMode == kRecords) {
-        const unsigned a16 = uid * 4u;
-        const unsigned a32 = uid * 8u + (static_cast<unsigned>(M.snap_off32) - static_cast<unsigned>(M.n16) * 8u);
-        const unsigned af = uid * 16u + (static_cast<unsigned>(M.snap_offF) - static_cast<unsigned>(M.n_int) * 16u);
-        return id < M.n16 ? a16 : (id < M.n_int ? a32 : af);
-    } else {
-        const unsigned af = uid * 16u + (static_cast<unsigned>(M.snap_offF) - static_cast<unsigned>(M.n_int) * 16u);
-        return id < M.n_int ? uid * 8u : af;
+        shift = id < M.n16 ? 2u : shift;
+        base = id < M.n16 ? 0u : base;
     }
+    return (uid << shift) + base;
 }
 
-// Dynamic LDS of the persistent kernel: the unit filter's arrays in a launch
+// Dynamic LDS of the persistent kernel: the sweep's window in a launch
 // of several units, else the 2-bit codes of the first D.n_lds binary columns
 // (other kernels run with D.n_lds = 0 and never touch it).
 extern __shared__ __align__(16) unsigned dyn_lds[];
@@ -386,6 +388,15 @@ __device__ __forceinline__ void row_extent(const DevMatrix &M, int r, int &start
     len = (b & ~(kRowAlign - 1)) - start - (a & (kRowAlign - 1));
 }
 
+// The lane's number, opaque to the optimizer: what is derived from it is
+// computed where it is used instead of being kept in registers across the
+// loops around (the sweep's registers decide its waves per SIMD).
+__device__ __forceinline__ int lane_here() {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
 // The values of a lane and of its partner in step h = 2^k of a butterfly whose
 // earlier steps ran (lanes of a group of h hold the same value): lane i ^ h,
 // or, where that is cheaper, another lane of the same partner group.  In
@@ -546,7 +557,7 @@ struct LaneEntries {
     // all lanes of a group return the same value.  Entries past the end of
     // the row hold zeros, which never replace the running value.
     __device__ __forceinline__ double eps_scan(int g, double run) const {
-        const int gbase = (threadIdx.x & 63) & ~(g - 1);
+        const int gbase = lane_here() & ~(g - 1);
         for (int j = 0; j < g; j++) {
 #pragma unroll
             for (int k = 0; k < K; k++) run = eps_max_step(run, __shfl(fabs(a[k]) * (u[k] - l[k]), gbase + j, 64));
@@ -622,19 +633,6 @@ __device__ __forceinline__ UnitStep unit_step(const DevMatrix &M, const DevState
     return r;
 }
 
-// Whether item b of a working unit (state V) has work in `step`: every item
-// when the unit processes all rows; otherwise a group item whose item mark,
-// or a seg / long item whose row mark, names the step.  Items still test
-// their rows one by one, so an item visited needlessly costs time, never a
-// different result.
-__device__ __forceinline__ bool item_has_work(const DevMatrix &M, const DevState &V, int b, int step,
-                                              bool all_rows) {
-    if (all_rows) return true;
-    const int row = M.item_row[b];
-    const int mark = row >= 0 ? coherent_load(&V.marks[row]) : coherent_load(&V.item_mark[b]);
-    return mark == step;
-}
-
 // Counts the wave's accepted candidates (`moved` per lane) of unit u in
 // `step` in one of the unit's kMoveLanes counters of the step (one
 // non-returning atomic per wave).  Whether the unit moved at all is recorded
@@ -660,14 +658,13 @@ __device__ __forceinline__ Sink make_sink(const DevState &V) {
 // sweep items
 // ---------------------------------------------------------------------------
 
-// Rows [first, first + nrows) of one tree-width bin: groups of 2^logg lanes,
-// K consecutive entries per lane.  Rows not marked for this step are
-// skipped (a pass with no marked row loads nothing).
+// Rows [first, first + nrows) of one tree-width bin, or the nrows rows listed
+// at list[first ..]: groups of 2^logg lanes, K consecutive entries per lane.
 template <int K, int kMode>
 __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int first, int nrows, int logg,
-                                          int step, bool all_rows) {
+                                          const int *list) {
     const DevState &V = S.V;
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_here();
     const int g = 1 << logg;
     const int gl = lane & (g - 1);
     const int per_pass = 64 >> logg;
@@ -675,9 +672,9 @@ __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int
     const int end = first + nrows;
     int moved = 0;
     for (int base = first; base < end; base += per_pass) {
-        const int r = base + (lane >> logg);
-        const bool take = r < end && (all_rows || V.marks[r] == step);
-        if (!__any(take)) continue;
+        int r = base + (lane >> logg);
+        const bool take = r < end;
+        if (list != nullptr && take) r = coherent_load(&list[r]);
         int start = 0, len = 0;
         double lhs = 0.0, rhs = 0.0;
         if (take) {
@@ -715,7 +712,7 @@ __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int
 __device__ __forceinline__ int long_item(const DevMatrix &M, const Sink &S, int r) {
     constexpr int K = kSegLen / 64;
     const DevState &V = S.V;
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_here();
     int start, len;
     row_extent(M, r, start, len);
     const double2 sd = M.sides[r];
@@ -750,7 +747,7 @@ __device__ __forceinline__ int long_item(const DevMatrix &M, const Sink &S, int 
 template <int kMode>
 __device__ __forceinline__ double split_eps_scan(const DevMatrix &M, const DevState &V, const int4 info, int start, int len) {
     constexpr int K = kSegLen / 64;
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_here();
     double run = 0.0;
     for (int b = 0; b < info.z; b += 64) {
         const int q = b + lane;
@@ -780,53 +777,47 @@ __device__ __forceinline__ void store_part(const DevState &V, int part, const La
     coherent_store_2i(&p->infs, E.infs, step);
 }
 
-// Segments [s, s + cnt) of split row lr (cnt <= kSegsPerItem) for unit u.
-// The wave reduces each kSegLen-entry segment like a kSegLen-wide group row,
-// stores the partials and counts them in; nobody waits.  The wave that
-// completes the row's count adds the partials in segment order and decides
-// the row gate; when it passes, the row's activity is stored and its
-// segments are queued for the apply phase that follows the sweep.
+// Reduces segment s of the split row (rows from `start`, `len` entries) whose
+// partials begin at part0 and stores the partial.
 template <int kMode>
-__device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, const DevState &V, int u, int lr, int s, int cnt,
-                         int *st, int step, bool all_rows, int unit_start) {
+__device__ __forceinline__ void segment_partial(const DevMatrix &M, const DevState &V, int part0, int s, int start,
+                                                int len, int step) {
     constexpr int K = kSegLen / 64;
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_here();
+    const int s0 = s * kSegLen;
+    LaneEntries<K, kMode> E;
+    E.load(M, V, start + s0, lane * K, len - s0);
+    E.template reduce<true>(64);
+    if (lane == 0) store_part(V, part0 + s, E, step);
+}
+
+// Segments [s, s + cnt) of split row lr (cnt <= kSegsPerItem; cnt < 0: the
+// one listed segment s of a step of marked rows) for unit u.  The wave
+// reduces each kSegLen-entry segment like a kSegLen-wide group row, stores
+// the partials and counts them in (a listed segment: off the segments that
+// the row has listed); nobody waits.  The wave that completes the row's count
+// adds the partials in segment order and decides the row gate; when it
+// passes, the row's activity is stored and its segments are queued for the
+// apply phase that follows the sweep.
+template <int kMode>
+__device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, const DevState &V, int u, int lr, int s,
+                                         int cnt, int *st, int step) {
+    const int lane = lane_here();
     const int4 info = M.seg_rows[lr];
     const int r = info.x;
     int start, len;
     row_extent(M, r, start, len);
-    // a segment computed earlier in this run none of whose columns moved in
-    // the previous step keeps its partial (its columns' bounds have not
-    // changed since it was computed: every change marks it); lane q reads
-    // segment q's stamp and mark
-    unsigned long long keep = 0ull;
-    if (!all_rows) {
-        bool kept = false;
-        if (lane < cnt) {
-            const int part = info.y + s + lane;
-            const int stamp = coherent_load(&V.seg_parts[part].stamp);
-            const int mark = coherent_load(&V.seg_marks[part]);
-            kept = stamp >= unit_start && mark != step;
-        }
-        keep = __ballot(kept);
-    }
-    for (int q = 0; q < cnt; q++) {
-        const int part = info.y + s + q;
-        if (!all_rows && ((keep >> q) & 1ull)) continue;
-        const int s0 = (s + q) * kSegLen;
-        LaneEntries<K, kMode> E;
-        E.load(M, V, start + s0, lane * K, len - s0);
-        E.template reduce<true>(64);
-        if (lane == 0) store_part(V, part, E, step);
-    }
+    const bool listed = cnt < 0;
+    const int end = s + (listed ? 1 : cnt);
+    for (int q = s; q < end; q++) segment_partial<kMode>(M, V, info.y, q, start, len, step);
     unsigned old = 0;
     if (lane == 0) {
         mem_wait();
-        old = __hip_atomic_fetch_add(&V.seg_count[lr], static_cast<unsigned>(cnt), __ATOMIC_RELAXED,
+        old = __hip_atomic_fetch_add(&V.seg_count[lr], static_cast<unsigned>(listed ? -1 : cnt), __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_AGENT);
     }
     old = __shfl(old, 0, 64);
-    if (old + cnt != static_cast<unsigned>(info.z)) return;
+    if (listed ? old != 1u : old + cnt != static_cast<unsigned>(info.z)) return;
 
     // the row is complete: the lanes load 64 partials at a time
     // (independent loads), which are then added in segment order
@@ -879,53 +870,254 @@ __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, 
     for (int q = lane; q < info.z; q += 64) coherent_store(&D.apply_tasks[pos + q], base + q);
 }
 
-// Unit and item of work index `it` (replicas: the launch's listed units,
-// n_items each; blocks: the item, whose unit it names).
-__device__ __forceinline__ void decode_work(const DevMatrix &M, const DevState &D, int it, int &u, int &b) {
-    if (M.replicas) {
-        const int k = it / M.n_items;
-        u = D.active[k];
-        b = it - k * M.n_items;
-    } else {
-        b = it;
-        u = M.items[b].x >> kItemUnitShift;
-    }
+// Lanes per row and entries per lane (log2) of a class of rows.
+__device__ __forceinline__ int class_logg(const DevMatrix &M, int c) {
+    return static_cast<int>(M.class_logg >> (4 * c)) & 15;
+}
+__device__ __forceinline__ int class_logk(const DevMatrix &M, int c) {
+    return static_cast<int>(M.class_logk >> (4 * c)) & 15;
 }
 
-// Sweep item `it` of `step` for a unit working in the step (us: its state):
-// skips unmarked rows, runs the item and records the unit's change.
-__device__ __forceinline__ void sweep_item(const DevMatrix &M, const DevState &D, int it, int step, int *st,
-                                           const UnitStep &us) {
-    int u, b;
-    decode_work(M, D, uniform(it), u, b);
+// The counters of unit u's lists for `step`, and the first place of class c's.
+__device__ __forceinline__ unsigned long long *list_counts(const DevState &D, int u, int step) {
+    return D.wl_cnt + (static_cast<size_t>(u) * 2 + (step & 1)) * kCountWords;
+}
+__device__ __forceinline__ int list_start(const DevMatrix &M, int u, int c) {
+    return M.list_at[(M.replicas ? 0 : u * kListStride) + c];
+}
+
+// Listed rows (class 0: segments) of unit u in `step`, lane c holding class
+// c's; the passes they take (segments and unsplit rows one each).
+__device__ __forceinline__ int listed_rows(const DevState &D, int u, int step) {
+    const int lane = lane_here();
+    if (lane >= kClasses) return 0;
+    const unsigned long long w = coherent_load(&list_counts(D, u, step)[lane >> 1]);
+    return static_cast<int>(lane & 1 ? w >> 32 : w & 0xffffffffull);
+}
+__device__ __forceinline__ int class_passes(const DevMatrix &M, int c, int rows) {
+    if (c < 2) return rows;
+    const int log_rows = 6 - class_logg(M, c);
+    return (rows + (1 << log_rows) - 1) >> log_rows;
+}
+// Passes of unit u's lists in `step`, by one lane.
+__device__ __forceinline__ int list_passes(const DevMatrix &M, const DevState &D, int u, int step) {
+    const unsigned long long *w = list_counts(D, u, step);
+    unsigned long long v[(kClasses + 1) / 2];
+#pragma unroll
+    for (int q = 0; q < (kClasses + 1) / 2; q++) v[q] = coherent_load(&w[q]);
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kClasses; c++)
+        n += class_passes(M, c, static_cast<int>(c & 1 ? v[c >> 1] >> 32 : v[c >> 1] & 0xffffffffull));
+    return n;
+}
+
+// Sweep items of unit u (a step of all rows).
+__device__ __forceinline__ int unit_items(const DevMatrix &M, int u) {
+    return M.replicas ? M.n_items : M.unit_item[u + 1] - M.unit_item[u];
+}
+
+// Piece `q` of the work of unit u in `step`: its q-th sweep item when every
+// row is processed, else the q-th pass of its lists (segments first, then
+// wide to narrow).  With 2^log_parts parts to an item, part `part` of it.
+// Records the unit's accepted candidates.
+__device__ __forceinline__ void sweep_piece(const DevMatrix &M, const DevState &D, int u, int q, bool all_rows,
+                                            int part, int log_parts, int step, int *st) {
     u = uniform(u);
-    b = uniform(b);
+    q = uniform(q);
     const DevState V = unit_view(M, D, u);
     const Sink S = make_sink(V);
-    int4 d = M.items[b];
-    d.x = uniform(d.x);
-    d.y = uniform(d.y);
-    d.z = uniform(d.z);
-    d.w = uniform(d.w);
-    const int kind = d.x & 15;
+    const int *list = nullptr;
+    int kind = kItemGroup, first = 0, n = 0, cnt = 0, logg = 0, logk = 0;
+    if (all_rows) {
+        const int4 d = M.items[(M.replicas ? 0 : uniform(M.unit_item[u])) + q];
+        kind = uniform(d.x) & 15;
+        logg = (uniform(d.x) >> 4) & 15;
+        logk = (uniform(d.x) >> 8) & 15;
+        first = uniform(d.y);
+        n = uniform(d.z);
+        cnt = uniform(d.w);
+        if (kind == kItemSeg) {
+            const int per = (cnt + (1 << log_parts) - 1) >> log_parts;
+            n += part * per;
+            cnt = min(per, cnt - part * per);
+            if (cnt <= 0) return;
+        } else if (kind == kItemGroup) {
+            const int log_unit = 6 - logg + log_parts;  // rows of one pass of every part
+            const int per = ((n + (1 << log_unit) - 1) >> log_unit) << (6 - logg);
+            first += part * per;
+            n = min(per, n - part * per);
+            if (n <= 0) return;
+        } else if (part > 0) {
+            return;
+        }
+    } else {
+        if (part > 0) return;  // a pass
+        const int lane = lane_here();
+        const int rows = listed_rows(D, u, step);
+        const int passes = lane < kClasses ? class_passes(M, lane, rows) : 0;
+        int upto = passes;  // inclusive running sum over the classes
+#pragma unroll
+        for (int h = 1; h < 16; h <<= 1) {
+            const int v = __shfl_up(upto, h, 64);
+            if (lane >= h) upto += v;
+        }
+        const unsigned long long above = __ballot(lane < kClasses && upto > q);
+        if (above == 0ull) return;
+        const int c = __ffsll(static_cast<long long>(above)) - 1;
+        const int at = q - (__shfl(upto, c, 64) - __shfl(passes, c, 64));
+        const int have = uniform(__shfl(rows, c, 64));
+        const int start = uniform(list_start(M, u, c));
+        if (c == 0) {
+            const int part = uniform(coherent_load(&V.wl_seg[start + at]));
+            kind = kItemSeg;
+            first = uniform(M.part_row[part]);
+            n = part - uniform(M.seg_rows[first].y);
+            cnt = -1;
+        } else if (c == 1) {
+            kind = kItemLong;
+            first = uniform(coherent_load(&V.wl[start + at]));
+        } else {
+            logg = class_logg(M, c);
+            logk = class_logk(M, c);
+            const int per_pass = 64 >> logg;
+            list = V.wl + start;
+            first = uniform(at * per_pass);
+            n = min(per_pass, have - first);
+        }
+    }
     int moved = 0;
     if (kind == kItemSeg) {
-        const int r = M.seg_rows[d.y].x;
-        if (us.all_rows || V.marks[r] == step) seg_item<kRecords>(M, D, V, u, d.y, d.z, d.w, st, step, us.all_rows, us.start);
+        seg_item<kRecords>(M, D, V, u, first, n, cnt, st, step);
         return;
     }
     if (kind == kItemLong) {
-        if (us.all_rows || V.marks[d.y] == step) moved = long_item(M, S, d.y);
+        moved = long_item(M, S, first);
     } else {
-        const int logg = (d.x >> 4) & 15;
-        const int logk = (d.x >> 8) & 15;
         switch (logk) {
-            case 0: moved = group_item<1, kRecords>(M, S, d.y, d.z, logg, step, us.all_rows); break;
-            case 1: moved = group_item<2, kRecords>(M, S, d.y, d.z, logg, step, us.all_rows); break;
-            default: moved = group_item<4, kRecords>(M, S, d.y, d.z, logg, step, us.all_rows); break;
+            case 0: moved = group_item<1, kRecords>(M, S, first, n, logg, list); break;
+            case 1: moved = group_item<2, kRecords>(M, S, first, n, logg, list); break;
+            default: moved = group_item<4, kRecords>(M, S, first, n, logg, list); break;
         }
     }
     note_change(D, u, step, moved);
+}
+
+// Running sums of the pieces of `win` units, slots (base + k) * groups + mine,
+// and their all-rows bits, in LDS (the whole workgroup).
+__device__ __forceinline__ void lay_out_window(const DevMatrix &M, const DevState &D, int step, int base, int win,
+                                               int mine, int groups, int *sums, unsigned *dense) {
+    const int lane = threadIdx.x & 63;
+    const int wg_wave = threadIdx.x >> 6;
+    __syncthreads();  // nobody still reads the previous window
+    for (int g = wg_wave * 64; g < win; g += blockDim.x) {
+        const int k = g + lane;
+        int n = 0;
+        UnitStep us{};
+        if (k < win) {
+            const int slot = (base + k) * groups + mine;
+            const int u = M.replicas ? D.active[slot] : slot;
+            us = unit_step_lane(M, D, u, step);
+            if (us.active) n = us.all_rows ? unit_items(M, u) : list_passes(M, D, u, step);
+        }
+        const unsigned long long b = __ballot(us.all_rows);
+        if (lane == 0) {
+            dense[g >> 5] = static_cast<unsigned>(b);
+            dense[(g >> 5) + 1] = static_cast<unsigned>(b >> 32);
+        }
+        sums[k] = n;
+    }
+    __syncthreads();
+    if (wg_wave == 0) {
+        int carry = 0;
+        for (int g = 0; g < win; g += 64) {
+            int v = sums[g + lane];
+#pragma unroll
+            for (int h = 1; h < 64; h <<= 1) {
+                const int o = __shfl_up(v, h, 64);
+                if (lane >= h) v += o;
+            }
+            sums[g + lane] = v + carry;
+            carry += __shfl(v, 63, 64);
+        }
+    }
+    __syncthreads();
+}
+
+// The sweep of a step over the waves of the grid: the pieces of every working
+// unit, one unit after the other, dealt out with the grid's stride.  With
+// several units, each workgroup lays out the running sums of their pieces in
+// LDS (`window`, kWindowLdsBytes) for up to kWindowUnits of them at a time;
+// a wave then finds its piece's unit with two ballots.  Also clears the
+// counters of the lists that the step's publish will fill.
+__device__ __forceinline__ void sweep_phase(const DevMatrix &M, const DevState &D, int step, int wave, int nwaves,
+                                            int n_units, unsigned *window, const UnitStep &one) {
+    int *st = status_row(D, step);
+    const int n_slots = M.replicas ? D.n_active : n_units;
+    if (M.mark_rows) {
+        const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+        for (int k = tid; k < n_slots * kCountWords; k += gridDim.x * blockDim.x) {
+            const int slot = k / kCountWords;
+            const int u = M.replicas ? D.active[slot] : slot;
+            coherent_store(&list_counts(D, u, step + 1)[k - slot * kCountWords], 0ull);
+        }
+    }
+    const bool single = n_slots == 1;
+    if (single && !one.active) return;
+    const int u1 = M.replicas ? uniform(D.active[0]) : 0;
+    int *sums = reinterpret_cast<int *>(window);            // kWindowUnits + 64
+    unsigned *dense = window + kWindowUnits + 64;           // all-rows bits
+    // Many bound vectors of one matrix: every workgroup works on the vectors
+    // of its own XCD (workgroups go round the 8 XCDs), slots x, x + 8, ...,
+    // so that an L2 holds the snapshots of an eighth of the vectors in work.
+    // Only the locality hangs on where a workgroup really runs.
+    const int groups = M.replicas && n_slots >= 64 && gridDim.x % 8 == 0 ? 8 : 1;
+    const int mine = groups == 8 ? blockIdx.x & 7 : 0;
+    if (groups == 8) {
+        const int waves = blockDim.x >> 6;
+        wave = uniform((blockIdx.x >> 3) * waves + (threadIdx.x >> 6));
+        nwaves = (gridDim.x >> 3) * waves;
+    }
+    const int own = (n_slots - mine + groups - 1) / groups;  // slots of this group
+    int shift = 0;  // pieces of the windows before
+    for (int base = 0; base < own; base += kWindowUnits) {
+        const int win = min(kWindowUnits, own - base);
+        const int blocks = (win + 63) / 64;
+        int total;
+        if (single) {
+            total = one.all_rows ? unit_items(M, u1) : uniform(list_passes(M, D, u1, step));
+        } else {
+            lay_out_window(M, D, step, base, win, mine, groups, sums, dense);
+            total = uniform(sums[blocks * 64 - 1]);
+        }
+        // items in up to 4 parts while the waves outnumber them: an item is
+        // four passes or more, a chain of about 4 us each
+        const int log_parts = total * 4 <= nwaves ? 2 : (total * 2 <= nwaves ? 1 : 0);
+        // the grid's stride goes on across the windows
+        int q = (wave - shift) % nwaves;
+        if (q < 0) q += nwaves;
+        for (; q < total << log_parts; q += nwaves) {
+            const int piece = q >> log_parts;
+            int u = u1, before = 0;
+            bool all_rows = one.all_rows;
+            if (!single) {
+                const int lane = lane_here();
+                int blk = 0;
+                if (blocks > 1)
+                    blk = uniform(__ffsll(static_cast<long long>(__ballot(
+                                      lane < blocks && sums[min(lane, blocks - 1) * 64 + 63] > piece))) - 1);
+                const int upto = sums[blk * 64 + lane];
+                const int k = uniform(__ffsll(static_cast<long long>(__ballot(upto > piece))) - 1);
+                before = uniform(k == 0 ? (blk == 0 ? 0 : sums[blk * 64 - 1]) : __shfl(upto, k - 1, 64));
+                const int at = blk * 64 + k;
+                const int slot = (base + at) * groups + mine;
+                u = M.replicas ? uniform(D.active[slot]) : slot;
+                all_rows = uniform((dense[at >> 5] >> (at & 31)) & 1u) != 0;
+            }
+            sweep_piece(M, D, u, piece - before, all_rows, q & ((1 << log_parts) - 1), log_parts, step, st);
+        }
+        shift = (shift + (total << log_parts)) % nwaves;
+    }
 }
 
 // Applies the candidates of queued task `task` = unit * n_seg_parts + segment
@@ -1005,6 +1197,69 @@ __device__ __forceinline__ bool decide_all_rows(const DevMatrix &M, const DevSta
     return valid && M.mark_rows && cnt >= limit;
 }
 
+// Marks column-to-row entries, N per lane (row[q], and its col_seg code, where
+// valid[q]), for `step` of unit u, the same unit on the lanes of each half of
+// the wave: the first to mark a row (a segment of a split row) lists it.  The
+// entries take their ranks within the half and class in LDS, and the places
+// of all classes in the unit's lists come from one atomic instruction (two
+// classes a word, six lanes) per N entries a lane: the counters of a unit lie
+// in one line, and every addition to it by a wave costs tens of nanoseconds.
+template <int N>
+__device__ __forceinline__ void mark_entries(const DevMatrix &M, const DevState &V, int u, const bool (&valid)[N],
+                                             const int (&row)[N], const int (&code)[N], int step) {
+    __shared__ unsigned ranks[16][2][16];  // per wave and half: rows per class, then their first places
+    const int lane = lane_here();
+    const int b = lane & 31;
+    unsigned *mine = ranks[threadIdx.x >> 6][lane >> 5];
+    bool first[N], any = false;
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        first[q] = false;
+        if (valid[q]) {
+            int *mark = code[q] >= 0 ? &V.seg_marks[code[q]] : &V.marks[row[q]];
+            first[q] = __hip_atomic_exchange(mark, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != step;
+        }
+        any |= first[q];
+    }
+    if (!__any(any)) return;
+    if (b < 16) mine[b] = 0u;
+    __builtin_amdgcn_wave_barrier();
+    unsigned rank[N];
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        rank[q] = 0u;
+        if (first[q])
+            rank[q] = __hip_atomic_fetch_add(&mine[code[q] >= 0 ? 0 : -1 - code[q]], 1u, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (b < (kClasses + 1) / 2) {
+        const unsigned n0 = __hip_atomic_load(&mine[2 * b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const unsigned n1 = __hip_atomic_load(&mine[2 * b + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if ((n0 | n1) != 0u) {
+            const unsigned long long old =
+                __hip_atomic_fetch_add(&list_counts(V, u, step)[b], n0 | (static_cast<unsigned long long>(n1) << 32),
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            mine[2 * b] = static_cast<unsigned>(list_start(M, u, 2 * b)) + static_cast<unsigned>(old);
+            mine[2 * b + 1] = static_cast<unsigned>(list_start(M, u, 2 * b + 1)) + static_cast<unsigned>(old >> 32);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        if (!first[q]) continue;
+        if (code[q] >= 0) {
+            coherent_store(&V.wl_seg[__hip_atomic_load(&mine[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + rank[q]],
+                           code[q]);
+            atomic_add_i(reinterpret_cast<int *>(&V.seg_count[M.part_row[code[q]]]), 1);
+        } else {
+            const unsigned at = __hip_atomic_load(&mine[-1 - code[q]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            coherent_store(&V.wl[at + rank[q]], row[q]);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ void publish_word(const DevMatrix &M, const DevState &D, int u, int w, unsigned bits,
                                              bool valid, int step, int all_rows_known) {
     const int lane = threadIdx.x & 63;
@@ -1032,12 +1287,13 @@ __device__ __forceinline__ void publish_word(const DevMatrix &M, const DevState 
         for (int h = 1; h < 16; h <<= 1) cw |= static_cast<unsigned>(__shfl_xor(static_cast<int>(cw), h, 64));
         if ((b & 15) == 0 && cw != 0u) atomic_or_u(&V.SB[id >> 4], cw);
     }
-    if (!M.mark_rows || !valid || all_rows) return;
+    const bool marks = M.mark_rows && valid && !all_rows;
+    if (!__any(marks)) return;
     // rows of the moved columns, flattened over the 32 lanes of the half:
     // exclusive prefix of the columns' lengths, then lane i marks entries
     // i, i + 32, ... found by a binary search over the prefix
-    const int c0 = moved ? M.col_ptr[id] : 0;
-    const int cn = moved ? M.col_ptr[id + 1] - c0 : 0;
+    const int c0 = moved && marks ? M.col_ptr[id] : 0;
+    const int cn = moved && marks ? M.col_ptr[id + 1] - c0 : 0;
     int pre = cn;
 #pragma unroll
     for (int d = 1; d < 32; d <<= 1) {
@@ -1045,12 +1301,14 @@ __device__ __forceinline__ void publish_word(const DevMatrix &M, const DevState 
         if (b >= d) pre += v;
     }
     const int total = __shfl(pre, 31, 32);
+    const int longest = max(total, __shfl_xor(total, 32, 64));  // of both halves, which go together
     pre -= cn;  // exclusive
     // kMarkBatch entries per lane at a time: their index loads are all issued
     // before the marks they name are stored
     constexpr int kMarkBatch = 4;
-    for (int base = 0; base < total; base += 32 * kMarkBatch) {  // same trip count on every lane of the half
-        int row[kMarkBatch], sp[kMarkBatch], ci[kMarkBatch];
+    for (int base = 0; base < longest; base += 32 * kMarkBatch) {
+        int row[kMarkBatch], sp[kMarkBatch];
+        bool in[kMarkBatch];
 #pragma unroll
         for (int q = 0; q < kMarkBatch; q++) {
             const int i = base + q * 32 + b;
@@ -1061,21 +1319,15 @@ __device__ __forceinline__ void publish_word(const DevMatrix &M, const DevState 
                 if (cand < 32 && __shfl(pre, cand, 32) <= i) lo = cand;
             }
             const int k = __shfl(c0, lo, 32) + i - __shfl(pre, lo, 32);
-            row[q] = -1;
+            row[q] = 0;
             sp[q] = -1;
-            ci[q] = -1;
-            if (i < total) {
+            in[q] = i < total;
+            if (in[q]) {
                 row[q] = M.col_rows[k];
                 sp[q] = M.col_seg[k];
-                ci[q] = M.col_item[k];
             }
         }
-#pragma unroll
-        for (int q = 0; q < kMarkBatch; q++) {
-            if (row[q] >= 0) coherent_store(&V.marks[row[q]], step + 1);
-            if (sp[q] >= 0) coherent_store(&V.seg_marks[sp[q]], step + 1);
-            if (ci[q] >= 0) coherent_store(&V.item_mark[ci[q]], step + 1);
-        }
+        mark_entries(M, V, u, in, row, sp, step + 1);
     }
 }
 
@@ -1229,41 +1481,19 @@ __device__ __forceinline__ bool step_skipped(const DevState &D, int step, int fi
     return coherent_load(&status_row(D, step - 1)[kStatusChanged]) == 0;
 }
 
-// The sweep of one step over a grid sized to the device (grid stride): each
-// wave tests 64 of its work items at once (one lane each: the unit's state
-// and the item's mark) and visits those with work, as the persistent kernel
-// does.  Many units' items then cost a few loads each instead of a wave.
+// The sweep of one step over a grid sized to the device.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void sweep_kernel(
-    DevMatrix M, DevState D_arg, int step, int guard, int first_step) {
-    // no LDS in the step kernels (a constant, so that the LDS reads compile out)
+    DevMatrix M, DevState D_arg, int step, int guard, int first_step, int n_units) {
+    // no LDS codes in the step kernels (a constant, so that the LDS reads compile out)
     DevState D = D_arg;
     D.n_lds = 0;
+    __shared__ unsigned window[kWindowLdsBytes / 4];
     if (guard && step_skipped(D, step, first_step)) return;
     const int waves = blockDim.x >> 6;
     const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));
-    const int nwaves = gridDim.x * waves;
-    const int n_work = M.replicas ? M.n_items * D.n_active : M.n_items;
-    const int lane = threadIdx.x & 63;
-    int *st = status_row(D, step);
-    for (int base = wave; base < n_work; base += 64 * nwaves) {
-        const int it = base + lane * nwaves;
-        bool on = false;
-        if (it < n_work) {
-            int u, b;
-            decode_work(M, D, it, u, b);
-            const UnitStep us = unit_step_lane(M, D, u, step);
-            on = us.active && item_has_work(M, unit_view(M, D, u), b, step, us.all_rows);
-        }
-        unsigned long long pending = __ballot(on);
-        while (pending) {
-            const int t = __ffsll(static_cast<long long>(pending)) - 1;
-            pending &= pending - 1;
-            const int itt = uniform(base + t * nwaves);
-            int uu, bb;
-            decode_work(M, D, itt, uu, bb);
-            sweep_item(M, D, itt, step, st, unit_step(M, D, uu, step));
-        }
-    }
+    UnitStep one{};
+    if ((M.replicas ? D.n_active : n_units) == 1) one = unit_step(M, D, M.replicas ? D.active[0] : 0, step);
+    sweep_phase(M, D, step, wave, gridDim.x * waves, n_units, window, one);
 }
 
 __global__ __launch_bounds__(256) void apply_split_kernel(DevMatrix M, DevState D_arg, int step, int guard,
@@ -1275,7 +1505,7 @@ __global__ __launch_bounds__(256) void apply_split_kernel(DevMatrix M, DevState 
     apply_phase(M, D, step, uniform(blockIdx.x * waves + (threadIdx.x >> 6)), gridDim.x * waves);
 }
 
-__global__ __launch_bounds__(256) void publish_kernel(DevMatrix M, DevState D_arg, int step, int guard,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void publish_kernel(DevMatrix M, DevState D_arg, int step, int guard,
                                                       int first_step, int n_units) {
     DevState D = D_arg;
     D.n_lds = 0;
@@ -1363,21 +1593,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const int waves = blockDim.x >> 6;
     const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));
     const int nwaves = gridDim.x * waves;
-    const int n_work = M.replicas ? M.n_items * D.n_active : M.n_items;
-    // Several units: at the start of a step every workgroup notes in LDS
-    // which units work in it, which of them process all rows, and their
-    // first steps (the state words do not change during the sweep), so that
-    // an item's unit costs no device-coherent loads.  One unit: every wave
-    // reads its state once per step.  Then each wave tests 64 of its items at
-    // once (lanes): items of idle units, and items none of whose rows are
-    // marked when their unit processes marked rows only, are not visited.
-    // (in the dynamic LDS, kFilterLdsBytes of it in launches of several units)
-    unsigned *works = dyn_lds;
-    unsigned *all_rows_of = dyn_lds + kMaxFilterUnits / 32;
-    int *start_of = reinterpret_cast<int *>(dyn_lds + 2 * (kMaxFilterUnits / 32));
     const int n_slots = M.replicas ? D.n_active : n_units;  // replicas: positions in the launch's list
-    const bool filter = n_slots > 1 && n_slots <= kMaxFilterUnits;
-    const int lane = threadIdx.x & 63;
     int steps = 0;
     for (int step = first_step; step < first_step + max_steps; step++) {
         int *st = status_row(D, step);
@@ -1394,68 +1610,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 for (int i = threadIdx.x; i < D.n_lds / 64; i += blockDim.x) dst[i] = src[i];
                 __syncthreads();
             }
-        } else if (filter) {
-            // the previous step's waves of this workgroup are past its
-            // barriers, so no wave still reads the entries overwritten here
-            for (int g = (threadIdx.x >> 6) * 64; g < n_slots; g += blockDim.x) {
-                const int k = g + lane;
-                UnitStep us{};
-                if (k < n_slots) us = unit_step_lane(M, D, M.replicas ? D.active[k] : k, step);
-                const unsigned long long bw = __ballot(k < n_slots && us.active);
-                const unsigned long long ba = __ballot(k < n_slots && us.all_rows);
-                if (lane == 0) {
-                    works[g >> 5] = static_cast<unsigned>(bw);
-                    works[(g >> 5) + 1] = static_cast<unsigned>(bw >> 32);
-                    all_rows_of[g >> 5] = static_cast<unsigned>(ba);
-                    all_rows_of[(g >> 5) + 1] = static_cast<unsigned>(ba >> 32);
-                }
-                if (k < n_slots) start_of[k] = us.start;
-            }
-            __syncthreads();
         }
-        // the wave's items in the order wave, wave + nwaves, ...: 64 at a time
-        if (n_slots != 1 || one.active) {
-            for (int base = wave; base < n_work; base += 64 * nwaves) {
-                const int it = base + lane * nwaves;
-                bool on = it < n_work;
-                int u = 0, b = 0;
-                UnitStep us = one;
-                if (on) {
-                    decode_work(M, D, it, u, b);
-                    if (filter) {
-                        const int k = M.replicas ? it / M.n_items : u;
-                        us.active = (works[k >> 5] >> (k & 31)) & 1u;
-                        us.all_rows = (all_rows_of[k >> 5] >> (k & 31)) & 1u;
-                        us.start = start_of[k];
-                    } else if (n_slots != 1) {
-                        us = unit_step_lane(M, D, u, step);
-                    }
-                    on = us.active && item_has_work(M, unit_view(M, D, u), b, step, us.all_rows);
-                }
-                unsigned long long pending = __ballot(on);
-                while (pending) {
-                    const int t = __ffsll(static_cast<long long>(pending)) - 1;
-                    pending &= pending - 1;
-                    // the picked item's unit state again, wave-uniform (no
-                    // per-lane state stays live across the item)
-                    const int itt = uniform(base + t * nwaves);
-                    UnitStep ut = one;
-                    if (n_slots != 1) {
-                        int uu, bb;
-                        decode_work(M, D, itt, uu, bb);
-                        if (filter) {
-                            const int k = uniform(M.replicas ? itt / M.n_items : uu);
-                            ut.active = true;
-                            ut.all_rows = (all_rows_of[k >> 5] >> (k & 31)) & 1u;
-                            ut.start = start_of[k];
-                        } else {
-                            ut = unit_step(M, D, uu, step);
-                        }
-                    }
-                    sweep_item(M, D, itt, step, st, ut);
-                }
-            }
-        }
+        sweep_phase(M, D, step, wave, nwaves, n_units, dyn_lds, one);
         if (!grid_barrier(D, nblocks, false)) { steps = -1; break; }
         if (coherent_load(&st[kStatusApply]) > 0) {
             apply_phase(M, D, step, wave, nwaves);
@@ -1584,15 +1740,15 @@ __device__ __forceinline__ int round_item(const DevMatrix &M, const DevState &V,
     d.y = uniform(d.y);
     d.z = uniform(d.z);
     if ((d.x & 15) == kItemSeg) {
-        seg_item<kMode>(M, V, V, 0, d.y, d.z, 1, st, step, true, 1);
+        seg_item<kMode>(M, V, V, 0, d.y, d.z, 1, st, step);
         return 0;
     }
     const int logg = (d.x >> 4) & 15;
     const Sink S = make_sink(V);
     switch ((d.x >> 8) & 15) {
-        case 0: return group_item<1, kMode>(M, S, d.y, d.z, logg, step, true);
-        case 1: return group_item<2, kMode>(M, S, d.y, d.z, logg, step, true);
-        default: return group_item<4, kMode>(M, S, d.y, d.z, logg, step, true);
+        case 0: return group_item<1, kMode>(M, S, d.y, d.z, logg, nullptr);
+        case 1: return group_item<2, kMode>(M, S, d.y, d.z, logg, nullptr);
+        default: return group_item<4, kMode>(M, S, d.y, d.z, logg, nullptr);
     }
 }
 
@@ -1879,6 +2035,8 @@ __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, in
         D.units[q.x] = s;
         for (int sl = 0; sl < kMoveSlots; sl++)
             for (int j = 0; j < kMoveLanes; j++) D.moved[moved_index(q.x, sl, j)] = 0;
+        if (D.wl_cnt != nullptr)
+            for (int j = 0; j < 2 * kCountWords; j++) D.wl_cnt[static_cast<size_t>(q.x) * 2 * kCountWords + j] = 0ull;
     }
     if (clear_status) {
         for (int k = tid; k < kStatusRows * kStatusWords; k += stride) D.status[k] = 0;
@@ -1960,7 +2118,6 @@ __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int 
         {
             for (int w = tid; w < M.nwords; w += stride) V.bm[w] = 0u;
             for (int r = tid; r < M.m; r += stride) V.marks[r] = 0;
-            for (int q = tid; q < M.n_items; q += stride) V.item_mark[q] = 0;
             for (int q = tid; q < M.n_seg_rows; q += stride) V.seg_count[q] = 0u;
             // segment marks too: their step stamps would otherwise match a
             // step of this run (steps restart with every run) and make it
@@ -1979,14 +2136,28 @@ __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int 
     }
 }
 
-// The snapshot block of a reference vector (records as load_kernel writes
+// The bitwise majority of up to three vectors (the first one where all
+// differ), column by column: a lower and an upper bound of one vector or of
+// two, whichever.  Any mixture is a valid reference.
+__device__ __forceinline__ double majority(double a, double b, double c) {
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b), z = __double_as_longlong(c);
+    return x != y && y == z ? b : a;
+}
+
+// The reference vector and its snapshot block (records as load_kernel writes
 // them).  Values outside a column's class leave a wrong record: a unit with
 // the same value there is refused, one with another drops the segment.
-__global__ __launch_bounds__(256) void load_reference_kernel(DevMatrix M, DevState V, const double *lbs,
-                                                             const double *ubs) {
+__global__ __launch_bounds__(256) void load_reference_kernel(DevMatrix M, DevState V, ReferenceVectors R, double *lbs,
+                                                             double *ubs) {
     for (int id = blockIdx.x * blockDim.x + threadIdx.x; id < M.n; id += gridDim.x * blockDim.x) {
         const int j = M.perm[id];
-        const double l = lbs[j], u = ubs[j];
+        double l = R.lb[0][j], u = R.ub[0][j];
+        if (R.n == 3) {
+            l = majority(l, R.lb[1][j], R.lb[2][j]);
+            u = majority(u, R.ub[1][j], R.ub[2][j]);
+        }
+        lbs[j] = l;
+        ubs[j] = u;
         if (id < M.n_int) {
             const bool fits = fits_int32(l) && fits_int32(u);
             const int il = fits ? static_cast<int>(l) : 0, iu = fits ? static_cast<int>(u) : 0;
@@ -2062,6 +2233,41 @@ __global__ __launch_bounds__(256) void drop_parts_kernel(DevMatrix M, DevState D
     }
 }
 
+// Computes the segment partials that hinted units do not have yet (no
+// reference, or dropped): a step of marked rows recomputes only listed
+// segments.  Each wave looks at `chunk` segments of a unit; units that process
+// every row in their first step compute theirs there.
+__global__ __launch_bounds__(256) void fill_parts_kernel(DevMatrix M, DevState D_arg, int n_list, const int *list,
+                                                         int start_step, int chunk) {
+    DevState D = D_arg;
+    D.n_lds = 0;
+    const int lane = threadIdx.x & 63;
+    // workgroups go round the 8 XCDs: a unit's keep to one, unit after unit, so
+    // that an L2 holds the snapshots in work
+    const int wg_parts = (blockDim.x >> 6) * chunk;
+    const int per_unit = (M.n_seg_parts + wg_parts - 1) / wg_parts;
+    const int xcd = blockIdx.x & 7, on_xcd = (n_list - xcd + 7) / 8;
+    for (int j = blockIdx.x >> 3; j < on_xcd * per_unit; j += gridDim.x >> 3) {
+        const int k = j / per_unit * 8 + xcd;
+        const int u = uniform(list[k]);
+        if (coherent_load(&D.units[u].markall) == start_step) continue;
+        const DevState V = unit_view(M, D, u);
+        {
+            const int p0 = uniform((j % per_unit) * wg_parts + (threadIdx.x >> 6) * chunk);
+            const int p = p0 + lane;
+            unsigned long long todo = __ballot(lane < chunk && p < M.n_seg_parts && V.seg_parts[p].stamp == 0);
+            while (todo) {
+                const int part = uniform(p0 + __ffsll(static_cast<long long>(todo)) - 1);
+                todo &= todo - 1;
+                const int4 info = M.seg_rows[M.part_row[part]];
+                int start, len;
+                row_extent(M, info.x, start, len);
+                segment_partial<kRecords>(M, V, info.y, part - info.y, start, len, start_step);
+            }
+        }
+    }
+}
+
 // Marks the rows of hinted columns (caller's column indices; unit k's hints
 // at hints[hint_ptr[k] .. hint_ptr[k + 1])) for the listed units' first step:
 // the bound vector differs from a propagated fixpoint only in these columns.
@@ -2071,14 +2277,19 @@ __global__ __launch_bounds__(256) void hint_kernel(DevMatrix M, DevState D, int 
     // a wave per hinted column, its lanes over the column's entries
     const int lane = threadIdx.x & 63;
     const int waves = gridDim.x * (blockDim.x >> 6);
-    const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int wave = uniform(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     for (int k = blockIdx.y; k < n_list; k += gridDim.y) {
-        const DevState V = unit_view(M, D, list[k]);
+        const int u = uniform(list[k]);
+        const DevState V = unit_view(M, D, u);
         for (int h = hint_ptr[k] + wave; h < hint_ptr[k + 1]; h += waves) {
             const int id = inv_perm[hints[h]];
-            for (int q = M.col_ptr[id] + lane; q < M.col_ptr[id + 1]; q += 64) {
-                V.marks[M.col_rows[q]] = start_step;
-                if (M.col_item[q] >= 0) V.item_mark[M.col_item[q]] = start_step;
+            const int end = M.col_ptr[id + 1];
+            for (int q0 = M.col_ptr[id]; q0 < end; q0 += 64) {
+                const int q = q0 + lane;
+                const bool in[1] = {q < end};
+                const int row[1] = {in[0] ? M.col_rows[q] : 0};
+                const int code[1] = {in[0] ? M.col_seg[q] : -1};
+                mark_entries(M, V, u, in, row, code, start_step);
             }
         }
     }
@@ -2312,13 +2523,19 @@ __global__ __launch_bounds__(256) void layout_rows_kernel(int mp, const long lon
 }
 
 // Column-to-row index: every entry of layout row r appends r to its column's
-// list (fill[] starts at col_ptr[]), for split rows (row_part[r] >= 0) the
-// entry's segment, and the group item holding the row (row_item[r], -1 for
-// split and long rows).  The order inside a column's list is not fixed; the
-// lists are used as sets (row, segment and item marking).  One wave per row.
+// list (fill[] starts at col_ptr[]) and, for split rows (row_part[r] >= 0),
+// the entry's segment, else -1 - the row's class.  The order inside a
+// column's list is not fixed; the lists are used as sets (marking).  One wave
+// per row.
+__device__ __forceinline__ int row_code(int len) {
+    if (len > kSegLen) return -2;  // class 1
+    const int log_width = len <= 1 ? 0 : 32 - __clz(len - 1);
+    return -1 - (10 - log_width);
+}
+
 __global__ __launch_bounds__(256) void layout_csc_kernel(int mp, const int *row_ptr_out, const int *col_out,
-                                                         const int *row_part, const int *row_item, int *fill,
-                                                         int *col_rows, int *col_seg, int *col_item) {
+                                                         const int *row_part, int *fill, int *col_rows,
+                                                         int *col_seg) {
     const int lane = threadIdx.x & 63;
     const int waves = gridDim.x * (blockDim.x >> 6);
     for (int r = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); r < mp; r += waves) {
@@ -2326,13 +2543,11 @@ __global__ __launch_bounds__(256) void layout_csc_kernel(int mp, const int *row_
         const int st = a & ~(kRowAlign - 1);
         const int len = (b & ~(kRowAlign - 1)) - st - (a & (kRowAlign - 1));
         const int part = row_part[r];
-        const int item = row_item[r];
         for (int e = lane; e < len; e += 64) {
             const int id = col_out[st + e] & kIdMask;
             const int slot = atomic_add_i(&fill[id], 1);
             col_rows[slot] = r;
-            col_seg[slot] = part >= 0 ? part + e / kSegLen : -1;
-            col_item[slot] = item;
+            col_seg[slot] = part >= 0 ? part + e / kSegLen : row_code(len);
         }
     }
 }
@@ -2408,25 +2623,23 @@ __global__ __launch_bounds__(256) void layout_rows_short_kernel(int r_begin, int
     }
 }
 
-// Column-to-row index entries of the short rows (never split: segment -1).
+// Column-to-row index entries of the short rows (never split).
 __global__ __launch_bounds__(256) void layout_csc_short_kernel(int r_begin, int mp, const int *row_ptr_out,
-                                                               const int *col_out, const int *row_item, int *fill,
-                                                               int *col_rows, int *col_seg, int *col_item) {
+                                                               const int *col_out, int *fill, int *col_rows,
+                                                               int *col_seg) {
     const int lane = threadIdx.x & 63;
     const int waves = gridDim.x * (blockDim.x >> 6);
     for (int r0 = r_begin + 64 * (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)); r0 < mp; r0 += 64 * waves) {
         const ShortRows R = short_rows(r0, mp, row_ptr_out, nullptr, nullptr);
-        const int item = row_item[r0 + min(lane, R.nrows - 1)];
         for (int base = R.S0; base < R.S1; base += 64) {
             const int e = base + lane;
             const int j = short_row_of(R, e);
-            const int rs = __shfl(R.st, j, 64), rl = __shfl(R.len, j, 64), it = __shfl(item, j, 64);
+            const int rs = __shfl(R.st, j, 64), rl = __shfl(R.len, j, 64);
             if (e >= R.S1 || e - rs >= rl) continue;
             const int id = col_out[e] & kIdMask;
             const int slot = atomic_add_i(&fill[id], 1);
             col_rows[slot] = r0 + j;
-            col_seg[slot] = -1;
-            col_item[slot] = it;
+            col_seg[slot] = row_code(rl);
         }
     }
 }

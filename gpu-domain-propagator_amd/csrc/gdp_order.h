@@ -38,9 +38,8 @@ void order_exclusive_sum(const int *in, int *out, int n, hipStream_t s);
 // row_ptr[r] |= plen[r] - len[r] for r < mp (the padding count).
 void order_pad_rows(int mp, const int *len, const int *plen, int *row_ptr, hipStream_t s);
 
-// row_item[r] = group item of layout row r; row_part[seg_rows[k].x] =
-// seg_rows[k].y.  Entries not written keep their values (the caller sets -1).
-void order_row_tables(int n_items, const int4 *items, int n_seg_rows, const int4 *seg_rows, int *row_item,
-                      int *row_part, hipStream_t s);
+// row_part[seg_rows[k].x] = seg_rows[k].y.  Entries not written keep their
+// values (the caller sets -1).
+void order_row_tables(int n_seg_rows, const int4 *seg_rows, int *row_part, hipStream_t s);
 
 }  // namespace gdp

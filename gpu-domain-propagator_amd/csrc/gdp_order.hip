@@ -113,18 +113,9 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(int mp, const int *len, c
         row_ptr[r] |= plen[r] - len[r];
 }
 
-// row_item[r] = the group item holding layout row r; row_part[r] = the first
-// segment of split row r.  Both start at -1 (set by the caller).  One wave
-// per item, then one thread per split row.
-__global__ __launch_bounds__(256) void row_tables_kernel(int n_items, const int4 *items, int n_seg_rows,
-                                                         const int4 *seg_rows, int *row_item, int *row_part) {
-    const int lane = threadIdx.x & 63;
-    const int waves = gridDim.x * (blockDim.x >> 6);
-    for (int q = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); q < n_items; q += waves) {
-        const int4 it = items[q];
-        if ((it.x & 15) != kItemGroup) continue;
-        for (int t = lane; t < it.z; t += 64) row_item[it.y + t] = q;
-    }
+// row_part[r] = the first segment of split row r (the others start at -1, set
+// by the caller).
+__global__ __launch_bounds__(256) void row_tables_kernel(int n_seg_rows, const int4 *seg_rows, int *row_part) {
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n_seg_rows; k += gridDim.x * blockDim.x)
         row_part[seg_rows[k].x] = seg_rows[k].y;
 }
@@ -333,11 +324,10 @@ void order_pad_rows(int mp, const int *len, const int *plen, int *row_ptr, hipSt
     check_order(hipGetLastError(), "pad rows launch");
 }
 
-void order_row_tables(int n_items, const int4 *items, int n_seg_rows, const int4 *seg_rows, int *row_item,
-                      int *row_part, hipStream_t s) {
-    const int grid = std::max(1, std::min(4096, std::max((n_items + 3) / 4, (n_seg_rows + 255) / 256)));
-    hipLaunchKernelGGL(row_tables_kernel, dim3(grid), dim3(256), 0, s, n_items, items, n_seg_rows, seg_rows,
-                       row_item, row_part);
+void order_row_tables(int n_seg_rows, const int4 *seg_rows, int *row_part, hipStream_t s) {
+    if (n_seg_rows < 1) return;
+    const int grid = std::max(1, std::min(1024, (n_seg_rows + 255) / 256));
+    hipLaunchKernelGGL(row_tables_kernel, dim3(grid), dim3(256), 0, s, n_seg_rows, seg_rows, row_part);
     check_order(hipGetLastError(), "row tables launch");
 }
 
