@@ -110,6 +110,7 @@ constexpr int kStatusApply = 2;    // split-row segments queued for the apply ph
 constexpr int kGlobalError = 0;    // a bounded device wait timed out
 constexpr int kGlobalSteps = 1;    // steps run by the persistent kernel
 constexpr int kGlobalTicket = 2;   // workgroups of unpack_rounds_kernel that are done
+constexpr int kGlobalEnvelope = 3; // some loaded vector left the envelope (runs that then return an error)
 constexpr int kGlobalWords = 8;
 
 // State of one unit (int32 words, read as 64-bit pairs).  A step's changes
@@ -141,6 +142,9 @@ constexpr int kMoveStride = 32;
 __host__ __device__ inline int moved_index(int u, int slot, int j) {
     return ((u * kMoveSlots + slot) * kMoveLanes + j) * kMoveStride;
 }
+
+// Progress word of launches that stop themselves: no further step runs.
+constexpr int kRoundsOver = 0x40000000;
 
 // Grid barrier words, each counter on its own 128-byte line.
 constexpr int kBarrierTop = 0;
@@ -229,6 +233,7 @@ struct DevState {
     int n_active;
     int n_lds;             // binary columns read from LDS (persistent launch of one unit; else 0)
     unsigned *SB;          // 2-bit codes of the binary columns (sb_words per unit)
+    int *host_word;        // pinned: the step that the guarded launches have started, or kRoundsOver
 };
 
 // A vector that the units of a launch mostly agree with (the base of a
@@ -263,7 +268,6 @@ struct ReferenceVectors {
 // snap_offF (the DevMatrix of these kernels has n16 = 0, snap_off32 = 0).
 constexpr int kPlanBins = 9;          // tree widths 2^8 .. 2^0
 constexpr int kMaxGatherBlocks = 512; // workgroups of the persistent launch
-constexpr int kRoundsOver = 0x40000000;  // host word: no further round runs
 // Where each tree-width bin's rows and items start (building the item list).
 struct RoundBins {
     int n_segs;
@@ -282,7 +286,6 @@ struct RoundPlan {
     unsigned long long *slots;        // arrivals of the persistent launch's barrier, two sets
     double *lbs, *ubs;                // the caller's vectors
     int mark_limit, max_rounds;
-    int *host_word;                   // pinned: progress of the launches (see round_kernel)
     UnitState *host_state;            // pinned: the outcome
 };
 

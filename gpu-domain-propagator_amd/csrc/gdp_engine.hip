@@ -62,7 +62,10 @@ __global__ void drop_parts_kernel(DevMatrix M, DevState D, int n_list, const int
 __global__ void hint_kernel(DevMatrix M, DevState D, int n_list, const int *list, const int *hint_ptr,
                             const int *hints, const int *inv_perm, int start_step);
 __global__ void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list, double *const *lbp,
-                              double *const *ubp);
+                              double *const *ubp, int checked);
+__global__ void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int *list, double **lbp,
+                                 double **ubp, double *lbs, double *ubs);
+__global__ void report_kernel(DevState D, int n_list, const int *list, UnitState *out);
 __global__ void delta_kernel(int n_list, double *const *lbp, double *const *ubp, const int *ptr, const int *cols,
                              const double *lv, const double *uv);
 __global__ void copy_pairs_kernel(long long n2, int count, double *const *ptrs);
@@ -106,23 +109,28 @@ T *dev_alloc(size_t count, std::vector<void *> &owned) {
 
 // Copies of 1 MiB and more from pageable host memory (the caller's arrays): the runtime
 // would stage them through its own pinned buffers, copying on one thread.
-// Here several threads copy each 32 MiB chunk into one of two pinned staging
+// Here several threads copy each chunk into one of two pinned staging
 // buffers while the DMA engine drains the other.  One copy at a time uses
 // them, and without them the copy is left to the runtime.  Returns when
 // every copy out of them has completed.
 //
-// Lifetime: the buffers (64 MiB of pinned memory) and the copy threads exist
-// while at least one problem does.  The first bulk copy creates them, and
-// the destruction of the last problem joins the threads and frees the
-// buffers, so nothing of them is left for the runtime's (or a profiler's)
-// teardown at process exit.
-constexpr size_t kStageChunk = 32u << 20;
+// Lifetime: the first bulk copy creates the buffers and the copy threads.
+// Copies below 64 MiB take buffers of 8 MiB, which stay with the threads for
+// the next problem (a stateless call creates and destroys its problem, and
+// paid 1.5 ms of allocating, freeing and joining each time); buffers of 32 MiB
+// go back when the last problem is destroyed.
+constexpr size_t kStageSmall = 8u << 20;
+constexpr size_t kStageLarge = 32u << 20;
 constexpr size_t kBulkMin = 1u << 20;
+// Bound vectors (both) of up to this size cross through a pinned block of the
+// problem's own instead of the shared staging.
+constexpr size_t kSmallBounds = 256u << 10;
 
 class Staging {
   public:
     std::mutex use;  // held for a whole bulk copy
     char *buf[2] = {nullptr, nullptr};
+    size_t chunk = 0;  // bytes of each
 
     // A problem starts / ends using the staging.
     void acquire() {
@@ -132,21 +140,22 @@ class Staging {
     void release() {
         std::lock_guard<std::mutex> use_lk(use);
         std::lock_guard<std::mutex> lk(life_);
-        if (--users_ > 0) return;
-        pool_.stop();
-        for (char *&b : buf) {
-            if (b) (void)hipHostFree(b);
-            b = nullptr;
-        }
+        if (--users_ > 0 || chunk <= kStageSmall) return;
+        drop();
     }
-    // With `use` held: whether both buffers exist (allocated here).
-    bool ready() {
+    // With `use` held: whether both buffers exist, large enough for a copy of
+    // `bytes` (allocated here).
+    bool ready(size_t bytes) {
+        const size_t want = bytes >= (64u << 20) ? kStageLarge : kStageSmall;
+        if (chunk < want) drop();
         for (char *&b : buf)
-            if (!b && hipHostMalloc(reinterpret_cast<void **>(&b), kStageChunk, hipHostMallocDefault) != hipSuccess) {
+            if (!b && hipHostMalloc(reinterpret_cast<void **>(&b), want, hipHostMallocPortable) != hipSuccess) {
                 b = nullptr;
                 (void)hipGetLastError();
+                drop();
                 return false;
             }
+        chunk = std::max(chunk, want);
         return true;
     }
     // With `use` held: copies `bytes` from src to dst with the copy threads.
@@ -168,6 +177,13 @@ class Staging {
     }
 
   private:
+    void drop() {
+        for (char *&b : buf) {
+            if (b) (void)hipHostFree(b);
+            b = nullptr;
+        }
+        chunk = 0;
+    }
     std::mutex life_;
     int users_ = 0;
     CopyPool pool_;
@@ -181,11 +197,12 @@ Staging &staging() {
 void upload_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
     Staging &st = staging();
     std::lock_guard<std::mutex> lock(st.use);
-    if (!st.ready()) {  // no pinned memory to spare: the runtime's own staged copy
+    if (!st.ready(bytes)) {  // no pinned memory to spare: the runtime's own staged copy
         check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s), "H2D");
         return;
     }
     char *const *buf = st.buf;
+    const size_t chunk = st.chunk;
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool used[2] = {false, false};
     auto release = [&]() {
@@ -197,8 +214,8 @@ void upload_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
     try {
         for (hipEvent_t &e : ev) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
         int k = 0;
-        for (size_t off = 0; off < bytes; off += kStageChunk, k ^= 1) {
-            const size_t len = std::min(kStageChunk, bytes - off);
+        for (size_t off = 0; off < bytes; off += chunk, k ^= 1) {
+            const size_t len = std::min(chunk, bytes - off);
             if (used[k]) check(hipEventSynchronize(ev[k]), "staging wait");  // its previous chunk has left
             st.copy(buf[k], static_cast<const char *>(src) + off, len);
             check(hipMemcpyAsync(static_cast<char *>(dst) + off, buf[k], len, hipMemcpyHostToDevice, s), "H2D");
@@ -218,12 +235,13 @@ void upload_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
 void download_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
     Staging &st = staging();
     std::lock_guard<std::mutex> lock(st.use);
-    if (!st.ready()) {
+    if (!st.ready(bytes)) {
         check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s), "D2H");
         check(hipStreamSynchronize(s), "D2H");
         return;
     }
     char *const *buf = st.buf;
+    const size_t chunk = st.chunk;
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool used[2] = {false, false};
     auto release = [&]() {
@@ -238,8 +256,8 @@ void download_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
         size_t prev_off = 0, prev_len = 0;
         int k = 0;
         // a buffer is filled again only after its previous chunk was copied out
-        for (size_t off = 0; off < bytes; off += kStageChunk, k ^= 1) {
-            const size_t len = std::min(kStageChunk, bytes - off);
+        for (size_t off = 0; off < bytes; off += chunk, k ^= 1) {
+            const size_t len = std::min(chunk, bytes - off);
             check(hipMemcpyAsync(buf[k], static_cast<const char *>(src) + off, len, hipMemcpyDeviceToHost, s), "D2H");
             check(hipEventRecord(ev[k], s), "event");
             used[k] = true;
@@ -322,6 +340,68 @@ HostSlots &host_slots() {
     static HostSlots *h = new HostSlots();  // outlives every problem
     return *h;
 }
+
+// Pinned host blocks for launch tables, outcomes and small bound vectors, by
+// powers of two from 4 KiB.  Freed blocks of up to 1 MiB are kept for the next
+// request, 16 MiB in all; the others go back to the runtime.
+class HostBlocks {
+  public:
+    void *take(size_t bytes, size_t *size) {
+        *size = 4096;
+        while (*size < bytes) *size *= 2;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            auto it = free_.find(*size);
+            if (it != free_.end() && !it->second.empty()) {
+                void *p = it->second.back();
+                it->second.pop_back();
+                kept_ -= *size;
+                return p;
+            }
+        }
+        void *p = nullptr;
+        check(hipHostMalloc(&p, *size, hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
+        return p;
+    }
+    void give(void *p, size_t size) {
+        if (!p) return;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (size <= (1u << 20) && kept_ + size <= (16u << 20)) {
+                free_[size].push_back(p);
+                kept_ += size;
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+
+  private:
+    std::mutex mu_;
+    std::unordered_map<size_t, std::vector<void *>> free_;
+    size_t kept_ = 0;
+};
+
+HostBlocks &host_blocks() {
+    static HostBlocks *h = new HostBlocks();  // outlives every problem
+    return *h;
+}
+
+// A pinned block of at least the bytes last asked for.
+struct HostBlock {
+    char *p = nullptr;
+    size_t size = 0;
+    char *get(size_t bytes) {
+        if (bytes > size) {
+            host_blocks().give(p, size);
+            p = nullptr;
+            size = 0;
+            p = static_cast<char *>(host_blocks().take(bytes, &size));
+        }
+        return p;
+    }
+    ~HostBlock() { host_blocks().give(p, size); }
+};
 
 // Phase times of a problem's creation, printed to stderr when the
 // environment variable GDP_TRACE_CREATE is set (a diagnostic of where the
@@ -463,7 +543,6 @@ struct Problem {
     const void *mega_fn_lds = nullptr;  // the same reading binary columns from LDS (one unit)
     // captured GPU_LOOP graphs, one per chunk of steps, for one launch shape
     std::vector<hipGraphExec_t> graphs;
-    std::vector<int> graph_last;
     long long graph_key = -1;
     std::mutex run_mutex;
     // double-buffered rounds (one bound vector; gdp_device.h, RoundPlan)
@@ -473,6 +552,8 @@ struct Problem {
     bool rounds_state = false;        // R's arrays are in the current run state
     int rounds_grid = 0, rounds_threads = 0;  // persistent launch
     HostSlot *host = nullptr;
+    HostBlock h_tables;               // pinned: launch tables of several units, then their outcomes
+    HostBlock h_bounds;               // pinned: small bound vectors on their way
     int servers = 0;                  // servers attached (they own the unit slots)
     bool graphs_enabled = true;       // GPU_LOOP may capture graphs of the current run state
     bool staging_held = false;
@@ -481,7 +562,6 @@ struct Problem {
         for (auto g : graphs)
             if (g) (void)hipGraphExecDestroy(g);
         graphs.clear();
-        graph_last.clear();
         graph_key = -1;
     }
 
@@ -589,6 +669,7 @@ void bind_state(Problem *P, char *base, int cap, bool rounds, bool lists = true)
     P->d_lbp = T.lbp;
     P->d_ubp = T.ubp;
     P->d_hint_ptr = T.hint_ptr;
+    P->D.host_word = P->host ? &P->host->word : nullptr;
     P->capacity = cap;
     P->n_units = P->replicas ? cap : P->n_inst;
 }
@@ -852,7 +933,7 @@ void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
     // phases: 1.3 persistent, 2.4 in the host loop).  3.1M nonzeros over 500,000
     // columns, 65 rounds: 2.4 ms (2.4 / 5.9).  19.3M nonzeros: 4.8 ms (3.1).
     constexpr int kMaxRoundEntries = 4 << 20;
-    if (!P->replicas || P->n_inst != 1 || n_padded > kMaxRoundEntries) return;
+    if (!P->replicas || P->n_inst != 1 || n_padded > (std::getenv("GDP_RMAX") ? std::atoi(std::getenv("GDP_RMAX")) : kMaxRoundEntries)) return;
     if (T.item_nnz != def.item_nnz || T.mega_blocks_per_cu != def.mega_blocks_per_cu ||
         T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
         !std::equal(T.group_log, T.group_log + 10, def.group_log))
@@ -895,7 +976,6 @@ void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
     M.snap_off32 = 0;
     M.snap_offF = (M.n_int * 8 + 15) / 16 * 16;
     M.snap_stride = M.snap_offF + 16LL * (M.n - M.n_int) + 16;
-    P->host = host_slots().take();
     int per_cu = 0;
     // at most 256 workgroups while the items allow it: the barrier grows with
     // them (1.2 us for 16, 3 us for 256, 4.3 us for 512), and a workgroup of 256
@@ -1218,6 +1298,7 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
             P->stats.n_units = replicas ? 0 : NI;
         }
 
+        P->host = host_slots().take();
         plan_rounds(P, R.start.data(), R.count.data(), n_padded);
 
         P->mega_threads = T.mega_threads == 256 || T.mega_threads == 1024 ? T.mega_threads : 512;
@@ -1332,24 +1413,30 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
     hipStream_t s = P->stream;
     DevMatrix &M = P->M;
     DevState &D = P->D;
-    // a few units' parameters on the stack: a single-vector run touches no heap
-    int4 few[8];
-    std::vector<int4> many;
-    if (n_list > 8) many.resize(n_list);
-    int4 *params = n_list > 8 ? many.data() : few;
-    for (int k = 0; k < n_list; k++) {
+    auto param = [&](int k) {
         const int u = list[k];
         const bool hinted = hint_ptr != nullptr && hint_ptr[k + 1] > hint_ptr[k] && M.mark_rows;
-        const int limit = P->mark_limit[P->replicas ? 0 : u];
-        params[k] = make_int4(u, limit, hinted ? 0 : 1, max_rounds[k]);
+        return make_int4(u, P->mark_limit[P->replicas ? 0 : u], hinted ? 0 : 1, max_rounds[k]);
+    };
+    if (n_list == 1) {
+        // a single vector: everything by kernel argument
+        hipLaunchKernelGGL(reset_one_kernel, dim3(1), dim3(256), 0, s, D, param(0), start, fresh ? 1 : 0, P->d_list,
+                           P->d_lbp, P->d_ubp, lbp[0], ubp[0]);
+    } else {
+        // the tables lie one after the other in the run state: one copy
+        const int n_tables = P->replicas ? n_list : 1;
+        char *const base = reinterpret_cast<char *>(P->d_list);
+        const size_t bytes = reinterpret_cast<char *>(P->d_ubp + n_tables) - base;
+        char *h = P->h_tables.get(bytes);
+        auto at = [&](const void *d) { return h + (static_cast<const char *>(d) - base); };
+        std::memcpy(h, list, sizeof(int) * n_list);
+        for (int k = 0; k < n_list; k++) reinterpret_cast<int4 *>(at(P->d_params))[k] = param(k);
+        std::memcpy(at(P->d_lbp), lbp, sizeof(double *) * n_tables);
+        std::memcpy(at(P->d_ubp), ubp, sizeof(double *) * n_tables);
+        check(hipMemcpyAsync(base, h, bytes, hipMemcpyHostToDevice, s), "H2D tables");
+        hipLaunchKernelGGL(unit_reset_kernel, dim3(std::max(1, std::min(64, (n_list + 255) / 256))), dim3(256), 0, s, D,
+                           n_list, P->d_params, start, fresh ? 1 : 0);
     }
-    upload(P->d_list, list, n_list, s);
-    upload(P->d_params, params, n_list, s);
-    const int n_tables = P->replicas ? n_list : 1;
-    upload(P->d_lbp, lbp, n_tables, s);
-    upload(P->d_ubp, ubp, n_tables, s);
-    hipLaunchKernelGGL(unit_reset_kernel, dim3(std::max(1, std::min(64, (n_list + 255) / 256))), dim3(256), 0, s, D,
-                       n_list, P->d_params, start, fresh ? 1 : 0);
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
     const int gy = P->replicas ? std::max(1, std::min(n_list, 1024)) : 1;
     ReferenceView ref;
@@ -1399,83 +1486,78 @@ void launch_step(Problem *P, int step, int guard, int first_step) {
                        step, guard, first_step, P->n_units);
 }
 
-// Runs steps 1.. for the listed units (loaded), at most max_rounds steps.
-// Returns the device time of the step loop.
-double run_steps(Problem *P, int sync_type, int max_rounds) {
+// Waits until the launches have started step `step` or are over; returns the
+// progress word.
+int wait_round(Problem *P, int step) {
+    const int *word = &P->host->word;
+    for (unsigned spins = 1;; spins++) {
+        const int w = __atomic_load_n(word, __ATOMIC_RELAXED);
+        if (w >= step) return w;
+        __builtin_ia32_pause();
+        if (spins % 8192 == 0) {
+            // an idle stream whose launches never got there, or a failed one
+            const hipError_t e = hipStreamQuery(P->stream);
+            if (e == hipErrorNotReady) continue;
+            check(e, "step launches");
+            const int end = __atomic_load_n(word, __ATOMIC_RELAXED);
+            if (end >= step) return end;
+            throw std::runtime_error("the step launches ended early");
+        }
+    }
+}
+
+// Steps that the launch loops run ahead of the host's look at the progress.
+constexpr int kAhead = 2;
+
+// Steps 1 .. max_rounds as captured graphs of graph_rounds steps (the launches
+// of one step by `launch`), kept for calls of the same key.  The next graph is
+// launched while the last steps of the previous one run.
+void run_graphs(Problem *P, long long key, int max_rounds, const std::function<void(int)> &launch) {
+    hipStream_t s = P->stream;
+    const int chunk = std::max(1, P->tuning.graph_rounds);
+    if (key != P->graph_key) {
+        P->drop_graphs();
+        P->graph_key = key;
+    }
+    for (int first = 1, ci = 0; first <= max_rounds; first += chunk, ci++) {
+        const int last = std::min(max_rounds, first + chunk - 1);
+        if (static_cast<int>(P->graphs.size()) <= ci) P->graphs.resize(ci + 1, nullptr);
+        if (!P->graphs[ci]) {
+            hipGraph_t graph;
+            check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture");
+            for (int step = first; step <= last; step++) launch(step);
+            check(hipStreamEndCapture(s, &graph), "end capture");
+            hipGraphExec_t exec;
+            check(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "instantiate");
+            (void)hipGraphDestroy(graph);
+            P->graphs[ci] = exec;
+        }
+        check(hipGraphLaunch(P->graphs[ci], s), "graph launch");
+        if (last < max_rounds && wait_round(P, std::max(first, last - 1)) == kRoundsOver) break;
+    }
+}
+
+// Issues steps 1.. for the listed units (loaded), at most max_rounds steps,
+// between the problem's two events.
+void run_steps(Problem *P, int sync_type, int max_rounds) {
     const DevMatrix &M = P->M;
     DevState &D = P->D;
     hipStream_t s = P->stream;
     check(hipEventRecord(P->ev0, s), "event");
-    if (sync_type == CPU_LOOP_ID) {
-        // one set of launches per step; the host reads the step's flags back
+    __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
+    if (sync_type == CPU_LOOP_ID || (sync_type == GPU_LOOP_ID && !P->graphs_enabled)) {
+        // one set of launches per step, which stop themselves once the run is
+        // over; they run ahead of the host's look at the progress by kAhead
+        // steps, so that the device never waits for it (without graphs, e.g.
+        // where nothing may be allocated, GPU_LOOP is the same)
         for (int step = 1; step <= max_rounds; step++) {
-            launch_step(P, step, 0, 1);
-            check(hipGetLastError(), "step launch");
-            int flags[kStatusWords];
-            int err = 0;
-            check(hipMemcpyAsync(flags, D.status + kStatusWords * (step % kStatusRows), sizeof(flags),
-                                 hipMemcpyDeviceToHost, s),
-                  "flags D2H");
-            check(hipMemcpyAsync(&err, D.global + kGlobalError, sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
-            check(hipStreamSynchronize(s), "step sync");
-            if (err) throw std::runtime_error("device wait timed out");
-            if (!flags[kStatusChanged]) break;
+            launch_step(P, step, 1, 1);
+            if (step > kAhead && wait_round(P, step - kAhead) == kRoundsOver) break;
         }
-    } else if (sync_type == GPU_LOOP_ID && !P->graphs_enabled) {
-        // the same chunks of self-stopping launches, issued without capture
-        // (no graph is created, so nothing is allocated)
-        const int chunk = std::max(1, P->tuning.graph_rounds);
-        for (int first = 1; first <= max_rounds; first += chunk) {
-            const int last = std::min(max_rounds, first + chunk - 1);
-            for (int step = first; step <= last; step++) launch_step(P, step, 1, 1);
-            check(hipGetLastError(), "step launch");
-            int flags[kStatusWords];
-            int err = 0;
-            check(hipMemcpyAsync(flags, D.status + kStatusWords * (last % kStatusRows), sizeof(flags),
-                                 hipMemcpyDeviceToHost, s),
-                  "flags D2H");
-            check(hipMemcpyAsync(&err, D.global + kGlobalError, sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
-            check(hipStreamSynchronize(s), "step sync");
-            if (err) throw std::runtime_error("device wait timed out");
-            if (!flags[kStatusChanged]) break;
-        }
+        check(hipGetLastError(), "step launch");
     } else if (sync_type == GPU_LOOP_ID) {
-        // captured chunks of steps whose launches stop themselves on the device
-        const int chunk = std::max(1, P->tuning.graph_rounds);
         const long long key = static_cast<long long>(D.n_active) * 1000 + max_rounds;
-        if (key != P->graph_key) {
-            P->drop_graphs();
-            P->graph_key = key;
-        }
-        for (int first = 1, ci = 0; first <= max_rounds; first += chunk, ci++) {
-            const int last = std::min(max_rounds, first + chunk - 1);
-            if (static_cast<int>(P->graphs.size()) <= ci) {
-                P->graphs.resize(ci + 1, nullptr);
-                P->graph_last.resize(ci + 1, 0);
-            }
-            if (!P->graphs[ci]) {
-                hipGraph_t graph;
-                check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture");
-                for (int step = first; step <= last; step++) launch_step(P, step, 1, 1);
-                check(hipStreamEndCapture(s, &graph), "end capture");
-                hipGraphExec_t exec;
-                check(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "instantiate");
-                (void)hipGraphDestroy(graph);
-                P->graphs[ci] = exec;
-                P->graph_last[ci] = last;
-            }
-            check(hipGraphLaunch(P->graphs[ci], s), "graph launch");
-            int flags[kStatusWords];
-            int err = 0;
-            check(hipMemcpyAsync(flags, D.status + kStatusWords * (last % kStatusRows), sizeof(flags),
-                                 hipMemcpyDeviceToHost, s),
-                  "flags D2H");
-            check(hipMemcpyAsync(&err, D.global + kGlobalError, sizeof(int), hipMemcpyDeviceToHost, s), "D2H");
-            check(hipStreamSynchronize(s), "graph sync");
-            if (err) throw std::runtime_error("device wait timed out");
-            // the next chunk is needed only if the chunk's last step still changed
-            if (!flags[kStatusChanged]) break;
-        }
+        run_graphs(P, key, max_rounds, [&](int step) { launch_step(P, step, 1, 1); });
     } else {
         int first = 1, steps = max_rounds, n_units = P->n_units;
         // dynamic LDS: the sweep's window for several units, else the
@@ -1502,16 +1584,8 @@ double run_steps(Problem *P, int sync_type, int max_rounds) {
             std::max(1LL, std::min<long long>(P->mega_grid, (need + waves_per_group - 1) / waves_per_group)));
         check(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(P->mega_threads), args, lds_bytes, s),
               "mega_kernel launch");
-        int g[kGlobalWords];
-        check(hipMemcpyAsync(g, D.global, sizeof(g), hipMemcpyDeviceToHost, s), "D2H");
-        check(hipStreamSynchronize(s), "mega sync");
-        if (g[kGlobalError] || g[kGlobalSteps] < 0) throw std::runtime_error("device wait timed out");
     }
     check(hipEventRecord(P->ev1, s), "event");
-    check(hipEventSynchronize(P->ev1), "event sync");
-    float ms = 0.f;
-    check(hipEventElapsedTime(&ms, P->ev0, P->ev1), "elapsed");
-    return ms;
 }
 
 std::vector<UnitState> read_units(Problem *P, int n_list, const int *list) {
@@ -1524,35 +1598,7 @@ std::vector<UnitState> read_units(Problem *P, int n_list, const int *list) {
     return out;
 }
 
-// State words of unit u (synchronous).
-UnitState read_unit(Problem *P, int u) {
-    UnitState st;
-    check(hipMemcpyAsync(&st, P->D.units + u, sizeof(UnitState), hipMemcpyDeviceToHost, P->stream), "unit D2H");
-    check(hipStreamSynchronize(P->stream), "unit sync");
-    return st;
-}
-
 // ---- double-buffered rounds of one bound vector ----
-
-// Waits until the launches have started round `step` or are over; returns
-// the progress word.
-int wait_round(Problem *P, int step) {
-    const int *word = &P->host->word;
-    for (unsigned spins = 1;; spins++) {
-        const int w = __atomic_load_n(word, __ATOMIC_RELAXED);
-        if (w >= step) return w;
-        __builtin_ia32_pause();
-        if (spins % 8192 == 0) {
-            // an idle stream whose launches never got there, or a failed one
-            const hipError_t e = hipStreamQuery(P->stream);
-            if (e == hipErrorNotReady) continue;
-            check(e, "round launches");
-            const int end = __atomic_load_n(word, __ATOMIC_RELAXED);
-            if (end >= step) return end;
-            throw std::runtime_error("the round launches ended early");
-        }
-    }
-}
 
 // Issues round `step`.
 void launch_round(Problem *P, int step) {
@@ -1563,29 +1609,9 @@ void launch_round(Problem *P, int step) {
                            dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
 }
 
-// Rounds 1 .. max_rounds, each one launch (two with split rows) that stops
-// itself on the device once the run is over; `first` .. `last` of them as one
-// captured graph.
-void launch_round_graph(Problem *P, int ci, int first, int last) {
-    hipStream_t s = P->stream;
-    if (static_cast<int>(P->graphs.size()) <= ci) {
-        P->graphs.resize(ci + 1, nullptr);
-        P->graph_last.resize(ci + 1, 0);
-    }
-    if (!P->graphs[ci]) {
-        hipGraph_t graph;
-        check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture");
-        for (int step = first; step <= last; step++) launch_round(P, step);
-        check(hipStreamEndCapture(s, &graph), "end capture");
-        hipGraphExec_t exec;
-        check(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "instantiate");
-        (void)hipGraphDestroy(graph);
-        P->graphs[ci] = exec;
-        P->graph_last[ci] = last;
-    }
-    check(hipGraphLaunch(P->graphs[ci], s), "graph launch");
-}
-
+// A complete run of one bound vector, each round one launch (two with split
+// rows) that stops itself on the device once the run is over, or all rounds
+// one persistent launch.
 RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds) {
     hipStream_t s = P->stream;
     RoundPlan &R = P->R;
@@ -1594,7 +1620,6 @@ RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, in
     R.ubs = d_ubs;
     R.max_rounds = max_rounds;
     R.mark_limit = P->mark_limit[0];
-    R.host_word = &P->host->word;
     R.host_state = &P->host->state;
     __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
@@ -1608,23 +1633,8 @@ RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, in
                                          dim3(P->rounds_threads), args, 0, s),
               "rounds_kernel launch");
     } else if (sync_type == GPU_LOOP_ID && P->graphs_enabled) {
-        // the next chunk is launched while the last rounds of the previous
-        // one run
-        const int chunk = std::max(1, P->tuning.graph_rounds);
-        const long long key = (1LL << 40) + max_rounds;
-        if (key != P->graph_key) {
-            P->drop_graphs();
-            P->graph_key = key;
-        }
-        for (int first = 1, ci = 0; first <= max_rounds; first += chunk, ci++) {
-            const int last = std::min(max_rounds, first + chunk - 1);
-            launch_round_graph(P, ci, first, last);
-            if (last < max_rounds && wait_round(P, std::max(first, last - 1)) == kRoundsOver) break;
-        }
+        run_graphs(P, (1LL << 40) + max_rounds, max_rounds, [&](int step) { launch_round(P, step); });
     } else {
-        // launches run ahead of the host's look at the progress by kAhead
-        // rounds, so that the device never waits for it
-        constexpr int kAhead = 2;
         for (int step = 1; step <= max_rounds; step++) {
             launch_round(P, step);
             if (step > kAhead && wait_round(P, step - kAhead) == kRoundsOver) break;
@@ -1644,67 +1654,69 @@ RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, in
     return r;
 }
 
-// A complete run of one bound vector (device pointers) as unit 0, from
-// round 1.  Host buffers stay on the stack.
-RunResult run_single(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds) {
-    if (sync_type < CPU_LOOP_ID || sync_type > MEGAKERNEL_ID) throw std::runtime_error("Unknown sync type");
-    if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
-    if (P->rounds_state) return run_rounds(P, d_lbs, d_ubs, sync_type, max_rounds);
-    const int list[1] = {0};
-    const int caps[1] = {max_rounds};
-    P->D.n_active = 1;
-    load_units(P, 1, list, &d_lbs, &d_ubs, nullptr, nullptr, caps, 1, true);
-    UnitState st = read_unit(P, 0);
-    if (st.envelope) throw std::runtime_error("bounds outside the problem's bound envelope");
-    double ms = 0.0;
-    if (!st.crossed) {
-        ms = run_steps(P, sync_type, max_rounds);
-        st = read_unit(P, 0);
-    }
-    RunResult r = outcome(st);
-    r.kernel_ms = ms;
-    const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
-    hipLaunchKernelGGL(unpack_kernel, dim3(gx, 1), dim3(256), 0, P->stream, P->M, P->D, 1, P->d_list, P->d_lbp,
-                       P->d_ubp);
-    check(hipGetLastError(), "unpack launch");
-    check(hipStreamSynchronize(P->stream), "unpack sync");
-    return r;
-}
-
-// A complete run of the listed units from round 1.
+// A complete run of the listed units from round 1.  The call waits once, for
+// the outcomes in pinned memory (a single vector's in the problem's own slot:
+// nothing is allocated).
 void run_units(Problem *P, int n_list, const int *list, double *const *lbp, double *const *ubp, const int *hint_ptr,
                const int *hints, int sync_type, int max_rounds, RunResult *out) {
     if (sync_type < CPU_LOOP_ID || sync_type > MEGAKERNEL_ID) throw std::runtime_error("Unknown sync type");
     if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
-    std::vector<int> caps(n_list, max_rounds);
+    hipStream_t s = P->stream;
+    std::vector<int> many;
+    if (n_list > 1) many.assign(n_list, max_rounds);
+    const int *caps = n_list > 1 ? many.data() : &max_rounds;
     P->D.n_active = P->replicas ? n_list : 0;
     // hinted vectors (children of propagated nodes) mostly agree with each other
     const bool related = P->replicas && n_list > 1 && P->M.n_seg_parts > 0 && P->M.mark_rows &&
                          hint_ptr != nullptr && hint_ptr[n_list] > 0;
     if (related) set_reference(P, lbp, ubp, n_list);
-    load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps.data(), 1, true, related);
-    // bounds outside the envelope are an error before any round
-    std::vector<UnitState> st = read_units(P, n_list, list);
+    load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps, 1, true, related);
+    run_steps(P, sync_type, max_rounds);
+    const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
+    const int gy = P->replicas ? std::max(1, std::min(n_list, 1024)) : 1;
+    hipLaunchKernelGGL(unpack_kernel, dim3(gx, gy), dim3(256), 0, s, P->M, P->D, n_list, P->d_list, P->d_lbp, P->d_ubp,
+                       1);
+    // (the tables' pinned copy is free again: the run has read it)
+    UnitState *st = &P->host->state;
+    if (n_list > 1) {
+        const size_t tables = reinterpret_cast<char *>(P->d_ubp + n_list) - reinterpret_cast<char *>(P->d_list);
+        const size_t at = (tables + 63) / 64 * 64;
+        char *h = P->h_tables.p;
+        if (P->h_tables.size < at + sizeof(UnitState) * n_list) {
+            check(hipStreamSynchronize(s), "sync");
+            h = P->h_tables.get(at + sizeof(UnitState) * n_list);
+        }
+        st = reinterpret_cast<UnitState *>(h + at);
+    }
+    hipLaunchKernelGGL(report_kernel, dim3(std::max(1, std::min(256, (n_list + 255) / 256))), dim3(256), 0, s, P->D,
+                       n_list, P->d_list, st);
+    check(hipGetLastError(), "run launches");
+    check(hipStreamSynchronize(s), "run");
     bool any_active = false;
-    for (const auto &u : st) {
-        if (u.envelope) throw std::runtime_error("bounds outside the problem's bound envelope");
-        any_active |= !u.crossed;
+    for (int k = 0; k < n_list; k++) {
+        if (st[k].error) throw std::runtime_error("device wait timed out");
+        // bounds outside the envelope are an error, the vectors left alone
+        if (st[k].envelope) throw std::runtime_error("bounds outside the problem's bound envelope");
+        any_active |= !st[k].crossed;
     }
-    double ms = 0.0;
-    if (any_active) {
-        ms = run_steps(P, sync_type, max_rounds);
-        st = read_units(P, n_list, list);
-    }
+    float ms = 0.f;
+    if (any_active) check(hipEventElapsedTime(&ms, P->ev0, P->ev1), "elapsed");
     for (int k = 0; k < n_list; k++) {
         out[k] = outcome(st[k]);
         out[k].kernel_ms = ms;
     }
-    const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
-    const int gy = P->replicas ? std::max(1, std::min(n_list, 1024)) : 1;
-    hipLaunchKernelGGL(unpack_kernel, dim3(gx, gy), dim3(256), 0, P->stream, P->M, P->D, n_list, P->d_list,
-                       P->d_lbp, P->d_ubp);
-    check(hipGetLastError(), "unpack launch");
-    check(hipStreamSynchronize(P->stream), "unpack sync");
+}
+
+// A complete run of one bound vector (device pointers) as unit 0, from
+// round 1.
+RunResult run_single(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds) {
+    if (sync_type < CPU_LOOP_ID || sync_type > MEGAKERNEL_ID) throw std::runtime_error("Unknown sync type");
+    if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
+    if (P->rounds_state) return run_rounds(P, d_lbs, d_ubs, sync_type, max_rounds);
+    const int list[1] = {0};
+    RunResult r;
+    run_units(P, 1, list, &d_lbs, &d_ubs, nullptr, nullptr, sync_type, max_rounds, &r);
+    return r;
 }
 
 }  // namespace
@@ -1783,12 +1795,26 @@ RunResult problem_propagate(Problem *P, double *lbs, double *ubs, int sync_type,
     double *d_b = nullptr;
     check(cached_malloc(&d_b, 2 * sizeof(double) * static_cast<size_t>(n)), "hipMalloc bounds");
     RunResult res;
+    const size_t nb = sizeof(double) * static_cast<size_t>(n);
     try {
-        upload(d_b, lbs, n, P->stream);
-        upload(d_b + n, ubs, n, P->stream);
-        res = propagate_device_locked(P, d_b, d_b + n, sync_type, max_rounds);
-        download(lbs, d_b, n, P->stream);
-        download(ubs, d_b + n, n, P->stream);
+        if (2 * nb <= kSmallBounds) {
+            // small vectors cross in one copy each way, through a pinned block
+            char *h = P->h_bounds.get(2 * nb);
+            std::memcpy(h, lbs, nb);
+            std::memcpy(h + nb, ubs, nb);
+            check(hipMemcpyAsync(d_b, h, 2 * nb, hipMemcpyHostToDevice, P->stream), "H2D bounds");
+            res = propagate_device_locked(P, d_b, d_b + n, sync_type, max_rounds);
+            check(hipMemcpyAsync(h, d_b, 2 * nb, hipMemcpyDeviceToHost, P->stream), "D2H bounds");
+            check(hipStreamSynchronize(P->stream), "D2H bounds");
+            std::memcpy(lbs, h, nb);
+            std::memcpy(ubs, h + nb, nb);
+        } else {
+            upload_bulk(d_b, lbs, nb, P->stream);
+            upload_bulk(d_b + n, ubs, nb, P->stream);
+            res = propagate_device_locked(P, d_b, d_b + n, sync_type, max_rounds);
+            download_bulk(lbs, d_b, nb, P->stream);
+            download_bulk(ubs, d_b + n, nb, P->stream);
+        }
     } catch (...) {
         (void)hipStreamSynchronize(P->stream);
         (void)cached_free(d_b);
@@ -1900,7 +1926,7 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
         res = outcome(st[0]);
         const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
         hipLaunchKernelGGL(unpack_kernel, dim3(gx, 1), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                           P->d_ubp);
+                           P->d_ubp, 0);
         check(hipGetLastError(), "unpack launch");
         check(hipStreamSynchronize(s), "unpack sync");
         check(hipMemcpy(lbs, d_b, n * sizeof(double), hipMemcpyDeviceToHost), "D2H lbs");
@@ -1958,7 +1984,7 @@ RunResult problem_propagate_measured(Problem *P, double *lbs, double *ubs, int m
             launch_step(P, step, 0, 1);
             check(hipGetLastError(), "step launch");
             hipLaunchKernelGGL(unpack_kernel, dim3(gx, 1), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                               P->d_ubp);
+                               P->d_ubp, 0);
             hipLaunchKernelGGL(measure_kernel, dim3(gx), dim3(256), 0, s, n, d_b, d_b + n, d_w, d_w + n, d_l,
                                d_l + n, d_prev, d_prev + n, part_f, part_i);
             hipLaunchKernelGGL(measure_total_kernel, dim3(1), dim3(64), 0, s, gx, part_f, part_i, out_f + step - 1,
@@ -1969,7 +1995,7 @@ RunResult problem_propagate_measured(Problem *P, double *lbs, double *ubs, int m
         }
         res = outcome(st[0]);
         hipLaunchKernelGGL(unpack_kernel, dim3(gx, 1), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                           P->d_ubp);
+                           P->d_ubp, 0);
         check(hipGetLastError(), "unpack launch");
         check(hipStreamSynchronize(s), "unpack sync");
         fin.resize(rounds);
@@ -2985,7 +3011,8 @@ int step_impl(Server *S) {
         upload(P->d_ubp, ubp.data(), fin.size(), s);
         const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
         hipLaunchKernelGGL(unpack_kernel, dim3(gx, std::max(1, std::min(static_cast<int>(fin.size()), 1024))),
-                           dim3(256), 0, s, P->M, P->D, static_cast<int>(fin.size()), P->d_list, P->d_lbp, P->d_ubp);
+                           dim3(256), 0, s, P->M, P->D, static_cast<int>(fin.size()), P->d_list, P->d_lbp, P->d_ubp,
+                           0);
         check(hipGetLastError(), "unpack launch");
         std::vector<Server::Done> out(fin.size());
         // delta requests (against the base vector) and in-place zero-copy

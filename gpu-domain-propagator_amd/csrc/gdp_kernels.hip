@@ -1488,7 +1488,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void s
     DevState D = D_arg;
     D.n_lds = 0;
     __shared__ unsigned window[kWindowLdsBytes / 4];
-    if (guard && step_skipped(D, step, first_step)) return;
+    const bool skipped = guard && step_skipped(D, step, first_step);
+    if (guard && blockIdx.x == 0 && threadIdx.x == 0)  // tells the host
+        __hip_atomic_store(D.host_word, skipped ? kRoundsOver : step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (skipped) return;
     const int waves = blockDim.x >> 6;
     const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));
     UnitStep one{};
@@ -1829,7 +1832,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void r
     const long long w0 = coherent_load(p), w2 = coherent_load(p + 2);
     const bool runs = (w0 >> 32) == 0 && w2 == 0 && (step == 1 || round_moved(D, step - 1));
     if (blockIdx.x == 0 && threadIdx.x == 0)
-        __hip_atomic_store(R.host_word, runs ? step : kRoundsOver, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(D.host_word, runs ? step : kRoundsOver, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (!runs) return;
     if (threadIdx.x == 0) any_moved = 0;
     __syncthreads();
@@ -2017,6 +2020,49 @@ __global__ __launch_bounds__(256) void unpack_rounds_kernel(DevMatrix M, DevStat
 // loading and reading bound vectors
 // ---------------------------------------------------------------------------
 
+// Resets the state words of unit q.x (q as in unit_reset_kernel).
+__device__ __forceinline__ void reset_unit(const DevState &D, const int4 q, int start_step) {
+    UnitState s = {};
+    s.start = start_step;
+    s.markall = q.z ? start_step : 0;
+    s.max_rounds = q.w;
+    s.mark_limit = q.y;
+    D.units[q.x] = s;
+    for (int sl = 0; sl < kMoveSlots; sl++)
+        for (int j = 0; j < kMoveLanes; j++) D.moved[moved_index(q.x, sl, j)] = 0;
+    if (D.wl_cnt != nullptr)
+        for (int j = 0; j < 2 * kCountWords; j++) D.wl_cnt[static_cast<size_t>(q.x) * 2 * kCountWords + j] = 0ull;
+}
+
+__device__ __forceinline__ void clear_run_words(const DevState &D, int tid, int stride) {
+    for (int k = tid; k < kStatusRows * kStatusWords; k += stride) D.status[k] = 0;
+    for (int k = tid; k < kGlobalWords; k += stride) D.global[k] = 0;
+    for (int k = tid; k < kBarrierWords; k += stride) D.barrier[k] = 0u;
+}
+
+// unit_reset_kernel and the launch tables for a single vector, all from the
+// arguments (no copy to the device): the listed unit and the vector's pointers.
+__global__ __launch_bounds__(256) void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int *list,
+                                                        double **lbp, double **ubp, double *lbs, double *ubs) {
+    if (threadIdx.x == 0) {
+        reset_unit(D, q, start_step);
+        list[0] = q.x;
+        lbp[0] = lbs;
+        ubp[0] = ubs;
+    }
+    if (clear_status) clear_run_words(D, threadIdx.x, blockDim.x);
+}
+
+// The state words of the listed units and the error word, to pinned host
+// memory.
+__global__ __launch_bounds__(256) void report_kernel(DevState D, int n_list, const int *list, UnitState *out) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n_list; k += gridDim.x * blockDim.x) {
+        UnitState s = D.units[list[k]];
+        s.error = D.global[kGlobalError];
+        out[k] = s;
+    }
+}
+
 // Resets the state words of the listed units, params[k] = {unit, mark
 // limit, all rows in round 1, round cap}: round 1 in `start_step`, every row
 // processed in that step unless marks come from changed-column hints.  With
@@ -2025,24 +2071,8 @@ __global__ __launch_bounds__(256) void unpack_rounds_kernel(DevMatrix M, DevStat
 __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status) {
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
-    for (int k = tid; k < n_list; k += stride) {
-        const int4 q = params[k];
-        UnitState s = {};
-        s.start = start_step;
-        s.markall = q.z ? start_step : 0;
-        s.max_rounds = q.w;
-        s.mark_limit = q.y;
-        D.units[q.x] = s;
-        for (int sl = 0; sl < kMoveSlots; sl++)
-            for (int j = 0; j < kMoveLanes; j++) D.moved[moved_index(q.x, sl, j)] = 0;
-        if (D.wl_cnt != nullptr)
-            for (int j = 0; j < 2 * kCountWords; j++) D.wl_cnt[static_cast<size_t>(q.x) * 2 * kCountWords + j] = 0ull;
-    }
-    if (clear_status) {
-        for (int k = tid; k < kStatusRows * kStatusWords; k += stride) D.status[k] = 0;
-        for (int k = tid; k < kGlobalWords; k += stride) D.global[k] = 0;
-        for (int k = tid; k < kBarrierWords; k += stride) D.barrier[k] = 0u;
-    }
+    for (int k = tid; k < n_list; k += stride) reset_unit(D, params[k], start_step);
+    if (clear_status) clear_run_words(D, tid, stride);
 }
 
 // Loads the bound vectors of the listed units (caller's column order: unit
@@ -2090,7 +2120,10 @@ __global__ __launch_bounds__(256) void load_kernel(DevMatrix M, DevState D, int 
                                   floor(uu) == uu;
                 // crossed input bounds make the vector infeasible, whatever
                 // the column's storage class
-                if (!fits && !eps_gt(l, uu)) atomic_or_i(&D.units[cu].envelope, 1);
+                if (!fits && !eps_gt(l, uu)) {
+                    atomic_or_i(&D.units[cu].envelope, 1);
+                    atomic_or_i(&D.global[kGlobalEnvelope], 1);
+                }
                 const int il = fits ? static_cast<int>(l) : 0, iu = fits ? static_cast<int>(uu) : 0;
                 V.AI[id] = make_int2(il, iu);
                 V.AX[id] = make_double2(-INFINITY, INFINITY);
@@ -2296,9 +2329,11 @@ __global__ __launch_bounds__(256) void hint_kernel(DevMatrix M, DevState D, int 
 }
 
 // Writes the accumulated bounds of the listed units back to the caller's
-// column order.
+// column order.  With `checked`, nothing when a loaded vector left the
+// envelope: the run is an error and leaves the vectors alone.
 __global__ __launch_bounds__(256) void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list,
-                                                     double *const *lbp, double *const *ubp) {
+                                                     double *const *lbp, double *const *ubp, int checked) {
+    if (checked && D.global[kGlobalEnvelope] != 0) return;
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     const int n_pass = M.replicas ? n_list : 1;  // blocks mode: one pass over all columns
