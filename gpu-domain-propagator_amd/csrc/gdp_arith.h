@@ -44,6 +44,21 @@ GDP_HD bool is_neg_inf(double x) { return x <= -kInf; }
 GDP_HD double round_upper(bool is_cont, double ub) { return is_cont ? ub : floor(ub + kEps); }
 GDP_HD double round_lower(bool is_cont, double lb) { return is_cont ? lb : ceil(lb - kEps); }
 
+// Storage class of a column from its bound envelope [l, u]: 0 = 2 x int16,
+// 1 = 2 x int32, 2 = 2 x double.
+GDP_HD int column_class(int vartype, double l, double u) {
+    if (vartype == kVarContinuous) return 2;
+    // both within the int32 range (false for NaN and infinities), then
+    // integral: exact through a 64-bit integer round trip in that range,
+    // without the library calls of floor()
+    if (!(l >= -2147483647.0 && l <= 2147483647.0 && u >= -2147483647.0 && u <= 2147483647.0)) return 2;
+    if (static_cast<double>(static_cast<long long>(l)) != l || static_cast<double>(static_cast<long long>(u)) != u)
+        return 2;
+    return l >= -32767.0 && l <= 32767.0 && u >= -32767.0 && u <= 32767.0 ? 0 : 1;
+}
+// An int16 column that needs 2 bits: its envelope lies in [0, 1].
+GDP_HD bool binary_envelope(double l, double u) { return l >= 0.0 && u <= 1.0; }
+
 // Contributions of a_k * x_k to the row's minimum and maximum activity and
 // whether they are infinite (propagation_methods.cuh:198-213).  An infinite
 // contribution is counted and contributes +0.0 to the finite part.

@@ -431,20 +431,6 @@ class CreateTrace {
     std::string line_;
 };
 
-// Storage class of a column from its bound envelope: 0 = 2 x int16,
-// 1 = 2 x int32, 2 = 2 x double.
-int column_class(int vartype, const double *env_lb, const double *env_ub, int j) {
-    if (vartype == kVarContinuous || !env_lb || !env_ub) return 2;
-    const double l = env_lb[j], u = env_ub[j];
-    // both within the int32 range (false for NaN and infinities), then
-    // integral: exact through a 64-bit integer round trip in that range,
-    // without the library calls of floor()
-    if (!(l >= -2147483647.0 && l <= 2147483647.0 && u >= -2147483647.0 && u <= 2147483647.0)) return 2;
-    if (static_cast<double>(static_cast<long long>(l)) != l || static_cast<double>(static_cast<long long>(u)) != u)
-        return 2;
-    return l >= -32767.0 && l <= 32767.0 && u >= -32767.0 && u <= 32767.0 ? 0 : 1;
-}
-
 // Input contract of the row structure (the column indices are checked on
 // the device while the layout is built).
 void validate(const InstanceView &v) {
@@ -736,15 +722,16 @@ class CsrUpload {
         for (void *p : mem_) (void)cached_free(p);
     }
 
-    void start(int device) {
-        th_ = std::thread([this, device] {
+    // vartypes false: the caller has filled `vartype` on the stream that reads it
+    void start(int device, bool vartypes) {
+        th_ = std::thread([this, device, vartypes] {
             try {
                 check(hipSetDevice(device), "hipSetDevice");
                 long long at = 0;
                 for (size_t i = 0; i < inst_.size(); i++) {
                     upload(col + at, inst_[i].col, inst_[i].nnz, stream_);
                     upload(val + at, inst_[i].val, inst_[i].nnz, stream_);
-                    upload(vartype + off_[i], inst_[i].vartype, inst_[i].n, stream_);
+                    if (vartypes) upload(vartype + off_[i], inst_[i].vartype, inst_[i].n, stream_);
                     at += inst_[i].nnz;
                 }
                 check(hipStreamSynchronize(stream_), "CSR upload");
@@ -828,6 +815,98 @@ void device_layout_build(CsrUpload &csr, const std::vector<int> &col_off, int mp
     }
     for (void *p : tmp) check(cached_free(p), "hipFree");
     trace.mark("free_temp");
+}
+
+// Internal column ids: perm[id] = column (-1: padding), internal[column] = id,
+// the first id of each storage class, the binary columns at the front of class
+// 0 and (blocks mode) the instance of each 32-id word.
+struct ColumnOrder {
+    int n_ids = 0, n_bin = 0;
+    int class_start[3] = {0, 0, 0};
+    std::vector<int> perm, internal, word_unit;  // of the order made on the host
+};
+
+ColumnOrder host_column_order(const std::vector<InstanceView> &inst, const std::vector<int> &col_off, bool replicas,
+                              bool compact) {
+    const int NI = static_cast<int>(inst.size());
+    const int n = col_off[NI];
+    ColumnOrder C;
+    std::vector<unsigned char> cls(n);
+    std::vector<int> cnt_ci(3 * static_cast<size_t>(NI), 0);
+    for (int i = 0; i < NI; i++)
+        for (int j = 0; j < inst[i].n; j++) {
+            const int c = compact && inst[i].env_lb && inst[i].env_ub
+                              ? column_class(inst[i].vartype[j], inst[i].env_lb[j], inst[i].env_ub[j])
+                              : 2;
+            cls[col_off[i] + j] = static_cast<unsigned char>(c);
+            cnt_ci[c * NI + i]++;
+        }
+    std::vector<int> start_ci(3 * static_cast<size_t>(NI));
+    long long n_ids_l = 0;
+    for (int c = 0; c < 3; c++) {
+        C.class_start[c] = static_cast<int>(n_ids_l);
+        for (int i = 0; i < NI; i++) {
+            start_ci[c * NI + i] = static_cast<int>(n_ids_l);
+            n_ids_l += cnt_ci[c * NI + i];
+            if (!replicas) n_ids_l = (n_ids_l + 31) / 32 * 32;
+            if (n_ids_l > kIdMask) throw std::runtime_error("too many columns");
+        }
+    }
+    C.n_ids = static_cast<int>(n_ids_l);
+    std::vector<unsigned char> binary;
+    if (replicas && NI == 1) {
+        binary.assign(n, 0);
+        for (int j = 0; j < inst[0].n; j++)
+            if (cls[j] == 0 && binary_envelope(inst[0].env_lb[j], inst[0].env_ub[j])) {
+                binary[j] = 1;
+                C.n_bin++;
+            }
+    }
+    C.perm.assign(C.n_ids, -1);
+    C.internal.resize(n);
+    std::vector<int> pos = start_ci;
+    int bin_pos = start_ci[0];
+    if (C.n_bin) pos[0] += C.n_bin;
+    for (int i = 0; i < NI; i++)
+        for (int j = 0; j < inst[i].n; j++) {
+            const int g = col_off[i] + j;
+            const int id = C.n_bin && binary[g] ? bin_pos++ : pos[cls[g] * NI + i]++;
+            C.internal[g] = id;
+            C.perm[id] = g;
+        }
+    if (!replicas) {
+        // every word lies in one (class, instance) range
+        C.word_unit.assign((C.n_ids + 31) / 32, 0);
+        for (int c = 0; c < 3; c++)
+            for (int i = 0; i < NI; i++) {
+                const int a0 = start_ci[c * NI + i], cnt = cnt_ci[c * NI + i];
+                for (int w = a0 / 32; w < (a0 + cnt + 31) / 32; w++) C.word_unit[w] = i;
+            }
+    }
+    return C;
+}
+
+// The same order for one instance's n columns, made on the device: vartype
+// and env (n lower bounds, then n upper bounds; null: every column FP64) are
+// device arrays, perm and internal are written.  Synchronous.
+ColumnOrder device_column_order(int n, const int *vartype, const double *env, int *perm, int *internal,
+                                std::vector<void *> &tmp, hipStream_t s) {
+    unsigned char *t_key = dev_alloc<unsigned char>(2 * static_cast<size_t>(n), tmp);
+    int *t_col = dev_alloc<int>(n, tmp);
+    int *t_tot = dev_alloc<int>(4, tmp);
+    check(hipMemsetAsync(t_tot, 0, sizeof(int) * 4, s), "memset totals");
+    order_column_keys(n, vartype, env, t_key, t_col, t_tot, s);
+    order_sort_rows(t_key, t_key + n, t_col, perm, n, s);
+    order_invert(n, perm, internal, s);
+    int tot[4];
+    check(hipMemcpyAsync(tot, t_tot, sizeof(tot), hipMemcpyDeviceToHost, s), "D2H totals");
+    check(hipStreamSynchronize(s), "column order");
+    ColumnOrder C;
+    C.n_ids = n;
+    C.n_bin = tot[0];
+    C.class_start[1] = tot[0] + tot[1];
+    C.class_start[2] = C.class_start[1] + tot[2];
+    return C;
 }
 
 // Layout rows as ordered on the device (gdp_order.hip): host copies of the
@@ -929,11 +1008,12 @@ void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
     const Tuning &T = P->tuning;
     // Every round processes every row, which costs about 8.5 ps per entry; the
     // three-phase rounds of larger problems skip the rows whose columns did not
-    // move.  200,000 rows, 2.2M nonzeros, 32 rounds: 0.80 ms a call (three
-    // phases: 1.3 persistent, 2.4 in the host loop).  3.1M nonzeros over 500,000
-    // columns, 65 rounds: 2.4 ms (2.4 / 5.9).  19.3M nonzeros: 4.8 ms (3.1).
+    // move.  ms a call (three phases: persistent / host loop): 200,000 rows,
+    // 2.2M nonzeros, 32 rounds 0.73 (1.15 / 1.03); 3.1M nonzeros over 500,000
+    // columns, 65 rounds 1.91 (2.39 / 1.92); 3.3M 1.16 (1.62 / 1.37); 5.5M 1.72
+    // (1.82 / 1.64); 7.8M 2.56 (1.90 / 1.75).
     constexpr int kMaxRoundEntries = 4 << 20;
-    if (!P->replicas || P->n_inst != 1 || n_padded > (std::getenv("GDP_RMAX") ? std::atoi(std::getenv("GDP_RMAX")) : kMaxRoundEntries)) return;
+    if (!P->replicas || P->n_inst != 1 || n_padded > kMaxRoundEntries) return;
     if (T.item_nnz != def.item_nnz || T.mega_blocks_per_cu != def.mega_blocks_per_cu ||
         T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
         !std::equal(T.group_log, T.group_log + 10, def.group_log))
@@ -1030,67 +1110,18 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         P->nnz = static_cast<int>(nnz_total);
 
         // ---- columns: internal ids by storage class, instance-major within a
-        // class; blocks mode pads each (class, instance) range to 32 ids ----
-        std::vector<unsigned char> cls(P->n);
-        std::vector<int> cnt_ci(3 * static_cast<size_t>(NI), 0);
-        for (int i = 0; i < NI; i++)
-            for (int j = 0; j < inst[i].n; j++) {
-                const int c =
-                    T.compact_bounds ? column_class(inst[i].vartype[j], inst[i].env_lb, inst[i].env_ub, j) : 2;
-                cls[col_off[i] + j] = static_cast<unsigned char>(c);
-                cnt_ci[c * NI + i]++;
-            }
-        std::vector<int> start_ci(3 * static_cast<size_t>(NI));
-        int class_start[3];
-        long long n_ids_l = 0;
-        for (int c = 0; c < 3; c++) {
-            class_start[c] = static_cast<int>(n_ids_l);
-            for (int i = 0; i < NI; i++) {
-                start_ci[c * NI + i] = static_cast<int>(n_ids_l);
-                n_ids_l += cnt_ci[c * NI + i];
-                if (!replicas) n_ids_l = (n_ids_l + 31) / 32 * 32;
-                if (n_ids_l > kIdMask) throw std::runtime_error("too many columns");
-            }
-        }
-        const int n_ids = static_cast<int>(n_ids_l);
-        // replicas mode: the binary columns (int16 class, envelope in [0, 1])
-        // take the first ids of their class
-        std::vector<unsigned char> binary;
-        int n_bin = 0;
-        if (replicas && NI == 1) {
-            binary.assign(P->n, 0);
-            for (int j = 0; j < inst[0].n; j++)
-                if (cls[j] == 0 && inst[0].env_lb[j] >= 0.0 && inst[0].env_ub[j] <= 1.0) {
-                    binary[j] = 1;
-                    n_bin++;
-                }
-        }
-        std::vector<int> perm(n_ids, -1), internal(P->n), word_unit;
-        {
-            std::vector<int> pos = start_ci;
-            int bin_pos = start_ci[0];
-            if (n_bin) pos[0] += n_bin;
-            for (int i = 0; i < NI; i++)
-                for (int j = 0; j < inst[i].n; j++) {
-                    const int g = col_off[i] + j;
-                    const int id = n_bin && binary[g] ? bin_pos++ : pos[cls[g] * NI + i]++;
-                    internal[g] = id;
-                    perm[id] = g;
-                }
-        }
-        const int nwords = (n_ids + 31) / 32;
-        if (!replicas) {
-            // every word lies in one (class, instance) range
-            word_unit.assign(nwords, 0);
-            for (int c = 0; c < 3; c++)
-                for (int i = 0; i < NI; i++) {
-                    const int a0 = start_ci[c * NI + i], cnt = cnt_ci[c * NI + i];
-                    for (int w = a0 / 32; w < (a0 + cnt + 31) / 32; w++) word_unit[w] = i;
-                }
-        }
-        P->stats.n16 = class_start[1] - class_start[0];
-        P->stats.n32 = class_start[2] - class_start[1];
-        P->stats.nf = n_ids - class_start[2];
+        // class; blocks mode pads each (class, instance) range to 32 ids.  In
+        // replicas mode the binary columns (int16 class, envelope in [0, 1])
+        // take the first ids of their class ----
+        // From 16K columns on a single instance's ids come from a sort on the
+        // device, under the copy of the nonzeros; below that the copies and the
+        // sort's launches cost more than the pass (creation, ms, host / device:
+        // 100,000 columns 2.40 / 1.48, 32,000 0.97 / 0.77, 16,000 0.69 / 0.66,
+        // 8,000 0.56 / 0.59).
+        constexpr int kDeviceColumns = 16 << 10;
+        const bool device_columns = replicas && P->n >= kDeviceColumns;
+        ColumnOrder C;
+        if (!device_columns) C = host_column_order(inst, col_off, replicas, T.compact_bounds);
 
         trace.mark("columns");
         // ---- device ----
@@ -1117,15 +1148,34 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         // (padding: column 0, coefficient 0), the padding count in the low
         // bits of the row starts ----
         constexpr int kLongBin = 10;
-        int *d_perm = dev_alloc<int>(n_ids, o);
+        int *d_perm = dev_alloc<int>(device_columns ? P->n : C.n_ids, o);
         P->d_inv_perm = dev_alloc<int>(P->n, o);
-        upload(d_perm, perm.data(), n_ids, s);
-        upload(P->d_inv_perm, internal.data(), P->n, s);
         CsrUpload csr(inst, col_off);
+        if (!device_columns) {
+            upload(d_perm, C.perm.data(), C.n_ids, s);
+            upload(P->d_inv_perm, C.internal.data(), P->n, s);
+        }
         int *d_rp = nullptr;
         double2 *d_sides = nullptr;
-        const RowOrder R =
-            device_row_order(inst, row_off, nnz_total, &d_rp, &d_sides, o, tmp, s, [&] { csr.start(P->device); });
+        const RowOrder R = device_row_order(inst, row_off, nnz_total, &d_rp, &d_sides, o, tmp, s, [&] {
+            if (!device_columns) {
+                csr.start(P->device, true);
+                return;
+            }
+            double *t_env = nullptr;
+            upload(csr.vartype, inst[0].vartype, P->n, s);
+            if (T.compact_bounds && inst[0].env_lb && inst[0].env_ub) {
+                t_env = dev_alloc<double>(2 * static_cast<size_t>(P->n), tmp);
+                upload(t_env, inst[0].env_lb, P->n, s);
+                upload(t_env + P->n, inst[0].env_ub, P->n, s);
+            }
+            csr.start(P->device, false);
+            C = device_column_order(P->n, csr.vartype, t_env, d_perm, P->d_inv_perm, tmp, s);
+        });
+        const int n_ids = C.n_ids, nwords = (n_ids + 31) / 32;
+        P->stats.n16 = C.class_start[1];
+        P->stats.n32 = C.class_start[2] - C.class_start[1];
+        P->stats.nf = n_ids - C.class_start[2];
         const int mp = R.mp;
         const int n_padded = R.n_padded;
         for (int b = 0; b <= kLongBin; b++) {
@@ -1220,8 +1270,8 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         DevMatrix &M = P->M;
         M.m = mp;
         M.n = n_ids;
-        M.n16 = class_start[1];
-        M.n_int = class_start[2];
+        M.n16 = C.class_start[1];
+        M.n_int = C.class_start[2];
         M.nwords = nwords;
         M.n_items = static_cast<int>(h_items.size());
         M.replicas = replicas ? 1 : 0;
@@ -1239,7 +1289,7 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         int *d_cseg = dev_alloc<int>(n_csc, o);
         int *d_unit_item = dev_alloc<int>(h_unit_item.size(), o);
         int *d_list_at = dev_alloc<int>(h_list_at.size(), o);
-        int *d_word_unit = dev_alloc<int>(word_unit.size(), o);
+        int *d_word_unit = dev_alloc<int>(C.word_unit.size(), o);
         // per layout row: first segment of a split row (-1: none)
         int *t_row_part = dev_alloc<int>(mp, tmp);
         trace.mark("device_setup_alloc");
@@ -1248,7 +1298,7 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         upload(d_list_at, h_list_at.data(), h_list_at.size(), s);
         upload(d_seg_rows, h_seg_rows.data(), h_seg_rows.size(), s);
         upload(d_part_row, h_part_row.data(), h_part_row.size(), s);
-        upload(d_word_unit, word_unit.data(), word_unit.size(), s);
+        upload(d_word_unit, C.word_unit.data(), C.word_unit.size(), s);
         check(hipMemsetAsync(t_row_part, 0xff, sizeof(int) * mp, s), "memset row tables");
         order_row_tables(M.n_seg_rows, d_seg_rows, t_row_part, s);
         check(hipStreamSynchronize(s), "upload");
@@ -1280,8 +1330,8 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         // snapshot block of a unit: int16 records, then int32, then FP64,
         // each class from a 16-byte boundary; the binary columns' codes in
         // 16-byte groups of 64 columns
-        M.n_bin = n_bin;
-        M.sb_words = (n_bin + 63) / 64 * 4;
+        M.n_bin = C.n_bin;
+        M.sb_words = (C.n_bin + 63) / 64 * 4;
         M.snap_off32 = (M.n16 * 4 + 15) / 16 * 16;
         M.snap_offF = M.snap_off32 + ((M.n_int - M.n16) * 8 + 15) / 16 * 16;
         M.snap_stride = M.snap_offF + 16LL * (M.n - M.n_int) + 16;
@@ -1320,11 +1370,11 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         // keep that many workgroups resident
         const int per_cu = mega_per_cu(P->mega_fn, kWindowLdsBytes);
         P->mega_grid = per_cu * P->cu_count;
-        int n_lds = std::min(n_bin, kMaxLdsBinBytes * 4) / 64 * 64;
+        int n_lds = std::min(C.n_bin, kMaxLdsBinBytes * 4) / 64 * 64;
         while (n_lds > 0 && mega_per_cu(P->mega_fn_lds, static_cast<size_t>(n_lds) / 4) < per_cu)
             n_lds = n_lds / 2 / 64 * 64;
         P->n_lds = n_lds;
-        P->stats.n_bin = n_bin;
+        P->stats.n_bin = C.n_bin;
         P->stats.n_lds = n_lds;
         int sweep_per_cu = 0;
         check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&sweep_per_cu, reinterpret_cast<const void *>(sweep_kernel),

@@ -1,4 +1,4 @@
-// gdp_order.h - device ordering of a problem's rows (gdp_order.hip).
+// gdp_order.h - device ordering of a problem's rows and columns (gdp_order.hip).
 //
 // Inputs on the device: the instances' row starts concatenated (instance i's
 // m_i + 1 entries from position row_off[i] + i), their sides concatenated
@@ -23,6 +23,16 @@ void order_row_keys(int M, int NI, const int *row_off, const int *rp_cat, unsign
 // Stable sort of the (key, row) pairs by the 4 key bits.
 void order_sort_rows(const unsigned char *keys, unsigned char *keys_sorted, const int *rows, int *rows_sorted, int M,
                      hipStream_t s);
+
+// keys[j], cols[j] = j for n columns: 0 binary, 1 other int16, 2 int32, 3 FP64
+// records; env holds the n lower, then the n upper bounds of the envelope
+// (null: every key is 3).  totals (4 entries, zeroed by the caller): columns
+// of each key.
+void order_column_keys(int n, const int *vartype, const double *env, unsigned char *keys, int *cols, int *totals,
+                       hipStream_t s);
+
+// inverse[perm[k]] = k for k < n.
+void order_invert(int n, const int *perm, int *inverse, hipStream_t s);
 
 // Per layout row r < mp (the nonempty rows, in sorted order): length,
 // padded length, source position, instance (inst may be null for one

@@ -1,4 +1,5 @@
-// gdp_order.hip - the order of a problem's rows, computed on the device.
+// gdp_order.hip - the order of a problem's rows (and, from the same sort, of
+// its columns), computed on the device.
 //
 // Layout rows are the nonempty rows of all instances, ordered by tree-width
 // bin (rows longer than kSegLen first, then the widths 2^9 down to 2^0), by
@@ -106,6 +107,32 @@ __global__ __launch_bounds__(256) void place_rows_kernel(int mp, int NI, const i
         if (!first && NI > 1) first = instance_of(order[r - 1], NI, row_off) != i;
         if (first) run_start[key * NI + i] = r;
     }
+}
+
+// The columns' ids are the same stable sort by storage class.  A few streaming
+// passes over 20 + 4 bytes a column; the sort's launches are the larger part.
+__global__ __launch_bounds__(256) void column_keys_kernel(int n, const int *vartype, const double *env,
+                                                          unsigned char *keys, int *cols, int *totals) {
+    __shared__ int s_tot[4];
+    if (threadIdx.x < 4) s_tot[threadIdx.x] = 0;
+    __syncthreads();
+    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
+        int key = 3;
+        if (env) {
+            const double l = env[j], u = env[n + j];
+            const int c = column_class(vartype[j], l, u);
+            key = c == 0 && binary_envelope(l, u) ? 0 : c + 1;
+        }
+        keys[j] = static_cast<unsigned char>(key);
+        cols[j] = j;
+        atomicAdd(&s_tot[key], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < 4 && s_tot[threadIdx.x]) atomicAdd(&totals[threadIdx.x], s_tot[threadIdx.x]);
+}
+
+__global__ __launch_bounds__(256) void invert_kernel(int n, const int *perm, int *inverse) {
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) inverse[perm[k]] = k;
 }
 
 __global__ __launch_bounds__(256) void pad_rows_kernel(int mp, const int *len, const int *plen, int *row_ptr) {
@@ -291,6 +318,17 @@ void order_sort_rows(const unsigned char *keys, unsigned char *keys_sorted, cons
     }
     (void)cached_free(tmp);
     check_order(e, "row sort");
+}
+
+void order_column_keys(int n, const int *vartype, const double *env, unsigned char *keys, int *cols, int *totals,
+                       hipStream_t s) {
+    hipLaunchKernelGGL(column_keys_kernel, dim3(grid_of(n)), dim3(256), 0, s, n, vartype, env, keys, cols, totals);
+    check_order(hipGetLastError(), "column keys launch");
+}
+
+void order_invert(int n, const int *perm, int *inverse, hipStream_t s) {
+    hipLaunchKernelGGL(invert_kernel, dim3(grid_of(n)), dim3(256), 0, s, n, perm, inverse);
+    check_order(hipGetLastError(), "invert launch");
 }
 
 void order_place_rows(int mp, int NI, const int *row_off, const long long *nnz_off, const int *rp_cat,
