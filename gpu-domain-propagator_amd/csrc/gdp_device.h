@@ -254,7 +254,7 @@ struct ReferenceVectors {
     int n;
 };
 
-// ---- double-buffered rounds (one bound vector) ----
+// ---- double-buffered rounds (one bound vector, or a batch) ----
 // Two blocks of bound records take turns: round s reads the bounds S_{s-1}
 // from block (s - 1) & 1 and folds its candidates into block s & 1, which
 // still holds S_{s-2}; the columns that round s - 1 moved are folded into it
@@ -268,6 +268,8 @@ struct ReferenceVectors {
 // snap_offF (the DevMatrix of these kernels has n16 = 0, snap_off32 = 0).
 constexpr int kPlanBins = 9;          // tree widths 2^8 .. 2^0
 constexpr int kMaxGatherBlocks = 512; // workgroups of the persistent launch
+constexpr int kMaxRoundUnits = 256;   // instances of a batch whose rounds run so (a multiple of 64)
+constexpr int kMaxSlotWords = (kMaxRoundUnits + 30) / 31;
 // Where each tree-width bin's rows and items start (building the item list).
 struct RoundBins {
     int n_segs;
@@ -286,7 +288,12 @@ struct RoundPlan {
     unsigned long long *slots;        // arrivals of the persistent launch's barrier, two sets
     double *lbs, *ubs;                // the caller's vectors
     int mark_limit, max_rounds;
-    UnitState *host_state;            // pinned: the outcome
+    UnitState *host_state;            // pinned: the outcome (of every unit)
+    // a batch: its instances side by side in the blocks
+    int n_units = 1;
+    int slot_words = 1;               // words of an arrival: 31 units each
+    const int *unit_item = nullptr;   // first item of each unit, and the end
+    int *run = nullptr, *upto = nullptr;  // launches: units of the round, running totals of their items
 };
 
 // State arrays of unit u (replicas mode); the shared arrays are unchanged.

@@ -47,7 +47,13 @@ template <int kThreads, bool kLds>
 __global__ void mega_kernel(DevMatrix M, DevState D, int first_step, int max_steps, int n_units);
 __global__ void plan_rounds_kernel(DevMatrix M, RoundBins B, int4 *items);
 __global__ void reset_rounds_kernel(DevState D, RoundPlan R);
+template <bool kUnits>
 __global__ void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin);
+__global__ void batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
+__global__ void batch_plan_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
+__global__ void batch_round_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
+__global__ void batch_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
+__global__ void unpack_batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
 __global__ void round_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
 __global__ void rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
@@ -625,7 +631,7 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
 }
 
 // The arrays of the double-buffered rounds (one bound vector), after those
-// of carve_state.  Returns the bytes needed.
+// of carve_state; R.slot_words and R.n_units are set.  Returns the bytes needed.
 size_t carve_rounds(const DevMatrix &Mr, char *base, RoundPlan &R) {
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -638,7 +644,9 @@ size_t carve_rounds(const DevMatrix &Mr, char *base, RoundPlan &R) {
         R.AX[k] = reinterpret_cast<double2 *>(take(Mr.n_int * sizeof(double2)));
         R.bm[k] = reinterpret_cast<unsigned *>(take(Mr.nwords * sizeof(unsigned)));
     }
-    R.slots = reinterpret_cast<unsigned long long *>(take(2 * kMaxGatherBlocks * sizeof(unsigned long long)));
+    R.slots = reinterpret_cast<unsigned long long *>(take(2 * kMaxGatherBlocks * R.slot_words * sizeof(unsigned long long)));
+    R.run = reinterpret_cast<int *>(take(R.n_units * sizeof(int)));
+    R.upto = reinterpret_cast<int *>(take(R.n_units * sizeof(int)));
     return off;
 }
 
@@ -672,7 +680,7 @@ void alloc_units(Problem *P, int cap) {
     DevState D{};
     UnitTables T;
     size_t bytes = carve_state(P->M, P->replicas, P->n_inst, cap, nullptr, D, T, true);
-    RoundPlan R;
+    RoundPlan R = P->R;
     if (P->rounds_ok) bytes += carve_rounds(P->Mr, nullptr, R);
     check(cached_malloc(&P->state_buf, bytes), "hipMalloc run state");
     bind_state(P, static_cast<char *>(P->state_buf), cap, P->rounds_ok);
@@ -1000,10 +1008,12 @@ RowOrder device_row_order(const std::vector<InstanceView> &inst, const std::vect
     return R;
 }
 
-// The plan of the double-buffered rounds of a single problem with default
-// tuning: start / count hold the first layout row and the rows of each bin
-// key (10 - log2 of the tree width).
-void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
+// The plan of the double-buffered rounds of a problem with default tuning:
+// start / count hold the first layout row and the rows of each (bin key,
+// instance) run (key: 10 - log2 of the tree width), first_part the first
+// split-row segment of each instance; part_row and seg_rows as in DevMatrix.
+void plan_rounds(Problem *P, const int *start, const int *count, const std::vector<int> &first_part,
+                 const std::vector<int> &part_row, const std::vector<int4> &seg_rows, int n_padded) {
     const Tuning def;
     const Tuning &T = P->tuning;
     // Every round processes every row, which costs about 8.5 ps per entry; the
@@ -1013,43 +1023,85 @@ void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
     // columns, 65 rounds 1.91 (2.39 / 1.92); 3.3M 1.16 (1.62 / 1.37); 5.5M 1.72
     // (1.82 / 1.64); 7.8M 2.56 (1.90 / 1.75).
     constexpr int kMaxRoundEntries = 4 << 20;
-    if (!P->replicas || P->n_inst != 1 || n_padded > kMaxRoundEntries) return;
+    // A batch leaves out the instances that are done, so its line lies higher,
+    // and higher still for small instances, whose numbers of rounds differ more.
+    // ms a call, persistent / loop, in brackets with three phases: 64 instances
+    // of 42,000 entries 0.99 / 0.95 (2.77 / 2.45), of 88,000 2.38 / 2.35 (4.05 /
+    // 3.54), of 122,000 2.25 / 2.22 (2.80 / 2.41), of 233,000 4.16 / 4.00 (4.46 /
+    // 4.07); 24 of 480,000 3.57 / 3.66 (4.08 / 3.52); 6 of 1.5M 2.99 / 3.10 (3.03 /
+    // 2.66); 16 of 2.1M 10.8 / 11.9 (7.4 in the loop).
+    constexpr int kMaxBatchEntries = 8 << 20;
+    constexpr int kSmallInstance = 256 << 10;
+    const int NI = P->n_inst;
+    if (P->replicas ? NI != 1 || n_padded > kMaxRoundEntries
+                    : NI > kMaxRoundUnits || n_padded > (n_padded / NI <= kSmallInstance ? 2 : 1) * kMaxBatchEntries)
+        return;
     if (T.item_nnz != def.item_nnz || T.mega_blocks_per_cu != def.mega_blocks_per_cu ||
         T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
         !std::equal(T.group_log, T.group_log + 10, def.group_log))
         return;
-    RoundBins B;
-    B.n_segs = P->M.n_seg_parts;
     // Entries per lane: few while the passes (256 lane entries of K each) still
     // find a free SIMD, because a pass is a chain of dependent loads, a butterfly
     // and divisions that grows with K.  Per persistent round with 1 / 2 / 4:
     // 33K entry slots 7.3 / 7.5 / 8.8 us, 115K 8.5 / 8.1 / 8.9 us, 330K 12.5 /
     // 10.3 / 10.4 us.
     const int logk_want = n_padded <= (64 << 10) ? 0 : (n_padded <= (512 << 10) ? 1 : 2);
-    int at = B.n_segs;
-    for (int q = 0; q < kPlanBins; q++) {
-        const int b = kPlanBins - 1 - q, key = 10 - b;
-        const int logk = std::max(std::min(logk_want, b), b - 6);
-        const int logg = b - logk;
-        B.logk[q] = logk;
-        B.logg[q] = logg;
-        B.rows_per_item[q] = 64 >> logg;
-        B.item0[q] = at;
-        B.row0[q] = start[key];
-        at += (count[key] + B.rows_per_item[q] - 1) / B.rows_per_item[q];
-    }
-    B.item0[kPlanBins] = at;
-    B.row0[kPlanBins] = P->M.m;
-    // bins without rows have no start of their own
-    for (int q = kPlanBins - 1; q >= 0; q--)
-        if (count[2 + q] == 0) B.row0[q] = B.row0[q + 1];
+    auto bin_logk = [&](int b) { return std::max(std::min(logk_want, b), b - 6); };
     RoundPlan &R = P->R;
-    R.n_items = at;
-    int4 *items = dev_alloc<int4>(at, P->owned);
-    R.items = items;
-    hipLaunchKernelGGL(plan_rounds_kernel, dim3(std::max(1, std::min(256, (at + 255) / 256))), dim3(256), 0, P->stream,
-                       P->M, B, items);
-    check(hipGetLastError(), "plan launch");
+    if (P->replicas) {
+        RoundBins B;
+        B.n_segs = P->M.n_seg_parts;
+        int at = B.n_segs;
+        for (int q = 0; q < kPlanBins; q++) {
+            const int b = kPlanBins - 1 - q, key = 10 - b;
+            const int logg = b - bin_logk(b);
+            B.logk[q] = bin_logk(b);
+            B.logg[q] = logg;
+            B.rows_per_item[q] = 64 >> logg;
+            B.item0[q] = at;
+            B.row0[q] = start[key];
+            at += (count[key] + B.rows_per_item[q] - 1) / B.rows_per_item[q];
+        }
+        B.item0[kPlanBins] = at;
+        B.row0[kPlanBins] = P->M.m;
+        // bins without rows have no start of their own
+        for (int q = kPlanBins - 1; q >= 0; q--)
+            if (count[2 + q] == 0) B.row0[q] = B.row0[q + 1];
+        R.n_items = at;
+        int4 *items = dev_alloc<int4>(at, P->owned);
+        R.items = items;
+        hipLaunchKernelGGL(plan_rounds_kernel, dim3(std::max(1, std::min(256, (at + 255) / 256))), dim3(256), 0,
+                           P->stream, P->M, B, items);
+        check(hipGetLastError(), "plan launch");
+    } else {
+        // instance after instance; a unit's runs are listed from the host
+        std::vector<int4> items;
+        std::vector<int> unit_item(NI + 1, 0);
+        items.reserve(static_cast<size_t>(n_padded) / 128 + 16 * static_cast<size_t>(NI));
+        for (int i = 0; i < NI; i++) {
+            const int parts_end = i + 1 < NI ? first_part[i + 1] : P->M.n_seg_parts;
+            for (int q = first_part[i]; q < parts_end; q++)
+                items.push_back(make_int4(kItemSeg, part_row[q], q - seg_rows[part_row[q]].y, 1));
+            for (int b = kPlanBins - 1; b >= 0; b--) {
+                const size_t run = static_cast<size_t>(10 - b) * NI + i;
+                const int logg = b - bin_logk(b), rows = 64 >> logg;
+                for (int q = 0; q < count[run]; q += rows)
+                    items.push_back(make_int4(kItemGroup | (logg << 4) | (bin_logk(b) << 8), start[run] + q,
+                                              std::min(rows, count[run] - q), 0));
+            }
+            unit_item[i + 1] = static_cast<int>(items.size());
+        }
+        R.n_items = static_cast<int>(items.size());
+        R.n_units = NI;
+        R.slot_words = (NI + 30) / 31;
+        int4 *d_items = dev_alloc<int4>(items.size(), P->owned);
+        int *d_unit_item = dev_alloc<int>(unit_item.size(), P->owned);
+        upload(d_items, items.data(), items.size(), P->stream);
+        upload(d_unit_item, unit_item.data(), unit_item.size(), P->stream);
+        check(hipStreamSynchronize(P->stream), "plan");
+        R.items = d_items;
+        R.unit_item = d_unit_item;
+    }
     DevMatrix &M = P->Mr;
     M = P->M;
     M.n16 = 0;
@@ -1061,9 +1113,9 @@ void plan_rounds(Problem *P, const int *start, const int *count, int n_padded) {
     // them (1.2 us for 16, 3 us for 256, 4.3 us for 512), and a workgroup of 256
     // threads spreads few items over more compute units
     P->rounds_threads = R.n_items <= 1024 ? 256 : (R.n_items <= 2048 ? 512 : 1024);
-    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(rounds_kernel),
-                                                       P->rounds_threads, 0),
-          "occupancy");
+    const void *fn = P->replicas ? reinterpret_cast<const void *>(rounds_kernel)
+                                 : reinterpret_cast<const void *>(batch_rounds_kernel);
+    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, P->rounds_threads, 0), "occupancy");
     const int waves = P->rounds_threads / 64;
     P->rounds_grid = std::max(1, std::min({per_cu * P->cu_count, kMaxGatherBlocks, (R.n_items + waves - 1) / waves}));
     P->rounds_ok = true;
@@ -1349,7 +1401,7 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         }
 
         P->host = host_slots().take();
-        plan_rounds(P, R.start.data(), R.count.data(), n_padded);
+        plan_rounds(P, R.start.data(), R.count.data(), first_part, h_part_row, h_seg_rows, n_padded);
 
         P->mega_threads = T.mega_threads == 256 || T.mega_threads == 1024 ? T.mega_threads : 512;
         P->mega_fn = P->mega_threads == 256    ? reinterpret_cast<const void *>(mega_kernel<256, false>)
@@ -1653,10 +1705,41 @@ std::vector<UnitState> read_units(Problem *P, int n_list, const int *list) {
 // Issues round `step`.
 void launch_round(Problem *P, int step) {
     const int grid = std::max(1, std::min(8 * P->cu_count, grid_for(P->R.n_items)));
+    const int apply_grid = std::max(1, std::min(1024, grid_for(P->Mr.n_seg_parts)));
+    if (!P->replicas) {
+        hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(kMaxRoundUnits), 0, P->stream, P->Mr, P->D, P->R, step);
+        hipLaunchKernelGGL(batch_round_kernel, dim3(grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+        if (P->Mr.n_seg_parts > 0)
+            hipLaunchKernelGGL(batch_apply_kernel, dim3(apply_grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+        return;
+    }
     hipLaunchKernelGGL(round_kernel, dim3(grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
     if (P->Mr.n_seg_parts > 0)
-        hipLaunchKernelGGL(round_apply_kernel, dim3(std::max(1, std::min(1024, grid_for(P->Mr.n_seg_parts)))),
-                           dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+        hipLaunchKernelGGL(round_apply_kernel, dim3(apply_grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+}
+
+// Issues the rounds of a loaded run, between the problem's two events.
+void issue_rounds(Problem *P, int sync_type, int max_rounds) {
+    hipStream_t s = P->stream;
+    check(hipEventRecord(P->ev0, s), "event");
+    if (sync_type == MEGAKERNEL_ID) {
+        void *args[] = {&P->Mr, &P->D, &P->R};
+        const void *fn = P->replicas ? reinterpret_cast<const void *>(rounds_kernel)
+                                     : reinterpret_cast<const void *>(batch_rounds_kernel);
+        check(hipLaunchCooperativeKernel(fn, dim3(P->rounds_grid), dim3(P->rounds_threads), args, 0, s),
+              "rounds launch");
+    } else if (sync_type == GPU_LOOP_ID && P->graphs_enabled) {
+        run_graphs(P, (1LL << 40) + max_rounds, max_rounds, [&](int step) { launch_round(P, step); });
+    } else {
+        for (int step = 1; step <= max_rounds; step++) {
+            launch_round(P, step);
+            if (step > kAhead && wait_round(P, step - kAhead) == kRoundsOver) break;
+        }
+        check(hipGetLastError(), "round launch");
+    }
+    if (sync_type != MEGAKERNEL_ID && !P->replicas)  // what the last round moved
+        hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(kMaxRoundUnits), 0, s, P->Mr, P->D, P->R, max_rounds + 1);
+    check(hipEventRecord(P->ev1, s), "event");
 }
 
 // A complete run of one bound vector, each round one launch (two with split
@@ -1674,24 +1757,9 @@ RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, in
     __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
     hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R);
-    hipLaunchKernelGGL(load_rounds_kernel, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
+    hipLaunchKernelGGL(load_rounds_kernel<false>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
     check(hipGetLastError(), "load launch");
-    check(hipEventRecord(P->ev0, s), "event");
-    if (sync_type == MEGAKERNEL_ID) {
-        void *args[] = {const_cast<DevMatrix *>(&M), &P->D, &R};
-        check(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(rounds_kernel), dim3(P->rounds_grid),
-                                         dim3(P->rounds_threads), args, 0, s),
-              "rounds_kernel launch");
-    } else if (sync_type == GPU_LOOP_ID && P->graphs_enabled) {
-        run_graphs(P, (1LL << 40) + max_rounds, max_rounds, [&](int step) { launch_round(P, step); });
-    } else {
-        for (int step = 1; step <= max_rounds; step++) {
-            launch_round(P, step);
-            if (step > kAhead && wait_round(P, step - kAhead) == kRoundsOver) break;
-        }
-        check(hipGetLastError(), "round launch");
-    }
-    check(hipEventRecord(P->ev1, s), "event");
+    issue_rounds(P, sync_type, max_rounds);
     hipLaunchKernelGGL(unpack_rounds_kernel, dim3(std::min(gx, 256)), dim3(256), 0, s, M, P->D, R);
     check(hipGetLastError(), "unpack launch");
     check(hipStreamSynchronize(s), "rounds sync");
@@ -1702,6 +1770,50 @@ RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, in
     if (!st.crossed) check(hipEventElapsedTime(&ms, P->ev0, P->ev1), "elapsed");
     r.kernel_ms = ms;
     return r;
+}
+
+// The outcomes of a finished run from its units' states.
+void run_outcomes(Problem *P, int n_list, const UnitState *st, RunResult *out) {
+    bool any_active = false;
+    for (int k = 0; k < n_list; k++) {
+        if (st[k].error) throw std::runtime_error("device wait timed out");
+        // bounds outside the envelope are an error, the vectors left alone
+        if (st[k].envelope) throw std::runtime_error("bounds outside the problem's bound envelope");
+        any_active |= !st[k].crossed;
+    }
+    float ms = 0.f;
+    if (any_active) check(hipEventElapsedTime(&ms, P->ev0, P->ev1), "elapsed");
+    for (int k = 0; k < n_list; k++) {
+        out[k] = outcome(st[k]);
+        out[k].kernel_ms = ms;
+    }
+}
+
+// A complete run of a batch, its rounds launches (two each, three with split
+// rows) or one persistent launch.
+void run_batch_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds, RunResult *out) {
+    if (sync_type < CPU_LOOP_ID || sync_type > MEGAKERNEL_ID) throw std::runtime_error("Unknown sync type");
+    if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
+    hipStream_t s = P->stream;
+    RoundPlan &R = P->R;
+    const DevMatrix &M = P->Mr;
+    const int NI = P->n_inst;
+    UnitState *st = reinterpret_cast<UnitState *>(P->h_tables.get(sizeof(UnitState) * NI));
+    R.lbs = d_lbs;
+    R.ubs = d_ubs;
+    R.max_rounds = max_rounds;
+    R.mark_limit = 1;
+    R.host_state = st;
+    const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
+    hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R);
+    hipLaunchKernelGGL(load_rounds_kernel<true>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
+    check(hipGetLastError(), "load launch");
+    __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
+    issue_rounds(P, sync_type, max_rounds);
+    hipLaunchKernelGGL(unpack_batch_rounds_kernel, dim3(gx), dim3(256), 0, s, M, P->D, R);
+    check(hipGetLastError(), "unpack launch");
+    check(hipStreamSynchronize(s), "rounds sync");
+    run_outcomes(P, NI, st, out);
 }
 
 // A complete run of the listed units from round 1.  The call waits once, for
@@ -1742,19 +1854,7 @@ void run_units(Problem *P, int n_list, const int *list, double *const *lbp, doub
                        n_list, P->d_list, st);
     check(hipGetLastError(), "run launches");
     check(hipStreamSynchronize(s), "run");
-    bool any_active = false;
-    for (int k = 0; k < n_list; k++) {
-        if (st[k].error) throw std::runtime_error("device wait timed out");
-        // bounds outside the envelope are an error, the vectors left alone
-        if (st[k].envelope) throw std::runtime_error("bounds outside the problem's bound envelope");
-        any_active |= !st[k].crossed;
-    }
-    float ms = 0.f;
-    if (any_active) check(hipEventElapsedTime(&ms, P->ev0, P->ev1), "elapsed");
-    for (int k = 0; k < n_list; k++) {
-        out[k] = outcome(st[k]);
-        out[k].kernel_ms = ms;
-    }
+    run_outcomes(P, n_list, st, out);
 }
 
 // A complete run of one bound vector (device pointers) as unit 0, from
@@ -2088,6 +2188,10 @@ void batch_propagate_device(Problem *P, double *d_lbs, double *d_ubs, int sync_t
     if (P->replicas) throw std::runtime_error("not a batch of instances");
     std::lock_guard<std::mutex> lock(P->run_mutex);
     ensure_units(P);
+    if (P->rounds_state) {
+        run_batch_rounds(P, d_lbs, d_ubs, sync_type, max_rounds, out);
+        return;
+    }
     std::vector<int> list(P->n_inst);
     for (int k = 0; k < P->n_inst; k++) list[k] = k;
     run_units(P, P->n_inst, list.data(), &d_lbs, &d_ubs, nullptr, nullptr, sync_type, max_rounds, out);

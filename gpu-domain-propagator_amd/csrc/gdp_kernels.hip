@@ -1670,8 +1670,11 @@ __device__ __forceinline__ DevState block_view(const DevMatrix &M, const DevStat
 // crossed.  Each wave takes `chunk` words of the bitmap at a time (one lane
 // each) and works through the nonzero ones two at a time, a half-wave per
 // word.
+// With kUnits (a batch), only words of the units in the run, run[u] != 0, are
+// folded: a unit that has crossed keeps the block of its last round as it is.
+template <bool kUnits>
 __device__ __forceinline__ bool carry_moved(const DevMatrix &M, const DevState &D, const RoundPlan &R, int step,
-                                            int wave, int nwaves) {
+                                            int wave, int nwaves, const int *run) {
     const DevState C = block_view(M, D, R, (step - 1) & 1);
     const DevState N = block_view(M, D, R, step & 1);
     const int lane = threadIdx.x & 63;
@@ -1696,10 +1699,18 @@ __device__ __forceinline__ bool carry_moved(const DevMatrix &M, const DevState &
             const unsigned wb = __shfl(bits, t < 0 ? 0 : t, 64);
             if (t < 0 || !((wb >> b) & 1u)) continue;
             const int id = (w0 + t) * 32 + b;
+            int unit = 0;
+            if constexpr (kUnits) {
+                unit = M.word_unit[w0 + t];
+                if (!run[unit]) continue;
+            }
             const AccRaw raw = acc_load(M, C, id);
             double l, u;
             acc_resolve(M, C, id, raw, l, u);
-            crossed |= eps_gt(l, u);
+            if (eps_gt(l, u)) {
+                crossed = true;
+                if constexpr (kUnits) atomic_max_i(&D.units[unit].infeasible, step - 1);
+            }
             if (id < M.n_int) {
                 atomic_max_i(&N.AI[id].x, static_cast<int>(static_cast<unsigned long long>(raw.w) & 0xffffffffull));
                 atomic_min_i(&N.AI[id].y, static_cast<int>(static_cast<unsigned long long>(raw.w) >> 32));
@@ -1759,37 +1770,48 @@ __device__ __forceinline__ int round_item(const DevMatrix &M, const DevState &V,
 // barrier's arrival slots for a run (one workgroup).
 __global__ __launch_bounds__(256) void reset_rounds_kernel(DevState D, RoundPlan R) {
     const int tid = threadIdx.x;
-    if (tid == 0) {
+    for (int u = tid; u < R.n_units; u += 256) {
         UnitState s = {};
         s.start = 1;
         s.markall = 1;
         s.max_rounds = R.max_rounds;
         s.mark_limit = R.mark_limit;
-        D.units[0] = s;
+        D.units[u] = s;
     }
     for (int k = tid; k < kStatusRows * kStatusWords; k += 256) D.status[k] = 0;
     for (int k = tid; k < kGlobalWords; k += 256) D.global[k] = 0;
-    for (int k = tid; k < 2 * kMoveLanes; k += 256) D.moved[moved_index(0, k & 1, k >> 1)] = 0;
-    for (int k = tid; k < 2 * kMaxGatherBlocks; k += 256) R.slots[k] = 0ull;
+    for (int k = tid; k < 2 * kMoveLanes * R.n_units; k += 256)
+        D.moved[moved_index(k / (2 * kMoveLanes), k & 1, (k >> 1) % kMoveLanes)] = 0;
+    for (int k = tid; k < 2 * kMaxGatherBlocks * R.slot_words; k += 256) R.slots[k] = 0ull;
 }
 
 // Loads the caller's vectors into both blocks and flags crossed bounds and
 // bounds outside a column's storage class (the storage classes of the
-// original matrix: n16, n_bin of the arguments).
+// original matrix: n16, n_bin of the arguments).  kUnits: a batch.
+template <bool kUnits>
 __global__ __launch_bounds__(256) void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin) {
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     const DevState A = block_view(M, D, R, 0), B = block_view(M, D, R, 1);
     for (int id = tid; id < M.n; id += stride) {
         const int j = M.perm[id];
-        const double l = R.lbs[j], u = R.ubs[j];
-        if (eps_gt(l, u)) atomic_or_i(&D.units[0].crossed, 1);
+        int unit = 0;
+        double l = 0.0, u = 0.0;
+        if (!kUnits || j >= 0) {  // a batch has padding ids
+            if constexpr (kUnits) unit = M.word_unit[id >> 5];
+            l = R.lbs[j];
+            u = R.ubs[j];
+        }
+        if (eps_gt(l, u)) atomic_or_i(&D.units[unit].crossed, 1);
         if (id < M.n_int) {
             const double lim = id < n16 ? 32767.0 : 2147483647.0;
             const double lo_lim = id < n_bin ? 0.0 : -lim, hi_lim = id < n_bin ? 1.0 : lim;
             const bool fits = l >= lo_lim && l <= hi_lim && u >= lo_lim && u <= hi_lim && floor(l) == l &&
                               floor(u) == u;
-            if (!fits && !eps_gt(l, u)) atomic_or_i(&D.units[0].envelope, 1);
+            if (!fits && !eps_gt(l, u)) {
+                atomic_or_i(&D.units[unit].envelope, 1);
+                if constexpr (kUnits) atomic_or_i(&D.global[kGlobalEnvelope], 1);
+            }
             const int2 v = make_int2(fits ? static_cast<int>(l) : 0, fits ? static_cast<int>(u) : 0);
             A.AI[id] = v;
             B.AI[id] = v;
@@ -1808,12 +1830,15 @@ __global__ __launch_bounds__(256) void load_rounds_kernel(DevMatrix M, DevState 
     for (int q = tid; q < M.n_seg_rows; q += stride) D.seg_count[q] = 0u;
 }
 
+template __global__ void load_rounds_kernel<false>(DevMatrix, DevState, RoundPlan, int, int);
+template __global__ void load_rounds_kernel<true>(DevMatrix, DevState, RoundPlan, int, int);
+
 // Whether a round moved a bound, for the launches: the round's number in any
 // of kMoveLanes words, each on its own line, by parity (the last rounds of
 // each parity, so that no round has to clear them).  Writers look first: a
 // store that every workgroup sends to one line costs about 50 ns each.
-__device__ __forceinline__ void note_round_moved(const DevState &D, int step) {
-    int *w = &D.moved[moved_index(0, step & 1, blockIdx.x % kMoveLanes)];
+__device__ __forceinline__ void note_round_moved(const DevState &D, int step, int unit = 0) {
+    int *w = &D.moved[moved_index(unit, step & 1, blockIdx.x % kMoveLanes)];
     if (coherent_load(w) != step) coherent_store(w, step);
 }
 __device__ __forceinline__ bool round_moved(const DevState &D, int step) {
@@ -1841,7 +1866,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void r
     const int nwaves = gridDim.x * waves;
     int *st = status_row(D, step);
     const DevState V = round_view(M, D, R, step);
-    if (step > 1 && carry_moved(M, D, R, step, wave, nwaves)) atomic_max_i(&D.units[0].infeasible, step - 1);
+    if (step > 1 && carry_moved<false>(M, D, R, step, wave, nwaves, nullptr)) atomic_max_i(&D.units[0].infeasible, step - 1);
     int moved = 0;
     for (int it = wave; it < R.n_items; it += nwaves) moved |= round_item<kWide>(M, V, R, it, step, st);
     if (__any(moved != 0) && (threadIdx.x & 63) == 0) any_moved = 1;
@@ -1931,7 +1956,7 @@ __global__ __launch_bounds__(1024) void rounds_kernel(DevMatrix M, DevState D, R
         int *st = status_row(D, step);
         const DevState V = round_view(M, D, R, step);
         unsigned flags = 0u;
-        if (step > 1 && carry_moved(M, D, R, step, wave, nwaves)) flags |= kCrossed;
+        if (step > 1 && carry_moved<false>(M, D, R, step, wave, nwaves, nullptr)) flags |= kCrossed;
         for (int it = wave; it < R.n_items; it += nwaves)
             if (round_item<kWideCoherent>(M, V, R, it, step, st)) flags |= kMoved;
         ok = gather_barrier(D, R, ++seq, flags, wg_flags, all);
@@ -1958,6 +1983,285 @@ __global__ __launch_bounds__(1024) void rounds_kernel(DevMatrix M, DevState D, R
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         D.units[0].infeasible = infeasible;
         D.moved[moved_index(0, last & 1, 0)] = last;
+    }
+}
+
+// The gather barrier with a bit per unit of a batch: a workgroup's arrival is
+// R.slot_words words, each the sequence number and the bits of 31 units (bit
+// 31: a crossed unit among them), so that every word shows by itself that it
+// has arrived.  All waves poll, 64 workgroups' words of one kind each.
+// own / all (LDS, 2 x kMaxSlotWords, zero at first): the workgroup's bits and
+// the union, two sets in turn.
+__device__ __forceinline__ bool gather_units(const DevState &D, const RoundPlan &R, unsigned seq,
+                                             unsigned (*own)[kMaxSlotWords], unsigned (*all)[kMaxSlotWords],
+                                             int *wg_ok) {
+    const int set = seq & 1;
+    mem_wait();
+    __syncthreads();
+    unsigned long long *slots = R.slots + static_cast<size_t>(set) * kMaxGatherBlocks * R.slot_words;
+    const int tid = threadIdx.x, lane = tid & 63, nb = gridDim.x;
+    if (tid < R.slot_words)
+        coherent_store(&slots[tid * kMaxGatherBlocks + blockIdx.x],
+                       (static_cast<unsigned long long>(seq) << 32) | own[set][tid]);
+    if (tid < kMaxSlotWords) {
+        own[set ^ 1][tid] = 0u;
+        all[set ^ 1][tid] = 0u;
+    }
+    const int groups = (nb + 63) / 64;
+    const long long t0 = wall_clock64();
+    for (int c = uniform(tid >> 6); c < groups * R.slot_words; c += blockDim.x >> 6) {
+        const int word = c / groups, k = (c - word * groups) * 64 + lane;
+        unsigned got = 0u;
+        while (true) {
+            const unsigned long long v = k < nb ? coherent_load(&slots[word * kMaxGatherBlocks + k])
+                                                : (static_cast<unsigned long long>(seq) << 32);
+            if (!__any(static_cast<unsigned>(v >> 32) != seq)) {
+                got = static_cast<unsigned>(v);
+                break;
+            }
+            if (wall_clock64() - t0 > kWaitTimeoutTicks || coherent_load(&D.global[kGlobalError])) {
+                if (lane == 0) {
+                    atomic_or_i(&D.global[kGlobalError], 1);
+                    *wg_ok = 0;
+                }
+                break;
+            }
+        }
+#pragma unroll
+        for (int h = 1; h < 64; h <<= 1) got |= static_cast<unsigned>(__shfl_xor(static_cast<int>(got), h, 64));
+        if (lane == 0 && got) atomicOr(&all[set][word], got);
+    }
+    __syncthreads();
+    return *wg_ok != 0;
+}
+
+// The running totals of the items of the instances in the run, by one wave.
+__device__ __forceinline__ void run_totals(int n_units, const int *run, const int *first, int *upto) {
+    const int lane = threadIdx.x & 63;
+    int before = 0;
+    for (int u0 = 0; u0 < n_units; u0 += 64) {
+        const int u = u0 + lane;
+        int inc = run[u] ? first[u + 1] - first[u] : 0;
+#pragma unroll
+        for (int h = 1; h < 64; h <<= 1) {
+            const int x = __shfl_up(inc, h, 64);
+            if (lane >= h) inc += x;
+        }
+        upto[u] = before + inc;
+        before += __shfl(inc, 63, 64);
+    }
+}
+// The instance whose item is the t-th of the round: one LDS read and a ballot
+// per 64 instances.
+__device__ __forceinline__ int run_unit(int n_units, const int *upto, int t) {
+    int u = 0;
+    for (int u0 = 0; u0 < n_units; u0 += 64)
+        u += __popcll(__ballot(upto[u0 + static_cast<int>(threadIdx.x & 63)] <= t));
+    return uniform(u);
+}
+
+// The rounds of a batch in one persistent launch: the instances side by side
+// in the two blocks, each round over the items of the instances that moved a
+// bound in the round before.  Every workgroup learns the moved and crossed
+// instances from the barrier and keeps its own list of them, with the running
+// totals of their items, in LDS.
+// Bound by the bounds' gathers while most instances run, by the barrier and
+// one pass's chain of loads, butterfly and divisions (8 us) in the tail.  64
+// instances of 42,000 entries, 58 rounds: 17 us a round (three phases: 47).
+__global__ __launch_bounds__(1024) void batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
+    __shared__ int run[kMaxRoundUnits];      // the instance takes part in the round
+    __shared__ int last[kMaxRoundUnits];     // its last round that moved a bound
+    __shared__ int first[kMaxRoundUnits + 1];  // its first item
+    __shared__ int upto[kMaxRoundUnits];     // items of the instances in the run up to and with this one
+    __shared__ unsigned own[2][kMaxSlotWords], all[2][kMaxSlotWords];
+    __shared__ int wg_ok;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int waves = blockDim.x >> 6;
+    const int wave = uniform(blockIdx.x * waves + (tid >> 6));
+    const int nwaves = gridDim.x * waves;
+    const int n_units = R.n_units;
+    for (int u = tid; u < kMaxRoundUnits; u += blockDim.x) {
+        // neither crossed nor outside the envelope
+        run[u] = u < n_units && coherent_load(reinterpret_cast<const long long *>(&D.units[u]) + 2) == 0;
+        last[u] = 0;
+    }
+    for (int u = tid; u <= n_units; u += blockDim.x) first[u] = R.unit_item[u];
+    if (tid < kMaxSlotWords) own[0][tid] = own[1][tid] = all[0][tid] = all[1][tid] = 0u;
+    if (tid == 0) wg_ok = 1;
+    __syncthreads();
+    unsigned seq = 0;
+    for (int step = 1; step <= R.max_rounds; step++) {
+        if (tid < 64) run_totals(n_units, run, first, upto);
+        __syncthreads();
+        const int total = upto[(n_units - 1) | 63];
+        if (total == 0) break;
+        int *st = status_row(D, step);
+        const DevState V = round_view(M, D, R, step);
+        const int set = (seq + 1) & 1;
+        if (step > 1 && carry_moved<true>(M, D, R, step, wave, nwaves, run))
+            for (int k = 0; k < R.slot_words; k++) atomicOr(&own[set][k], 1u << 31);
+        for (int t = wave; t < total; t += nwaves) {
+            const int u = run_unit(n_units, upto, t);
+            const int it = uniform(first[u + 1] - upto[u]) + t;
+            const int moved = round_item<kWideCoherent>(M, V, R, it, step, st);
+            if (__any(moved != 0) && lane == 0) atomicOr(&own[set][u / 31], 1u << (u % 31));
+        }
+        if (!gather_units(D, R, ++seq, own, all, &wg_ok)) break;
+        unsigned *seen = all[seq & 1];
+        bool crossed = false;
+        if (M.n_seg_parts > 0) {
+            const int count = coherent_load(&st[kStatusApply]);
+            if (count > 0) {
+                // (the bits of the round go on into the second barrier)
+                const int set2 = (seq + 1) & 1;
+                if (tid < R.slot_words) atomicOr(&own[set2][tid], seen[tid]);
+                for (int t = wave; t < count; t += nwaves) {
+                    const int task = coherent_load(&D.apply_tasks[t]);
+                    int u;
+                    const int moved = apply_split_task<kWideCoherent>(M, V, task, u);
+                    u = uniform(M.seg_rows[M.part_row[uniform(task)]].w);
+                    if (__any(moved != 0) && lane == 0) atomicOr(&own[set2][u / 31], 1u << (u % 31));
+                }
+                if (!gather_units(D, R, ++seq, own, all, &wg_ok)) break;
+                seen = all[seq & 1];
+            }
+        }
+        for (int k = 0; k < R.slot_words; k++) crossed |= (seen[k] >> 31) != 0;
+        for (int u = tid; u < n_units; u += blockDim.x) {
+            if (!run[u]) continue;
+            // (a workgroup ahead may already report crossings of this round)
+            if (crossed && coherent_load(&D.units[u].infeasible) == step - 1)
+                run[u] = 0;
+            else if ((seen[u / 31] >> (u % 31)) & 1u)
+                last[u] = step;
+            else
+                run[u] = 0;
+        }
+        __syncthreads();
+    }
+    if (blockIdx.x == 0)
+        for (int u = tid; u < n_units; u += blockDim.x) D.units[u].changed[last[u] & 1] = last[u];
+}
+
+// The rounds of a batch as launches.  Before round `step`, one workgroup finds
+// the instances that take part in it, notes the last rounds that moved a
+// bound, and tells the host how far the run is.
+__global__ __launch_bounds__(kMaxRoundUnits) void batch_plan_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+    __shared__ int run[kMaxRoundUnits], first[kMaxRoundUnits + 1], upto[kMaxRoundUnits];
+    const int u = threadIdx.x;
+    int in = 0;
+    if (u < R.n_units) {
+        first[u] = R.unit_item[u];
+        if (u == R.n_units - 1) first[u + 1] = R.unit_item[u + 1];
+        const UnitState &s = D.units[u];
+        if (step == 1) {
+            in = s.crossed == 0 && s.envelope == 0;
+        } else if (R.run[u] && s.infeasible == 0) {
+            for (int j = 0; j < kMoveLanes; j++) in |= D.moved[moved_index(u, (step - 1) & 1, j)] == step - 1;
+            if (in) D.units[u].changed[(step - 1) & 1] = step - 1;
+        }
+        R.run[u] = in;
+    }
+    run[u] = in;
+    __syncthreads();
+    if (u < 64) run_totals(R.n_units, run, first, upto);
+    __syncthreads();
+    if (u < R.n_units) R.upto[u] = upto[u];
+    if (u == 0)
+        __hip_atomic_store(D.host_word, upto[R.n_units - 1] > 0 ? step : kRoundsOver, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Round `step` of a batch; bounds as in batch_rounds_kernel, the kernel
+// boundaries in the barrier's place.  64 instances of 42,000 entries: 16 us a
+// round with its plan (three phases: 42).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void batch_round_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+    __shared__ int run[kMaxRoundUnits], first[kMaxRoundUnits + 1], upto[kMaxRoundUnits];
+    __shared__ unsigned moved_units[kMaxRoundUnits / 32];
+    const int tid = threadIdx.x;
+    const int n_units = R.n_units;
+    const int total = R.upto[n_units - 1];
+    if (total == 0) return;
+    run[tid] = tid < n_units ? R.run[tid] : 0;
+    upto[tid] = tid < n_units ? R.upto[tid] : total;
+    if (tid < n_units) first[tid + 1] = R.unit_item[tid + 1];
+    if (tid < kMaxRoundUnits / 32) moved_units[tid] = 0u;
+    __syncthreads();
+    const int wave = uniform(blockIdx.x * 4 + (tid >> 6));
+    const int nwaves = gridDim.x * 4;
+    int *st = status_row(D, step);
+    const DevState V = round_view(M, D, R, step);
+    if (step > 1) carry_moved<true>(M, D, R, step, wave, nwaves, run);
+    for (int t = wave; t < total; t += nwaves) {
+        const int u = run_unit(n_units, upto, t);
+        const int it = uniform(first[u + 1] - upto[u]) + t;
+        const int moved = round_item<kWide>(M, V, R, it, step, st);
+        if (__any(moved != 0) && (tid & 63) == 0) atomicOr(&moved_units[u >> 5], 1u << (u & 31));
+    }
+    __syncthreads();
+    if ((moved_units[tid >> 5] >> (tid & 31)) & 1u) note_round_moved(D, step, tid);
+}
+
+// The candidates of the batch's split rows whose gate passed in the round.
+__global__ __launch_bounds__(256) void batch_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+    const int count = coherent_load(&status_row(D, step)[kStatusApply]);
+    const DevState V = round_view(M, D, R, step);
+    for (int t = blockIdx.x * 4 + (threadIdx.x >> 6); t < count; t += gridDim.x * 4) {
+        const int task = uniform(coherent_load(&D.apply_tasks[t]));
+        int u;
+        const int moved = apply_split_task<kWide>(M, V, task, u);
+        if (__any(moved != 0) && (threadIdx.x & 63) == 0)
+            note_round_moved(D, step, M.seg_rows[M.part_row[task]].w);
+    }
+}
+
+// Writes the final bounds of a batch to the caller's vectors (not when some
+// input was outside its envelope), finds crossed bounds of the instances' last
+// rounds, and the last workgroup to finish writes the outcomes to pinned host
+// memory.
+__global__ __launch_bounds__(256) void unpack_batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
+    if (D.global[kGlobalEnvelope] == 0) {
+        const DevState A = block_view(M, D, R, 0), B = block_view(M, D, R, 1);
+        const int stride = gridDim.x * blockDim.x;
+        for (int id = blockIdx.x * blockDim.x + threadIdx.x; id < M.n; id += stride) {
+            const int j = M.perm[id];
+            if (j < 0) continue;
+            const int unit = M.word_unit[id >> 5];
+            const int c0 = D.units[unit].changed[0], c1 = D.units[unit].changed[1];
+            const int last = c0 > c1 ? c0 : c1;
+            const bool odd = last & 1;
+            double l, u;
+            if (id < M.n_int) {
+                const int2 a = odd ? B.AI[id] : A.AI[id];
+                l = static_cast<double>(a.x);
+                u = static_cast<double>(a.y);
+                if (a.x == kAiHigh || a.y == kAiLow) {
+                    const double2 x = odd ? B.AX[id] : A.AX[id];
+                    l = x.x > l ? x.x : l;
+                    u = x.y < u ? x.y : u;
+                }
+            } else {
+                const double2 a = odd ? B.AF[id - M.n_int] : A.AF[id - M.n_int];
+                l = a.x;
+                u = a.y;
+            }
+            if (last > 0 && eps_gt(l, u)) atomic_max_i(&D.units[unit].infeasible, last);
+            R.lbs[j] = l;
+            R.ubs[j] = u;
+        }
+    }
+    __shared__ int final_wg;
+    mem_wait();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        final_wg = atomic_add_i(&D.global[kGlobalTicket], 1) == static_cast<int>(gridDim.x) - 1;
+    __syncthreads();
+    if (!final_wg) return;
+    for (int u = threadIdx.x; u < R.n_units; u += blockDim.x) {
+        UnitState s = D.units[u];
+        s.infeasible = coherent_load(&D.units[u].infeasible);
+        s.error = coherent_load(&D.global[kGlobalError]);
+        R.host_state[u] = s;
     }
 }
 
