@@ -113,6 +113,17 @@ constexpr int kGlobalTicket = 2;   // workgroups of unpack_rounds_kernel that ar
 constexpr int kGlobalEnvelope = 3; // some loaded vector left the envelope (runs that then return an error)
 constexpr int kGlobalWords = 8;
 
+// Words of a run state that outlive its runs: row marks hold the step plus the
+// epoch, which starts beyond every earlier mark with each run, so that no run
+// has to clear them; whether an exact integer accumulator (AX) was written.
+constexpr int kPersistEpoch = 0;
+constexpr int kPersistAx = 1;
+constexpr int kPersistWords = 2;
+constexpr int kPersistAt = 32;    // first of them, from the global words
+constexpr int kEpochSteps = 128;  // steps of a run, rounded up
+// Loads and unpacks of this many vectors keep a vector to one XCD.
+constexpr int kVectorsByXcd = 64;
+
 // State of one unit (int32 words, read as 64-bit pairs).  A step's changes
 // go to slot step & 1 of `changed`, and step s asks slot (s - 1) & 1 whether
 // the unit moved in its previous round: writers and readers of one step
@@ -228,6 +239,7 @@ struct DevState {
     int *status;           // kStatusRows * kStatusWords ring
     int *global;           // kGlobalWords
     unsigned *barrier;     // kBarrierWords
+    int *persist;          // kPersistWords
     int *apply_tasks;      // unit * n_seg_parts + segment, per step
     const int *active;     // units of the launch (replicas mode)
     int n_active;
@@ -242,7 +254,7 @@ struct DevState {
 // starts with them in place of its own wherever it has the same bounds.
 struct ReferenceView {
     const SegPart *parts = nullptr;  // null: no reference
-    const double *lbs = nullptr, *ubs = nullptr;  // caller's column order
+    const double *lbs = nullptr, *ubs = nullptr;  // by internal id
     unsigned *diff = nullptr;        // per listed unit: columns that differ (nwords each)
     int *n_diff = nullptr;           // per listed unit: words of diff that are not zero
     int start = 0;                   // step that the copied partials are stamped with

@@ -58,9 +58,11 @@ __global__ void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
 __global__ void round_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
 __global__ void rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
-__global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status);
+__global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status,
+                                  int epoch);
+__global__ void clean_ax_kernel(DevState D, long long count);
 __global__ void load_kernel(DevMatrix M, DevState D, int n_list, const int *list, const double *const *lbp,
-                            const double *const *ubp, ReferenceView ref);
+                            const double *const *ubp, ReferenceView ref, int per_unit, int all);
 __global__ void load_reference_kernel(DevMatrix M, DevState V, ReferenceVectors R, double *lbs, double *ubs);
 __global__ void reference_parts_kernel(DevMatrix M, DevState V, SegPart *parts);
 __global__ void fill_parts_kernel(DevMatrix M, DevState D, int n_list, const int *list, int start_step, int chunk);
@@ -68,8 +70,8 @@ __global__ void drop_parts_kernel(DevMatrix M, DevState D, int n_list, const int
 __global__ void hint_kernel(DevMatrix M, DevState D, int n_list, const int *list, const int *hint_ptr,
                             const int *hints, const int *inv_perm, int start_step);
 __global__ void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list, double *const *lbp,
-                              double *const *ubp, int checked);
-__global__ void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int *list, double **lbp,
+                              double *const *ubp, int per_unit, int checked);
+__global__ void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int epoch, int *list, double **lbp,
                                  double **ubp, double *lbs, double *ubs);
 __global__ void report_kernel(DevState D, int n_list, const int *list, UnitState *out);
 __global__ void delta_kernel(int n_list, double *const *lbp, double *const *ubp, const int *ptr, const int *cols,
@@ -506,6 +508,8 @@ struct Problem {
     std::vector<void *> owned;       // matrix layout
     void *state_buf = nullptr;       // run state owned by the problem (carve_state), or null
     int capacity = 0;                // units with state arrays (replicas)
+    bool borrowed = false;           // the run state is not the problem's own
+    unsigned epoch = 0;              // of the marks in the own run state (kPersistEpoch)
     int n_units = 0;                 // entries of D.units
     std::vector<int> inst_ncols;     // blocks: columns per instance
     std::vector<int> mark_limit;     // per instance (blocks) or for every unit (replicas)
@@ -612,7 +616,7 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
     D.units = reinterpret_cast<UnitState *>(take(units * sizeof(UnitState)));
     D.moved = reinterpret_cast<int *>(take(units * kMoveSlots * kMoveLanes * kMoveStride * sizeof(int)));
     D.status = reinterpret_cast<int *>(take(kStatusRows * kStatusWords * sizeof(int)));
-    D.global = reinterpret_cast<int *>(take(kGlobalWords * sizeof(int)));
+    D.global = reinterpret_cast<int *>(take((kPersistAt + kPersistWords) * sizeof(int)));
     D.barrier = reinterpret_cast<unsigned *>(take(kBarrierWords * sizeof(unsigned)));
     T.list = reinterpret_cast<int *>(take(units * sizeof(int)));
     T.params = reinterpret_cast<int4 *>(take(units * sizeof(int4)));
@@ -627,6 +631,7 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
         D.wl_cnt = reinterpret_cast<unsigned long long *>(take(units * 2 * kCountWords * sizeof(unsigned long long)));
     }
     D.active = T.list;
+    D.persist = D.global ? D.global + kPersistAt : nullptr;
     return off;
 }
 
@@ -668,6 +673,37 @@ void bind_state(Problem *P, char *base, int cap, bool rounds, bool lists = true)
     P->n_units = P->replicas ? cap : P->n_inst;
 }
 
+// Clears the marks of the problem's own run state; their epochs start again.
+void clear_marks(Problem *P) {
+    const size_t k = P->replicas ? static_cast<size_t>(P->capacity) : 1;
+    check(hipMemsetAsync(P->D.marks, 0, sizeof(int) * k * P->M.m, P->stream), "memset marks");
+    if (P->M.n_seg_parts > 0)
+        check(hipMemsetAsync(P->D.seg_marks, 0, sizeof(int) * k * P->M.n_seg_parts, P->stream), "memset marks");
+    P->epoch = 0;
+}
+
+// The epoch of a new run of up to kEpochSteps steps.
+int next_epoch(Problem *P) {
+    if (P->borrowed) return 0;
+    if (P->epoch >= 1u << 30) clear_marks(P);
+    P->epoch += kEpochSteps;
+    return static_cast<int>(P->epoch);
+}
+
+// Grid of load_kernel and unpack_kernel: four columns a thread from the
+// number of vectors that fill the chip so, one column a thread for few.
+struct VectorGrid {
+    int per_unit, grid;
+};
+VectorGrid vector_grid(int n, int n_vectors) {
+    const int per_thread = n_vectors >= 16 ? 4 : 1;
+    VectorGrid g;
+    g.per_unit = std::max(1, std::min(1024, (n + 256 * per_thread - 1) / (256 * per_thread)));
+    const long long vectors = n_vectors >= kVectorsByXcd ? (n_vectors + 7) / 8 * 8LL : n_vectors;
+    g.grid = static_cast<int>(std::min<long long>(1 << 18, vectors * g.per_unit));
+    return g;
+}
+
 // Device state of `cap` units (replicas) or of the batch (blocks), owned by
 // the problem.
 void alloc_units(Problem *P, int cap) {
@@ -692,6 +728,13 @@ void alloc_units(Problem *P, int cap) {
     check(hipMemsetAsync(P->D.bm, 0, sizeof(unsigned) * k * M.nwords, P->stream), "memset");
     check(hipMemsetAsync(P->D.barrier, 0, sizeof(unsigned) * kBarrierWords, P->stream), "memset");
     check(hipMemsetAsync(P->D.global, 0, sizeof(int) * kGlobalWords, P->stream), "memset");
+    // what the loads leave alone: row marks, exact integer accumulators
+    clear_marks(P);
+    check(hipMemsetAsync(P->D.persist, 0, sizeof(int) * kPersistWords, P->stream), "memset");
+    const long long n_ax = static_cast<long long>(k) * M.n_int;
+    if (n_ax > 0)
+        hipLaunchKernelGGL(clean_ax_kernel, dim3(static_cast<int>(std::min<long long>(2048, (n_ax + 255) / 256))),
+                           dim3(256), 0, P->stream, P->D, n_ax);
     check(hipStreamSynchronize(P->stream), "alloc sync");
     P->stats.n_units = P->n_units;
 }
@@ -1520,10 +1563,11 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
         const bool hinted = hint_ptr != nullptr && hint_ptr[k + 1] > hint_ptr[k] && M.mark_rows;
         return make_int4(u, P->mark_limit[P->replicas ? 0 : u], hinted ? 0 : 1, max_rounds[k]);
     };
+    const int epoch = fresh ? next_epoch(P) : 0;
     if (n_list == 1) {
         // a single vector: everything by kernel argument
-        hipLaunchKernelGGL(reset_one_kernel, dim3(1), dim3(256), 0, s, D, param(0), start, fresh ? 1 : 0, P->d_list,
-                           P->d_lbp, P->d_ubp, lbp[0], ubp[0]);
+        hipLaunchKernelGGL(reset_one_kernel, dim3(1), dim3(256), 0, s, D, param(0), start, fresh ? 1 : 0, epoch,
+                           P->d_list, P->d_lbp, P->d_ubp, lbp[0], ubp[0]);
     } else {
         // the tables lie one after the other in the run state: one copy
         const int n_tables = P->replicas ? n_list : 1;
@@ -1536,19 +1580,20 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
         std::memcpy(at(P->d_lbp), lbp, sizeof(double *) * n_tables);
         std::memcpy(at(P->d_ubp), ubp, sizeof(double *) * n_tables);
         check(hipMemcpyAsync(base, h, bytes, hipMemcpyHostToDevice, s), "H2D tables");
-        hipLaunchKernelGGL(unit_reset_kernel, dim3(std::max(1, std::min(64, (n_list + 255) / 256))), dim3(256), 0, s, D,
-                           n_list, P->d_params, start, fresh ? 1 : 0);
+        hipLaunchKernelGGL(unit_reset_kernel, dim3(std::max(1, std::min(256, (n_list + 3) / 4))), dim3(256), 0, s, D,
+                           n_list, P->d_params, start, fresh ? 1 : 0, epoch);
     }
-    const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
-    const int gy = P->replicas ? std::max(1, std::min(n_list, 1024)) : 1;
+    const VectorGrid g = vector_grid(M.n, P->replicas ? n_list : 1);
     ReferenceView ref;
     if (referenced) ref = reference_view(P, n_list, start);
-    hipLaunchKernelGGL(load_kernel, dim3(gx, gy), dim3(256), 0, s, M, D, n_list, P->d_list, P->d_lbp, P->d_ubp, ref);
+    hipLaunchKernelGGL(load_kernel, dim3(g.grid), dim3(256), 0, s, M, D, n_list, P->d_list, P->d_lbp, P->d_ubp, ref,
+                       g.per_unit, P->borrowed ? 1 : 0);
     if (referenced) {
         // walking the columns of up to this many words costs less than an
         // eighth of the unit's segments
         const int limit = std::max(16, M.nwords / 64);
-        hipLaunchKernelGGL(drop_parts_kernel, dim3(std::max(1, std::min(8, (M.nwords + 255) / 256)), gy), dim3(256), 0, s,
+        hipLaunchKernelGGL(drop_parts_kernel, dim3(std::max(1, std::min(8, (M.nwords + 255) / 256)),
+                                                   std::max(1, std::min(n_list, 1024))), dim3(256), 0, s,
                            M, D, n_list, P->d_list, ref, limit);
     }
     check(hipGetLastError(), "load launch");
@@ -1583,7 +1628,10 @@ void launch_step(Problem *P, int step, int guard, int first_step) {
                        P->n_units);
     if (M.n_seg_parts > 0)
         hipLaunchKernelGGL(apply_split_kernel, dim3(apply_grid), dim3(256), 0, s, M, D, step, guard, first_step);
-    const long long pub_waves = static_cast<long long>(P->replicas ? D.n_active : 1) * ((M.nwords + 7) / 8);
+    // 8 bitmap words a wave, 64 from where that still fills the chip
+    const long long pub_units = P->replicas ? D.n_active : 1;
+    long long pub_waves = pub_units * ((M.nwords + 7) / 8);
+    if (P->replicas && pub_units * ((M.nwords + 63) / 64) >= 4096) pub_waves = pub_units * ((M.nwords + 63) / 64);
     hipLaunchKernelGGL(publish_kernel, dim3(std::max(1, std::min(8192, grid_for(pub_waves)))), dim3(256), 0, s, M, D,
                        step, guard, first_step, P->n_units);
 }
@@ -1834,10 +1882,9 @@ void run_units(Problem *P, int n_list, const int *list, double *const *lbp, doub
     if (related) set_reference(P, lbp, ubp, n_list);
     load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps, 1, true, related);
     run_steps(P, sync_type, max_rounds);
-    const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
-    const int gy = P->replicas ? std::max(1, std::min(n_list, 1024)) : 1;
-    hipLaunchKernelGGL(unpack_kernel, dim3(gx, gy), dim3(256), 0, s, P->M, P->D, n_list, P->d_list, P->d_lbp, P->d_ubp,
-                       1);
+    const VectorGrid g = vector_grid(P->M.n, P->replicas ? n_list : 1);
+    hipLaunchKernelGGL(unpack_kernel, dim3(g.grid), dim3(256), 0, s, P->M, P->D, n_list, P->d_list, P->d_lbp, P->d_ubp,
+                       g.per_unit, 1);
     // (the tables' pinned copy is free again: the run has read it)
     UnitState *st = &P->host->state;
     if (n_list > 1) {
@@ -2019,6 +2066,7 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
             if (step == 1 ? st[0].crossed != 0 : !active_after(st[0], step - 1)) break;
             RoundWork w;
             const bool all_rows = !M.mark_rows || st[0].markall == step;
+            const int mark = step + static_cast<int>(P->epoch);
             if (!all_rows) {
                 check(hipMemcpy(marks.data(), P->D.marks, sizeof(int) * M.m, hipMemcpyDeviceToHost), "D2H marks");
                 if (M.n_seg_parts > 0)
@@ -2039,10 +2087,10 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
             for (int r = 0; r < M.m; r++) {
                 if (!all_rows) {
                     // a split row is processed when one of its segments is marked
-                    bool marked = marks[r] == step;
+                    bool marked = marks[r] == mark;
                     if (split_of[r] >= 0) {
                         const int4 sr = seg_rows[split_of[r]];
-                        marked = std::find(&seg_marks[sr.y], &seg_marks[sr.y] + sr.z, step) != &seg_marks[sr.y] + sr.z;
+                        marked = std::find(&seg_marks[sr.y], &seg_marks[sr.y] + sr.z, mark) != &seg_marks[sr.y] + sr.z;
                     }
                     if (!marked) continue;
                 }
@@ -2057,7 +2105,7 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
                 }
                 for (int g = 0; g < seg_rows[q].z; g++) {
                     const int part = seg_rows[q].y + g;
-                    if (!all_rows && seg_stamp[part] >= 1 && seg_marks[part] != step) continue;
+                    if (!all_rows && seg_stamp[part] >= 1 && seg_marks[part] != mark) continue;
                     seg_stamp[part] = step;
                     count_entries(start, g * kSegLen, std::min(len, (g + 1) * kSegLen));
                 }
@@ -2075,8 +2123,8 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
         }
         res = outcome(st[0]);
         const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
-        hipLaunchKernelGGL(unpack_kernel, dim3(gx, 1), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                           P->d_ubp, 0);
+        hipLaunchKernelGGL(unpack_kernel, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
+                           P->d_ubp, gx, 0);
         check(hipGetLastError(), "unpack launch");
         check(hipStreamSynchronize(s), "unpack sync");
         check(hipMemcpy(lbs, d_b, n * sizeof(double), hipMemcpyDeviceToHost), "D2H lbs");
@@ -2133,8 +2181,8 @@ RunResult problem_propagate_measured(Problem *P, double *lbs, double *ubs, int m
             if (step == 1 ? st[0].crossed != 0 : !active_after(st[0], step - 1)) break;
             launch_step(P, step, 0, 1);
             check(hipGetLastError(), "step launch");
-            hipLaunchKernelGGL(unpack_kernel, dim3(gx, 1), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                               P->d_ubp, 0);
+            hipLaunchKernelGGL(unpack_kernel, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
+                               P->d_ubp, gx, 0);
             hipLaunchKernelGGL(measure_kernel, dim3(gx), dim3(256), 0, s, n, d_b, d_b + n, d_w, d_w + n, d_l,
                                d_l + n, d_prev, d_prev + n, part_f, part_i);
             hipLaunchKernelGGL(measure_total_kernel, dim3(1), dim3(64), 0, s, gx, part_f, part_i, out_f + step - 1,
@@ -2144,8 +2192,8 @@ RunResult problem_propagate_measured(Problem *P, double *lbs, double *ubs, int m
             rounds = step;
         }
         res = outcome(st[0]);
-        hipLaunchKernelGGL(unpack_kernel, dim3(gx, 1), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                           P->d_ubp, 0);
+        hipLaunchKernelGGL(unpack_kernel, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
+                           P->d_ubp, gx, 0);
         check(hipGetLastError(), "unpack launch");
         check(hipStreamSynchronize(s), "unpack sync");
         fin.resize(rounds);
@@ -2247,8 +2295,10 @@ class BorrowedState {
         bind_state(P, base, 1, P->rounds_ok && need + carve_rounds(P->Mr, nullptr, R) <= kScratchBytes,
                    need <= kScratchBytes);
         P->graphs_enabled = false;
+        P->borrowed = true;
     }
     ~BorrowedState() {
+        P_->borrowed = false;
         P_->D = D_;
         P_->d_list = list_;
         P_->d_params = params_;
@@ -2566,6 +2616,7 @@ struct Server {
         if (cs) (void)hipStreamDestroy(cs);
         if (attached) {
             std::lock_guard<std::mutex> lock(P->run_mutex);
+            P->epoch += (static_cast<unsigned>(step) / kEpochSteps + 1) * kEpochSteps;  // its marks
             P->servers--;
         }
     }
@@ -2687,7 +2738,8 @@ Server *server_create(Problem *P, int64_t hbm_budget, int max_slots) {
         P->servers++;
         S->attached = true;
         // fresh status ring for the server's steps
-        hipLaunchKernelGGL(unit_reset_kernel, dim3(1), dim3(256), 0, P->stream, P->D, 0, P->d_params, 0, 1);
+        hipLaunchKernelGGL(unit_reset_kernel, dim3(1), dim3(256), 0, P->stream, P->D, 0, P->d_params, 0, 1,
+                           next_epoch(P));
         check(hipStreamSynchronize(P->stream), "server init");
     } catch (...) {
         delete S;
@@ -3164,9 +3216,9 @@ int step_impl(Server *S) {
         upload(P->d_lbp, lbp.data(), fin.size(), s);
         upload(P->d_ubp, ubp.data(), fin.size(), s);
         const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
-        hipLaunchKernelGGL(unpack_kernel, dim3(gx, std::max(1, std::min(static_cast<int>(fin.size()), 1024))),
-                           dim3(256), 0, s, P->M, P->D, static_cast<int>(fin.size()), P->d_list, P->d_lbp, P->d_ubp,
-                           0);
+        const VectorGrid g = vector_grid(P->M.n, static_cast<int>(fin.size()));
+        hipLaunchKernelGGL(unpack_kernel, dim3(g.grid), dim3(256), 0, s, P->M, P->D, static_cast<int>(fin.size()),
+                           P->d_list, P->d_lbp, P->d_ubp, g.per_unit, 0);
         check(hipGetLastError(), "unpack launch");
         std::vector<Server::Done> out(fin.size());
         // delta requests (against the base vector) and in-place zero-copy

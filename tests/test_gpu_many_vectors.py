@@ -1,0 +1,84 @@
+"""Loads, unpacks and publishes of many bound vectors, and what a run state
+keeps from one run to the next: each vector bit for bit the round-synchronous
+oracle's.
+
+Sizes: vectors around the line from which a vector's workgroups share an XCD
+(64) and not a multiple of 8; columns around a workgroup's 1024 and a wave's
+64, binary columns ending inside a wave; as many bitmap words as make a
+publishing wave take 64 of them.
+"""
+import numpy as np
+import pytest
+
+import fixtures
+from gdp_amd import interface as I
+from gdp_amd.instances import powerlaw_mip, small_mip, tighten_node
+
+pytestmark = pytest.mark.gpu
+
+SYNCS = [I.CPU_LOOP, I.GPU_LOOP, I.MEGAKERNEL]
+
+
+def _children(inst, oracle, count, seed):
+    lb, ub = oracle.jacobi(inst)[:2]
+    rng = np.random.default_rng(seed)
+    out = []
+    for _ in range(count):
+        l, u, cols = tighten_node(inst, rng, 1, 9, lb, ub)
+        out.append((l, u, cols, oracle.jacobi(inst.with_bounds(l, u))))
+    return out
+
+
+def _run(p, nodes, pick, sync, hints=True):
+    got = p.propagate_nodes([nodes[k][0] for k in pick], [nodes[k][1] for k in pick],
+                            hints=[nodes[k][2] for k in pick] if hints else None, sync_type=sync)
+    for i, (k, g) in enumerate(zip(pick, got)):
+        exp = nodes[k][3]
+        np.testing.assert_array_equal(g.lbs, exp[0], err_msg=f"vector {i} of {len(pick)} sync={sync}")
+        np.testing.assert_array_equal(g.ubs, exp[1], err_msg=f"vector {i} of {len(pick)} sync={sync}")
+        assert (g.rounds, g.infeasible, g.capped) == exp[2:]
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 1023, 1025, 4100])
+def test_columns_and_vectors(gpu, oracle, n):
+    inst = powerlaw_mip(seed=n, m=2 * n + 30, n=n, len_hi=max(8, n // 2), s=1.7)
+    nodes = _children(inst, oracle, 7, n)
+    print(f"many vectors: n={n}", flush=True)
+    p = I.Problem(inst)
+    try:
+        for count in (1, 15, 16, 63, 64, 67):
+            for sync in SYNCS:
+                _run(p, nodes, [k % 7 for k in range(count)], sync, hints=count != 67)
+    finally:
+        p.close()
+
+
+@pytest.mark.parametrize("hints", [True, False])
+def test_wide_publish(gpu, oracle, hints):
+    inst = small_mip(seed=8, m=9000, n=30000, len_hi=9)
+    nodes = _children(inst, oracle, 5, 3)
+    p = I.Problem(inst)
+    try:
+        for sync in SYNCS:
+            print(f"many vectors: 300, sync={sync} hints={hints}", flush=True)
+            _run(p, nodes, [k % 5 for k in range(300)], sync, hints)
+    finally:
+        p.close()
+
+
+def test_integers_beyond_int32_and_back(gpu, oracle):
+    """A run that needs the exact integer accumulators, then runs of the same
+    state that must find them clean, several times over."""
+    inst = fixtures.int32_overflow()
+    tight_ub = inst.ub.copy()
+    ints = np.flatnonzero((inst.vartype != 3) & (inst.ub < 1e9) & (inst.lb > -1e9))
+    tight_ub[ints] = inst.lb[ints]
+    nodes = [(inst.lb, inst.ub, np.arange(inst.n, dtype=np.int32), oracle.jacobi(inst)),
+             (inst.lb, tight_ub, ints.astype(np.int32), oracle.jacobi(inst.with_bounds(inst.lb, tight_ub)))]
+    p = I.Problem(inst)
+    try:
+        for sync in SYNCS:
+            for pick in ([1, 1, 1], [1, 0, 1], [1, 1, 0], [0, 1, 1], [1, 1, 1]):
+                _run(p, nodes, pick, sync, hints=False)
+    finally:
+        p.close()
