@@ -272,14 +272,23 @@ struct ReferenceVectors {
 // still holds S_{s-2}; the columns that round s - 1 moved are folded into it
 // in the same phase (maximum and minimum commute), so that at the end of the
 // round it holds S_s.  A round is then one phase, with one kernel boundary or
-// one grid barrier, in place of sweep, apply and publish.  Every round
-// processes every row: no marks.  Crossed bounds of round s - 1 are found
+// one grid barrier, in place of sweep, apply and publish.  No marks:
+// from kMinTestItems items on, every workgroup copies the bitmap of the columns
+// that the round before moved to LDS, and a pass looks its columns up there
+// before it gathers anything; rows without a moved column would repeat the
+// candidates they had.  (On average over the rounds 35 to 55% of the entries lie
+// in rows with a moved column.)  Crossed bounds of round s - 1 are found
 // while its moved columns are folded in round s, whose own candidates are
 // then dropped with their block.
 // Records: int32 pairs for the integer columns, then FP64 pairs from byte
 // snap_offF (the DevMatrix of these kernels has n16 = 0, snap_off32 = 0).
 constexpr int kPlanBins = 9;          // tree widths 2^8 .. 2^0
 constexpr int kMaxGatherBlocks = 512; // workgroups of the persistent launch
+// Items from which a round looks for unmoved rows: one a wave of the persistent
+// launch.  Below, a round is the latency of one pass, which a lookup makes longer
+// (77,000 nonzeros: 7.3 us a round without, 7.8 with; 2.2M: 23 without, 18 with).
+constexpr int kMinTestItems = 4096;
+constexpr int kMaxBitWords = 16 << 10; // LDS copy of the moved columns: 64 KB
 constexpr int kMaxRoundUnits = 256;   // instances of a batch whose rounds run so (a multiple of 64)
 constexpr int kMaxSlotWords = (kMaxRoundUnits + 30) / 31;
 // Where each tree-width bin's rows and items start (building the item list).
@@ -296,7 +305,8 @@ struct RoundPlan {
     const int4 *items;                // as DevMatrix's: one segment of a split row, or one pass of rows
     char *block[2];
     double2 *AX[2];                   // exact integer values beyond int32, per block
-    unsigned *bm[2];                  // columns moved in a round, by parity
+    unsigned *bm[3];                  // columns moved in a round, by round % 3
+    int bit_words;                    // words of a workgroup's LDS copy of one (a power of two)
     unsigned long long *slots;        // arrivals of the persistent launch's barrier, two sets
     double *lbs, *ubs;                // the caller's vectors
     int mark_limit, max_rounds;

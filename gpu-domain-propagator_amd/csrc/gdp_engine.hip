@@ -49,13 +49,17 @@ __global__ void plan_rounds_kernel(DevMatrix M, RoundBins B, int4 *items);
 __global__ void reset_rounds_kernel(DevState D, RoundPlan R);
 template <bool kUnits>
 __global__ void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin);
+template <bool kTest>
 __global__ void batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void batch_plan_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
+template <bool kTest>
 __global__ void batch_round_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
 __global__ void batch_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
 __global__ void unpack_batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
+template <bool kTest>
 __global__ void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
 __global__ void round_apply_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
+template <bool kTest>
 __global__ void rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status,
@@ -647,8 +651,8 @@ size_t carve_rounds(const DevMatrix &Mr, char *base, RoundPlan &R) {
     for (int k = 0; k < 2; k++) {
         R.block[k] = take(static_cast<size_t>(Mr.snap_stride));
         R.AX[k] = reinterpret_cast<double2 *>(take(Mr.n_int * sizeof(double2)));
-        R.bm[k] = reinterpret_cast<unsigned *>(take(Mr.nwords * sizeof(unsigned)));
     }
+    for (unsigned *&bm : R.bm) bm = reinterpret_cast<unsigned *>(take((Mr.nwords + 1) / 2 * 8));
     R.slots = reinterpret_cast<unsigned long long *>(take(2 * kMaxGatherBlocks * R.slot_words * sizeof(unsigned long long)));
     R.run = reinterpret_cast<int *>(take(R.n_units * sizeof(int)));
     R.upto = reinterpret_cast<int *>(take(R.n_units * sizeof(int)));
@@ -1051,6 +1055,15 @@ RowOrder device_row_order(const std::vector<InstanceView> &inst, const std::vect
     return R;
 }
 
+// The persistent kernel of the problem's double-buffered rounds.
+const void *rounds_fn(const Problem *P) {
+    if (P->replicas)
+        return P->R.bit_words > 0 ? reinterpret_cast<const void *>(rounds_kernel<true>)
+                                  : reinterpret_cast<const void *>(rounds_kernel<false>);
+    return P->R.bit_words > 0 ? reinterpret_cast<const void *>(batch_rounds_kernel<true>)
+                              : reinterpret_cast<const void *>(batch_rounds_kernel<false>);
+}
+
 // The plan of the double-buffered rounds of a problem with default tuning:
 // start / count hold the first layout row and the rows of each (bin key,
 // instance) run (key: 10 - log2 of the tree width), first_part the first
@@ -1059,25 +1072,23 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
                  const std::vector<int> &part_row, const std::vector<int4> &seg_rows, int n_padded) {
     const Tuning def;
     const Tuning &T = P->tuning;
-    // Every round processes every row, which costs about 8.5 ps per entry; the
-    // three-phase rounds of larger problems skip the rows whose columns did not
-    // move.  ms a call (three phases: persistent / host loop): 200,000 rows,
-    // 2.2M nonzeros, 32 rounds 0.73 (1.15 / 1.03); 3.1M nonzeros over 500,000
-    // columns, 65 rounds 1.91 (2.39 / 1.92); 3.3M 1.16 (1.62 / 1.37); 5.5M 1.72
-    // (1.82 / 1.64); 7.8M 2.56 (1.90 / 1.75).
-    constexpr int kMaxRoundEntries = 4 << 20;
-    // A batch leaves out the instances that are done, so its line lies higher,
-    // and higher still for small instances, whose numbers of rounds differ more.
-    // ms a call, persistent / loop, in brackets with three phases: 64 instances
-    // of 42,000 entries 0.99 / 0.95 (2.77 / 2.45), of 88,000 2.38 / 2.35 (4.05 /
-    // 3.54), of 122,000 2.25 / 2.22 (2.80 / 2.41), of 233,000 4.16 / 4.00 (4.46 /
-    // 4.07); 24 of 480,000 3.57 / 3.66 (4.08 / 3.52); 6 of 1.5M 2.99 / 3.10 (3.03 /
-    // 2.66); 16 of 2.1M 10.8 / 11.9 (7.4 in the loop).
-    constexpr int kMaxBatchEntries = 8 << 20;
-    constexpr int kSmallInstance = 256 << 10;
+    // Every round streams every row's columns and works on the rows with moved
+    // ones (8.5 ps per entry when all are); the three-phase rounds of larger
+    // problems never touch the others.  ms a call, persistent / loop, in brackets
+    // with three phases: 200,000 rows, 2.2M nonzeros, 32 rounds 0.64 / 0.65 (1.15
+    // / 1.03); 3.1M over 500,000 columns, 65 rounds 1.4 (2.4 / 1.9); 5.5M 1.24 /
+    // 1.20 (1.80 / 1.65); 7.8M 1.65 / 1.69 (1.91 / 1.76); 9.0M with long rows 1.56
+    // / 1.47 (1.60 / 1.47); 12.6M over 1M columns, 2 rounds 0.25 (0.17); 20.1M 3.4
+    // / 3.3 (2.6 / 3.0).
+    constexpr int kMaxRoundEntries = 8 << 20;
+    // A batch leaves out the instances that are done, so its line lies higher:
+    // 64 instances of 42,000 entries 0.98 / 1.01 (2.77 / 2.45), of 88,000 2.2 (4.05 /
+    // 3.54), of 244,000 3.79 / 3.77 (4.87 / 4.42); 24 of 470,000 2.43 / 2.52 (3.11 /
+    // 2.82); 6 of 1.7M 2.14 / 2.22 (2.71 / 2.41); 8 of 2.8M 3.60 / 3.59 (3.49 / 3.46);
+    // 16 of 2.0M 7.7 / 7.9 (6.9 / 6.9).
+    constexpr int kMaxBatchEntries = 16 << 20;
     const int NI = P->n_inst;
-    if (P->replicas ? NI != 1 || n_padded > kMaxRoundEntries
-                    : NI > kMaxRoundUnits || n_padded > (n_padded / NI <= kSmallInstance ? 2 : 1) * kMaxBatchEntries)
+    if (P->replicas ? NI != 1 || n_padded > kMaxRoundEntries : NI > kMaxRoundUnits || n_padded > kMaxBatchEntries)
         return;
     if (T.item_nnz != def.item_nnz || T.mega_blocks_per_cu != def.mega_blocks_per_cu ||
         T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
@@ -1156,9 +1167,15 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     // them (1.2 us for 16, 3 us for 256, 4.3 us for 512), and a workgroup of 256
     // threads spreads few items over more compute units
     P->rounds_threads = R.n_items <= 1024 ? 256 : (R.n_items <= 2048 ? 512 : 1024);
-    const void *fn = P->replicas ? reinterpret_cast<const void *>(rounds_kernel)
-                                 : reinterpret_cast<const void *>(batch_rounds_kernel);
-    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, P->rounds_threads, 0), "occupancy");
+    // moved columns in LDS: up to 512K have a bit of their own
+    R.bit_words = 0;
+    if (R.n_items >= kMinTestItems) {
+        R.bit_words = 64;
+        while (R.bit_words < M.nwords && R.bit_words < kMaxBitWords) R.bit_words *= 2;
+    }
+    const size_t lds = sizeof(unsigned) * R.bit_words;
+    const void *fn = rounds_fn(P);
+    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, P->rounds_threads, lds), "occupancy");
     const int waves = P->rounds_threads / 64;
     P->rounds_grid = std::max(1, std::min({per_cu * P->cu_count, kMaxGatherBlocks, (R.n_items + waves - 1) / waves}));
     P->rounds_ok = true;
@@ -1752,16 +1769,21 @@ std::vector<UnitState> read_units(Problem *P, int n_list, const int *list) {
 
 // Issues round `step`.
 void launch_round(Problem *P, int step) {
-    const int grid = std::max(1, std::min(8 * P->cu_count, grid_for(P->R.n_items)));
+    // with a copy of the moved columns in LDS few large workgroups, all resident
+    const size_t lds = sizeof(unsigned) * P->R.bit_words;
+    const bool small = lds == 0;
+    const int threads = small ? 256 : 512;
+    const int waves = threads / 64;
+    const int grid = std::max(1, std::min((small ? 8 : 2) * P->cu_count, (P->R.n_items + waves - 1) / waves));
     const int apply_grid = std::max(1, std::min(1024, grid_for(P->Mr.n_seg_parts)));
     if (!P->replicas) {
         hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(kMaxRoundUnits), 0, P->stream, P->Mr, P->D, P->R, step);
-        hipLaunchKernelGGL(batch_round_kernel, dim3(grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+        hipLaunchKernelGGL(lds > 0 ? batch_round_kernel<true> : batch_round_kernel<false>, dim3(grid), dim3(threads), lds, P->stream, P->Mr, P->D, P->R, step);
         if (P->Mr.n_seg_parts > 0)
             hipLaunchKernelGGL(batch_apply_kernel, dim3(apply_grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
         return;
     }
-    hipLaunchKernelGGL(round_kernel, dim3(grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+    hipLaunchKernelGGL(lds > 0 ? round_kernel<true> : round_kernel<false>, dim3(grid), dim3(threads), lds, P->stream, P->Mr, P->D, P->R, step);
     if (P->Mr.n_seg_parts > 0)
         hipLaunchKernelGGL(round_apply_kernel, dim3(apply_grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
 }
@@ -1772,9 +1794,8 @@ void issue_rounds(Problem *P, int sync_type, int max_rounds) {
     check(hipEventRecord(P->ev0, s), "event");
     if (sync_type == MEGAKERNEL_ID) {
         void *args[] = {&P->Mr, &P->D, &P->R};
-        const void *fn = P->replicas ? reinterpret_cast<const void *>(rounds_kernel)
-                                     : reinterpret_cast<const void *>(batch_rounds_kernel);
-        check(hipLaunchCooperativeKernel(fn, dim3(P->rounds_grid), dim3(P->rounds_threads), args, 0, s),
+        check(hipLaunchCooperativeKernel(rounds_fn(P), dim3(P->rounds_grid), dim3(P->rounds_threads), args,
+                                         sizeof(unsigned) * P->R.bit_words, s),
               "rounds launch");
     } else if (sync_type == GPU_LOOP_ID && P->graphs_enabled) {
         run_graphs(P, (1LL << 40) + max_rounds, max_rounds, [&](int step) { launch_round(P, step); });

@@ -446,6 +446,14 @@ __device__ __forceinline__ int step_add(int v) {
     return a + b;
 }
 
+// The columns that the previous round moved, a bit each, in LDS: bit id of
+// word (id / 32) & mask (larger problems share words, which lets rows through
+// that have no moved column).  words null: every row counts as moved.
+struct MovedBits {
+    const unsigned *words;
+    unsigned mask;
+};
+
 // K consecutive entries of one lane: loads, contributions, pairwise tree of
 // the K contributions in natural order, and the cross-lane reduction.
 // A sweep is bound by its instructions as much as by its gathers (200,000
@@ -466,27 +474,54 @@ struct LaneEntries {
     __device__ __forceinline__ int max_inf() const { return infs >> 16; }
 
     __device__ __forceinline__ void load(const DevMatrix &M, const DevState &D, int base, int first, int len) {
-        // the lane's K entries in one go (base + first is a multiple of K and
-        // the row is padded to a multiple of kRowAlign, a multiple of K), a
-        // lane past the end the padding entries behind the last row
-        const size_t e = static_cast<size_t>(first < len ? base + first : M.n_padded);
-        const int *cp = M.col + e;
-        const double *vp = M.val + e;
+        const int e = place(M, base, first, len);
+        columns(M, e);
+        coefficients(M, e);
+        bounds(M, D);
+    }
+    // Where the lane's K entries lie (base + first is a multiple of K and the
+    // row is padded to a multiple of kRowAlign, a multiple of K): for a lane
+    // past the end, the padding entries behind the last row.
+    static __device__ __forceinline__ int place(const DevMatrix &M, int base, int first, int len) {
+        return first < len ? base + first : M.n_padded;
+    }
+    __device__ __forceinline__ void columns(const DevMatrix &M, int e) {
+        const int *cp = M.col + static_cast<size_t>(e);
         if constexpr (K == 4) {
             const int4 c = *reinterpret_cast<const int4 *>(cp);
-            const double2 v0 = *reinterpret_cast<const double2 *>(vp);
-            const double2 v1 = *reinterpret_cast<const double2 *>(vp + 2);
             jp[0] = c.x; jp[1] = c.y; jp[2] = c.z; jp[3] = c.w;
-            a[0] = v0.x; a[1] = v0.y; a[2] = v1.x; a[3] = v1.y;
         } else if constexpr (K == 2) {
             const int2 c = *reinterpret_cast<const int2 *>(cp);
-            const double2 v0 = *reinterpret_cast<const double2 *>(vp);
             jp[0] = c.x; jp[1] = c.y;
-            a[0] = v0.x; a[1] = v0.y;
         } else {
             jp[0] = *cp;
+        }
+    }
+    // Whether a bound of one of the lane's columns moved.
+    __device__ __forceinline__ bool moved(const MovedBits &B) const {
+        unsigned any = 0u;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const unsigned id = static_cast<unsigned>(jp[k] & kIdMask);
+            any |= B.words[(id >> 5) & B.mask] >> (id & 31);
+        }
+        return any & 1u;
+    }
+    __device__ __forceinline__ void coefficients(const DevMatrix &M, int e) {
+        const double *vp = M.val + static_cast<size_t>(e);
+        if constexpr (K == 4) {
+            const double2 v0 = *reinterpret_cast<const double2 *>(vp);
+            const double2 v1 = *reinterpret_cast<const double2 *>(vp + 2);
+            a[0] = v0.x; a[1] = v0.y; a[2] = v1.x; a[3] = v1.y;
+        } else if constexpr (K == 2) {
+            const double2 v0 = *reinterpret_cast<const double2 *>(vp);
+            a[0] = v0.x; a[1] = v0.y;
+        } else {
             a[0] = *vp;
         }
+    }
+    // The bounds, and the lane's contributions.
+    __device__ __forceinline__ void bounds(const DevMatrix &M, const DevState &D) {
         // every gather first, then the decoding and the contributions; binary
         // columns held in LDS are read there instead
         uint4 rec[K];
@@ -662,9 +697,11 @@ __device__ __forceinline__ Sink make_sink(const DevState &V) {
 
 // Rows [first, first + nrows) of one tree-width bin, or the nrows rows listed
 // at list[first ..]: groups of 2^logg lanes, K consecutive entries per lane.
-template <int K, int kMode>
+// With kTest, rows none of whose columns moved are left out: their lanes take
+// the padding entries.
+template <int K, int kMode, bool kTest = false>
 __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int first, int nrows, int logg,
-                                          const int *list) {
+                                          const int *list, const MovedBits &B = MovedBits{nullptr, 0u}) {
     const DevState &V = S.V;
     const int lane = lane_here();
     const int g = 1 << logg;
@@ -686,7 +723,22 @@ __device__ __forceinline__ int group_item(const DevMatrix &M, const Sink &S, int
             rhs = sd.y;
         }
         LaneEntries<K, kMode> E;
-        E.load(M, V, start, gl * K, len);
+        int e = E.place(M, start, gl * K, len);
+        E.columns(M, e);
+        if constexpr (kTest) {
+            if (B.words != nullptr) {
+                const unsigned long long rows = __ballot(E.moved(B));
+                if (rows == 0ull) continue;
+                if ((rows & gmask) == 0ull) {
+                    len = 0;
+                    e = M.n_padded;
+#pragma unroll
+                    for (int k = 0; k < K; k++) E.jp[k] = M.n;
+                }
+            }
+        }
+        E.coefficients(M, e);
+        E.bounds(M, V);
         E.template reduce<false>(g);
         const double minact = 0.0 + E.tmin;
         const double maxact = 0.0 + E.tmax;
@@ -801,9 +853,9 @@ __device__ __forceinline__ void segment_partial(const DevMatrix &M, const DevSta
 // adds the partials in segment order and decides the row gate; when it
 // passes, the row's activity is stored and its segments are queued for the
 // apply phase that follows the sweep.
-template <int kMode>
+template <int kMode, bool kTest = false>
 __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, const DevState &V, int u, int lr, int s,
-                                         int cnt, int *st, int step) {
+                                         int cnt, int *st, int step, const MovedBits &B = MovedBits{nullptr, 0u}) {
     const int lane = lane_here();
     const int4 info = M.seg_rows[lr];
     const int r = info.x;
@@ -811,15 +863,41 @@ __device__ __forceinline__ void seg_item(const DevMatrix &M, const DevState &D, 
     row_extent(M, r, start, len);
     const bool listed = cnt < 0;
     const int end = s + (listed ? 1 : cnt);
-    for (int q = s; q < end; q++) segment_partial<kMode>(M, V, info.y, q, start, len, step);
+    unsigned add = static_cast<unsigned>(listed ? -1 : cnt);
+    if constexpr (kTest) {
+        // a segment without moved columns keeps its partial of the round
+        // before; the upper half of the row's count holds the others
+        constexpr int K = kSegLen / 64;
+        const bool countable = info.z < 0x8000;
+        for (int q = s; q < end; q++) {
+            if (B.words != nullptr && countable) {
+                LaneEntries<K, kMode> E;
+                E.columns(M, E.place(M, start + q * kSegLen, lane * K, len - q * kSegLen));
+                if (!__any(E.moved(B))) continue;
+            }
+            if (countable) add += 0x10000u;
+            segment_partial<kMode>(M, V, info.y, q, start, len, step);
+        }
+    } else {
+        for (int q = s; q < end; q++) segment_partial<kMode>(M, V, info.y, q, start, len, step);
+    }
     unsigned old = 0;
     if (lane == 0) {
         mem_wait();
-        old = __hip_atomic_fetch_add(&V.seg_count[lr], static_cast<unsigned>(listed ? -1 : cnt), __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
+        old = __hip_atomic_fetch_add(&V.seg_count[lr], add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     old = __shfl(old, 0, 64);
-    if (listed ? old != 1u : old + cnt != static_cast<unsigned>(info.z)) return;
+    if constexpr (kTest) {
+        const unsigned now = old + add;
+        const bool countable = info.z < 0x8000;
+        if ((countable ? now & 0xffffu : now) != static_cast<unsigned>(info.z)) return;
+        if (countable && now >> 16 == 0u) {  // nothing of the row moved
+            if (lane == 0) coherent_store(&V.seg_count[lr], 0u);
+            return;
+        }
+    } else {
+        if (listed ? old != 1u : old + cnt != static_cast<unsigned>(info.z)) return;
+    }
 
     // the row is complete: the lanes load 64 partials at a time
     // (independent loads), which are then added in segment order
@@ -1649,6 +1727,54 @@ template __global__ void mega_kernel<1024, true>(DevMatrix, DevState, int, int, 
 // double-buffered rounds of one bound vector (gdp_device.h, RoundPlan)
 // ---------------------------------------------------------------------------
 
+// The bitmap of the columns that round `step` moves.  Three take turns: round
+// s reads the one of round s - 1 while it writes its own and clears that of
+// round s + 1.
+__device__ __forceinline__ unsigned *moved_bitmap(const RoundPlan &R, int step) {
+    const int k = step % 3;
+    return k == 0 ? R.bm[0] : (k == 1 ? R.bm[1] : R.bm[2]);
+}
+
+// The columns that the round before `step` moved, copied to LDS by the whole
+// workgroup, if the round has n_items enough for it; else every row counts as
+// moved.  Eight loads a thread are in flight (one at a time, 64 KB took 8 us).
+// Every thread calls it; ends with a barrier.
+template <int kMode, bool kTest>
+__device__ __forceinline__ MovedBits load_moved_bits(const DevMatrix &M, const RoundPlan &R, int step, int n_items,
+                                                     unsigned *words) {
+    if constexpr (!kTest) {
+        __syncthreads();
+        return MovedBits{nullptr, 0u};
+    }
+    if (step == 1 || n_items < kMinTestItems) {
+        __syncthreads();
+        return MovedBits{nullptr, 0u};
+    }
+    constexpr int kFlight = 8;
+    const long long *bm = reinterpret_cast<const long long *>(moved_bitmap(R, step - 1));
+    long long *out = reinterpret_cast<long long *>(words);
+    const int n = R.bit_words / 2, have = (M.nwords + 1) / 2;  // (the bitmaps are a multiple of 8 bytes)
+    const int stride = static_cast<int>(blockDim.x);
+    for (int w0 = threadIdx.x; w0 < n; w0 += kFlight * stride) {
+        long long v[kFlight];
+#pragma unroll
+        for (int q = 0; q < kFlight; q++) {
+            const int w = w0 + q * stride;
+            v[q] = 0;
+            if (w < n && w < have) v[q] = kMode == kWideCoherent ? coherent_load(&bm[w]) : bm[w];
+        }
+#pragma unroll
+        for (int q = 0; q < kFlight; q++) {
+            const int w = w0 + q * stride;
+            if (w >= n) break;
+            for (int x = w + n; x < have; x += n) v[q] |= kMode == kWideCoherent ? coherent_load(&bm[x]) : bm[x];
+            out[w] = v[q];
+        }
+    }
+    __syncthreads();
+    return MovedBits{words, static_cast<unsigned>(R.bit_words - 1)};
+}
+
 // The state of round `step`: records read from block (step - 1) & 1,
 // candidates and moved-column bits into the other parity's arrays.
 __device__ __forceinline__ DevState round_view(const DevMatrix &M, const DevState &D, const RoundPlan &R, int step) {
@@ -1659,7 +1785,7 @@ __device__ __forceinline__ DevState round_view(const DevMatrix &M, const DevStat
     V.AI = reinterpret_cast<int2 *>(nxt);
     V.AF = reinterpret_cast<double2 *>(nxt + M.snap_offF);
     V.AX = odd ? R.AX[1] : R.AX[0];
-    V.bm = odd ? R.bm[1] : R.bm[0];
+    V.bm = moved_bitmap(R, step);
     V.n_lds = 0;
     return V;
 }
@@ -1671,22 +1797,23 @@ __device__ __forceinline__ DevState block_view(const DevMatrix &M, const DevStat
     V.AI = reinterpret_cast<int2 *>(block);
     V.AF = reinterpret_cast<double2 *>(block + M.snap_offF);
     V.AX = parity ? R.AX[1] : R.AX[0];
-    V.bm = parity ? R.bm[1] : R.bm[0];
     return V;
 }
 
 // Folds the columns that round step - 1 moved into the block of round `step`
-// and clears their bits.  Returns whether one of the lane's columns is
+// and clears the bitmap of the next round (without kTest its own).  Returns whether one of the lane's columns is
 // crossed.  Each wave takes `chunk` words of the bitmap at a time (one lane
 // each) and works through the nonzero ones two at a time, a half-wave per
 // word.
 // With kUnits (a batch), only words of the units in the run, run[u] != 0, are
 // folded: a unit that has crossed keeps the block of its last round as it is.
-template <bool kUnits>
+template <bool kUnits, bool kTest>
 __device__ __forceinline__ bool carry_moved(const DevMatrix &M, const DevState &D, const RoundPlan &R, int step,
                                             int wave, int nwaves, const int *run) {
     const DevState C = block_view(M, D, R, (step - 1) & 1);
     const DevState N = block_view(M, D, R, step & 1);
+    unsigned *bm = moved_bitmap(R, step - 1);
+    unsigned *next_bm = moved_bitmap(R, step + 1);
     const int lane = threadIdx.x & 63;
     const int half = lane >> 5, b = lane & 31;
     int chunk = (M.nwords + nwaves - 1) / nwaves;
@@ -1694,8 +1821,15 @@ __device__ __forceinline__ bool carry_moved(const DevMatrix &M, const DevState &
     bool crossed = false;
     for (int w0 = (nwaves - 1 - wave) * chunk; w0 < M.nwords; w0 += nwaves * chunk) {
         const int w = w0 + lane;
-        const unsigned bits = lane < chunk && w < M.nwords ? coherent_load(&C.bm[w]) : 0u;
-        if (bits) coherent_store(&C.bm[w], 0u);
+        unsigned bits = 0u;
+        if (lane < chunk && w < M.nwords) {
+            bits = coherent_load(&bm[w]);
+            if constexpr (kTest) {
+                if (coherent_load(&next_bm[w]) != 0u) coherent_store(&next_bm[w], 0u);
+            } else if (bits) {  // nobody else reads it
+                coherent_store(&bm[w], 0u);
+            }
+        }
         unsigned long long pending = __ballot(bits != 0u);
         while (pending) {
             const int t0 = __ffsll(static_cast<long long>(pending)) - 1;
@@ -1756,23 +1890,23 @@ __global__ __launch_bounds__(256) void plan_rounds_kernel(DevMatrix M, RoundBins
 }
 
 // Item `it` of a round.  Returns the lane's accepted candidates.
-template <int kMode>
+template <int kMode, bool kTest>
 __device__ __forceinline__ int round_item(const DevMatrix &M, const DevState &V, const RoundPlan &R, int it, int step,
-                                          int *st) {
+                                          int *st, const MovedBits &B) {
     int4 d = R.items[uniform(it)];
     d.x = uniform(d.x);
     d.y = uniform(d.y);
     d.z = uniform(d.z);
     if ((d.x & 15) == kItemSeg) {
-        seg_item<kMode>(M, V, V, 0, d.y, d.z, 1, st, step);
+        seg_item<kMode, kTest>(M, V, V, 0, d.y, d.z, 1, st, step, B);
         return 0;
     }
     const int logg = (d.x >> 4) & 15;
     const Sink S = make_sink(V);
     switch ((d.x >> 8) & 15) {
-        case 0: return group_item<1, kMode>(M, S, d.y, d.z, logg, nullptr);
-        case 1: return group_item<2, kMode>(M, S, d.y, d.z, logg, nullptr);
-        default: return group_item<4, kMode>(M, S, d.y, d.z, logg, nullptr);
+        case 0: return group_item<1, kMode, kTest>(M, S, d.y, d.z, logg, nullptr, B);
+        case 1: return group_item<2, kMode, kTest>(M, S, d.y, d.z, logg, nullptr, B);
+        default: return group_item<4, kMode, kTest>(M, S, d.y, d.z, logg, nullptr, B);
     }
 }
 
@@ -1833,9 +1967,10 @@ __global__ __launch_bounds__(256) void load_rounds_kernel(DevMatrix M, DevState 
         }
     }
     if (tid == 0) A.AF[M.n - M.n_int] = B.AF[M.n - M.n_int] = make_double2(0.0, 0.0);  // the padding entries' column
-    for (int w = tid; w < M.nwords; w += stride) {
-        A.bm[w] = 0u;
-        B.bm[w] = 0u;
+    for (int w = tid; w < (M.nwords + 1) / 2 * 2; w += stride) {
+        R.bm[0][w] = 0u;
+        R.bm[1][w] = 0u;
+        R.bm[2][w] = 0u;
     }
     for (int q = tid; q < M.n_seg_rows; q += stride) D.seg_count[q] = 0u;
 }
@@ -1861,7 +1996,9 @@ __device__ __forceinline__ bool round_moved(const DevState &D, int step) {
 // the run goes on (input usable, not infeasible, the previous round moved a
 // bound); the first workgroup tells the host: its word becomes `step` when
 // the round runs, else kRoundsOver.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void round_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+template <bool kTest>
+__global__ __launch_bounds__(kTest ? 512 : 256) __attribute__((amdgpu_waves_per_eu(kTest ? 4 : 5))) void round_kernel(
+    DevMatrix M, DevState D, RoundPlan R, int step) {
     __shared__ int any_moved;
     const long long *p = reinterpret_cast<const long long *>(&D.units[0]);
     const long long w0 = coherent_load(p), w2 = coherent_load(p + 2);
@@ -1870,15 +2007,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void r
         __hip_atomic_store(D.host_word, runs ? step : kRoundsOver, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (!runs) return;
     if (threadIdx.x == 0) any_moved = 0;
-    __syncthreads();
+    const MovedBits B = load_moved_bits<kWide, kTest>(M, R, step, R.n_items, dyn_lds);
     const int waves = blockDim.x >> 6;
     const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));
     const int nwaves = gridDim.x * waves;
     int *st = status_row(D, step);
     const DevState V = round_view(M, D, R, step);
-    if (step > 1 && carry_moved<false>(M, D, R, step, wave, nwaves, nullptr)) atomic_max_i(&D.units[0].infeasible, step - 1);
+    if (step > 1 && carry_moved<false, kTest>(M, D, R, step, wave, nwaves, nullptr)) atomic_max_i(&D.units[0].infeasible, step - 1);
     int moved = 0;
-    for (int it = wave; it < R.n_items; it += nwaves) moved |= round_item<kWide>(M, V, R, it, step, st);
+    for (int it = wave; it < R.n_items; it += nwaves) moved |= round_item<kWide, kTest>(M, V, R, it, step, st, B);
     if (__any(moved != 0) && (threadIdx.x & 63) == 0) any_moved = 1;
     __syncthreads();
     if (threadIdx.x == 0 && any_moved) note_round_moved(D, step);
@@ -1949,6 +2086,7 @@ __device__ __forceinline__ bool gather_barrier(const DevState &D, const RoundPla
 // device-coherent loads (nothing is invalidated between the rounds, so the
 // matrix stays in the caches); one barrier per round, and a second one in
 // rounds in which a split row passed its gate.
+template <bool kTest>
 __global__ __launch_bounds__(1024) void rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
     constexpr unsigned kMoved = 1u, kCrossed = 2u;
     const long long w2 = coherent_load(reinterpret_cast<const long long *>(&D.units[0]) + 2);
@@ -1965,10 +2103,11 @@ __global__ __launch_bounds__(1024) void rounds_kernel(DevMatrix M, DevState D, R
     for (int step = 1; ok && step <= R.max_rounds; step++) {
         int *st = status_row(D, step);
         const DevState V = round_view(M, D, R, step);
+        const MovedBits B = load_moved_bits<kWideCoherent, kTest>(M, R, step, R.n_items, dyn_lds);
         unsigned flags = 0u;
-        if (step > 1 && carry_moved<false>(M, D, R, step, wave, nwaves, nullptr)) flags |= kCrossed;
+        if (step > 1 && carry_moved<false, kTest>(M, D, R, step, wave, nwaves, nullptr)) flags |= kCrossed;
         for (int it = wave; it < R.n_items; it += nwaves)
-            if (round_item<kWideCoherent>(M, V, R, it, step, st)) flags |= kMoved;
+            if (round_item<kWideCoherent, kTest>(M, V, R, it, step, st, B)) flags |= kMoved;
         ok = gather_barrier(D, R, ++seq, flags, wg_flags, all);
         unsigned seen = all;
         if (ok && M.n_seg_parts > 0) {
@@ -2078,6 +2217,7 @@ __device__ __forceinline__ int run_unit(int n_units, const int *upto, int t) {
 // Bound by the bounds' gathers while most instances run, by the barrier and
 // one pass's chain of loads, butterfly and divisions (8 us) in the tail.  64
 // instances of 42,000 entries, 58 rounds: 17 us a round (three phases: 47).
+template <bool kTest>
 __global__ __launch_bounds__(1024) void batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
     __shared__ int run[kMaxRoundUnits];      // the instance takes part in the round
     __shared__ int last[kMaxRoundUnits];     // its last round that moved a bound
@@ -2105,15 +2245,16 @@ __global__ __launch_bounds__(1024) void batch_rounds_kernel(DevMatrix M, DevStat
         __syncthreads();
         const int total = upto[(n_units - 1) | 63];
         if (total == 0) break;
+        const MovedBits B = load_moved_bits<kWideCoherent, kTest>(M, R, step, total, dyn_lds);
         int *st = status_row(D, step);
         const DevState V = round_view(M, D, R, step);
         const int set = (seq + 1) & 1;
-        if (step > 1 && carry_moved<true>(M, D, R, step, wave, nwaves, run))
+        if (step > 1 && carry_moved<true, kTest>(M, D, R, step, wave, nwaves, run))
             for (int k = 0; k < R.slot_words; k++) atomicOr(&own[set][k], 1u << 31);
         for (int t = wave; t < total; t += nwaves) {
             const int u = run_unit(n_units, upto, t);
             const int it = uniform(first[u + 1] - upto[u]) + t;
-            const int moved = round_item<kWideCoherent>(M, V, R, it, step, st);
+            const int moved = round_item<kWideCoherent, kTest>(M, V, R, it, step, st, B);
             if (__any(moved != 0) && lane == 0) atomicOr(&own[set][u / 31], 1u << (u % 31));
         }
         if (!gather_units(D, R, ++seq, own, all, &wg_ok)) break;
@@ -2185,31 +2326,36 @@ __global__ __launch_bounds__(kMaxRoundUnits) void batch_plan_kernel(DevMatrix M,
 // Round `step` of a batch; bounds as in batch_rounds_kernel, the kernel
 // boundaries in the barrier's place.  64 instances of 42,000 entries: 16 us a
 // round with its plan (three phases: 42).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void batch_round_kernel(DevMatrix M, DevState D, RoundPlan R, int step) {
+template <bool kTest>
+__global__ __launch_bounds__(kTest ? 512 : 256) __attribute__((amdgpu_waves_per_eu(kTest ? 4 : 5))) void batch_round_kernel(
+    DevMatrix M, DevState D, RoundPlan R, int step) {
     __shared__ int run[kMaxRoundUnits], first[kMaxRoundUnits + 1], upto[kMaxRoundUnits];
     __shared__ unsigned moved_units[kMaxRoundUnits / 32];
     const int tid = threadIdx.x;
     const int n_units = R.n_units;
     const int total = R.upto[n_units - 1];
     if (total == 0) return;
-    run[tid] = tid < n_units ? R.run[tid] : 0;
-    upto[tid] = tid < n_units ? R.upto[tid] : total;
+    if (tid < kMaxRoundUnits) {
+        run[tid] = tid < n_units ? R.run[tid] : 0;
+        upto[tid] = tid < n_units ? R.upto[tid] : total;
+    }
     if (tid < n_units) first[tid + 1] = R.unit_item[tid + 1];
     if (tid < kMaxRoundUnits / 32) moved_units[tid] = 0u;
-    __syncthreads();
-    const int wave = uniform(blockIdx.x * 4 + (tid >> 6));
-    const int nwaves = gridDim.x * 4;
+    const MovedBits B = load_moved_bits<kWide, kTest>(M, R, step, total, dyn_lds);
+    const int waves = blockDim.x >> 6;
+    const int wave = uniform(blockIdx.x * waves + (tid >> 6));
+    const int nwaves = gridDim.x * waves;
     int *st = status_row(D, step);
     const DevState V = round_view(M, D, R, step);
-    if (step > 1) carry_moved<true>(M, D, R, step, wave, nwaves, run);
+    if (step > 1) carry_moved<true, kTest>(M, D, R, step, wave, nwaves, run);
     for (int t = wave; t < total; t += nwaves) {
         const int u = run_unit(n_units, upto, t);
         const int it = uniform(first[u + 1] - upto[u]) + t;
-        const int moved = round_item<kWide>(M, V, R, it, step, st);
+        const int moved = round_item<kWide, kTest>(M, V, R, it, step, st, B);
         if (__any(moved != 0) && (tid & 63) == 0) atomicOr(&moved_units[u >> 5], 1u << (u & 31));
     }
     __syncthreads();
-    if ((moved_units[tid >> 5] >> (tid & 31)) & 1u) note_round_moved(D, step, tid);
+    if (tid < n_units && ((moved_units[tid >> 5] >> (tid & 31)) & 1u)) note_round_moved(D, step, tid);
 }
 
 // The candidates of the batch's split rows whose gate passed in the round.
@@ -2224,6 +2370,15 @@ __global__ __launch_bounds__(256) void batch_apply_kernel(DevMatrix M, DevState 
             note_round_moved(D, step, M.seg_rows[M.part_row[task]].w);
     }
 }
+
+template __global__ void round_kernel<false>(DevMatrix, DevState, RoundPlan, int);
+template __global__ void round_kernel<true>(DevMatrix, DevState, RoundPlan, int);
+template __global__ void rounds_kernel<false>(DevMatrix, DevState, RoundPlan);
+template __global__ void rounds_kernel<true>(DevMatrix, DevState, RoundPlan);
+template __global__ void batch_round_kernel<false>(DevMatrix, DevState, RoundPlan, int);
+template __global__ void batch_round_kernel<true>(DevMatrix, DevState, RoundPlan, int);
+template __global__ void batch_rounds_kernel<false>(DevMatrix, DevState, RoundPlan);
+template __global__ void batch_rounds_kernel<true>(DevMatrix, DevState, RoundPlan);
 
 // Writes the final bounds of a batch to the caller's vectors (not when some
 // input was outside its envelope), finds crossed bounds of the instances' last

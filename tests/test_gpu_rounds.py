@@ -1,4 +1,4 @@
-"""Double-buffered rounds: single problems of up to 4M padded entries with
+"""Double-buffered rounds: single problems of up to 8M padded entries with
 default tuning run each round as one phase (one launch, or one barrier of the
 persistent launch).  Checked bit for bit against the round-synchronous oracle
 and against the three-phase rounds, which an explicit work-item size selects,
@@ -51,8 +51,8 @@ def test_widths_and_remainders(gpu, oracle, width, m):
     _check(_rows_of(width, m, max(700, 2 * width), width + m), oracle, tunings=(None, {"item_nnz": 1024}))
 
 
-# about 11 nonzeros a row, 16.5 padded entry slots
-@pytest.mark.parametrize("m", [5000, 6000, 40000, 44000, 130000, 330000, 380000])
+# about 11 nonzeros a row, 12.5 padded entries
+@pytest.mark.parametrize("m", [5000, 6000, 40000, 44000, 130000, 330000, 380000, 650000, 700000])
 def test_plan_thresholds(gpu, oracle, m):
     inst = small_mip(seed=m, m=m, n=m // 2 + 1)
     print(f"rounds: m {m} nnz {inst.nnz}", flush=True)
