@@ -210,6 +210,7 @@ struct DevMatrix {
     const int *perm;       // internal id -> caller's column (-1: padding id)
     const int *word_unit;  // blocks mode: unit of each bitmap word
     int snap_off32;        // byte offset of S32 in a unit's snapshot block
+    int snap_offB;         // byte offset of SB
     int snap_offF;         // byte offset of SF
     long long snap_stride; // bytes between the snapshot blocks of two units
     int n_bin;             // binary columns: internal ids [0, n_bin) (replicas mode; blocks: 0)
@@ -245,6 +246,7 @@ struct DevState {
     int n_active;
     int n_lds;             // binary columns read from LDS (persistent launch of one unit; else 0)
     unsigned *SB;          // 2-bit codes of the binary columns (sb_words per unit)
+    int n_codes;           // binary columns read from their codes in SB (kRecords)
     int *host_word;        // pinned: the step that the guarded launches have started, or kRoundsOver
 };
 
@@ -338,7 +340,7 @@ __device__ __forceinline__ DevState unit_view(const DevMatrix &M, const DevState
     V.seg_marks += k * M.n_seg_parts;
     V.seg_state += k * M.n_seg_rows;
     V.seg_count += k * M.n_seg_rows;
-    V.SB += k * M.sb_words;
+    V.SB = reinterpret_cast<unsigned *>(reinterpret_cast<char *>(D.SB) + snap);
     return V;
 }
 

@@ -610,7 +610,8 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
     D.AX = reinterpret_cast<double2 *>(take(k * M.n_int * sizeof(double2)));
     D.AF = reinterpret_cast<double2 *>(take(k * nf * sizeof(double2)));
     D.bm = reinterpret_cast<unsigned *>(take(k * M.nwords * sizeof(unsigned)));
-    D.SB = reinterpret_cast<unsigned *>(take(k * M.sb_words * sizeof(unsigned)));
+    D.SB = reinterpret_cast<unsigned *>(snap ? snap + M.snap_offB : nullptr);
+    D.n_codes = replicas ? M.n_bin : 0;
     D.marks = reinterpret_cast<int *>(take(k * M.m * sizeof(int)));
     D.seg_parts = reinterpret_cast<SegPart *>(take(k * M.n_seg_parts * sizeof(SegPart)));
     D.seg_marks = reinterpret_cast<int *>(take(k * M.n_seg_parts * sizeof(int)));
@@ -1439,13 +1440,14 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         M.perm = d_perm;
         M.word_unit = d_word_unit;
 
-        // snapshot block of a unit: int16 records, then int32, then FP64,
-        // each class from a 16-byte boundary; the binary columns' codes in
-        // 16-byte groups of 64 columns
+        // snapshot block of a unit: int16 records, then int32, then the binary
+        // columns' codes in 16-byte groups of 64 columns, then FP64, each from a
+        // 16-byte boundary
         M.n_bin = C.n_bin;
         M.sb_words = (C.n_bin + 63) / 64 * 4;
         M.snap_off32 = (M.n16 * 4 + 15) / 16 * 16;
-        M.snap_offF = M.snap_off32 + ((M.n_int - M.n16) * 8 + 15) / 16 * 16;
+        M.snap_offB = M.snap_off32 + ((M.n_int - M.n16) * 8 + 15) / 16 * 16;
+        M.snap_offF = M.snap_offB + 4 * M.sb_words;
         M.snap_stride = M.snap_offF + 16LL * (M.n - M.n_int) + 16;
         check(hipStreamSynchronize(s), "upload");
         {

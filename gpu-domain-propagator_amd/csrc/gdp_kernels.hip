@@ -119,8 +119,15 @@ constexpr int kRecords = 0, kWide = 1, kWideCoherent = 2;
 // Byte offset of the record of internal column `id` in the unit's block: the
 // record's size and the class's base picked by class, then one shift and add
 // (picking among the three finished offsets becomes branches).
+// Binary columns id < D.n_codes are read from their 2-bit codes, 16 columns a
+// word: 50,000 of them take 12.5 KB where the records take 200, so that a
+// compute unit at work on one vector of many finds them in its L1: a sweep is
+// bound by its requests to the L2 (116 a ns, half of what 128 channels could
+// take at one a clock), one per gathered record.  256 vectors, 200,000 rows:
+// 2.09 -> 1.94 ms in the persistent launch; one vector of 1M rows in the loop, whose
+// 62 KB of codes fit an L1 by half: 3.02 -> 2.67.
 template <int kMode>
-__device__ __forceinline__ unsigned record_offset(const DevMatrix &M, int id) {
+__device__ __forceinline__ unsigned record_offset(const DevMatrix &M, const DevState &D, int id) {
     const unsigned uid = static_cast<unsigned>(id);
     const unsigned base32 = static_cast<unsigned>(M.snap_off32) - static_cast<unsigned>(M.n16) * 8u;
     const unsigned baseF = static_cast<unsigned>(M.snap_offF) - static_cast<unsigned>(M.n_int) * 16u;
@@ -129,6 +136,8 @@ __device__ __forceinline__ unsigned record_offset(const DevMatrix &M, int id) {
     if constexpr (kMode == kRecords) {
         shift = id < M.n16 ? 2u : shift;
         base = id < M.n16 ? 0u : base;
+        const unsigned code_word = static_cast<unsigned>(M.snap_offB) + (uid >> 4 << 2);
+        return id < D.n_codes ? code_word : (uid << shift) + base;
     }
     return (uid << shift) + base;
 }
@@ -154,7 +163,7 @@ __device__ __forceinline__ uint4 load_record(const DevMatrix &M, const DevState 
 }
 
 // Bounds of `id` from its record; of a binary column id < D.n_lds from its
-// 2-bit code in LDS instead.
+// 2-bit code in LDS instead, of one id < D.n_codes from its code in `c`.
 template <int kMode>
 __device__ __forceinline__ void decode_bounds(const DevMatrix &M, const DevState &D, int id, const uint4 c, double &l,
                                               double &u) {
@@ -163,8 +172,8 @@ __device__ __forceinline__ void decode_bounds(const DevMatrix &M, const DevState
         const bool c16 = id < M.n16;
         il = c16 ? static_cast<short>(c.x & 0xffffu) : il;
         iu = c16 ? static_cast<int>(c.x) >> 16 : iu;
-        if (id < D.n_lds) {
-            const unsigned code = dyn_lds[id >> 4] >> ((id & 15) * 2);
+        if (id < D.n_lds || id < D.n_codes) {
+            const unsigned code = (id < D.n_lds ? dyn_lds[id >> 4] : c.x) >> ((id & 15) * 2);
             il = static_cast<int>(code & 1u);
             iu = static_cast<int>(((code >> 1) & 1u) ^ 1u);
         }
@@ -179,7 +188,7 @@ __device__ __forceinline__ void decode_bounds(const DevMatrix &M, const DevState
 // Bounds of internal column `id` at the start of the round.
 template <int kMode>
 __device__ __forceinline__ void load_bounds(const DevMatrix &M, const DevState &D, int id, double &l, double &u) {
-    const unsigned off = id < D.n_lds ? kNoRecord : record_offset<kMode>(M, id);
+    const unsigned off = id < D.n_lds ? kNoRecord : record_offset<kMode>(M, D, id);
     decode_bounds<kMode>(M, D, id, load_record<kMode>(M, D, off), l, u);
 }
 
@@ -528,7 +537,7 @@ struct LaneEntries {
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int id = jp[k] & kIdMask;
-            rec[k] = load_record<kMode>(M, D, id < D.n_lds ? kNoRecord : record_offset<kMode>(M, id));
+            rec[k] = load_record<kMode>(M, D, id < D.n_lds ? kNoRecord : record_offset<kMode>(M, D, id));
         }
         dmax = 0.0;
         bool any = false;
@@ -1357,12 +1366,10 @@ __device__ __forceinline__ void publish_word(const DevMatrix &M, const DevState 
         accumulated(M, V, id, l, uu);
         store_snapshot(M, V, id, l, uu);
         if (eps_gt(l, uu)) atomic_max_i(&D.units[u].infeasible, step);
-        if (id < D.n_lds) code = (l >= 1.0 ? 1u : 0u) | (uu < 1.0 ? 2u : 0u);
+        if (id < D.n_lds || id < D.n_codes) code = (l >= 1.0 ? 1u : 0u) | (uu < 1.0 ? 2u : 0u);
     }
-    if (D.n_lds > 0) {
-        // the launch reads these columns from LDS (one unit, reloaded at the
-        // start of every propagation): the new code bits of each 16
-        // columns, ORed into their table word
+    if (__any(code != 0u)) {
+        // the new code bits of each 16 columns, ORed into their table word
         unsigned cw = code << ((id & 15) * 2);
 #pragma unroll
         for (int h = 1; h < 16; h <<= 1) cw |= static_cast<unsigned>(__shfl_xor(static_cast<int>(cw), h, 64));
@@ -1499,9 +1506,9 @@ __device__ __forceinline__ void publish_phase(const DevMatrix &M, const DevState
                         acc_resolve(M, V, ids[i], raw[i], l, uu);
                         store_snapshot(M, V, ids[i], l, uu);
                         if (eps_gt(l, uu)) atomic_max_i(&D.units[u].infeasible, step);
-                        if (ids[i] < D.n_lds) code = (l >= 1.0 ? 1u : 0u) | (uu < 1.0 ? 2u : 0u);
+                        if (ids[i] < D.n_lds || ids[i] < D.n_codes) code = (l >= 1.0 ? 1u : 0u) | (uu < 1.0 ? 2u : 0u);
                     }
-                    if (D.n_lds > 0) {
+                    if (__any(code != 0u)) {
                         unsigned cw = code << ((ids[i] & 15) * 2);
 #pragma unroll
                         for (int h = 1; h < 16; h <<= 1)
@@ -1677,9 +1684,10 @@ template <int kThreads, bool kLds>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void mega_kernel(DevMatrix M, DevState D_arg, int first_step, int max_steps,
                                                         int n_units) {
     // kLds: a launch of one unit that reads binary columns from LDS; without
-    // it n_lds is a constant 0, and the LDS reads and code updates compile out
+    // it n_lds is a constant 0, and the LDS reads compile out (with it n_codes)
     DevState D = D_arg;
-    if constexpr (!kLds) D.n_lds = 0;
+    if constexpr (kLds) D.n_codes = 0;
+    else D.n_lds = 0;
     const unsigned nblocks = gridDim.x;
     const int waves = blockDim.x >> 6;
     const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));

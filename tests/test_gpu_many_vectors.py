@@ -82,3 +82,29 @@ def test_integers_beyond_int32_and_back(gpu, oracle):
                 _run(p, nodes, pick, sync, hints=False)
     finally:
         p.close()
+
+
+@pytest.mark.parametrize("n_bin", [1, 15, 16, 17, 63, 64, 65, 200])
+def test_binary_codes(gpu, oracle, n_bin):
+    """Binary columns read from their codes: counts around a code word (16
+    columns) and a 16-byte group (64), before other classes, one vector and
+    several."""
+    inst = small_mip(seed=n_bin, m=600, n=300)
+    lb, ub, vt = inst.lb.copy(), inst.ub.copy(), inst.vartype.copy()
+    ints = np.flatnonzero(vt != 3)
+    ub[ints] = np.maximum(ub[ints], lb[ints] + 2)
+    pick = np.random.default_rng(n_bin).permutation(inst.n)[:n_bin]
+    vt[pick], lb[pick], ub[pick] = 1, 0.0, 1.0
+    inst = inst.__class__(**{**inst.__dict__, "lb": lb, "ub": ub, "vartype": vt})
+    exp = oracle.jacobi(inst)
+    p = I.Problem(inst, {"item_nnz": 512})
+    try:
+        assert p.stats().n_binary == n_bin
+        for sync in SYNCS:
+            for count in (1, 3):
+                for g in p.propagate_nodes([lb] * count, [ub] * count, sync_type=sync):
+                    np.testing.assert_array_equal(g.lbs, exp[0])
+                    np.testing.assert_array_equal(g.ubs, exp[1])
+                    assert (g.rounds, g.infeasible, g.capped) == exp[2:]
+    finally:
+        p.close()
