@@ -113,14 +113,22 @@ constexpr int kGlobalTicket = 2;   // workgroups of unpack_rounds_kernel that ar
 constexpr int kGlobalEnvelope = 3; // some loaded vector left the envelope (runs that then return an error)
 constexpr int kGlobalWords = 8;
 
-// Words of a run state that outlive its runs: row marks hold the step plus the
-// epoch, which starts beyond every earlier mark with each run, so that no run
-// has to clear them; whether an exact integer accumulator (AX) was written.
+// Words of a run state that outlive its runs: row marks hold the step's stamp
+// plus the epoch, which starts beyond every earlier mark with each run, so that
+// no run has to clear them; whether an exact integer accumulator (AX) was
+// written.
 constexpr int kPersistEpoch = 0;
 constexpr int kPersistAx = 1;
 constexpr int kPersistWords = 2;
 constexpr int kPersistAt = 32;    // first of them, from the global words
-constexpr int kEpochSteps = 128;  // steps of a run, rounded up
+constexpr int kEpochStamps = 256; // stamps of a run, rounded up
+// A step's stamps: of rows marked by the publish before it, and of rows marked
+// by the hints of a vector that starts in it.  A server's slot may hold marks of
+// its last vector for the very step in which the next one starts (the last one
+// moved bounds, and crossed them or reached its cap, in the step before).
+__host__ __device__ inline unsigned mark_stamp(int step, bool hint) {
+    return 2u * static_cast<unsigned>(step) + (hint ? 1u : 0u);
+}
 // Loads and unpacks of this many vectors keep a vector to one XCD.
 constexpr int kVectorsByXcd = 64;
 

@@ -687,11 +687,12 @@ void clear_marks(Problem *P) {
     P->epoch = 0;
 }
 
-// The epoch of a new run of up to kEpochSteps steps.
+// The epoch of a new run of up to kMaxRounds steps.
+static_assert(2 * (kMaxRounds + 1) + 1 < kEpochStamps, "a run's stamps lie before the next epoch");
 int next_epoch(Problem *P) {
     if (P->borrowed) return 0;
     if (P->epoch >= 1u << 30) clear_marks(P);
-    P->epoch += kEpochSteps;
+    P->epoch += kEpochStamps;
     return static_cast<int>(P->epoch);
 }
 
@@ -2089,7 +2090,7 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
             if (step == 1 ? st[0].crossed != 0 : !active_after(st[0], step - 1)) break;
             RoundWork w;
             const bool all_rows = !M.mark_rows || st[0].markall == step;
-            const int mark = step + static_cast<int>(P->epoch);
+            const int mark = static_cast<int>(mark_stamp(step, false) + P->epoch);
             if (!all_rows) {
                 check(hipMemcpy(marks.data(), P->D.marks, sizeof(int) * M.m, hipMemcpyDeviceToHost), "D2H marks");
                 if (M.n_seg_parts > 0)
@@ -2639,7 +2640,7 @@ struct Server {
         if (cs) (void)hipStreamDestroy(cs);
         if (attached) {
             std::lock_guard<std::mutex> lock(P->run_mutex);
-            P->epoch += (static_cast<unsigned>(step) / kEpochSteps + 1) * kEpochSteps;  // its marks
+            P->epoch += (mark_stamp(step, true) / kEpochStamps + 1) * kEpochStamps;  // its marks
             P->servers--;
         }
     }

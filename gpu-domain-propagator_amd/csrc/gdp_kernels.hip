@@ -1293,14 +1293,15 @@ __device__ __forceinline__ bool decide_all_rows(const DevMatrix &M, const DevSta
 // of all classes in the unit's lists come from one atomic instruction (two
 // classes a word, six lanes) per N entries a lane: the counters of a unit lie
 // in one line, and every addition to it by a wave costs tens of nanoseconds.
-template <int N>
+// kHint: marks of a vector's first step (mark_stamp).
+template <bool kHint, int N>
 __device__ __forceinline__ void mark_entries(const DevMatrix &M, const DevState &V, int u, const bool (&valid)[N],
                                              const int (&row)[N], const int (&code)[N], int step) {
     __shared__ unsigned ranks[16][2][16];  // per wave and half: rows per class, then their first places
     const int lane = lane_here();
     const int b = lane & 31;
     unsigned *mine = ranks[threadIdx.x >> 6][lane >> 5];
-    const int stamp = static_cast<int>(static_cast<unsigned>(step) + static_cast<unsigned>(V.persist[kPersistEpoch]));
+    const int stamp = static_cast<int>(mark_stamp(step, kHint) + static_cast<unsigned>(V.persist[kPersistEpoch]));
     bool first[N], any = false;
 #pragma unroll
     for (int q = 0; q < N; q++) {
@@ -1415,7 +1416,7 @@ __device__ __forceinline__ void publish_word(const DevMatrix &M, const DevState 
                 sp[q] = M.col_seg[k];
             }
         }
-        mark_entries(M, V, u, in, row, sp, step + 1);
+        mark_entries<false>(M, V, u, in, row, sp, step + 1);
     }
 }
 
@@ -2851,7 +2852,7 @@ __global__ __launch_bounds__(256) void hint_kernel(DevMatrix M, DevState D, int 
                 const bool in[1] = {q < end};
                 const int row[1] = {in[0] ? M.col_rows[q] : 0};
                 const int code[1] = {in[0] ? M.col_seg[q] : -1};
-                mark_entries(M, V, u, in, row, code, start_step);
+                mark_entries<true>(M, V, u, in, row, code, start_step);
             }
         }
     }

@@ -108,3 +108,49 @@ def test_binary_codes(gpu, oracle, n_bin):
                     assert (g.rounds, g.infeasible, g.capped) == exp[2:]
     finally:
         p.close()
+
+
+@pytest.mark.parametrize("n, slots", [(63, 5), (65, 70), (4100, 12), (30000, 3)])
+def test_server_changes(gpu, oracle, n, slots):
+    """A server's changed columns, listed by the unpack: columns around a wave,
+    more requests than slots, full vectors beside deltas, and (30,000 columns
+    from the unpropagated bounds) more changes than a list holds."""
+    inst = small_mip(seed=n, m=2 * n, n=n, len_hi=9)
+    base = oracle.jacobi(inst) if n < 30000 else (inst.lb, inst.ub)
+    rng = np.random.default_rng(n)
+    p = I.Problem(inst)
+    server = I.Server(p, 4 << 30, slots)
+    try:
+        server.set_base(base[0], base[1])
+        print(f"server changes: n={n} slots={server.slots}", flush=True)
+        want = []
+        for k in range(2 * slots if n < 30000 else slots):
+            l, u, cols = tighten_node(inst, rng, 1, 9, base[0], base[1])
+            exp = oracle.jacobi(inst.with_bounds(l, u))
+            if n == 30000:  # the base is no fixpoint: every row in round 1
+                want.append((server.submit(l, u), True, exp))
+            elif k % 3 == 2:
+                want.append((server.submit(l, u, hints=cols), True, exp))
+            else:
+                want.append((server.submit_delta(cols, l[cols], u[cols]), False, exp))
+        if n == 30000:
+            every = np.arange(n, dtype=np.int32)
+            want.append((server.submit_delta(every, inst.lb, inst.ub), False, oracle.jacobi(inst)))
+            assert int(np.sum((want[-1][2][0] != inst.lb) | (want[-1][2][1] != inst.ub))) > 4096
+        while server.pending():
+            server.step()
+        for ticket, full, exp in want:
+            if full:
+                got = server.result(ticket)
+                lb, ub, info = got.lbs, got.ubs, got
+            else:
+                cols, cl, cu, info = server.result_changes(ticket)
+                lb, ub = base[0].copy(), base[1].copy()
+                lb[cols], ub[cols] = cl, cu
+                assert len(np.unique(cols)) == len(cols)
+            np.testing.assert_array_equal(lb, exp[0])
+            np.testing.assert_array_equal(ub, exp[1])
+            assert (info.rounds, bool(info.infeasible), bool(info.capped)) == exp[2:]
+    finally:
+        server.close()
+        p.close()
