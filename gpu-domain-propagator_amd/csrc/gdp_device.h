@@ -270,6 +270,16 @@ struct ReferenceView {
     int start = 0;                   // step that the copied partials are stamped with
 };
 
+// Columns in which finished vectors differ from others: vector k's indices and
+// bounds in region k (of cap) of cols / vl / vu, their number in cnt[k] (zero on
+// entry; it may exceed cap).
+struct ChangeLists {
+    const double *const *lb = nullptr, *const *ub = nullptr;
+    int cap = 0;
+    int *cnt = nullptr, *cols = nullptr;
+    double *vl = nullptr, *vu = nullptr;
+};
+
 // Up to three vectors whose bitwise majority is the reference.
 struct ReferenceVectors {
     const double *lb[3], *ub[3];

@@ -73,18 +73,17 @@ __global__ void fill_parts_kernel(DevMatrix M, DevState D, int n_list, const int
 __global__ void drop_parts_kernel(DevMatrix M, DevState D, int n_list, const int *list, ReferenceView ref, int limit);
 __global__ void hint_kernel(DevMatrix M, DevState D, int n_list, const int *list, const int *hint_ptr,
                             const int *hints, const int *inv_perm, int start_step);
+template <bool kDiff>
 __global__ void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list, double *const *lbp,
-                              double *const *ubp, int per_unit, int checked);
+                              double *const *ubp, int per_unit, int checked, ChangeLists L);
 __global__ void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int epoch, int *list, double **lbp,
                                  double **ubp, double *lbs, double *ubs);
 __global__ void report_kernel(DevState D, int n_list, const int *list, UnitState *out);
 __global__ void delta_kernel(int n_list, double *const *lbp, double *const *ubp, const int *ptr, const int *cols,
                              const double *lv, const double *uv);
 __global__ void copy_pairs_kernel(long long n2, int count, double *const *ptrs);
-__global__ void diff_kernel(int n, int n_list, double *const *lbp, double *const *ubp, const double *const *blp,
-                            const double *const *bup, int cap, int *cnt, int *cols, double *vl, double *vu);
 __global__ void compact_changes_kernel(int nd, int cap, const int *cnt, const int *cols, const double *vl,
-                                       const double *vu, int *off, int *kcols, double *kl, double *ku);
+                                       const double *vu, int *cnt_out, int *off, int *kcols, double *kl, double *ku);
 __global__ void layout_rows_kernel(int mp, const long long *src_start, const int *row_inst, const int *inst_col_off,
                                    const int *col_in, const double *val_in, const int *row_ptr_out,
                                    const int *internal, const int *vartype, int *col_out, double *val_out,
@@ -1907,8 +1906,8 @@ void run_units(Problem *P, int n_list, const int *list, double *const *lbp, doub
     load_units(P, n_list, list, lbp, ubp, hint_ptr, hints, caps, 1, true, related);
     run_steps(P, sync_type, max_rounds);
     const VectorGrid g = vector_grid(P->M.n, P->replicas ? n_list : 1);
-    hipLaunchKernelGGL(unpack_kernel, dim3(g.grid), dim3(256), 0, s, P->M, P->D, n_list, P->d_list, P->d_lbp, P->d_ubp,
-                       g.per_unit, 1);
+    hipLaunchKernelGGL(unpack_kernel<false>, dim3(g.grid), dim3(256), 0, s, P->M, P->D, n_list, P->d_list, P->d_lbp, P->d_ubp,
+                       g.per_unit, 1, ChangeLists());
     // (the tables' pinned copy is free again: the run has read it)
     UnitState *st = &P->host->state;
     if (n_list > 1) {
@@ -2147,8 +2146,8 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
         }
         res = outcome(st[0]);
         const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
-        hipLaunchKernelGGL(unpack_kernel, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                           P->d_ubp, gx, 0);
+        hipLaunchKernelGGL(unpack_kernel<false>, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
+                           P->d_ubp, gx, 0, ChangeLists());
         check(hipGetLastError(), "unpack launch");
         check(hipStreamSynchronize(s), "unpack sync");
         check(hipMemcpy(lbs, d_b, n * sizeof(double), hipMemcpyDeviceToHost), "D2H lbs");
@@ -2205,8 +2204,8 @@ RunResult problem_propagate_measured(Problem *P, double *lbs, double *ubs, int m
             if (step == 1 ? st[0].crossed != 0 : !active_after(st[0], step - 1)) break;
             launch_step(P, step, 0, 1);
             check(hipGetLastError(), "step launch");
-            hipLaunchKernelGGL(unpack_kernel, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                               P->d_ubp, gx, 0);
+            hipLaunchKernelGGL(unpack_kernel<false>, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
+                               P->d_ubp, gx, 0, ChangeLists());
             hipLaunchKernelGGL(measure_kernel, dim3(gx), dim3(256), 0, s, n, d_b, d_b + n, d_w, d_w + n, d_l,
                                d_l + n, d_prev, d_prev + n, part_f, part_i);
             hipLaunchKernelGGL(measure_total_kernel, dim3(1), dim3(64), 0, s, gx, part_f, part_i, out_f + step - 1,
@@ -2216,8 +2215,8 @@ RunResult problem_propagate_measured(Problem *P, double *lbs, double *ubs, int m
             rounds = step;
         }
         res = outcome(st[0]);
-        hipLaunchKernelGGL(unpack_kernel, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
-                           P->d_ubp, gx, 0);
+        hipLaunchKernelGGL(unpack_kernel<false>, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
+                           P->d_ubp, gx, 0, ChangeLists());
         check(hipGetLastError(), "unpack launch");
         check(hipStreamSynchronize(s), "unpack sync");
         fin.resize(rounds);
@@ -2565,10 +2564,10 @@ struct Server {
     int *d_ccnt = nullptr, *d_ccols = nullptr;
     double *d_cl = nullptr, *d_cu = nullptr;
     int *h_ccnt = nullptr, *h_ccols = nullptr;
-    // the changes packed for the copy back: columns and bounds, each
-    // vector's start (device, then pinned host)
-    int *d_kcols = nullptr, *d_off = nullptr, *h_off = nullptr;
-    double *d_kl = nullptr, *d_ku = nullptr;
+    // the changes packed into pinned memory: columns and bounds, each vector's
+    // count and start
+    int *h_off = nullptr;
+    HostBlock h_states;                  // pinned: the states of a step's slots
     double *h_cl = nullptr, *h_cu = nullptr;
     int diff_slots = 0;
     std::vector<double *> slot_lb, slot_ub;
@@ -2618,9 +2617,6 @@ struct Server {
         if (d_base) (void)cached_free(d_base);
         if (inbox) (void)hipHostFree(inbox);
         if (outbox) (void)hipHostFree(outbox);
-        for (void *q : {static_cast<void *>(d_kcols), static_cast<void *>(d_off), static_cast<void *>(d_kl),
-                        static_cast<void *>(d_ku)})
-            if (q) (void)cached_free(q);
         if (h_off) (void)hipHostFree(h_off);
         for (void *q : {static_cast<void *>(h_ccnt), static_cast<void *>(h_ccols), static_cast<void *>(h_cl),
                         static_cast<void *>(h_cu)})
@@ -2719,10 +2715,6 @@ Server *server_create(Problem *P, int64_t hbm_budget, int max_slots) {
         check(hipHostMalloc(reinterpret_cast<void **>(&S->h_ccols), sizeof(int) * dc, 0), "hipHostMalloc");
         check(hipHostMalloc(reinterpret_cast<void **>(&S->h_cl), sizeof(double) * dc, 0), "hipHostMalloc");
         check(hipHostMalloc(reinterpret_cast<void **>(&S->h_cu), sizeof(double) * dc, 0), "hipHostMalloc");
-        check(cached_malloc(&S->d_kcols, sizeof(int) * dc), "hipMalloc");
-        check(cached_malloc(&S->d_kl, sizeof(double) * dc), "hipMalloc");
-        check(cached_malloc(&S->d_ku, sizeof(double) * dc), "hipMalloc");
-        check(cached_malloc(&S->d_off, sizeof(int) * (slots + 1)), "hipMalloc");
         check(hipHostMalloc(reinterpret_cast<void **>(&S->h_off), sizeof(int) * (slots + 1), 0), "hipHostMalloc");
         // pinned staging for request and result vectors (up to 1 GiB each)
         const int entries = static_cast<int>(
@@ -3206,7 +3198,13 @@ int step_impl(Server *S) {
     P->D.n_active = static_cast<int>(active.size());
     launch_step(P, S->step, 0, S->step);
     check(hipGetLastError(), "step launch");
-    std::vector<UnitState> st = read_units(P, static_cast<int>(active.size()), active.data());  // synchronizes
+    // the states come back in pinned memory: one wait
+    const int n_act = static_cast<int>(active.size());
+    const UnitState *st = reinterpret_cast<const UnitState *>(S->h_states.get(sizeof(UnitState) * S->slots));
+    hipLaunchKernelGGL(report_kernel, dim3((n_act + 255) / 256), dim3(256), 0, s, P->D, n_act, P->d_list,
+                       const_cast<UnitState *>(st));
+    check(hipGetLastError(), "report launch");
+    check(hipStreamSynchronize(s), "step");
     {
         std::lock_guard<std::mutex> lk(S->mu);
         for (int e : used_inbox) S->inbox_free.push_back(e);
@@ -3215,9 +3213,7 @@ int step_impl(Server *S) {
     }
     if (!used_inbox.empty()) S->space_cv.notify_all();
     keep.clear();
-    int err = 0;
-    check(hipMemcpy(&err, P->D.global + kGlobalError, sizeof(int), hipMemcpyDeviceToHost), "D2H");
-    if (err) throw std::runtime_error("device wait timed out");
+    if (st[0].error) throw std::runtime_error("device wait timed out");
     t_retire = Clock::now();
     // ---- retire finished slots: unpack and copy the results out ----
     std::vector<int> fin;
@@ -3240,57 +3236,50 @@ int step_impl(Server *S) {
         upload(P->d_lbp, lbp.data(), fin.size(), s);
         upload(P->d_ubp, ubp.data(), fin.size(), s);
         const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
-        const VectorGrid g = vector_grid(P->M.n, static_cast<int>(fin.size()));
-        hipLaunchKernelGGL(unpack_kernel, dim3(g.grid), dim3(256), 0, s, P->M, P->D, static_cast<int>(fin.size()),
-                           P->d_list, P->d_lbp, P->d_ubp, g.per_unit, 0);
-        check(hipGetLastError(), "unpack launch");
-        std::vector<Server::Done> out(fin.size());
         // delta requests (against the base vector) and in-place zero-copy
-        // requests (against their own input): the columns that differ, found
-        // on the device, so that only they cross PCIe
-        std::vector<int> dq;  // indices into fin of diffed requests
-        std::vector<double *> dl, du;
-        std::vector<const double *> bl, bu;
-        for (size_t q = 0; q < fin.size(); q++)
-            if (S->slot_delta[fin[q]] || S->slot_inplace[fin[q]]) {
-                const int k = fin[q];
-                dq.push_back(static_cast<int>(q));
-                dl.push_back(S->slot_lb[k]);
-                du.push_back(S->slot_ub[k]);
-                bl.push_back(S->slot_delta[k] ? S->d_base : S->orig_lb(k));
-                bu.push_back(S->slot_delta[k] ? S->d_base + n : S->orig_ub(k));
-            }
-        if (!dq.empty()) {
-            const int nd = static_cast<int>(dq.size());
-            upload(P->d_lbp, dl.data(), nd, s);
-            upload(P->d_ubp, du.data(), nd, s);
+        // requests (against their own input): the columns that differ, listed
+        // by the unpack, packed into pinned memory, so that only they cross PCIe
+        const int nd = static_cast<int>(fin.size());
+        std::vector<const double *> bl(nd, nullptr), bu(nd, nullptr);
+        bool any_diff = false;
+        for (int q = 0; q < nd; q++) {
+            const int k = fin[q];
+            if (!S->slot_delta[k] && !S->slot_inplace[k]) continue;
+            bl[q] = S->slot_delta[k] ? S->d_base : S->orig_lb(k);
+            bu[q] = S->slot_delta[k] ? S->d_base + n : S->orig_ub(k);
+            any_diff = true;
+        }
+        const VectorGrid g = vector_grid(P->M.n, nd);
+        if (any_diff) {
             upload(S->d_blp, const_cast<double **>(bl.data()), nd, s);
             upload(S->d_bup, const_cast<double **>(bu.data()), nd, s);
             check(hipMemsetAsync(S->d_ccnt, 0, sizeof(int) * nd, s), "memset");
-            hipLaunchKernelGGL(diff_kernel, dim3(gx, std::max(1, std::min(nd, 1024))), dim3(256), 0, s,
-                               static_cast<int>(n), nd, P->d_lbp, P->d_ubp, S->d_blp, S->d_bup,
-                               Server::kDiffCap, S->d_ccnt, S->d_ccols, S->d_cl, S->d_cu);
-            check(hipGetLastError(), "diff launch");
-            // packed on the device, so that only the changes cross PCIe
+            ChangeLists L;
+            L.lb = S->d_blp;
+            L.ub = S->d_bup;
+            L.cap = Server::kDiffCap;
+            L.cnt = S->d_ccnt;
+            L.cols = S->d_ccols;
+            L.vl = S->d_cl;
+            L.vu = S->d_cu;
+            hipLaunchKernelGGL(unpack_kernel<true>, dim3(g.grid), dim3(256), 0, s, P->M, P->D, nd, P->d_list, P->d_lbp,
+                               P->d_ubp, g.per_unit, 0, L);
             hipLaunchKernelGGL(compact_changes_kernel, dim3(std::max(1, std::min(nd, 1024))), dim3(256), 0, s, nd,
-                               Server::kDiffCap, S->d_ccnt, S->d_ccols, S->d_cl, S->d_cu, S->d_off, S->d_kcols,
-                               S->d_kl, S->d_ku);
-            check(hipGetLastError(), "compact launch");
-            check(hipMemcpyAsync(S->h_ccnt, S->d_ccnt, sizeof(int) * nd, hipMemcpyDeviceToHost, s), "D2H");
-            check(hipMemcpyAsync(S->h_off, S->d_off, sizeof(int) * (nd + 1), hipMemcpyDeviceToHost, s), "D2H");
+                               Server::kDiffCap, S->d_ccnt, S->d_ccols, S->d_cl, S->d_cu, S->h_ccnt, S->h_off,
+                               S->h_ccols, S->h_cl, S->h_cu);
+        } else {
+            hipLaunchKernelGGL(unpack_kernel<false>, dim3(g.grid), dim3(256), 0, s, P->M, P->D, nd, P->d_list, P->d_lbp,
+                               P->d_ubp, g.per_unit, 0, ChangeLists());
+        }
+        check(hipGetLastError(), "unpack launch");
+        std::vector<Server::Done> out(fin.size());
+        if (any_diff) {
             check(hipStreamSynchronize(s), "diff sync");
-            const size_t total = static_cast<size_t>(S->h_off[nd]);
-            if (total > 0) {
-                check(hipMemcpyAsync(S->h_ccols, S->d_kcols, sizeof(int) * total, hipMemcpyDeviceToHost, s), "D2H");
-                check(hipMemcpyAsync(S->h_cl, S->d_kl, sizeof(double) * total, hipMemcpyDeviceToHost, s), "D2H");
-                check(hipMemcpyAsync(S->h_cu, S->d_ku, sizeof(double) * total, hipMemcpyDeviceToHost, s), "D2H");
-                check(hipStreamSynchronize(s), "diff sync");
-            }
             for (int j = 0; j < nd; j++) {
                 const int c = S->h_ccnt[j];
-                if (c > Server::kDiffCap) continue;  // too many: the full vector below
-                const int k = fin[dq[j]];
-                Server::Done &d = out[dq[j]];
+                if (!bl[j] || c > Server::kDiffCap) continue;  // not asked for or too many: the full vector below
+                const int k = fin[j];
+                Server::Done &d = out[j];
                 const size_t o = static_cast<size_t>(S->h_off[j]);
                 if (S->slot_inplace[k]) {
                     // the caller's buffers hold the input: write the changes

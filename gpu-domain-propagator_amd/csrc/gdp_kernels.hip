@@ -2863,9 +2863,14 @@ __global__ __launch_bounds__(256) void hint_kernel(DevMatrix M, DevState D, int 
 // envelope: the run is an error and leaves the vectors alone.  256 vectors of
 // 100,000 columns: 174 us (336 with one column in flight, over all XCDs and
 // with the exact accumulators read for every column).
+// With kDiff (a server's finished requests) it also lists the columns in which
+// a vector differs, bit for bit, from the one at L.lb[k], L.ub[k] (null: not
+// asked for): the differing lanes of a wave take their places from one atomic.
+// A pass of its own over vectors and bases took three times the unpack.
+template <bool kDiff>
 __global__ __launch_bounds__(256) void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list,
                                                      double *const *lbp, double *const *ubp, int per_unit,
-                                                     int checked) {
+                                                     int checked, ChangeLists L) {
     if (checked && D.global[kGlobalEnvelope] != 0) return;
     // blocks mode: one pass over all columns
     for_vectors(M.replicas ? n_list : 1, per_unit, [&](int k, int b) {
@@ -2873,7 +2878,14 @@ __global__ __launch_bounds__(256) void unpack_kernel(DevMatrix M, DevState D, in
         const DevState V = unit_view(M, D, list[k]);
         double *lbs = lbp[M.replicas ? k : 0];
         double *ubs = ubp[M.replicas ? k : 0];
-        for (int i0 = tid; i0 < M.n; i0 += 4 * stride) {
+        const int lane = static_cast<int>(threadIdx.x & 63);
+        const double *base_l = nullptr, *base_u = nullptr;
+        if constexpr (kDiff) {
+            base_l = L.lb[k];
+            base_u = L.ub[k];
+        }
+        for (int w0 = tid - lane; w0 < M.n; w0 += 4 * stride) {
+            const int i0 = w0 + lane;
             int col[4];
             int2 ai[4];
             double2 af[4];
@@ -2887,9 +2899,10 @@ __global__ __launch_bounds__(256) void unpack_kernel(DevMatrix M, DevState D, in
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 const int id = i0 + q * stride;
-                if (col[q] < 0) continue;
-                double l, u;
-                if (id < M.n_int) {
+                if (!kDiff && col[q] < 0) continue;
+                double l = 0.0, u = 0.0;
+                if (col[q] < 0) {
+                } else if (id < M.n_int) {
                     l = static_cast<double>(ai[q].x);
                     u = static_cast<double>(ai[q].y);
                     if (ai[q].x == kAiHigh || ai[q].y == kAiLow) {
@@ -2901,12 +2914,36 @@ __global__ __launch_bounds__(256) void unpack_kernel(DevMatrix M, DevState D, in
                     l = af[q].x;
                     u = af[q].y;
                 }
-                lbs[col[q]] = l;
-                ubs[col[q]] = u;
+                if (col[q] >= 0) {
+                    lbs[col[q]] = l;
+                    ubs[col[q]] = u;
+                }
+                if constexpr (kDiff) {
+                    if (base_l == nullptr) continue;
+                    const bool differs = col[q] >= 0 &&
+                                         (__double_as_longlong(l) != __double_as_longlong(base_l[col[q]]) ||
+                                          __double_as_longlong(u) != __double_as_longlong(base_u[col[q]]));
+                    const unsigned long long all = __ballot(differs);
+                    if (all == 0ull) continue;
+                    int at = 0;
+                    if (lane == 0) at = atomic_add_i(&L.cnt[k], __popcll(all));
+                    at = __shfl(at, 0, 64) + __popcll(all & ((1ull << lane) - 1ull));
+                    if (differs && at < L.cap) {
+                        const size_t to = static_cast<size_t>(k) * L.cap + at;
+                        L.cols[to] = col[q];
+                        L.vl[to] = l;
+                        L.vu[to] = u;
+                    }
+                }
             }
         }
     });
 }
+
+template __global__ void unpack_kernel<false>(DevMatrix, DevState, int, const int *, double *const *, double *const *,
+                                              int, int, ChangeLists);
+template __global__ void unpack_kernel<true>(DevMatrix, DevState, int, const int *, double *const *, double *const *,
+                                             int, int, ChangeLists);
 
 // Writes the changed columns of delta requests into their bound vectors:
 // vector k gets lbs[cols[h]] = lv[h], ubs[cols[h]] = uv[h] for h in
@@ -2931,34 +2968,6 @@ __global__ __launch_bounds__(256) void copy_pairs_kernel(long long n2, int count
         for (long long i = blockIdx.x * static_cast<long long>(blockDim.x) + threadIdx.x; i < h;
              i += static_cast<long long>(gridDim.x) * blockDim.x)
             dst[i] = src[i];
-    }
-}
-
-// Columns in which vector k (lbp[k], ubp[k]) differs from the base vector,
-// bit for bit: their indices and bounds go to region k (capacity cap) of
-// cols / vl / vu, their number to cnt[k] (which may exceed cap).  cnt must be
-// zero on entry.
-__global__ __launch_bounds__(256) void diff_kernel(int n, int n_list, double *const *lbp, double *const *ubp,
-                                                   const double *const *blp, const double *const *bup, int cap,
-                                                   int *cnt, int *cols, double *vl, double *vu) {
-    for (int k = blockIdx.y; k < n_list; k += gridDim.y) {
-        const double *l = lbp[k];
-        const double *u = ubp[k];
-        const double *base_l = blp[k];
-        const double *base_u = bup[k];
-        for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-            const double a = l[j], b = u[j];
-            if (__double_as_longlong(a) == __double_as_longlong(base_l[j]) &&
-                __double_as_longlong(b) == __double_as_longlong(base_u[j]))
-                continue;
-            const int pos = atomic_add_i(&cnt[k], 1);
-            if (pos < cap) {
-                const size_t q = static_cast<size_t>(k) * cap + pos;
-                cols[q] = j;
-                vl[q] = a;
-                vu[q] = b;
-            }
-        }
     }
 }
 
@@ -3023,12 +3032,13 @@ __global__ __launch_bounds__(64) void measure_total_kernel(int parts, const doub
 }
 
 
-// Packs the changed columns that diff_kernel found for nd vectors (vector
-// k's cnt[k] entries at [k * cap, ...), none when cnt[k] > cap) into
-// consecutive positions: vector k's start into off[k], the total into
-// off[nd].  One workgroup per vector; each sums the counts before its own.
+// Packs the changed columns listed for nd vectors (vector k's cnt[k] entries
+// at [k * cap, ...), none when cnt[k] > cap) into consecutive positions of
+// pinned host memory: vector k's count into cnt_out[k], its start into off[k],
+// the total into off[nd].  One workgroup per vector; each sums the counts
+// before its own.
 __global__ __launch_bounds__(256) void compact_changes_kernel(int nd, int cap, const int *cnt, const int *cols,
-                                                              const double *vl, const double *vu, int *off,
+                                                              const double *vl, const double *vu, int *cnt_out, int *off,
                                                               int *kcols, double *kl, double *ku) {
     __shared__ int part[256];
     for (int k = blockIdx.x; k < nd; k += gridDim.x) {
@@ -3046,6 +3056,7 @@ __global__ __launch_bounds__(256) void compact_changes_kernel(int nd, int cap, c
         const int o = part[0];
         const int c = cnt[k] <= cap ? cnt[k] : 0;
         if (threadIdx.x == 0) {
+            cnt_out[k] = cnt[k];
             off[k] = o;
             if (k == nd - 1) off[nd] = o + c;
         }
