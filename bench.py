@@ -527,7 +527,7 @@ def summarize_steps(d, out_md):
     trace.sort(key=lambda r: int(r["Start_Timestamp"]))
     props, cur = [], None
     for r in trace:
-        name = r["Kernel_Name"].split("(")[0].split("::")[-1]
+        name = r["Kernel_Name"].split("(")[0].split("::")[-1].split("<")[0]
         dur = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3
         if name == "load_kernel":
             cur = {"steps": [], "start": int(r["Start_Timestamp"])}
