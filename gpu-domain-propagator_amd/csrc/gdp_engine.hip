@@ -1608,28 +1608,31 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
     hipLaunchKernelGGL(load_kernel, dim3(g.grid), dim3(256), 0, s, M, D, n_list, P->d_list, P->d_lbp, P->d_ubp, ref,
                        g.per_unit, P->borrowed ? 1 : 0);
     if (referenced) {
-        // walking the columns of up to this many words costs less than an
-        // eighth of the unit's segments
-        const int limit = std::max(16, M.nwords / 64);
+        // Walking the columns of up to this many words drops few enough segments
+        // to be worth it.  256 vectors, up to 50 of 100,000 columns changed: with a
+        // line of nwords / 64 = 48 words five vectors dropped and recomputed all
+        // their 2784 segments, 100 us of fill_parts_kernel.
+        const int limit = std::max(16, M.nwords / 16);
         hipLaunchKernelGGL(drop_parts_kernel, dim3(std::max(1, std::min(8, (M.nwords + 255) / 256)),
                                                    std::max(1, std::min(n_list, 1024))), dim3(256), 0, s,
                            M, D, n_list, P->d_list, ref, limit);
     }
     check(hipGetLastError(), "load launch");
     if (hint_ptr != nullptr && M.mark_rows && hint_ptr[n_list] > 0) {
-        if (M.n_seg_parts > 0) {
-            // segments a wave looks at: few while the units are few
-            const int chunk = std::max(1, std::min(4, n_list / 16));
-            const long long wgs = static_cast<long long>((n_list + 7) / 8) * 8 *
-                                  ((M.n_seg_parts + 4 * chunk - 1) / (4 * chunk));
-            hipLaunchKernelGGL(fill_parts_kernel, dim3(static_cast<int>(std::min<long long>(wgs, 1 << 20))), dim3(256), 0,
-                               s, M, D, n_list, P->d_list, start, chunk);
-        }
         reserve_hints(P, hint_ptr[n_list]);
         upload(P->d_hint_ptr, hint_ptr, n_list + 1, s);
         upload(P->d_hints, hints, hint_ptr[n_list], s);
         hipLaunchKernelGGL(hint_kernel, dim3(16, std::max(1, std::min(n_list, 1024))), dim3(256), 0, s, M, D, n_list,
                            P->d_list, P->d_hint_ptr, P->d_hints, P->d_inv_perm, start);
+        if (M.n_seg_parts > 0) {
+            // segments a wave looks at: few while the units are few, more where
+            // most have their partial from a reference
+            const int chunk = std::max(1, std::min(referenced ? 16 : 4, n_list / (referenced ? 8 : 16)));
+            const long long wgs = static_cast<long long>((n_list + 7) / 8) * 8 *
+                                  ((M.n_seg_parts + 4 * chunk - 1) / (4 * chunk));
+            hipLaunchKernelGGL(fill_parts_kernel, dim3(static_cast<int>(std::min<long long>(wgs, 1 << 20))), dim3(256), 0,
+                               s, M, D, n_list, P->d_list, start, chunk);
+        }
         check(hipGetLastError(), "hint launch");
     }
 }

@@ -2798,8 +2798,11 @@ __global__ __launch_bounds__(256) void drop_parts_kernel(DevMatrix M, DevState D
 
 // Computes the segment partials that hinted units do not have yet (no
 // reference, or dropped): a step of marked rows recomputes only listed
-// segments.  Each wave looks at `chunk` segments of a unit; units that process
-// every row in their first step compute theirs there.
+// segments.  Those that the hints have listed are left to the first step: a
+// dropped segment mostly is one, because it holds a column in which the unit
+// differs.  Each wave looks at `chunk` segments of a unit; units that process
+// every row in their first step compute theirs there.  256 vectors, 2784 segments:
+// 160 us with the listed segments and four a wave, 17 without and 16 a wave.
 __global__ __launch_bounds__(256) void fill_parts_kernel(DevMatrix M, DevState D_arg, int n_list, const int *list,
                                                          int start_step, int chunk) {
     DevState D = D_arg;
@@ -2807,6 +2810,7 @@ __global__ __launch_bounds__(256) void fill_parts_kernel(DevMatrix M, DevState D
     const int lane = threadIdx.x & 63;
     // workgroups go round the 8 XCDs: a unit's keep to one, unit after unit, so
     // that an L2 holds the snapshots in work
+    const int listed = static_cast<int>(mark_stamp(start_step, true) + static_cast<unsigned>(D.persist[kPersistEpoch]));
     const int wg_parts = (blockDim.x >> 6) * chunk;
     const int per_unit = (M.n_seg_parts + wg_parts - 1) / wg_parts;
     const int xcd = blockIdx.x & 7, on_xcd = (n_list - xcd + 7) / 8;
@@ -2818,7 +2822,8 @@ __global__ __launch_bounds__(256) void fill_parts_kernel(DevMatrix M, DevState D
         {
             const int p0 = uniform((j % per_unit) * wg_parts + (threadIdx.x >> 6) * chunk);
             const int p = p0 + lane;
-            unsigned long long todo = __ballot(lane < chunk && p < M.n_seg_parts && V.seg_parts[p].stamp == 0);
+            unsigned long long todo = __ballot(lane < chunk && p < M.n_seg_parts && V.seg_parts[p].stamp == 0 &&
+                                               V.seg_marks[p] != listed);
             while (todo) {
                 const int part = uniform(p0 + __ffsll(static_cast<long long>(todo)) - 1);
                 todo &= todo - 1;
