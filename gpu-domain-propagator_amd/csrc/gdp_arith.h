@@ -40,10 +40,6 @@ GDP_HD bool eps_gt(double x, double y) { return (x - y) > kEps; }
 GDP_HD bool is_pos_inf(double x) { return x >= kInf; }
 GDP_HD bool is_neg_inf(double x) { return x <= -kInf; }
 
-// Integer rounding of a candidate bound (propagation_methods.cuh:40-52).
-GDP_HD double round_upper(bool is_cont, double ub) { return is_cont ? ub : floor(ub + kEps); }
-GDP_HD double round_lower(bool is_cont, double lb) { return is_cont ? lb : ceil(lb - kEps); }
-
 // Storage class of a column from its bound envelope [l, u]: 0 = 2 x int16,
 // 1 = 2 x int32, 2 = 2 x double.
 GDP_HD int column_class(int vartype, double l, double u) {
@@ -96,12 +92,13 @@ GDP_HD bool row_gate(double minact, double maxact, int min_inf, int max_inf,
 GDP_HD double eps_max_step(double running, double d) { return eps_gt(d, running) ? d : running; }
 
 // Candidate bound of one variable from one side of a row
-// (propagation_methods.cuh:78-134): an upper bound v + l or a lower bound
+// (propagation_methods.cuh:40-52, :78-134): an upper bound v + l or a lower bound
 // v + u, v the side's slack or surplus over the coefficient; `num_inf` is the
 // infinity count of the activity it is derived from, and the other bound
 // drops out when it is the one infinite contribution.  Lower bounds are
-// computed mirrored (ceil(v - eps) = -floor(-v + eps), exactly), so that both
-// kinds share their instructions in a wave.  Returns whether it tightens.
+// computed mirrored (ceil(v - eps) = -floor(-v + eps); v = eps gives +0, whose
+// sign only the accepted bounds need), so that both kinds share their
+// instructions in a wave.  Returns whether it tightens.
 GDP_HD bool candidate(bool upper, double v, int num_inf, double l, double u, bool is_cont, double &nb) {
     if (num_inf == 0) {
         v += upper ? l : u;
@@ -109,9 +106,10 @@ GDP_HD bool candidate(bool upper, double v, int num_inf, double l, double u, boo
         return false;
     }
     const double x = upper ? v : -v;
-    const double w = round_upper(is_cont, x);
+    const double w = is_cont ? x : floor(x + kEps);
     if (!eps_lt(w, upper ? u : -l)) return false;
     nb = upper ? w : -w;
+    if (!upper && !is_cont && x == -kEps) nb = 0.0;
     return true;
 }
 
