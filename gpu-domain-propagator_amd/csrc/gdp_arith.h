@@ -153,4 +153,14 @@ GDP_HD int tighten_variable(double a, double lhs, double rhs, double minact, dou
     return r;
 }
 
+// Whether the launch of double-buffered round `step` runs, as far as the unit's
+// state says (`infeasible`: the round that crossed bounds, 0: none; `unusable`:
+// crossed or outside the envelope as loaded).  The launch itself reports the
+// crossings of round step - 1, so that value says nothing: waves that start
+// late must decide as the first ones did, for the barriers of their workgroup.
+// An earlier crossing is a smaller number.
+GDP_HD bool round_runs(int step, int infeasible, bool unusable) {
+    return !unusable && (infeasible == 0 || infeasible == step - 1);
+}
+
 }  // namespace gdp

@@ -2011,7 +2011,7 @@ __global__ __launch_bounds__(kTest ? 512 : 256) __attribute__((amdgpu_waves_per_
     __shared__ int any_moved;
     const long long *p = reinterpret_cast<const long long *>(&D.units[0]);
     const long long w0 = coherent_load(p), w2 = coherent_load(p + 2);
-    const bool runs = (w0 >> 32) == 0 && w2 == 0 && (step == 1 || round_moved(D, step - 1));
+    const bool runs = round_runs(step, static_cast<int>(w0 >> 32), w2 != 0) && (step == 1 || round_moved(D, step - 1));
     if (blockIdx.x == 0 && threadIdx.x == 0)
         __hip_atomic_store(D.host_word, runs ? step : kRoundsOver, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (!runs) return;
