@@ -416,7 +416,10 @@ struct HostBlock {
 
 // Phase times of a problem's creation, printed to stderr when the
 // environment variable GDP_TRACE_CREATE is set (a diagnostic of where the
-// creation time goes: host ordering, allocations, copies, device layout).
+// creation time goes: host ordering, allocations, copies, device layout), and
+// the bytes of a run state: the least one, with the lists of marked rows, and
+// with the arrays of the double-buffered rounds too (0: runs take the three
+// phases).
 class CreateTrace {
   public:
     CreateTrace() : on_(std::getenv("GDP_TRACE_CREATE") != nullptr), t0_(Clock::now()), last_(t0_) {}
@@ -430,6 +433,9 @@ class CreateTrace {
         std::snprintf(buf, sizeof(buf), " %s=%.2f", phase, ms(last_, t));
         line_ += buf;
         last_ = t;
+    }
+    void bytes(const char *name, size_t value) {
+        if (on_) line_ += std::string(" ") + name + "=" + std::to_string(value);
     }
 
   private:
@@ -1091,8 +1097,10 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     const int NI = P->n_inst;
     if (P->replicas ? NI != 1 || n_padded > kMaxRoundEntries : NI > kMaxRoundUnits || n_padded > kMaxBatchEntries)
         return;
+    // (row_marking and mark_limit say how the three phases choose their rows)
     if (T.item_nnz != def.item_nnz || T.mega_blocks_per_cu != def.mega_blocks_per_cu ||
         T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
+        T.row_marking != def.row_marking || T.mark_limit != def.mark_limit ||
         !std::equal(T.group_log, T.group_log + 10, def.group_log))
         return;
     // Entries per lane: few while the passes (256 lane entries of K each) still
@@ -1464,6 +1472,15 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
 
         P->host = host_slots().take();
         plan_rounds(P, R.start.data(), R.count.data(), first_part, h_part_row, h_seg_rows, n_padded);
+        {
+            DevState D{};
+            UnitTables T;
+            RoundPlan plan = P->R;
+            const size_t lists = carve_state(M, replicas, NI, 1, nullptr, D, T, true);
+            trace.bytes("state_bytes", carve_state(M, replicas, NI, 1, nullptr, D, T, false));
+            trace.bytes("with_lists", lists);
+            trace.bytes("with_rounds", P->rounds_ok ? lists + carve_rounds(P->Mr, nullptr, plan) : 0);
+        }
 
         P->mega_threads = T.mega_threads == 256 || T.mega_threads == 1024 ? T.mega_threads : 512;
         P->mega_fn = P->mega_threads == 256    ? reinterpret_cast<const void *>(mega_kernel<256, false>)
