@@ -171,8 +171,11 @@ constexpr int kBarrierGen = 32;
 constexpr int kBarrierGroup = 64;  // + 32 * group, 8 groups
 constexpr int kBarrierWords = 64 + 32 * 8;
 
-// wall_clock64 runs at 100 MHz on CDNA; give up a wait after 1 s
-constexpr long long kWaitTimeoutTicks = 100000000LL;
+// wall_clock64 runs at 100 MHz on CDNA.  A wait inside a launch is given up
+// after 1 s, or after GDP_WAIT_US microseconds where that is set when the
+// problem is created.
+constexpr long long kWaitTicksPerUs = 100;
+constexpr long long kWaitDefaultUs = 1000000;
 
 // Partial activity of one segment of a split row.
 struct SegPart {
@@ -255,6 +258,7 @@ struct DevState {
     int n_lds;             // binary columns read from LDS (persistent launch of one unit; else 0)
     unsigned *SB;          // 2-bit codes of the binary columns (sb_words per unit)
     int n_codes;           // binary columns read from their codes in SB (kRecords)
+    long long wait_ticks;  // bound of a wait inside a launch
     int *host_word;        // pinned: the step that the guarded launches have started, or kRoundsOver
 };
 

@@ -1205,6 +1205,8 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         P->n_inst = static_cast<int>(inst.size());
         if (tuning) P->tuning = *tuning;
         const Tuning &T = P->tuning;
+        const char *wait_us = std::getenv("GDP_WAIT_US");
+        P->D.wait_ticks = kWaitTicksPerUs * (wait_us ? std::max(0LL, std::atoll(wait_us)) : kWaitDefaultUs);
         const int NI = P->n_inst;
         std::vector<int> col_off(NI + 1, 0), row_off(NI + 1, 0);
         long long nnz_total = 0;

@@ -1660,7 +1660,7 @@ __device__ __forceinline__ bool grid_barrier(const DevState &D, unsigned nblocks
                     ok = 0;
                     break;
                 }
-                if (wall_clock64() - t0 > kWaitTimeoutTicks) {
+                if (wall_clock64() - t0 > D.wait_ticks) {
                     atomic_or_i(&D.global[kGlobalError], 1);
                     ok = 0;
                     break;
@@ -2071,7 +2071,7 @@ __device__ __forceinline__ bool gather_barrier(const DevState &D, const RoundPla
                     got |= static_cast<unsigned>(v);
                     break;
                 }
-                if (wall_clock64() - t0 > kWaitTimeoutTicks || coherent_load(&D.global[kGlobalError])) {
+                if (wall_clock64() - t0 > D.wait_ticks || coherent_load(&D.global[kGlobalError])) {
                     ok = false;
                     break;
                 }
@@ -2177,7 +2177,7 @@ __device__ __forceinline__ bool gather_units(const DevState &D, const RoundPlan 
                 got = static_cast<unsigned>(v);
                 break;
             }
-            if (wall_clock64() - t0 > kWaitTimeoutTicks || coherent_load(&D.global[kGlobalError])) {
+            if (wall_clock64() - t0 > D.wait_ticks || coherent_load(&D.global[kGlobalError])) {
                 if (lane == 0) {
                     atomic_or_i(&D.global[kGlobalError], 1);
                     *wg_ok = 0;
@@ -2390,11 +2390,11 @@ template __global__ void batch_rounds_kernel<false>(DevMatrix, DevState, RoundPl
 template __global__ void batch_rounds_kernel<true>(DevMatrix, DevState, RoundPlan);
 
 // Writes the final bounds of a batch to the caller's vectors (not when some
-// input was outside its envelope), finds crossed bounds of the instances' last
+// input was outside its envelope or a wait failed), finds crossed bounds of the instances' last
 // rounds, and the last workgroup to finish writes the outcomes to pinned host
 // memory.
 __global__ __launch_bounds__(256) void unpack_batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
-    if (D.global[kGlobalEnvelope] == 0) {
+    if (D.global[kGlobalEnvelope] == 0 && D.global[kGlobalError] == 0) {
         const DevState A = block_view(M, D, R, 0), B = block_view(M, D, R, 1);
         const int stride = gridDim.x * blockDim.x;
         for (int id = blockIdx.x * blockDim.x + threadIdx.x; id < M.n; id += stride) {
@@ -2440,7 +2440,7 @@ __global__ __launch_bounds__(256) void unpack_batch_rounds_kernel(DevMatrix M, D
 }
 
 // Writes the final bounds to the caller's vectors (not when the input was
-// outside the envelope), finds crossed bounds of the last round, and the last
+// outside the envelope or a wait failed), finds crossed bounds of the last round, and the last
 // workgroup to finish writes the outcome to pinned host memory.
 __global__ __launch_bounds__(256) void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R) {
     const long long *p = reinterpret_cast<const long long *>(&D.units[0]);
@@ -2456,7 +2456,7 @@ __global__ __launch_bounds__(256) void unpack_rounds_kernel(DevMatrix M, DevStat
     }
     last = uniform(infeasible ? infeasible : last);
     const DevState V = block_view(M, D, R, last & 1);
-    if ((w2 >> 32) == 0) {
+    if ((w2 >> 32) == 0 && D.global[kGlobalError] == 0) {
         const int stride = gridDim.x * blockDim.x;
         bool crossed = false;
         for (int id = blockIdx.x * blockDim.x + threadIdx.x; id < M.n; id += stride) {
@@ -2864,8 +2864,9 @@ __global__ __launch_bounds__(256) void hint_kernel(DevMatrix M, DevState D, int 
 }
 
 // Writes the accumulated bounds of the listed units back to the caller's
-// column order.  With `checked`, nothing when a loaded vector left the
-// envelope: the run is an error and leaves the vectors alone.  256 vectors of
+// column order.  Nothing when a wait of the run failed or, with `checked`, a
+// loaded vector left the envelope: the run is an error and leaves the vectors
+// alone.  256 vectors of
 // 100,000 columns: 174 us (336 with one column in flight, over all XCDs and
 // with the exact accumulators read for every column).
 // With kDiff (a server's finished requests) it also lists the columns in which
@@ -2876,7 +2877,7 @@ template <bool kDiff>
 __global__ __launch_bounds__(256) void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list,
                                                      double *const *lbp, double *const *ubp, int per_unit,
                                                      int checked, ChangeLists L) {
-    if (checked && D.global[kGlobalEnvelope] != 0) return;
+    if (D.global[kGlobalError] != 0 || (checked && D.global[kGlobalEnvelope] != 0)) return;
     // blocks mode: one pass over all columns
     for_vectors(M.replicas ? n_list : 1, per_unit, [&](int k, int b) {
         const int tid = b * 256 + static_cast<int>(threadIdx.x), stride = per_unit * 256;
