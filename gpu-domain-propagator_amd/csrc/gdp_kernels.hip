@@ -1092,10 +1092,10 @@ __device__ __forceinline__ void sweep_piece(const DevMatrix &M, const DevState &
     note_change(D, u, step, moved);
 }
 
-// Running sums of the pieces of `win` units, slots (base + k) * groups + mine,
-// and their all-rows bits, in LDS (the whole workgroup).
+// Running sums of the pieces of the units of slots [base, base + win), and
+// their all-rows bits, in LDS (the whole workgroup).
 __device__ __forceinline__ void lay_out_window(const DevMatrix &M, const DevState &D, int step, int base, int win,
-                                               int mine, int groups, int *sums, unsigned *dense) {
+                                               int *sums, unsigned *dense) {
     const int lane = threadIdx.x & 63;
     const int wg_wave = threadIdx.x >> 6;
     __syncthreads();  // nobody still reads the previous window
@@ -1104,7 +1104,7 @@ __device__ __forceinline__ void lay_out_window(const DevMatrix &M, const DevStat
         int n = 0;
         UnitStep us{};
         if (k < win) {
-            const int slot = (base + k) * groups + mine;
+            const int slot = base + k;
             const int u = M.replicas ? D.active[slot] : slot;
             us = unit_step_lane(M, D, u, step);
             if (us.active) n = us.all_rows ? unit_items(M, u) : list_passes(M, D, u, step);
@@ -1156,36 +1156,41 @@ __device__ __forceinline__ void sweep_phase(const DevMatrix &M, const DevState &
     const int u1 = M.replicas ? uniform(D.active[0]) : 0;
     int *sums = reinterpret_cast<int *>(window);            // kWindowUnits + 64
     unsigned *dense = window + kWindowUnits + 64;           // all-rows bits
-    // Many bound vectors of one matrix: every workgroup works on the vectors
-    // of its own XCD (workgroups go round the 8 XCDs), slots x, x + 8, ...,
-    // so that an L2 holds the snapshots of an eighth of the vectors in work.
-    // Only the locality hangs on where a workgroup really runs.
-    const int groups = M.replicas && n_slots >= 64 && gridDim.x % 8 == 0 ? 8 : 1;
-    const int mine = groups == 8 ? blockIdx.x & 7 : 0;
-    if (groups == 8) {
+    // Many bound vectors of one matrix: the workgroups of an XCD (they go round
+    // the 8 XCDs) take an eighth of the pieces that lies together, so that an
+    // L2 holds the snapshots of an eighth of the vectors in work, and every
+    // workgroup has work whichever vectors still need any (one vector of 64 with
+    // 4.4M nonzeros and 32 rounds of work: 2.5 ms; 5.8 with every eighth vector
+    // to an XCD).  Only the locality hangs on where a workgroup really runs.
+    const bool by_xcd = M.replicas && n_slots >= 64 && gridDim.x % 8 == 0;
+    const int xcd = blockIdx.x & 7;
+    const int chip_waves = nwaves;
+    if (by_xcd) {
         const int waves = blockDim.x >> 6;
         wave = uniform((blockIdx.x >> 3) * waves + (threadIdx.x >> 6));
         nwaves = (gridDim.x >> 3) * waves;
     }
-    const int own = (n_slots - mine + groups - 1) / groups;  // slots of this group
     int shift = 0;  // pieces of the windows before
-    for (int base = 0; base < own; base += kWindowUnits) {
-        const int win = min(kWindowUnits, own - base);
+    for (int base = 0; base < n_slots; base += kWindowUnits) {
+        const int win = min(kWindowUnits, n_slots - base);
         const int blocks = (win + 63) / 64;
         int total;
         if (single) {
             total = one.all_rows ? unit_items(M, u1) : uniform(list_passes(M, D, u1, step));
         } else {
-            lay_out_window(M, D, step, base, win, mine, groups, sums, dense);
+            lay_out_window(M, D, step, base, win, sums, dense);
             total = uniform(sums[blocks * 64 - 1]);
         }
         // items in up to 4 parts while the waves outnumber them: an item is
         // four passes or more, a chain of about 4 us each
-        const int log_parts = total * 4 <= nwaves ? 2 : (total * 2 <= nwaves ? 1 : 0);
+        const int log_parts = total * 4 <= chip_waves ? 2 : (total * 2 <= chip_waves ? 1 : 0);
+        const int parts = total << log_parts;
+        const int begin = by_xcd ? (parts >> 3) * xcd + ((parts & 7) * xcd >> 3) : 0;
+        const int end = by_xcd ? (parts >> 3) * (xcd + 1) + ((parts & 7) * (xcd + 1) >> 3) : parts;
         // the grid's stride goes on across the windows
         int q = (wave - shift) % nwaves;
         if (q < 0) q += nwaves;
-        for (; q < total << log_parts; q += nwaves) {
+        for (q += begin; q < end; q += nwaves) {
             const int piece = q >> log_parts;
             int u = u1, before = 0;
             bool all_rows = one.all_rows;
@@ -1199,13 +1204,13 @@ __device__ __forceinline__ void sweep_phase(const DevMatrix &M, const DevState &
                 const int k = uniform(__ffsll(static_cast<long long>(__ballot(upto > piece))) - 1);
                 before = uniform(k == 0 ? (blk == 0 ? 0 : sums[blk * 64 - 1]) : __shfl(upto, k - 1, 64));
                 const int at = blk * 64 + k;
-                const int slot = (base + at) * groups + mine;
+                const int slot = base + at;
                 u = M.replicas ? uniform(D.active[slot]) : slot;
                 all_rows = uniform((dense[at >> 5] >> (at & 31)) & 1u) != 0;
             }
             sweep_piece(M, D, u, piece - before, all_rows, q & ((1 << log_parts) - 1), log_parts, step, st);
         }
-        shift = (shift + (total << log_parts)) % nwaves;
+        shift = (shift + end - begin) % nwaves;
     }
 }
 
