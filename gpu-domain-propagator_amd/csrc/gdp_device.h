@@ -108,9 +108,8 @@ constexpr int kStatusChanged = 0;  // some unit moved a bound in the step
 constexpr int kStatusApply = 2;    // split-row segments queued for the apply phase
 // Words of the problem-wide status block (separate from the ring).
 constexpr int kGlobalError = 0;    // a bounded device wait timed out
-constexpr int kGlobalSteps = 1;    // steps run by the persistent kernel
-constexpr int kGlobalTicket = 2;   // workgroups of unpack_rounds_kernel that are done
-constexpr int kGlobalEnvelope = 3; // some loaded vector left the envelope (runs that then return an error)
+constexpr int kGlobalTicket = 1;   // workgroups of unpack_rounds_kernel that are done
+constexpr int kGlobalEnvelope = 2; // some loaded vector left the envelope (runs that then return an error)
 constexpr int kGlobalWords = 8;
 
 // Words of a run state that outlive its runs: row marks hold the step's stamp
@@ -171,11 +170,8 @@ constexpr int kBarrierGen = 32;
 constexpr int kBarrierGroup = 64;  // + 32 * group, 8 groups
 constexpr int kBarrierWords = 64 + 32 * 8;
 
-// wall_clock64 runs at 100 MHz on CDNA.  A wait inside a launch is given up
-// after 1 s, or after GDP_WAIT_US microseconds where that is set when the
-// problem is created.
-constexpr long long kWaitTicksPerUs = 100;
-constexpr long long kWaitDefaultUs = 1000000;
+// wall_clock64 runs at 100 MHz on CDNA; give up a wait after 1 s
+constexpr long long kWaitTimeoutTicks = 100000000LL;
 
 // Partial activity of one segment of a split row.
 struct SegPart {
@@ -258,7 +254,6 @@ struct DevState {
     int n_lds;             // binary columns read from LDS (persistent launch of one unit; else 0)
     unsigned *SB;          // 2-bit codes of the binary columns (sb_words per unit)
     int n_codes;           // binary columns read from their codes in SB (kRecords)
-    long long wait_ticks;  // bound of a wait inside a launch
     int *host_word;        // pinned: the step that the guarded launches have started, or kRoundsOver
 };
 

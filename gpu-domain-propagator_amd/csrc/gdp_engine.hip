@@ -46,7 +46,7 @@ __global__ void publish_kernel(DevMatrix M, DevState D, int step, int guard, int
 template <int kThreads, bool kLds>
 __global__ void mega_kernel(DevMatrix M, DevState D, int first_step, int max_steps, int n_units);
 __global__ void plan_rounds_kernel(DevMatrix M, RoundBins B, int4 *items);
-__global__ void reset_rounds_kernel(DevState D, RoundPlan R);
+__global__ void reset_rounds_kernel(DevState D, RoundPlan R, int fail);
 template <bool kUnits>
 __global__ void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin);
 template <bool kTest>
@@ -63,7 +63,7 @@ template <bool kTest>
 __global__ void rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unpack_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status,
-                                  int epoch);
+                                  int epoch, int fail);
 __global__ void clean_ax_kernel(DevState D, long long count);
 __global__ void load_kernel(DevMatrix M, DevState D, int n_list, const int *list, const double *const *lbp,
                             const double *const *ubp, ReferenceView ref, int per_unit, int all);
@@ -76,7 +76,7 @@ __global__ void hint_kernel(DevMatrix M, DevState D, int n_list, const int *list
 template <bool kDiff>
 __global__ void unpack_kernel(DevMatrix M, DevState D, int n_list, const int *list, double *const *lbp,
                               double *const *ubp, int per_unit, int checked, ChangeLists L);
-__global__ void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int epoch, int *list, double **lbp,
+__global__ void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int epoch, int fail, int *list, double **lbp,
                                  double **ubp, double *lbs, double *ubs);
 __global__ void report_kernel(DevState D, int n_list, const int *list, UnitState *out);
 __global__ void delta_kernel(int n_list, double *const *lbp, double *const *ubp, const int *ptr, const int *cols,
@@ -560,6 +560,7 @@ struct Problem {
     HostBlock h_tables;               // pinned: launch tables of several units, then their outcomes
     HostBlock h_bounds;               // pinned: small bound vectors on their way
     int servers = 0;                  // servers attached (they own the unit slots)
+    bool fail_waits = false;          // GDP_FAIL_WAITS
     bool graphs_enabled = true;       // GPU_LOOP may capture graphs of the current run state
     bool staging_held = false;
 
@@ -1205,8 +1206,9 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         P->n_inst = static_cast<int>(inst.size());
         if (tuning) P->tuning = *tuning;
         const Tuning &T = P->tuning;
-        const char *wait_us = std::getenv("GDP_WAIT_US");
-        P->D.wait_ticks = kWaitTicksPerUs * (wait_us ? std::max(0LL, std::atoll(wait_us)) : kWaitDefaultUs);
+        // for tests of error handling: every run ends as if a device wait had
+        // lasted too long (the waits see the error word, every kernel ends)
+        P->fail_waits = std::getenv("GDP_FAIL_WAITS") != nullptr;
         const int NI = P->n_inst;
         std::vector<int> col_off(NI + 1, 0), row_off(NI + 1, 0);
         long long nnz_total = 0;
@@ -1605,7 +1607,7 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
     if (n_list == 1) {
         // a single vector: everything by kernel argument
         hipLaunchKernelGGL(reset_one_kernel, dim3(1), dim3(256), 0, s, D, param(0), start, fresh ? 1 : 0, epoch,
-                           P->d_list, P->d_lbp, P->d_ubp, lbp[0], ubp[0]);
+                           P->fail_waits ? 1 : 0, P->d_list, P->d_lbp, P->d_ubp, lbp[0], ubp[0]);
     } else {
         // the tables lie one after the other in the run state: one copy
         const int n_tables = P->replicas ? n_list : 1;
@@ -1619,7 +1621,7 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
         std::memcpy(at(P->d_ubp), ubp, sizeof(double *) * n_tables);
         check(hipMemcpyAsync(base, h, bytes, hipMemcpyHostToDevice, s), "H2D tables");
         hipLaunchKernelGGL(unit_reset_kernel, dim3(std::max(1, std::min(256, (n_list + 3) / 4))), dim3(256), 0, s, D,
-                           n_list, P->d_params, start, fresh ? 1 : 0, epoch);
+                           n_list, P->d_params, start, fresh ? 1 : 0, epoch, P->fail_waits ? 1 : 0);
     }
     const VectorGrid g = vector_grid(M.n, P->replicas ? n_list : 1);
     ReferenceView ref;
@@ -1849,7 +1851,7 @@ RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, in
     R.host_state = &P->host->state;
     __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
-    hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R);
+    hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R, P->fail_waits ? 1 : 0);
     hipLaunchKernelGGL(load_rounds_kernel<false>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
     check(hipGetLastError(), "load launch");
     issue_rounds(P, sync_type, max_rounds);
@@ -1898,7 +1900,7 @@ void run_batch_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, i
     R.mark_limit = 1;
     R.host_state = st;
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
-    hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R);
+    hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R, P->fail_waits ? 1 : 0);
     hipLaunchKernelGGL(load_rounds_kernel<true>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
     check(hipGetLastError(), "load launch");
     __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
@@ -2777,7 +2779,7 @@ Server *server_create(Problem *P, int64_t hbm_budget, int max_slots) {
         S->attached = true;
         // fresh status ring for the server's steps
         hipLaunchKernelGGL(unit_reset_kernel, dim3(1), dim3(256), 0, P->stream, P->D, 0, P->d_params, 0, 1,
-                           next_epoch(P));
+                           next_epoch(P), P->fail_waits ? 1 : 0);
         check(hipStreamSynchronize(P->stream), "server init");
     } catch (...) {
         delete S;

@@ -1665,7 +1665,7 @@ __device__ __forceinline__ bool grid_barrier(const DevState &D, unsigned nblocks
                     ok = 0;
                     break;
                 }
-                if (wall_clock64() - t0 > D.wait_ticks) {
+                if (wall_clock64() - t0 > kWaitTimeoutTicks) {
                     atomic_or_i(&D.global[kGlobalError], 1);
                     ok = 0;
                     break;
@@ -1684,8 +1684,7 @@ __device__ __forceinline__ bool grid_barrier(const DevState &D, unsigned nblocks
 // stride, all meet at a barrier, and all read the same status words, so all
 // take the same decision to go on: the run ends after a step in which no
 // unit moved a bound.  Phases of a step: sweep; apply of the split rows when
-// the sweep queued any; publish.  The number of steps run goes to the global
-// status block (-1 after a failed wait).
+// the sweep queued any; publish.
 template <int kThreads, bool kLds>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void mega_kernel(DevMatrix M, DevState D_arg, int first_step, int max_steps,
                                                         int n_units) {
@@ -1699,7 +1698,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const int wave = uniform(blockIdx.x * waves + (threadIdx.x >> 6));
     const int nwaves = gridDim.x * waves;
     const int n_slots = M.replicas ? D.n_active : n_units;  // replicas: positions in the launch's list
-    int steps = 0;
     for (int step = first_step; step < first_step + max_steps; step++) {
         int *st = status_row(D, step);
         UnitStep one{};
@@ -1717,17 +1715,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             }
         }
         sweep_phase(M, D, step, wave, nwaves, n_units, dyn_lds, one);
-        if (!grid_barrier(D, nblocks, false)) { steps = -1; break; }
+        if (!grid_barrier(D, nblocks, false)) return;
         if (coherent_load(&st[kStatusApply]) > 0) {
             apply_phase(M, D, step, wave, nwaves);
-            if (!grid_barrier(D, nblocks, false)) { steps = -1; break; }
+            if (!grid_barrier(D, nblocks, false)) return;
         }
         publish_phase(M, D, step, wave, nwaves, n_units);
-        if (!grid_barrier(D, nblocks, true)) { steps = -1; break; }
-        steps = step - first_step + 1;
+        if (!grid_barrier(D, nblocks, true)) return;
         if (!coherent_load(&st[kStatusChanged])) break;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) D.global[kGlobalSteps] = steps;
 }
 
 template __global__ void mega_kernel<256, false>(DevMatrix, DevState, int, int, int);
@@ -1925,8 +1921,9 @@ __device__ __forceinline__ int round_item(const DevMatrix &M, const DevState &V,
 }
 
 // Resets the state words, the status ring, the global words and the
-// barrier's arrival slots for a run (one workgroup).
-__global__ __launch_bounds__(256) void reset_rounds_kernel(DevState D, RoundPlan R) {
+// barrier's arrival slots for a run (one workgroup).  `fail`: the error word of
+// a failed wait is set from the start.
+__global__ __launch_bounds__(256) void reset_rounds_kernel(DevState D, RoundPlan R, int fail) {
     const int tid = threadIdx.x;
     for (int u = tid; u < R.n_units; u += 256) {
         UnitState s = {};
@@ -1937,7 +1934,7 @@ __global__ __launch_bounds__(256) void reset_rounds_kernel(DevState D, RoundPlan
         D.units[u] = s;
     }
     for (int k = tid; k < kStatusRows * kStatusWords; k += 256) D.status[k] = 0;
-    for (int k = tid; k < kGlobalWords; k += 256) D.global[k] = 0;
+    for (int k = tid; k < kGlobalWords; k += 256) D.global[k] = k == kGlobalError ? fail : 0;
     for (int k = tid; k < 2 * kMoveLanes * R.n_units; k += 256)
         D.moved[moved_index(k / (2 * kMoveLanes), k & 1, (k >> 1) % kMoveLanes)] = 0;
     for (int k = tid; k < 2 * kMaxGatherBlocks * R.slot_words; k += 256) R.slots[k] = 0ull;
@@ -2076,7 +2073,7 @@ __device__ __forceinline__ bool gather_barrier(const DevState &D, const RoundPla
                     got |= static_cast<unsigned>(v);
                     break;
                 }
-                if (wall_clock64() - t0 > D.wait_ticks || coherent_load(&D.global[kGlobalError])) {
+                if (wall_clock64() - t0 > kWaitTimeoutTicks || coherent_load(&D.global[kGlobalError])) {
                     ok = false;
                     break;
                 }
@@ -2182,7 +2179,7 @@ __device__ __forceinline__ bool gather_units(const DevState &D, const RoundPlan 
                 got = static_cast<unsigned>(v);
                 break;
             }
-            if (wall_clock64() - t0 > D.wait_ticks || coherent_load(&D.global[kGlobalError])) {
+            if (wall_clock64() - t0 > kWaitTimeoutTicks || coherent_load(&D.global[kGlobalError])) {
                 if (lane == 0) {
                     atomic_or_i(&D.global[kGlobalError], 1);
                     *wg_ok = 0;
@@ -2451,6 +2448,7 @@ __global__ __launch_bounds__(256) void unpack_rounds_kernel(DevMatrix M, DevStat
     const long long *p = reinterpret_cast<const long long *>(&D.units[0]);
     const int infeasible = static_cast<int>(coherent_load(p) >> 32);
     const long long w2 = coherent_load(p + 2);
+    const int error = coherent_load(&D.global[kGlobalError]);
     // the last round that moved a bound
     const int lane = threadIdx.x & 63;
     int last = lane < 2 * kMoveLanes ? coherent_load(&D.moved[moved_index(0, lane & 1, lane >> 1)]) : 0;
@@ -2461,7 +2459,7 @@ __global__ __launch_bounds__(256) void unpack_rounds_kernel(DevMatrix M, DevStat
     }
     last = uniform(infeasible ? infeasible : last);
     const DevState V = block_view(M, D, R, last & 1);
-    if ((w2 >> 32) == 0 && D.global[kGlobalError] == 0) {
+    if ((w2 >> 32) == 0 && error == 0) {
         const int stride = gridDim.x * blockDim.x;
         bool crossed = false;
         for (int id = blockIdx.x * blockDim.x + threadIdx.x; id < M.n; id += stride) {
@@ -2520,16 +2518,16 @@ __device__ __forceinline__ void reset_unit(const DevState &D, const int4 q, int 
         D.wl_cnt[static_cast<size_t>(q.x) * 2 * kCountWords + lane] = 0ull;
 }
 
-__device__ __forceinline__ void clear_run_words(const DevState &D, int tid, int stride, int epoch) {
+__device__ __forceinline__ void clear_run_words(const DevState &D, int tid, int stride, int epoch, int fail) {
     if (tid == 0) D.persist[kPersistEpoch] = epoch;
     for (int k = tid; k < kStatusRows * kStatusWords; k += stride) D.status[k] = 0;
-    for (int k = tid; k < kGlobalWords; k += stride) D.global[k] = 0;
+    for (int k = tid; k < kGlobalWords; k += stride) D.global[k] = k == kGlobalError ? fail : 0;
     for (int k = tid; k < kBarrierWords; k += stride) D.barrier[k] = 0u;
 }
 
 // unit_reset_kernel and the launch tables for a single vector, all from the
 // arguments (no copy to the device): the listed unit and the vector's pointers.
-__global__ __launch_bounds__(256) void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int epoch, int *list,
+__global__ __launch_bounds__(256) void reset_one_kernel(DevState D, int4 q, int start_step, int clear_status, int epoch, int fail, int *list,
                                                         double **lbp, double **ubp, double *lbs, double *ubs) {
     if (threadIdx.x < 64) reset_unit(D, q, start_step);
     if (threadIdx.x == 0) {
@@ -2537,7 +2535,7 @@ __global__ __launch_bounds__(256) void reset_one_kernel(DevState D, int4 q, int 
         lbp[0] = lbs;
         ubp[0] = ubs;
     }
-    if (clear_status) clear_run_words(D, threadIdx.x, blockDim.x, epoch);
+    if (clear_status) clear_run_words(D, threadIdx.x, blockDim.x, epoch, fail);
 }
 
 // The state words of the listed units and the error word, to pinned host
@@ -2553,14 +2551,15 @@ __global__ __launch_bounds__(256) void report_kernel(DevState D, int n_list, con
 // Resets the state words of the listed units, params[k] = {unit, mark
 // limit, all rows in round 1, round cap}: round 1 in `start_step`, every row
 // processed in that step unless marks come from changed-column hints.  With
-// `clear_status`, also clears the step-status ring, the global words and the
-// barrier and starts the marks' epoch.
+// `clear_status`, also clears the step-status ring, the global words (`fail`:
+// the error word is set from the start) and the barrier and starts the marks'
+// epoch.
 __global__ void unit_reset_kernel(DevState D, int n_list, const int4 *params, int start_step, int clear_status,
-                                  int epoch) {
+                                  int epoch, int fail) {
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     for (int k = tid >> 6; k < n_list; k += stride >> 6) reset_unit(D, params[k], start_step);
-    if (clear_status) clear_run_words(D, tid, stride, epoch);
+    if (clear_status) clear_run_words(D, tid, stride, epoch, fail);
 }
 
 // The passes over all columns of many vectors (load, unpack).  Workgroup j of
