@@ -48,7 +48,7 @@ __global__ void mega_kernel(DevMatrix M, DevState D, int first_step, int max_ste
 __global__ void plan_rounds_kernel(DevMatrix M, RoundBins B, int4 *items);
 __global__ void reset_rounds_kernel(DevState D, RoundPlan R, int fail);
 template <bool kUnits>
-__global__ void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin);
+__global__ void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin, int first);
 template <bool kTest>
 __global__ void batch_rounds_kernel(DevMatrix M, DevState D, RoundPlan R);
 __global__ void batch_plan_kernel(DevMatrix M, DevState D, RoundPlan R, int step);
@@ -555,6 +555,7 @@ struct Problem {
     DevMatrix Mr{};                   // the matrix with the rounds' record layout
     RoundPlan R{};
     bool rounds_state = false;        // R's arrays are in the current run state
+    bool rounds_loaded = false;       // they have been loaded once in the own run state
     int rounds_grid = 0, rounds_threads = 0;  // persistent launch
     HostSlot *host = nullptr;
     HostBlock h_tables;               // pinned: launch tables of several units, then their outcomes
@@ -743,6 +744,7 @@ void alloc_units(Problem *P, int cap) {
     // what the loads leave alone: row marks, exact integer accumulators
     clear_marks(P);
     check(hipMemsetAsync(P->D.persist, 0, sizeof(int) * kPersistWords, P->stream), "memset");
+    P->rounds_loaded = false;
     const long long n_ax = static_cast<long long>(k) * M.n_int;
     if (n_ax > 0)
         hipLaunchKernelGGL(clean_ax_kernel, dim3(static_cast<int>(std::min<long long>(2048, (n_ax + 255) / 256))),
@@ -1837,6 +1839,14 @@ void issue_rounds(Problem *P, int sync_type, int max_rounds) {
     check(hipEventRecord(P->ev1, s), "event");
 }
 
+// Whether a load of the rounds is the first one into its run state.
+bool first_load(Problem *P) {
+    if (P->borrowed) return true;
+    const bool first = !P->rounds_loaded;
+    P->rounds_loaded = true;
+    return first;
+}
+
 // A complete run of one bound vector, each round one launch (two with split
 // rows) that stops itself on the device once the run is over, or all rounds
 // one persistent launch.
@@ -1852,7 +1862,8 @@ RunResult run_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, in
     __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
     hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R, P->fail_waits ? 1 : 0);
-    hipLaunchKernelGGL(load_rounds_kernel<false>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
+    hipLaunchKernelGGL(load_rounds_kernel<false>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin,
+                       first_load(P) ? 1 : 0);
     check(hipGetLastError(), "load launch");
     issue_rounds(P, sync_type, max_rounds);
     hipLaunchKernelGGL(unpack_rounds_kernel, dim3(std::min(gx, 256)), dim3(256), 0, s, M, P->D, R);
@@ -1901,7 +1912,8 @@ void run_batch_rounds(Problem *P, double *d_lbs, double *d_ubs, int sync_type, i
     R.host_state = st;
     const int gx = std::max(1, std::min(1024, (M.n + 255) / 256));
     hipLaunchKernelGGL(reset_rounds_kernel, dim3(1), dim3(256), 0, s, P->D, R, P->fail_waits ? 1 : 0);
-    hipLaunchKernelGGL(load_rounds_kernel<true>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin);
+    hipLaunchKernelGGL(load_rounds_kernel<true>, dim3(gx), dim3(256), 0, s, M, P->D, R, P->M.n16, P->M.n_bin,
+                       first_load(P) ? 1 : 0);
     check(hipGetLastError(), "load launch");
     __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
     issue_rounds(P, sync_type, max_rounds);
