@@ -458,6 +458,17 @@ void validate(const InstanceView &v) {
         if (v.row_ptr[i + 1] < v.row_ptr[i]) throw std::runtime_error("row_ptrs not monotone");
 }
 
+// Accepted candidates of a step from which the next one processes all rows.
+// Marking pays while the rows it marks stay below an eighth of the rows (1M
+// rows: 2.80 ms with a quarter, 2.75 with an eighth, 2.78 with a sixteenth;
+// batches and node vectors the same with all three).  A candidate marks the
+// rows of its column: the mean length nnz / n, and at least the row it came
+// from.  (Without that row: 2.2M entries over 16M columns 1.83 ms, with it 0.95;
+// 5.5M over 5M 1.64 and 1.40.)
+long long default_mark_limit(const InstanceView &v) {
+    return static_cast<long long>(v.m) * v.n / (8LL * (static_cast<long long>(v.nnz) + v.n));
+}
+
 // Outcome of one unit from its state words (the reference's round-count
 // convention: the final no-change round counts).
 RunResult outcome(const UnitState &s) {
@@ -1221,14 +1232,8 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
             P->inst_ncols.push_back(inst[i].n);
         }
         if (nnz_total > 0x7fffff00LL || col_off[NI] > kIdMask) throw std::runtime_error("problem too large");
-        // row marking pays while the rows it marks (about accepted candidates
-        // x mean column length) stay below an eighth of the rows (1M rows: 2.80
-        // ms with a quarter, 2.75 with an eighth, 2.78 with a sixteenth; batches
-        // and node vectors the same with all three)
         for (int i = 0; i < NI; i++) {
-            const long long lim = T.mark_limit > 0 ? T.mark_limit
-                                                    : static_cast<long long>(inst[i].m) * inst[i].n /
-                                                          (8LL * std::max(1, inst[i].nnz));
+            const long long lim = T.mark_limit > 0 ? T.mark_limit : default_mark_limit(inst[i]);
             P->mark_limit.push_back(static_cast<int>(std::max(64LL, std::min(lim, 1LL << 30))));
         }
         if (replicas) P->mark_limit.resize(1);
@@ -2501,7 +2506,7 @@ Tuning autotune(const std::vector<InstanceView> &instances, const double *lbs, c
             // the full-sweep threshold: the default and larger ones (marks
             // pushed in more rounds)
             const auto &v = instances[0];
-            const long long def = std::max(64LL, static_cast<long long>(v.m) * v.n / (8LL * std::max(1, v.nnz)));
+            const long long def = std::max(64LL, default_mark_limit(v));
             for (long long f : {4LL, 16LL}) {
                 Tuning t = best;
                 t.mark_limit = static_cast<int>(std::min(def * f, 1LL << 30));
