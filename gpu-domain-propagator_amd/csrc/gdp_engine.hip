@@ -419,7 +419,7 @@ struct HostBlock {
 // creation time goes: host ordering, allocations, copies, device layout), and
 // the bytes of a run state: the least one, with the lists of marked rows, and
 // with the arrays of the double-buffered rounds too (0: runs take the three
-// phases).
+// phases; rounds_launched 0: all but persistent ones do).
 class CreateTrace {
   public:
     CreateTrace() : on_(std::getenv("GDP_TRACE_CREATE") != nullptr), t0_(Clock::now()), last_(t0_) {}
@@ -562,11 +562,13 @@ struct Problem {
     long long graph_key = -1;
     std::mutex run_mutex;
     // double-buffered rounds (one bound vector; gdp_device.h, RoundPlan)
-    bool rounds_ok = false;           // the problem's single runs take them
+    bool rounds_ok = false;           // the problem's persistent runs take them
+    bool rounds_launch = false;       // its launched runs too
     DevMatrix Mr{};                   // the matrix with the rounds' record layout
     RoundPlan R{};
     bool rounds_state = false;        // R's arrays are in the current run state
     bool rounds_loaded = false;       // they have been loaded once in the own run state
+    int rounds_work = 0;              // waves that find work in a round
     int rounds_grid = 0, rounds_threads = 0;  // persistent launch
     HostSlot *host = nullptr;
     HostBlock h_tables;               // pinned: launch tables of several units, then their outcomes
@@ -1108,6 +1110,16 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     // 2.82); 6 of 1.7M 2.14 / 2.22 (2.71 / 2.41); 8 of 2.8M 3.60 / 3.59 (3.49 / 3.46);
     // 16 of 2.0M 7.7 / 7.9 (6.9 / 6.9).
     constexpr int kMaxBatchEntries = 16 << 20;
+    // Rounds that look for unmoved rows copy the bitmap of the columns once for
+    // every workgroup, so that they lose to the three phases in wide systems; two
+    // launched workgroups a compute unit do sooner than the persistent ones.  us a
+    // call, loop / graph / persistent, in brackets with three phases: 5.5M entries
+    // over 2.5M columns 1410 / 1440 / 1280 (1510 / 1530 / 1600); 6.3M over 3M 1230
+    // / 1270 / 1100 (1190 / 1230 / 1290); 2.2M over 4M 780 / 830 / 620 (690 / 750 /
+    // 770); 1.5M over 5M 810 / 850 / 630 (720 / 780 / 780); 3.1M over 6M 920 / 950 /
+    // 700 (620 / 640 / 640); 6.2M over 8M 1630 / 1660 / 1220 (960 / 970 / 940).
+    // Smaller systems do not look: 0.22M over 8M 380 / 390 / 390 (620 / 640 / 570).
+    constexpr int kLaunchTestWords = 5 * kMaxBitWords, kPersistentTestWords = 10 * kMaxBitWords;
     const int NI = P->n_inst;
     if (P->replicas ? NI != 1 || n_padded > kMaxRoundEntries : NI > kMaxRoundUnits || n_padded > kMaxBatchEntries)
         return;
@@ -1125,6 +1137,7 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     const int logk_want = n_padded <= (64 << 10) ? 0 : (n_padded <= (512 << 10) ? 1 : 2);
     auto bin_logk = [&](int b) { return std::max(std::min(logk_want, b), b - 6); };
     RoundPlan &R = P->R;
+    auto persistent_pays = [&] { return R.n_items < kMinTestItems || P->M.nwords <= kPersistentTestWords; };
     if (P->replicas) {
         RoundBins B;
         B.n_segs = P->M.n_seg_parts;
@@ -1145,6 +1158,7 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
         for (int q = kPlanBins - 1; q >= 0; q--)
             if (count[2 + q] == 0) B.row0[q] = B.row0[q + 1];
         R.n_items = at;
+        if (!persistent_pays()) return;
         int4 *items = dev_alloc<int4>(at, P->owned);
         R.items = items;
         hipLaunchKernelGGL(plan_rounds_kernel, dim3(std::max(1, std::min(256, (at + 255) / 256))), dim3(256), 0,
@@ -1169,6 +1183,7 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
             unit_item[i + 1] = static_cast<int>(items.size());
         }
         R.n_items = static_cast<int>(items.size());
+        if (!persistent_pays()) return;
         R.n_units = NI;
         R.slot_words = (NI + 30) / 31;
         int4 *d_items = dev_alloc<int4>(items.size(), P->owned);
@@ -1186,10 +1201,15 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     M.snap_offF = (M.n_int * 8 + 15) / 16 * 16;
     M.snap_stride = M.snap_offF + 16LL * (M.n - M.n_int) + 16;
     int per_cu = 0;
-    // at most 256 workgroups while the items allow it: the barrier grows with
+    // A wave per item, and one per 64 words of the bitmap of moved columns where
+    // there are more of those (1000 entries over 16M columns 566 -> 480 us, 336
+    // over 1M 102 -> 74; a wave per 8 words made the barriers longer than it
+    // gained: 11,000 over 1M 122 -> 147 us persistent, 122 so).
+    // At most 256 workgroups while the work allows it: the barrier grows with
     // them (1.2 us for 16, 3 us for 256, 4.3 us for 512), and a workgroup of 256
     // threads spreads few items over more compute units
-    P->rounds_threads = R.n_items <= 1024 ? 256 : (R.n_items <= 2048 ? 512 : 1024);
+    P->rounds_work = std::max(R.n_items, (M.nwords + 63) / 64);
+    P->rounds_threads = P->rounds_work <= 1024 ? 256 : (P->rounds_work <= 2048 ? 512 : 1024);
     // moved columns in LDS: up to 512K have a bit of their own
     R.bit_words = 0;
     if (R.n_items >= kMinTestItems) {
@@ -1200,8 +1220,14 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     const void *fn = rounds_fn(P);
     check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, P->rounds_threads, lds), "occupancy");
     const int waves = P->rounds_threads / 64;
-    P->rounds_grid = std::max(1, std::min({per_cu * P->cu_count, kMaxGatherBlocks, (R.n_items + waves - 1) / waves}));
+    P->rounds_grid = std::max(1, std::min({per_cu * P->cu_count, kMaxGatherBlocks, (P->rounds_work + waves - 1) / waves}));
     P->rounds_ok = true;
+    P->rounds_launch = R.n_items < kMinTestItems || M.nwords <= kLaunchTestWords;
+}
+
+// Whether a run takes the double-buffered rounds.
+bool takes_rounds(const Problem *P, int sync_type) {
+    return P->rounds_state && (sync_type == MEGAKERNEL_ID || P->rounds_launch);
 }
 
 Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tuning *tuning) {
@@ -1491,6 +1517,7 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
             trace.bytes("state_bytes", carve_state(M, replicas, NI, 1, nullptr, D, T, false));
             trace.bytes("with_lists", lists);
             trace.bytes("with_rounds", P->rounds_ok ? lists + carve_rounds(P->Mr, nullptr, plan) : 0);
+            trace.bytes("rounds_launched", P->rounds_launch ? 1 : 0);
         }
 
         P->mega_threads = T.mega_threads == 256 || T.mega_threads == 1024 ? T.mega_threads : 512;
@@ -1807,7 +1834,7 @@ void launch_round(Problem *P, int step) {
     const bool small = lds == 0;
     const int threads = small ? 256 : 512;
     const int waves = threads / 64;
-    const int grid = std::max(1, std::min((small ? 8 : 2) * P->cu_count, (P->R.n_items + waves - 1) / waves));
+    const int grid = std::max(1, std::min((small ? 8 : 2) * P->cu_count, (P->rounds_work + waves - 1) / waves));
     const int apply_grid = std::max(1, std::min(1024, grid_for(P->Mr.n_seg_parts)));
     if (!P->replicas) {
         hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(kMaxRoundUnits), 0, P->stream, P->Mr, P->D, P->R, step);
@@ -1973,7 +2000,7 @@ void run_units(Problem *P, int n_list, const int *list, double *const *lbp, doub
 RunResult run_single(Problem *P, double *d_lbs, double *d_ubs, int sync_type, int max_rounds) {
     if (sync_type < CPU_LOOP_ID || sync_type > MEGAKERNEL_ID) throw std::runtime_error("Unknown sync type");
     if (max_rounds < 1 || max_rounds > kMaxRounds) throw std::runtime_error("max_rounds out of range");
-    if (P->rounds_state) return run_rounds(P, d_lbs, d_ubs, sync_type, max_rounds);
+    if (takes_rounds(P, sync_type)) return run_rounds(P, d_lbs, d_ubs, sync_type, max_rounds);
     const int list[1] = {0};
     RunResult r;
     run_units(P, 1, list, &d_lbs, &d_ubs, nullptr, nullptr, sync_type, max_rounds, &r);
@@ -2300,7 +2327,7 @@ void batch_propagate_device(Problem *P, double *d_lbs, double *d_ubs, int sync_t
     if (P->replicas) throw std::runtime_error("not a batch of instances");
     std::lock_guard<std::mutex> lock(P->run_mutex);
     ensure_units(P);
-    if (P->rounds_state) {
+    if (takes_rounds(P, sync_type)) {
         run_batch_rounds(P, d_lbs, d_ubs, sync_type, max_rounds, out);
         return;
     }

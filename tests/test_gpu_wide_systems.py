@@ -1,5 +1,8 @@
 """Systems of many more columns than entries, against the round-synchronous
 oracle, and the rules that look at the number of columns."""
+import re
+import time
+
 import numpy as np
 import pytest
 
@@ -7,6 +10,79 @@ from gdp_amd import interface as I
 from gdp_amd.instances import small_mip
 
 pytestmark = pytest.mark.gpu
+
+SYNCS = [I.CPU_LOOP, I.GPU_LOOP, I.MEGAKERNEL]
+
+
+def _traced(make, monkeypatch, capfd):
+    """The problem, and whether its persistent and its launched runs take the
+    double-buffered rounds."""
+    monkeypatch.setenv("GDP_TRACE_CREATE", "1")
+    capfd.readouterr()
+    p = make()
+    monkeypatch.delenv("GDP_TRACE_CREATE")
+    err = capfd.readouterr().err
+    return p, tuple(int(re.search(rf" {k}=(\d+)", err).group(1)) > 0 for k in ("with_rounds", "rounds_launched"))
+
+
+# 5000 items look for unmoved rows: launches up to 2.6M columns, persistent runs
+# up to 5.2M; few items never look
+@pytest.mark.parametrize("m,n,route", [
+    (100_000, 5 << 19, (True, True)), (100_000, (5 << 19) + 33, (True, False)), (100_000, 10 << 19, (True, False)),
+    (100_000, (10 << 19) + 33, (False, False)), (30, 1_000_003, (True, True)), (50_000, 6_000_001, (True, True))])
+def test_routes_of_wide_systems(gpu, oracle, monkeypatch, capfd, m, n, route):
+    inst = small_mip(seed=3, m=m, n=n)
+    exp = oracle.jacobi(inst)
+    p, got = _traced(lambda: I.Problem(inst), monkeypatch, capfd)
+    try:
+        assert got == route
+        for sync in SYNCS + [I.MEGAKERNEL, I.CPU_LOOP]:  # the routes share a run state
+            out = p.propagate(inst.lb, inst.ub, sync)
+            np.testing.assert_array_equal(out.lbs, exp[0])
+            np.testing.assert_array_equal(out.ubs, exp[1])
+            assert (out.rounds, out.infeasible, out.capped) == exp[2:]
+    finally:
+        p.close()
+
+
+def test_routes_of_a_wide_batch(gpu, oracle, monkeypatch, capfd):
+    xs = [small_mip(seed=k, m=14_000 + k, n=700_000 + k) for k in range(8)]
+    exp = [oracle.jacobi(x) for x in xs]
+    b, got = _traced(lambda: I.Batch(xs), monkeypatch, capfd)
+    try:
+        assert got == (False, False)
+        for sync in SYNCS:
+            for out, e in zip(b.propagate(sync_type=sync), exp):
+                np.testing.assert_array_equal(out.lbs, e[0])
+                np.testing.assert_array_equal(out.ubs, e[1])
+                assert (out.rounds, out.infeasible, out.capped) == e[2:]
+    finally:
+        b.close()
+
+
+def test_wide_systems_are_not_slower_than_the_three_phases(gpu):
+    """3.1M entries over 12M columns: rounds that copy the bitmap of the columns
+    for every workgroup took 1.6 to 2.5 times as long."""
+    inst = small_mip(seed=1, m=100_000, n=12_000_000, len_hi=60)
+    took = {}
+    for tuning in (None, {"item_nnz": 1024}):
+        p = I.Problem(inst, tuning)
+        lb, ub = I.DeviceArray(inst.lb), I.DeviceArray(inst.ub)
+        for sync in SYNCS:
+            times = []
+            for _ in range(7):
+                lb.upload(inst.lb)
+                ub.upload(inst.ub)
+                t = time.perf_counter()
+                p.propagate_device(lb.ptr, ub.ptr, sync)
+                times.append(time.perf_counter() - t)
+            took[tuning is None, sync] = sorted(times)[2]
+        p.close()
+        lb.free()
+        ub.free()
+    print(took, flush=True)
+    for sync in SYNCS:
+        assert took[True, sync] < 1.4 * took[False, sync], took
 
 
 def test_a_candidate_marks_at_least_its_row(gpu, oracle):
