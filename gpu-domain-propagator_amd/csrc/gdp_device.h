@@ -216,7 +216,8 @@ struct DevMatrix {
     unsigned long long class_logg, class_logk;  // lanes per row and entries per lane (log2), 4 bits a class
     const int *perm;       // internal id -> caller's column (-1: padding id)
     const int *word_unit;  // blocks mode: unit of each bitmap word
-    int snap_off32;        // byte offset of S32 in a unit's snapshot block
+    int snap_off32;        // byte offset of S32 in a unit's snapshot block (these three: bits of a
+                           // 32-bit unsigned number, below 2^31 in the rounds)
     int snap_offB;         // byte offset of SB
     int snap_offF;         // byte offset of SF
     long long snap_stride; // bytes between the snapshot blocks of two units

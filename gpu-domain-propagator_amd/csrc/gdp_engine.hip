@@ -624,13 +624,13 @@ size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char 
     const size_t nf = static_cast<size_t>(M.n - M.n_int);
     char *snap = take(k * static_cast<size_t>(M.snap_stride));
     D.S16 = reinterpret_cast<unsigned *>(snap);
-    D.S32 = reinterpret_cast<int2 *>(snap ? snap + M.snap_off32 : nullptr);
-    D.SF = reinterpret_cast<double2 *>(snap ? snap + M.snap_offF : nullptr);
+    D.S32 = reinterpret_cast<int2 *>(snap ? snap + static_cast<unsigned>(M.snap_off32) : nullptr);
+    D.SF = reinterpret_cast<double2 *>(snap ? snap + static_cast<unsigned>(M.snap_offF) : nullptr);
     D.AI = reinterpret_cast<int2 *>(take(k * M.n_int * sizeof(int2)));
     D.AX = reinterpret_cast<double2 *>(take(k * M.n_int * sizeof(double2)));
     D.AF = reinterpret_cast<double2 *>(take(k * nf * sizeof(double2)));
     D.bm = reinterpret_cast<unsigned *>(take(k * M.nwords * sizeof(unsigned)));
-    D.SB = reinterpret_cast<unsigned *>(snap ? snap + M.snap_offB : nullptr);
+    D.SB = reinterpret_cast<unsigned *>(snap ? snap + static_cast<unsigned>(M.snap_offB) : nullptr);
     D.n_codes = replicas ? M.n_bin : 0;
     D.marks = reinterpret_cast<int *>(take(k * M.m * sizeof(int)));
     D.seg_parts = reinterpret_cast<SegPart *>(take(k * M.n_seg_parts * sizeof(SegPart)));
@@ -1119,10 +1119,13 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     // 770); 1.5M over 5M 810 / 850 / 630 (720 / 780 / 780); 3.1M over 6M 920 / 950 /
     // 700 (620 / 640 / 640); 6.2M over 8M 1630 / 1660 / 1220 (960 / 970 / 940).
     // Smaller systems do not look: 0.22M over 8M 380 / 390 / 390 (620 / 640 / 570).
+    // Their records (int32 pairs at least) are addressed with 32 bits.
+    constexpr int kMaxRoundWords = 1 << 21;
     constexpr int kLaunchTestWords = 5 * kMaxBitWords, kPersistentTestWords = 10 * kMaxBitWords;
     const int NI = P->n_inst;
     if (P->replicas ? NI != 1 || n_padded > kMaxRoundEntries : NI > kMaxRoundUnits || n_padded > kMaxBatchEntries)
         return;
+    if (P->M.nwords > kMaxRoundWords) return;
     // (row_marking and mark_limit say how the three phases choose their rows)
     if (T.item_nnz != def.item_nnz || T.mega_blocks_per_cu != def.mega_blocks_per_cu ||
         T.mega_threads != def.mega_threads || T.max_split_segs != def.max_split_segs ||
@@ -1490,10 +1493,15 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         // 16-byte boundary
         M.n_bin = C.n_bin;
         M.sb_words = (C.n_bin + 63) / 64 * 4;
-        M.snap_off32 = (M.n16 * 4 + 15) / 16 * 16;
-        M.snap_offB = M.snap_off32 + ((M.n_int - M.n16) * 8 + 15) / 16 * 16;
-        M.snap_offF = M.snap_offB + 4 * M.sb_words;
-        M.snap_stride = M.snap_offF + 16LL * (M.n - M.n_int) + 16;
+        const long long off32 = (4LL * M.n16 + 15) / 16 * 16;
+        const long long offB = off32 + (8LL * (M.n_int - M.n16) + 15) / 16 * 16;
+        const long long offF = offB + 4LL * M.sb_words;
+        M.snap_stride = offF + 16LL * (M.n - M.n_int) + 16;
+        // (records are addressed with 32 bits)
+        if (M.snap_stride > 0xffffffffLL) throw std::runtime_error("too many columns");
+        M.snap_off32 = static_cast<int>(static_cast<unsigned>(off32));
+        M.snap_offB = static_cast<int>(static_cast<unsigned>(offB));
+        M.snap_offF = static_cast<int>(static_cast<unsigned>(offF));
         check(hipStreamSynchronize(s), "upload");
         {
             // device bytes of one more bound vector's state (the run state
@@ -1585,8 +1593,8 @@ void set_reference(Problem *P, double *const *lbp, double *const *ubp, int n_vec
     P->ref_ub = P->ref_lb + n;
     DevState V{};
     V.S16 = reinterpret_cast<unsigned *>(P->ref_block);
-    V.S32 = reinterpret_cast<int2 *>(P->ref_block + M.snap_off32);
-    V.SF = reinterpret_cast<double2 *>(P->ref_block + M.snap_offF);
+    V.S32 = reinterpret_cast<int2 *>(P->ref_block + static_cast<unsigned>(M.snap_off32));
+    V.SF = reinterpret_cast<double2 *>(P->ref_block + static_cast<unsigned>(M.snap_offF));
     ReferenceVectors R{};
     R.n = std::min(3, n_vectors);
     for (int k = 0; k < R.n; k++) {

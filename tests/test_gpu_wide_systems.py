@@ -45,6 +45,30 @@ def test_routes_of_wide_systems(gpu, oracle, monkeypatch, capfd, m, n, route):
         p.close()
 
 
+# beyond 2^26 columns a round's records would need offsets of more than 31 bits
+@pytest.mark.parametrize("n,rounds", [(1 << 26, True), ((1 << 26) + 1, False)])
+def test_columns_of_the_rounds(gpu, oracle, monkeypatch, capfd, n, rounds):
+    small = small_mip(seed=2, m=40, n=60)
+    at = np.sort(np.random.default_rng(1).choice(n, 60, replace=False))
+    lb, ub, vt = np.zeros(n), np.ones(n), np.zeros(n, np.int32)
+    lb[at], ub[at], vt[at] = small.lb, small.ub, small.vartype
+    inst = small.__class__(**{**small.__dict__, "n": n, "col": at[small.col].astype(np.int32), "lb": lb, "ub": ub,
+                              "vartype": vt})
+    exp = oracle.jacobi(small)
+    p, got = _traced(lambda: I.Problem(inst), monkeypatch, capfd)
+    try:
+        assert got == (rounds, rounds)
+        for sync in SYNCS:
+            out = p.propagate(lb, ub, sync)
+            np.testing.assert_array_equal(out.lbs[at], exp[0])
+            np.testing.assert_array_equal(out.ubs[at], exp[1])
+            assert (out.rounds, out.infeasible, out.capped) == exp[2:]
+            out.lbs[at], out.ubs[at] = 0.0, 1.0
+            assert not out.lbs.any() and (out.ubs == 1.0).all()
+    finally:
+        p.close()
+
+
 def test_routes_of_a_wide_batch(gpu, oracle, monkeypatch, capfd):
     xs = [small_mip(seed=k, m=14_000 + k, n=700_000 + k) for k in range(8)]
     exp = [oracle.jacobi(x) for x in xs]
