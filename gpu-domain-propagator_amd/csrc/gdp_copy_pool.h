@@ -14,6 +14,17 @@
 
 namespace gdp {
 
+// Copies of this size and more from or to pageable host memory are bulk copies.
+constexpr size_t kBulkMin = 1u << 20;
+
+// The staging's lock for a copy of `bytes`: a bulk copy waits for it, a smaller
+// one (bound vectors) does without the staging when another problem's copy has
+// it (the lock returned then owns nothing).
+inline std::unique_lock<std::mutex> staging_lock(std::mutex &use, size_t bytes) {
+    if (bytes >= kBulkMin) return std::unique_lock<std::mutex>(use);
+    return std::unique_lock<std::mutex>(use, std::try_to_lock);
+}
+
 class CopyPool {
   public:
     static constexpr size_t kBlock = 256u << 10;  // blocks dealt out in turn

@@ -122,8 +122,10 @@ T *dev_alloc(size_t count, std::vector<void *> &owned) {
 // would stage them through its own pinned buffers, copying on one thread.
 // Here several threads copy each chunk into one of two pinned staging
 // buffers while the DMA engine drains the other.  One copy at a time uses
-// them, and without them the copy is left to the runtime.  Returns when
-// every copy out of them has completed.
+// them, and without them the copy is left to the runtime.  Bound vectors below
+// 1 MiB use them too while they are free (node calls of 60,000 columns 1.3 ->
+// 0.75 ms), but never wait for them.  Returns when every copy out of them has
+// completed.
 //
 // Lifetime: the first bulk copy creates the buffers and the copy threads.
 // Copies below 64 MiB take buffers of 8 MiB, which stay with the threads for
@@ -132,7 +134,6 @@ T *dev_alloc(size_t count, std::vector<void *> &owned) {
 // go back when the last problem is destroyed.
 constexpr size_t kStageSmall = 8u << 20;
 constexpr size_t kStageLarge = 32u << 20;
-constexpr size_t kBulkMin = 1u << 20;
 // Bound vectors (both) of up to this size cross through a pinned block of the
 // problem's own instead of the shared staging.
 constexpr size_t kSmallBounds = 256u << 10;
@@ -207,8 +208,8 @@ Staging &staging() {
 
 void upload_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
     Staging &st = staging();
-    std::lock_guard<std::mutex> lock(st.use);
-    if (!st.ready(bytes)) {  // no pinned memory to spare: the runtime's own staged copy
+    const std::unique_lock<std::mutex> lock = staging_lock(st.use, bytes);
+    if (!lock.owns_lock() || !st.ready(bytes)) {  // in use, or no pinned memory to spare: the runtime's own staged copy
         check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s), "H2D");
         return;
     }
@@ -245,8 +246,8 @@ void upload_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
 // Synchronous.
 void download_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
     Staging &st = staging();
-    std::lock_guard<std::mutex> lock(st.use);
-    if (!st.ready(bytes)) {
+    const std::unique_lock<std::mutex> lock = staging_lock(st.use, bytes);
+    if (!lock.owns_lock() || !st.ready(bytes)) {
         check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s), "D2H");
         check(hipStreamSynchronize(s), "D2H");
         return;
