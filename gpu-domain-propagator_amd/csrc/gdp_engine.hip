@@ -36,6 +36,7 @@
 #include "gdp_devmem.h"
 #include "gdp_engine.h"
 #include "gdp_host.h"
+#include "gdp_host_blocks.h"
 #include "gdp_order.h"
 
 namespace gdp {
@@ -353,67 +354,17 @@ HostSlots &host_slots() {
     return *h;
 }
 
-// Pinned host blocks for launch tables, outcomes and small bound vectors, by
-// powers of two from 4 KiB.  Freed blocks of up to 1 MiB are kept for the next
-// request, 16 MiB in all; the others go back to the runtime.
-class HostBlocks {
-  public:
-    void *take(size_t bytes, size_t *size) {
-        *size = 4096;
-        while (*size < bytes) *size *= 2;
-        {
-            std::lock_guard<std::mutex> lk(mu_);
-            auto it = free_.find(*size);
-            if (it != free_.end() && !it->second.empty()) {
-                void *p = it->second.back();
-                it->second.pop_back();
-                kept_ -= *size;
-                return p;
-            }
-        }
-        void *p = nullptr;
-        check(hipHostMalloc(&p, *size, hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
-        return p;
-    }
-    void give(void *p, size_t size) {
-        if (!p) return;
-        {
-            std::lock_guard<std::mutex> lk(mu_);
-            if (size <= (1u << 20) && kept_ + size <= (16u << 20)) {
-                free_[size].push_back(p);
-                kept_ += size;
-                return;
-            }
-        }
-        (void)hipHostFree(p);
-    }
-
-  private:
-    std::mutex mu_;
-    std::unordered_map<size_t, std::vector<void *>> free_;
-    size_t kept_ = 0;
-};
+void *pinned_alloc(size_t bytes) {
+    void *p = nullptr;
+    check(hipHostMalloc(&p, bytes, hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
+    return p;
+}
+void pinned_free(void *p) { (void)hipHostFree(p); }
 
 HostBlocks &host_blocks() {
-    static HostBlocks *h = new HostBlocks();  // outlives every problem
+    static HostBlocks *h = new HostBlocks(pinned_alloc, pinned_free);  // outlives every problem
     return *h;
 }
-
-// A pinned block of at least the bytes last asked for.
-struct HostBlock {
-    char *p = nullptr;
-    size_t size = 0;
-    char *get(size_t bytes) {
-        if (bytes > size) {
-            host_blocks().give(p, size);
-            p = nullptr;
-            size = 0;
-            p = static_cast<char *>(host_blocks().take(bytes, &size));
-        }
-        return p;
-    }
-    ~HostBlock() { host_blocks().give(p, size); }
-};
 
 // Phase times of a problem's creation, printed to stderr when the
 // environment variable GDP_TRACE_CREATE is set (a diagnostic of where the
@@ -572,8 +523,8 @@ struct Problem {
     int rounds_work = 0;              // waves that find work in a round
     int rounds_grid = 0, rounds_threads = 0;  // persistent launch
     HostSlot *host = nullptr;
-    HostBlock h_tables;               // pinned: launch tables of several units, then their outcomes
-    HostBlock h_bounds;               // pinned: small bound vectors on their way
+    HostBlock h_tables{host_blocks()};  // pinned: launch tables of several units, then their outcomes
+    HostBlock h_bounds{host_blocks()};  // pinned: small bound vectors on their way
     int servers = 0;                  // servers attached (they own the unit slots)
     bool fail_waits = false;          // GDP_FAIL_WAITS
     bool graphs_enabled = true;       // GPU_LOOP may capture graphs of the current run state
@@ -2644,7 +2595,7 @@ struct Server {
     // the changes packed into pinned memory: columns and bounds, each vector's
     // count and start
     int *h_off = nullptr;
-    HostBlock h_states;                  // pinned: the states of a step's slots
+    HostBlock h_states{host_blocks()};   // pinned: the states of a step's slots
     double *h_cl = nullptr, *h_cu = nullptr;
     int diff_slots = 0;
     std::vector<double *> slot_lb, slot_ub;

@@ -1,5 +1,6 @@
 """What the process shares of pinned host memory, on the CPU: the lock of the
-staging of bulk copies (csrc/gdp_copy_pool.h)."""
+staging of bulk copies (csrc/gdp_copy_pool.h) and the pool of blocks
+(csrc/gdp_host_blocks.h)."""
 import os
 import subprocess
 
@@ -8,7 +9,7 @@ import pytest
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.mark.parametrize("driver", ["staging_lock_driver"])
+@pytest.mark.parametrize("driver", ["staging_lock_driver", "host_blocks_driver"])
 def test_native(tmp_path, driver):
     exe = tmp_path / driver
     subprocess.run(["g++", "-O2", "-std=c++17", "-pthread", "-Wall", "-I",
