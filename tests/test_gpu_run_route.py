@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from gdp_amd import interface as I
-from gdp_amd.instances import small_mip
+from gdp_amd.instances import INF, Instance, small_mip
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +42,48 @@ def test_options_reach_the_phases_they_describe(gpu, oracle, monkeypatch, capfd,
             np.testing.assert_array_equal(out.ubs, exp[1])
         finally:
             p.close()
+
+
+ARRAY_BYTES = 64 << 20  # of the allocation-free call
+
+
+def _blocks(rows, n):
+    """`rows` rows over disjoint columns, 80% of them integer, the others continuous."""
+    per = n // rows
+    rng = np.random.default_rng(4)
+    val = rng.integers(1, 9, n).astype(float)
+    return Instance(rows, n, np.arange(n, dtype=np.int32), (np.arange(rows + 1) * per).astype(np.int32), val,
+                    np.full(rows, -INF), rng.integers(5, 500, rows).astype(float), np.zeros(n), np.full(n, 60.0),
+                    np.where(rng.random(n) < 0.8, 1, 3).astype(np.int32))
+
+
+# what the array holds: everything; the lists of marked rows, but not the rounds'
+# arrays; not even the lists (every step then processes all rows)
+@pytest.mark.parametrize("make,lists,rounds", [
+    (lambda: _blocks(2000, 800_000), True, True), (lambda: _blocks(2000, 1_000_000), True, False),
+    (lambda: small_mip(seed=6, m=2_000_000, n=1_800_000, len_lo=2, len_hi=2), False, False)],
+    ids=["rounds", "lists", "neither"])
+def test_what_the_allocation_free_array_holds(gpu, oracle, monkeypatch, capfd, make, lists, rounds):
+    inst = make()
+    exp = oracle.jacobi(inst)
+    p, got = _bytes(lambda: I.Problem(inst), monkeypatch, capfd)
+    try:
+        print(got, flush=True)
+        assert got[0] == p.stats().run_state_bytes <= ARRAY_BYTES
+        assert got[2] > 0 and (got[1] <= ARRAY_BYTES, got[2] <= ARRAY_BYTES) == (lists, rounds), got
+        for sync in (I.CPU_LOOP, I.GPU_LOOP, I.MEGAKERNEL):
+            dl, du = I.DeviceArray(inst.lb), I.DeviceArray(inst.ub)
+            for _ in range(2):  # from the bounds, then from their fixpoint
+                info = p.propagate_device_no_alloc(dl.ptr, du.ptr, sync)
+                np.testing.assert_array_equal(dl.numpy(), exp[0])
+                np.testing.assert_array_equal(du.numpy(), exp[1])
+            assert info.rounds == 1
+            dl.upload(inst.lb)
+            du.upload(inst.ub)
+            info = p.propagate_device_no_alloc(dl.ptr, du.ptr, sync)
+            assert (info.rounds, bool(info.infeasible), bool(info.capped)) == exp[2:]
+            dl.free()
+            du.free()
+        assert p.stats().n_units == 0
+    finally:
+        p.close()
