@@ -561,8 +561,8 @@ namespace {
 // counters), the problem-wide status ring, global words and barrier, and
 // the launch tables the host fills (listed units, reset parameters,
 // bound-vector pointers, hint starts).  With base null only the size is
-// computed.  Without `lists` (the allocation-free entry point, where they do
-// not fit) every step processes all rows.  Returns the bytes needed.
+// computed; without `lists`, which take no more than the marks do, the size that
+// run_state_bytes reports.  Returns the bytes needed.
 size_t carve_state(const DevMatrix &M, bool replicas, int n_inst, int cap, char *base, DevState &D,
                    UnitTables &T, bool lists) {
     size_t off = 0;
@@ -634,10 +634,9 @@ size_t carve_rounds(const DevMatrix &Mr, char *base, RoundPlan &R) {
 
 // Points the problem's run state at `base` (cap units, see carve_state);
 // with `rounds`, the arrays of the double-buffered rounds follow.
-void bind_state(Problem *P, char *base, int cap, bool rounds, bool lists = true) {
+void bind_state(Problem *P, char *base, int cap, bool rounds) {
     UnitTables T;
-    const size_t off = carve_state(P->M, P->replicas, P->n_inst, cap, base, P->D, T, lists);
-    P->M.mark_rows = lists && P->tuning.row_marking ? 1 : 0;
+    const size_t off = carve_state(P->M, P->replicas, P->n_inst, cap, base, P->D, T, true);
     if (rounds) carve_rounds(P->Mr, base + off, P->R);
     P->rounds_state = rounds;
     P->d_list = T.list;
@@ -2302,11 +2301,16 @@ void batch_propagate_device(Problem *P, double *d_lbs, double *d_ubs, int sync_t
 
 // The run state of the allocation-free entry point lives in this fixed array
 // of device memory, which every device the library runs on holds until the
-// process ends.  In host code `scratch` names a host-side stand-in, not the
+// process ends: kScratchBytes for what run_state_bytes counts, and as much again
+// for the lists of marked rows, which never take more than the marks do, and for
+// the rounds' arrays where they fit.  (With 64 MiB for everything, systems whose
+// lists did not fit processed all rows in every step: 11M nonzeros 4.3 ms, 2.3 so.)
+// In host code `scratch` names a host-side stand-in, not the
 // device array: its device address comes from hipGetSymbolAddress (once per
 // device, with that device current), and only that address is handed to
 // kernels.
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+constexpr size_t kScratchArray = 2 * kScratchBytes;
+static __device__ __align__(256) unsigned char scratch[kScratchArray];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -2337,14 +2341,13 @@ class BorrowedState {
         : P_(P), D_(P->D), list_(P->d_list), params_(P->d_params), lbp_(P->d_lbp), ubp_(P->d_ubp),
           hint_ptr_(P->d_hint_ptr), capacity_(P->capacity), n_units_(P->n_units), graphs_(P->graphs_enabled),
           R_(P->R), rounds_state_(P->rounds_state) {
-        // the lists of marked rows and the double-buffered rounds where their
-        // arrays fit too
+        // the double-buffered rounds where their arrays fit too
         DevState D{};
         UnitTables T;
         RoundPlan R;
         const size_t need = carve_state(P->M, P->replicas, P->n_inst, 1, nullptr, D, T, true);
-        bind_state(P, base, 1, P->rounds_ok && need + carve_rounds(P->Mr, nullptr, R) <= kScratchBytes,
-                   need <= kScratchBytes);
+        if (need > kScratchArray) throw std::runtime_error("run state beyond the allocation-free array");
+        bind_state(P, base, 1, P->rounds_ok && need + carve_rounds(P->Mr, nullptr, R) <= kScratchArray);
         P->graphs_enabled = false;
         P->borrowed = true;
     }
@@ -2359,7 +2362,6 @@ class BorrowedState {
         P_->capacity = capacity_;
         P_->n_units = n_units_;
         P_->graphs_enabled = graphs_;
-        P_->M.mark_rows = P_->tuning.row_marking ? 1 : 0;
         P_->R = R_;
         P_->rounds_state = rounds_state_;
     }

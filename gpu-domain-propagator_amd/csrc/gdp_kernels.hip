@@ -2518,7 +2518,7 @@ __device__ __forceinline__ void reset_unit(const DevState &D, const int4 q, int 
     }
     static_assert(kMoveSlots * kMoveLanes == 64 && 2 * kCountWords <= 64, "a lane per counter");
     D.moved[moved_index(q.x, lane / kMoveLanes, lane % kMoveLanes)] = 0;
-    if (D.wl_cnt != nullptr && lane < 2 * kCountWords)
+    if (lane < 2 * kCountWords)
         D.wl_cnt[static_cast<size_t>(q.x) * 2 * kCountWords + lane] = 0ull;
 }
 

@@ -60,10 +60,10 @@ typedef struct {
     long long unit_state_bytes; /* device bytes of one bound vector's state */
     int mega_threads;           /* persistent kernel: workgroup size */
     int mega_grid;              /* persistent kernel: workgroups */
-    long long run_state_bytes;  /* device bytes of the run state of one propagation:
-                                   allocated by the problem on its first propagation,
-                                   taken from the fixed device array by
-                                   gdpPropagateDeviceNoAlloc */
+    long long run_state_bytes;  /* device bytes of the least run state of one propagation,
+                                   which gdpPropagateDeviceNoAlloc limits; the state that the
+                                   problem allocates on its first propagation holds lists of
+                                   work and the arrays of its rounds besides */
     int n_binary;               /* integer columns whose envelope lies in [0, 1]
                                    (single problems; 0 for batches) */
     int n_lds_binary;           /* of them, the columns whose bounds a persistent
@@ -117,11 +117,12 @@ GDP_RETCODE gdpPropagateDevice(gdp_problem p, double *d_lbs, double *d_ubs, cons
  * the reference.  For callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The run
  * state (unit state, split-row partials, status words, counters, launch
- * tables; gdp_problem_stats.run_state_bytes) lives in one fixed array of
- * GDP_NOALLOC_SCRATCH_BYTES (64 MiB) of device memory that the library holds
- * on every device it runs on until the process ends, instead of the
- * problem's own state, which is never allocated for a problem run only this
- * way.  Problems whose run state exceeds the array return GDP_ERROR.  The
+ * tables; gdp_problem_stats.run_state_bytes, at most
+ * GDP_NOALLOC_SCRATCH_BYTES: 64 MiB) lives in one fixed array of device memory
+ * (128 MiB: as much again holds lists of work and the arrays of faster rounds)
+ * that the library holds on every device it runs on until the process ends,
+ * instead of the problem's own state, which is never allocated for a problem run only this
+ * way.  Problems whose run state exceeds the limit return GDP_ERROR.  The
  * problem's device must be the current device.  The array is shared by all
  * problems on a device and keeps the last call's contents; every call resets
  * what it reads.  Calls on one device are serialised by the library (calls

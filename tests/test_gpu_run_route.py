@@ -2,6 +2,7 @@
 creation (with_rounds: bytes of the run state with the arrays of the
 double-buffered rounds, 0 where runs take the three phases)."""
 import re
+import time
 
 import numpy as np
 import pytest
@@ -44,7 +45,7 @@ def test_options_reach_the_phases_they_describe(gpu, oracle, monkeypatch, capfd,
             p.close()
 
 
-ARRAY_BYTES = 64 << 20  # of the allocation-free call
+STATE_BYTES, ARRAY_BYTES = 64 << 20, 128 << 20  # of the allocation-free call
 
 
 def _blocks(rows, n):
@@ -57,20 +58,20 @@ def _blocks(rows, n):
                     np.where(rng.random(n) < 0.8, 1, 3).astype(np.int32))
 
 
-# what the array holds: everything; the lists of marked rows, but not the rounds'
-# arrays; not even the lists (every step then processes all rows)
-@pytest.mark.parametrize("make,lists,rounds", [
-    (lambda: _blocks(2000, 800_000), True, True), (lambda: _blocks(2000, 1_000_000), True, False),
-    (lambda: small_mip(seed=6, m=2_000_000, n=1_800_000, len_lo=2, len_hi=2), False, False)],
-    ids=["rounds", "lists", "neither"])
-def test_what_the_allocation_free_array_holds(gpu, oracle, monkeypatch, capfd, make, lists, rounds):
+# what the array holds beside the run state: lists of marked rows and the rounds'
+# arrays, or only the lists (always: the marks leave room for them)
+@pytest.mark.parametrize("make,rounds", [
+    (lambda: _blocks(2000, 1_000_000), True), (lambda: _blocks(2000, 1_900_000), False),
+    (lambda: small_mip(seed=6, m=2_000_000, n=1_800_000, len_lo=2, len_hi=2), False)],
+    ids=["rounds", "lists", "many rows"])
+def test_what_the_allocation_free_array_holds(gpu, oracle, monkeypatch, capfd, make, rounds):
     inst = make()
     exp = oracle.jacobi(inst)
     p, got = _bytes(lambda: I.Problem(inst), monkeypatch, capfd)
     try:
         print(got, flush=True)
-        assert got[0] == p.stats().run_state_bytes <= ARRAY_BYTES
-        assert got[2] > 0 and (got[1] <= ARRAY_BYTES, got[2] <= ARRAY_BYTES) == (lists, rounds), got
+        assert got[0] == p.stats().run_state_bytes <= STATE_BYTES
+        assert got[1] <= ARRAY_BYTES and got[2] > 0 and (got[2] <= ARRAY_BYTES) == rounds, got
         for sync in (I.CPU_LOOP, I.GPU_LOOP, I.MEGAKERNEL):
             dl, du = I.DeviceArray(inst.lb), I.DeviceArray(inst.ub)
             for _ in range(2):  # from the bounds, then from their fixpoint
@@ -87,3 +88,29 @@ def test_what_the_allocation_free_array_holds(gpu, oracle, monkeypatch, capfd, m
         assert p.stats().n_units == 0
     finally:
         p.close()
+
+
+def test_many_rows_keep_their_marks_without_allocation(gpu):
+    """11M nonzeros, a state of 64.4 MB and lists beyond 64 MiB: without the lists,
+    every step processed all rows and took 1.8 times as long."""
+    inst = small_mip(seed=1, m=1_000_000, n=2_000_000)
+    p = I.Problem(inst)
+    dl, du = I.DeviceArray(inst.lb), I.DeviceArray(inst.ub)
+    took = []
+    try:
+        assert p.stats().run_state_bytes <= STATE_BYTES
+        for fn in (p.propagate_device, p.propagate_device_no_alloc):
+            times = []
+            for _ in range(7):
+                dl.upload(inst.lb)
+                du.upload(inst.ub)
+                t = time.perf_counter()
+                fn(dl.ptr, du.ptr, I.CPU_LOOP)
+                times.append(time.perf_counter() - t)
+            took.append(sorted(times)[2] * 1e3)
+        print(f"own state {took[0]:.2f} ms, array {took[1]:.2f} ms", flush=True)
+        assert took[1] < 1.3 * took[0]
+    finally:
+        p.close()
+        dl.free()
+        du.free()
