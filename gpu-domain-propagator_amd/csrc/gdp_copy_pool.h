@@ -14,6 +14,15 @@
 
 namespace gdp {
 
+// The one T of the process, made on first use and never destroyed: at the
+// process's end its threads wait for work, and joining them there crashes a
+// forked child, which does not have them.
+template <typename T>
+T &process_wide() {
+    static T *t = new T();
+    return *t;
+}
+
 // Copies of this size and more from or to pageable host memory are bulk copies.
 constexpr size_t kBulkMin = 1u << 20;
 

@@ -202,10 +202,7 @@ class Staging {
     CopyPool pool_;
 };
 
-Staging &staging() {
-    static Staging st;
-    return st;
-}
+Staging &staging() { return process_wide<Staging>(); }
 
 void upload_bulk(void *dst, const void *src, size_t bytes, hipStream_t s) {
     Staging &st = staging();
