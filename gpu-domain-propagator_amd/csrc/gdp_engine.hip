@@ -2812,13 +2812,14 @@ void server_set_base(Server *S, const double *lbs, const double *ubs) {
     check(hipMemcpy(S->d_base + S->n, ubs, sizeof(double) * S->n, hipMemcpyHostToDevice), "H2D base");
     S->base_lb.assign(lbs, lbs + S->n);
     S->base_ub.assign(ubs, ubs + S->n);
-    S->has_base = true;
     // requests mostly agree with the base: its segment partials are theirs
+    // (admissions take them for granted, so the server has no base without them)
     if (S->P->M.n_seg_parts > 0 && S->P->M.mark_rows) {
         double *lb = S->d_base, *ub = S->d_base + S->n;
         set_reference(S->P, &lb, &ub, 1);
         check(hipStreamSynchronize(S->P->stream), "reference sync");
     }
+    S->has_base = true;
 }
 
 namespace {
