@@ -1949,7 +1949,8 @@ __global__ __launch_bounds__(256) void reset_rounds_kernel(DevState D, RoundPlan
 template <bool kUnits>
 __global__ __launch_bounds__(256) void load_rounds_kernel(DevMatrix M, DevState D, RoundPlan R, int n16, int n_bin,
                                                           int first) {
-    const bool ax = first || D.persist[kPersistAx] != 0;
+    const int used = D.persist[kPersistAx];  // (of a new state: anything)
+    const bool ax = (first | used) != 0;
     const int tid = blockIdx.x * blockDim.x + threadIdx.x;
     const int stride = gridDim.x * blockDim.x;
     const DevState A = block_view(M, D, R, 0), B = block_view(M, D, R, 1);
