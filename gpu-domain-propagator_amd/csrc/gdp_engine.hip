@@ -408,14 +408,16 @@ void validate(const InstanceView &v) {
 }
 
 // Accepted candidates of a step from which the next one processes all rows.
-// Marking pays while the rows it marks stay below an eighth of the rows (1M
-// rows: 2.80 ms with a quarter, 2.75 with an eighth, 2.78 with a sixteenth;
+// Marking pays while the rows it marks stay below about a sixth of the rows (ms
+// a call, persistent / loop, with a quarter, a sixth, an eighth: 12.4M entries
+// over 2M columns 7.04 / 7.02, 7.05 / 7.03, 7.13 / 7.06; 1M rows of 42M entries
+// 5.54 / 5.88, 5.53 / 5.88, 5.59 / 5.99; of 19M 2.64 / 2.65, 2.57 / 2.61 with both;
 // batches and node vectors the same with all three).  A candidate marks the
 // rows of its column: the mean length nnz / n, and at least the row it came
 // from.  (Without that row: 2.2M entries over 16M columns 1.83 ms, with it 0.95;
 // 5.5M over 5M 1.64 and 1.40.)
 long long default_mark_limit(const InstanceView &v) {
-    return static_cast<long long>(v.m) * v.n / (8LL * (static_cast<long long>(v.nnz) + v.n));
+    return static_cast<long long>(v.m) * v.n / (6LL * (static_cast<long long>(v.nnz) + v.n));
 }
 
 // Outcome of one unit from its state words (the reference's round-count

@@ -44,7 +44,7 @@ typedef struct {
     int row_marking;         /* 1 (default): a round processes only rows with a column
                                 that moved in the previous round; 0: every row */
     int mark_limit;          /* accepted candidates of a round from which the next round
-                                processes every row instead (0: default max(64, m n / (8 (nnz + n)))) */
+                                processes every row instead (0: default max(64, m n / (6 (nnz + n)))) */
     int group_log[10];       /* lanes per row (log2) for rows of width 2^b; -1: default */
 } gdp_tuning;
 

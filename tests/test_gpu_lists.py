@@ -82,3 +82,21 @@ def test_many_windows(gpu, oracle, count):
     _run(inst, nodes, [k % 12 for k in range(count)], I.MEGAKERNEL)
     if count < 2000:
         _run(inst, nodes, [k % 12 for k in range(count)], I.CPU_LOOP)
+
+
+@pytest.mark.parametrize("seed", [2, 3, 5, 7])
+def test_rounds_after_few_candidates_process_marked_rows(gpu, seed):
+    """A round processes every row after max(64, m n / (6 (nnz + n))) accepted
+    candidates or more, else marked rows.  These runs have a round between an
+    eighth and a sixth."""
+    inst = small_mip(seed=seed, m=8000, n=40_000, len_hi=60, fixed_frac=0.02)
+    p = I.Problem(inst)
+    try:
+        out, rows, _, _, accepted = p.work_profile(inst.lb, inst.ub)
+    finally:
+        p.close()
+    limit = max(64, inst.m * inst.n // (6 * (inst.nnz + inst.n)))
+    between = [a for a in accepted if inst.m * inst.n // (8 * (inst.nnz + inst.n)) <= a < limit]
+    assert between, (list(accepted), limit)
+    for k in range(out.rounds - 1):
+        assert (rows[k + 1] == inst.m) == (accepted[k] >= limit), (k, list(rows), list(accepted), limit)
