@@ -520,9 +520,8 @@ def summarize(d, kernel="mega_kernel"):
 
 def summarize_steps(d, out_md):
     """Per-round durations of the step kernels (sweep, apply, publish) of the
-    CPU_LOOP propagations in a rocprofv3 kernel trace under d: one row per
-    round of the last propagation of each round count (the timed ones come
-    after the warmup), written as a markdown table to out_md."""
+    fastest CPU_LOOP propagation in a rocprofv3 kernel trace under d: one row
+    per round, written as a markdown table to out_md."""
     trace = _csv_rows(f"{d}/**/*kernel_trace.csv")
     trace.sort(key=lambda r: int(r["Start_Timestamp"]))
     props, cur = [], None
@@ -543,36 +542,31 @@ def summarize_steps(d, out_md):
             cur["wall"] = (int(r["End_Timestamp"]) - cur["start"]) / 1e3
             props.append(cur)
             cur = None
-    last = {}  # the fastest propagation of each round count (a timed one)
-    for p in props:
-        k = len(p["steps"])
-        if k not in last or p["wall"] < last[k]["wall"]:
-            last[k] = p
+    p = min(props, key=lambda q: q["wall"])  # the fastest propagation: a timed step
     with open(out_md, "w") as fh:
         fh.write("# Step kernels per round (CPU_LOOP launches)\n\n")
         fh.write("Commands (from the repository root, `cd /tmp && export TMPDIR=/tmp` first):\n\n")
         fh.write(f"    rocprofv3 --kernel-trace --stats --output-format csv -d {d} -o steps -- python3 bench.py "
                  "--sync 0 --steps 3 --warmup 1 --no-cpu --no-batch --no-serve --no-extra --no-tune\n")
         fh.write(f"    python3 bench.py --summarize-steps {d} {out_md}\n\n")
-        fh.write("Durations in microseconds from the kernel trace, one propagation per round count "
-                 "(the fastest one from its load to its unpack: a timed step).\n\n")
-        for k in sorted(last):
-            p = last[k]
-            tot = [sum(x[i] for x in p["steps"]) for i in range(3)]
-            fh.write(f"## {k} rounds: sweep {tot[0]:.0f} us, apply {tot[1]:.0f} us, publish {tot[2]:.0f} us, "
-                     f"load to unpack {p['wall']:.0f} us\n\n| round | sweep | apply | publish |\n|---|---|---|---|\n")
-            for i, x in enumerate(p["steps"]):
-                fh.write(f"| {i + 1} | {x[0]:.1f} | {x[1]:.1f} | {x[2]:.1f} |\n")
-            fh.write("\n")
+        tot = [sum(x[i] for x in p["steps"]) for i in range(3)]
+        fh.write(f"Durations in microseconds from the kernel trace of the fastest propagation: sweep {tot[0]:.0f}, "
+                 f"apply {tot[1]:.0f}, publish {tot[2]:.0f}, load to unpack {p['wall']:.0f}.  The host issues launches "
+                 "two steps ahead: those past the last round stop themselves.\n\n"
+                 "| round | sweep | apply | publish |\n|---|---|---|---|\n")
+        for i, x in enumerate(p["steps"]):
+            fh.write(f"| {i + 1} | {x[0]:.1f} | {x[1]:.1f} | {x[2]:.1f} |\n")
     print(f"wrote {out_md}")
 
 
 def summarize_batch(d, out_md):
     """The batched leg from a rocprofv3 kernel trace under d of a bench run
-    whose stdout (the JSON line) is in d/bench.out: the last 260 mega_kernel
-    dispatches are the 4 launches of the tuned batch and the 256 plain
-    launches, in that order."""
-    trace = [r for r in _csv_rows(f"{d}/**/*kernel_trace.csv") if "mega_kernel" in r["Kernel_Name"]]
+    whose stdout (the JSON line) is in d/bench.out: the last 260 persistent
+    launches (mega_kernel, or rounds_kernel of single problems) are the 4
+    launches of the tuned batch and the 256 plain launches, in that order."""
+    trace = [r for r in _csv_rows(f"{d}/**/*kernel_trace.csv")
+             if "mega_kernel" in r["Kernel_Name"] or "rounds_kernel<" in r["Kernel_Name"] and
+             not any(k in r["Kernel_Name"] for k in ("load_rounds", "reset_rounds", "plan_rounds", "unpack_"))]
     trace.sort(key=lambda r: int(r["Start_Timestamp"]))
     dur = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e6 for r in trace]
     grid = [int(r.get("Grid_Size_X") or r.get("Grid_Size") or 0) // max(1, int(r.get("Workgroup_Size_X") or
