@@ -147,18 +147,32 @@ __device__ __forceinline__ unsigned record_offset(const DevMatrix &M, const DevS
 // (other kernels run with D.n_lds = 0 and never touch it).
 extern __shared__ __align__(16) unsigned dyn_lds[];
 
-// The 16 bytes from byte `off` of the unit's snapshot block (a multiple of 4),
-// zeros from kNoRecord.  One buffer load whatever the record's class: the
-// record's own bytes come first, so nothing has to be picked out of an
-// aligned chunk, the address takes no 64-bit arithmetic, and the lanes
-// without an entry are cut off by the bounds check instead of by masks.
+// The bytes from byte `off` of the unit's snapshot block (a multiple of the
+// record's size), the record's own first, zeros from kNoRecord.  One 16-byte
+// buffer load whatever the record's class: the address takes no 64-bit
+// arithmetic, and the lanes without an entry are cut off by the bounds check
+// instead of by masks.  Of blocks with 4-byte records it is the aligned 16 bytes
+// that hold the record, picked apart: from the record's own first byte every
+// tenth load crossed into a second line, and a sweep is bound by such requests
+// (ms a call: 12.4M entries over 2M columns 8.11 -> 7.90 persistent, 8.00 -> 7.79 in
+// the loop; 16M with rows of up to 50,000 3.54 -> 3.53 and 3.54 -> 3.45; 1M rows 2.83
+// -> 2.84 and 2.86 -> 2.80; 256 node vectors 2.84 -> 2.86).  Where records have 8
+// bytes or 16, every sixteenth crosses, and picking gains nothing.
 constexpr unsigned kNoRecord = 0xfffffff0u;
 template <int kMode>
 __device__ __forceinline__ uint4 load_record(const DevMatrix &M, const DevState &D, unsigned off) {
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(D.S16, 0, static_cast<int>(M.snap_stride), 0x00020000);
     constexpr int kSc1 = 16;
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(off), 0,
+    const unsigned at = kMode == kRecords ? off & ~15u : off;
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at), 0,
                                                          kMode == kWideCoherent ? kSc1 : 0);
+    if constexpr (kMode == kRecords) {
+        // bits 3 and 2 of the offset as masks: two bit-field extracts, three inserts
+        const unsigned upper = static_cast<unsigned>(static_cast<int>(off << 28) >> 31);
+        const unsigned odd = static_cast<unsigned>(static_cast<int>(off << 29) >> 31);
+        const unsigned x = (v[2] & upper) | (v[0] & ~upper), y = (v[3] & upper) | (v[1] & ~upper);
+        return make_uint4((y & odd) | (x & ~odd), y, v[2], v[3]);
+    }
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
