@@ -33,7 +33,7 @@ struct Tuning {
     int block_threads = 256;  // threads per workgroup (multiple of 64)
     int mega_blocks_per_cu = 0;  // 0: occupancy limit
     int mega_threads = 512;   // workgroup size of the persistent kernel: 256, 512 or 1024
-    int graph_rounds = 8;     // rounds per captured graph for GPU_LOOP
+    int graph_rounds = 8;     // rounds per graph for GPU_LOOP
     int max_split_segs = -1;  // rows with more segments run on one wave (-1: split all, 0: none)
     int compact_bounds = 1;   // 0: keep every column in 16-byte FP64 records
     int row_marking = 1;      // 0: every round processes every row of an active unit

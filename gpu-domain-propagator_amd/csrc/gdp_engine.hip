@@ -7,7 +7,7 @@
 // width, columns relabelled by bound storage class, integrality folded into
 // the column index, a column-to-row index for row marking); rounds are
 // round-synchronous steps (sweep, apply of split rows, publish); GPU_LOOP is
-// a captured HIP graph of step launches that stop themselves on the device;
+// a HIP graph of step launches that stop themselves on the device;
 // several bound vectors or instances can share the launches (units).
 #include <hip/hip_runtime.h>
 
@@ -508,7 +508,7 @@ struct Problem {
     int sweep_grid = 0;               // workgroups of the step sweep kernel (all resident)
     const void *mega_fn = nullptr;
     const void *mega_fn_lds = nullptr;  // the same reading binary columns from LDS (one unit)
-    // captured GPU_LOOP graphs, one per chunk of steps, for one launch shape
+    // GPU_LOOP graphs, one per chunk of steps, for one launch shape
     std::vector<hipGraphExec_t> graphs;
     long long graph_key = -1;
     std::mutex run_mutex;
@@ -526,7 +526,7 @@ struct Problem {
     HostBlock h_bounds{host_blocks()};  // pinned: small bound vectors on their way
     int servers = 0;                  // servers attached (they own the unit slots)
     bool fail_waits = false;          // GDP_FAIL_WAITS
-    bool graphs_enabled = true;       // GPU_LOOP may capture graphs of the current run state
+    bool graphs_enabled = true;       // GPU_LOOP may keep graphs of the current run state
     bool staging_held = false;
 
     void drop_graphs() {
@@ -1650,25 +1650,54 @@ void load_units(Problem *P, int n_list, const int *list, double *const *lbp, dou
     }
 }
 
+// Where launches go: to a stream, or into a graph, each node after the one
+// before.  Graphs are built from their nodes, not captured: while any thread of
+// the process captures, hipDeviceSynchronize and copies through the null stream
+// fail in the other threads and end the capture.
+struct LaunchTarget {
+    hipStream_t stream = nullptr;
+    hipGraph_t graph = nullptr;
+    hipGraphNode_t last = nullptr;
+};
+template <typename T>
+struct AsDeclared {
+    using type = T;
+};
+template <typename... Args>
+void launch(LaunchTarget &to, void (*kernel)(Args...), int grid, int threads, size_t lds,
+            typename AsDeclared<Args>::type... args) {
+    void *params[] = {&args...};
+    if (!to.graph) {
+        check(hipLaunchKernel(reinterpret_cast<const void *>(kernel), dim3(grid), dim3(threads), params, lds, to.stream),
+              "step launch");
+        return;
+    }
+    hipKernelNodeParams node = {};
+    node.func = reinterpret_cast<void *>(kernel);
+    node.gridDim = dim3(grid);
+    node.blockDim = dim3(threads);
+    node.sharedMemBytes = static_cast<unsigned>(lds);
+    node.kernelParams = params;
+    hipGraphNode_t before = to.last;
+    check(hipGraphAddKernelNode(&to.last, to.graph, before ? &before : nullptr, before ? 1 : 0, &node), "graph node");
+}
+
 // One step of the listed units (already uploaded as the active list).
-void launch_step(Problem *P, int step, int guard, int first_step) {
+void launch_step(Problem *P, LaunchTarget &to, int step, int guard, int first_step) {
     const DevMatrix &M = P->M;
     const DevState &D = P->D;
-    hipStream_t s = P->stream;
     const long long n_work = P->replicas ? static_cast<long long>(M.n_items) * D.n_active : M.n_items;
     const int apply_grid = std::max(1, std::min(1024, grid_for(static_cast<long long>(M.n_seg_parts) *
                                                                  (P->replicas ? D.n_active : 1))));
     const int sweep_grid = static_cast<int>(std::min<long long>(grid_for(n_work), P->sweep_grid));
-    hipLaunchKernelGGL(sweep_kernel, dim3(sweep_grid), dim3(256), 0, s, M, D, step, guard, first_step,
-                       P->n_units);
-    if (M.n_seg_parts > 0)
-        hipLaunchKernelGGL(apply_split_kernel, dim3(apply_grid), dim3(256), 0, s, M, D, step, guard, first_step);
+    launch(to, sweep_kernel, sweep_grid, 256, 0, M, D, step, guard, first_step, P->n_units);
+    if (M.n_seg_parts > 0) launch(to, apply_split_kernel, apply_grid, 256, 0, M, D, step, guard, first_step);
     // 8 bitmap words a wave, 64 from where that still fills the chip
     const long long pub_units = P->replicas ? D.n_active : 1;
     long long pub_waves = pub_units * ((M.nwords + 7) / 8);
     if (P->replicas && pub_units * ((M.nwords + 63) / 64) >= 4096) pub_waves = pub_units * ((M.nwords + 63) / 64);
-    hipLaunchKernelGGL(publish_kernel, dim3(std::max(1, std::min(8192, grid_for(pub_waves)))), dim3(256), 0, s, M, D,
-                       step, guard, first_step, P->n_units);
+    launch(to, publish_kernel, std::max(1, std::min(8192, grid_for(pub_waves))), 256, 0, M, D, step, guard, first_step,
+           P->n_units);
 }
 
 // Waits until the launches have started step `step` or are over; returns the
@@ -1694,10 +1723,11 @@ int wait_round(Problem *P, int step) {
 // Steps that the launch loops run ahead of the host's look at the progress.
 constexpr int kAhead = 2;
 
-// Steps 1 .. max_rounds as captured graphs of graph_rounds steps (the launches
-// of one step by `launch`), kept for calls of the same key.  The next graph is
+// Steps 1 .. max_rounds as graphs of graph_rounds steps (the launches of one
+// step by `step_launches`), kept for calls of the same key.  The next graph is
 // launched while the last steps of the previous one run.
-void run_graphs(Problem *P, long long key, int max_rounds, const std::function<void(int)> &launch) {
+void run_graphs(Problem *P, long long key, int max_rounds,
+                const std::function<void(LaunchTarget &, int)> &step_launches) {
     hipStream_t s = P->stream;
     const int chunk = std::max(1, P->tuning.graph_rounds);
     if (key != P->graph_key) {
@@ -1708,13 +1738,17 @@ void run_graphs(Problem *P, long long key, int max_rounds, const std::function<v
         const int last = std::min(max_rounds, first + chunk - 1);
         if (static_cast<int>(P->graphs.size()) <= ci) P->graphs.resize(ci + 1, nullptr);
         if (!P->graphs[ci]) {
-            hipGraph_t graph;
-            check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture");
-            for (int step = first; step <= last; step++) launch(step);
-            check(hipStreamEndCapture(s, &graph), "end capture");
-            hipGraphExec_t exec;
-            check(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "instantiate");
-            (void)hipGraphDestroy(graph);
+            LaunchTarget to;
+            check(hipGraphCreate(&to.graph, 0), "graph");
+            hipGraphExec_t exec = nullptr;
+            try {
+                for (int step = first; step <= last; step++) step_launches(to, step);
+                check(hipGraphInstantiate(&exec, to.graph, nullptr, nullptr, 0), "instantiate");
+            } catch (...) {
+                (void)hipGraphDestroy(to.graph);
+                throw;
+            }
+            (void)hipGraphDestroy(to.graph);
             P->graphs[ci] = exec;
         }
         check(hipGraphLaunch(P->graphs[ci], s), "graph launch");
@@ -1728,6 +1762,7 @@ void run_steps(Problem *P, int sync_type, int max_rounds) {
     const DevMatrix &M = P->M;
     DevState &D = P->D;
     hipStream_t s = P->stream;
+    LaunchTarget to{s};
     check(hipEventRecord(P->ev0, s), "event");
     __atomic_store_n(&P->host->word, 0, __ATOMIC_RELAXED);
     if (sync_type == CPU_LOOP_ID || (sync_type == GPU_LOOP_ID && !P->graphs_enabled)) {
@@ -1736,13 +1771,13 @@ void run_steps(Problem *P, int sync_type, int max_rounds) {
         // steps, so that the device never waits for it (without graphs, e.g.
         // where nothing may be allocated, GPU_LOOP is the same)
         for (int step = 1; step <= max_rounds; step++) {
-            launch_step(P, step, 1, 1);
+            launch_step(P, to, step, 1, 1);
             if (step > kAhead && wait_round(P, step - kAhead) == kRoundsOver) break;
         }
         check(hipGetLastError(), "step launch");
     } else if (sync_type == GPU_LOOP_ID) {
         const long long key = static_cast<long long>(D.n_active) * 1000 + max_rounds;
-        run_graphs(P, key, max_rounds, [&](int step) { launch_step(P, step, 1, 1); });
+        run_graphs(P, key, max_rounds, [&](LaunchTarget &g, int step) { launch_step(P, g, step, 1, 1); });
     } else {
         int first = 1, steps = max_rounds, n_units = P->n_units;
         // dynamic LDS: the sweep's window for several units, else the
@@ -1786,7 +1821,7 @@ std::vector<UnitState> read_units(Problem *P, int n_list, const int *list) {
 // ---- double-buffered rounds of one bound vector ----
 
 // Issues round `step`.
-void launch_round(Problem *P, int step) {
+void launch_round(Problem *P, LaunchTarget &to, int step) {
     // with a copy of the moved columns in LDS few large workgroups, all resident
     const size_t lds = sizeof(unsigned) * P->R.bit_words;
     const bool small = lds == 0;
@@ -1795,20 +1830,20 @@ void launch_round(Problem *P, int step) {
     const int grid = std::max(1, std::min((small ? 8 : 2) * P->cu_count, (P->rounds_work + waves - 1) / waves));
     const int apply_grid = std::max(1, std::min(1024, grid_for(P->Mr.n_seg_parts)));
     if (!P->replicas) {
-        hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(kMaxRoundUnits), 0, P->stream, P->Mr, P->D, P->R, step);
-        hipLaunchKernelGGL(lds > 0 ? batch_round_kernel<true> : batch_round_kernel<false>, dim3(grid), dim3(threads), lds, P->stream, P->Mr, P->D, P->R, step);
-        if (P->Mr.n_seg_parts > 0)
-            hipLaunchKernelGGL(batch_apply_kernel, dim3(apply_grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+        launch(to, batch_plan_kernel, 1, kMaxRoundUnits, 0, P->Mr, P->D, P->R, step);
+        launch(to, lds > 0 ? batch_round_kernel<true> : batch_round_kernel<false>, grid, threads, lds, P->Mr, P->D, P->R,
+               step);
+        if (P->Mr.n_seg_parts > 0) launch(to, batch_apply_kernel, apply_grid, 256, 0, P->Mr, P->D, P->R, step);
         return;
     }
-    hipLaunchKernelGGL(lds > 0 ? round_kernel<true> : round_kernel<false>, dim3(grid), dim3(threads), lds, P->stream, P->Mr, P->D, P->R, step);
-    if (P->Mr.n_seg_parts > 0)
-        hipLaunchKernelGGL(round_apply_kernel, dim3(apply_grid), dim3(256), 0, P->stream, P->Mr, P->D, P->R, step);
+    launch(to, lds > 0 ? round_kernel<true> : round_kernel<false>, grid, threads, lds, P->Mr, P->D, P->R, step);
+    if (P->Mr.n_seg_parts > 0) launch(to, round_apply_kernel, apply_grid, 256, 0, P->Mr, P->D, P->R, step);
 }
 
 // Issues the rounds of a loaded run, between the problem's two events.
 void issue_rounds(Problem *P, int sync_type, int max_rounds) {
     hipStream_t s = P->stream;
+    LaunchTarget to{s};
     check(hipEventRecord(P->ev0, s), "event");
     if (sync_type == MEGAKERNEL_ID) {
         void *args[] = {&P->Mr, &P->D, &P->R};
@@ -1816,10 +1851,10 @@ void issue_rounds(Problem *P, int sync_type, int max_rounds) {
                                          sizeof(unsigned) * P->R.bit_words, s),
               "rounds launch");
     } else if (sync_type == GPU_LOOP_ID && P->graphs_enabled) {
-        run_graphs(P, (1LL << 40) + max_rounds, max_rounds, [&](int step) { launch_round(P, step); });
+        run_graphs(P, (1LL << 40) + max_rounds, max_rounds, [&](LaunchTarget &g, int step) { launch_round(P, g, step); });
     } else {
         for (int step = 1; step <= max_rounds; step++) {
-            launch_round(P, step);
+            launch_round(P, to, step);
             if (step > kAhead && wait_round(P, step - kAhead) == kRoundsOver) break;
         }
         check(hipGetLastError(), "round launch");
@@ -2032,8 +2067,7 @@ RunResult problem_propagate_device(Problem *P, double *d_lbs, double *d_ubs, int
 }
 
 // The whole call holds the problem's lock: the bound vectors travel on the
-// problem's stream, which another thread's call may otherwise be capturing
-// into a graph (GPU_LOOP) or waiting on.
+// problem's stream, which another thread's call may otherwise be using.
 RunResult problem_propagate(Problem *P, double *lbs, double *ubs, int sync_type, int max_rounds) {
     std::lock_guard<std::mutex> lock(P->run_mutex);
     check_no_server(P);
@@ -2159,7 +2193,8 @@ RunResult problem_work_profile(Problem *P, double *lbs, double *ubs, int max_rou
                     count_entries(start, g * kSegLen, std::min(len, (g + 1) * kSegLen));
                 }
             }
-            launch_step(P, step, 0, 1);
+            LaunchTarget to{s};
+            launch_step(P, to, step, 0, 1);
             check(hipGetLastError(), "step launch");
             int cnt[kMoveLanes * kMoveStride];
             check(hipMemcpyAsync(cnt, P->D.moved + moved_index(0, step % kMoveSlots, 0), sizeof(cnt),
@@ -2228,7 +2263,8 @@ RunResult problem_propagate_measured(Problem *P, double *lbs, double *ubs, int m
         int rounds = 0;
         for (int step = 1; step <= max_rounds; step++) {
             if (step == 1 ? st[0].crossed != 0 : !active_after(st[0], step - 1)) break;
-            launch_step(P, step, 0, 1);
+            LaunchTarget to{s};
+            launch_step(P, to, step, 0, 1);
             check(hipGetLastError(), "step launch");
             hipLaunchKernelGGL(unpack_kernel<false>, dim3(gx), dim3(256), 0, s, P->M, P->D, 1, P->d_list, P->d_lbp,
                                P->d_ubp, gx, 0, ChangeLists());
@@ -2332,7 +2368,7 @@ char *scratch_address(int dev) {
 }
 
 // Runs the problem on a borrowed run state for the lifetime of the object:
-// the owned state (if any), its launch tables and its captured graphs are
+// the owned state (if any), its launch tables and its graphs are
 // set aside and restored afterwards.
 class BorrowedState {
   public:
@@ -3226,7 +3262,8 @@ int step_impl(Server *S) {
     if (active.empty()) return 0;
     upload(P->d_list, active.data(), active.size(), s);
     P->D.n_active = static_cast<int>(active.size());
-    launch_step(P, S->step, 0, S->step);
+    LaunchTarget to{s};
+    launch_step(P, to, S->step, 0, S->step);
     check(hipGetLastError(), "step launch");
     // the states come back in pinned memory: one wait
     const int n_act = static_cast<int>(active.size());
@@ -3265,7 +3302,6 @@ int step_impl(Server *S) {
         upload(P->d_list, fin.data(), fin.size(), s);
         upload(P->d_lbp, lbp.data(), fin.size(), s);
         upload(P->d_ubp, ubp.data(), fin.size(), s);
-        const int gx = std::max(1, std::min(1024, (P->M.n + 255) / 256));
         // delta requests (against the base vector) and in-place zero-copy
         // requests (against their own input): the columns that differ, listed
         // by the unpack, packed into pinned memory, so that only they cross PCIe

@@ -1587,7 +1587,7 @@ __device__ __forceinline__ void publish_phase(const DevMatrix &M, const DevState
 // step kernels (CPU_LOOP, GPU_LOOP)
 // ---------------------------------------------------------------------------
 
-// With `guard` (captured graphs), a launch first checks on the device whether
+// With `guard`, a launch first checks on the device whether
 // the previous step changed anything; if not, the run is over and the launch
 // does nothing.
 __device__ __forceinline__ bool step_skipped(const DevState &D, int step, int first_step) {

@@ -37,7 +37,7 @@ typedef enum GDP_Vartype GDP_VARTYPE;
 
 /* How propagation rounds are driven (reference src/def.h:36-41).
  *   CPU_LOOP   - one kernel launch per round, host reads the change flag.
- *   GPU_LOOP   - rounds run without host round-trips from a captured HIP
+ *   GPU_LOOP   - rounds run without host round-trips from a HIP
  *                graph of round launches that exit early on the device once
  *                the fixpoint is reached (HIP has no dynamic parallelism).
  *   MEGAKERNEL - one persistent launch iterates all rounds with device-wide

@@ -35,7 +35,7 @@ typedef struct {
     int item_nnz;            /* target nonzeros per work item (0: default, 1024) */
     int mega_blocks_per_cu;  /* persistent grid: workgroups per CU (0: occupancy) */
     int mega_threads;        /* persistent kernel workgroup size: 256, 512 (default) or 1024 */
-    int graph_rounds;        /* rounds per captured graph in GPU_LOOP (0: 8) */
+    int graph_rounds;        /* rounds per graph in GPU_LOOP (0: 8) */
     int max_split_segs;      /* rows longer than 256 entries with up to this many
                                 256-entry segments are split into one wave per
                                 segment (-1: default, all; 0: never split) */
@@ -127,7 +127,7 @@ GDP_RETCODE gdpPropagateDevice(gdp_problem p, double *d_lbs, double *d_ubs, cons
  * problems on a device and keeps the last call's contents; every call resets
  * what it reads.  Calls on one device are serialised by the library (calls
  * that overlapped on one array would race).  Supports every sync type;
- * GPU_LOOP issues its self-stopping launches without capturing a graph. */
+ * GPU_LOOP issues its self-stopping launches without a graph. */
 #define GDP_NOALLOC_SCRATCH_BYTES (64LL << 20)
 GDP_RETCODE gdpPropagateDeviceNoAlloc(gdp_problem p, double *d_lbs, double *d_ubs, const int sync_type,
                                       const int max_rounds, gdp_run_info *info);

@@ -62,3 +62,38 @@ def test_two_threads(gpu, oracle, kept):
     for th in threads:
         th.join()
     assert not errors, errors
+
+
+def test_graphs_beside_synchronising_calls(gpu, oracle):
+    """New graphs of launches are made while another thread copies through the
+    null stream and waits for the device: neither disturbs the other.  (Captures
+    were ended by such calls, which failed themselves.)"""
+    inst = small_mip(seed=3, m=300, n=200)
+    exp = oracle.jacobi(inst)
+    stop, errors, copies = threading.Event(), [], [0]
+    array = I.DeviceArray(inst.lb)
+
+    def copy():
+        try:
+            while not stop.is_set():
+                array.upload(inst.lb)
+                copies[0] += 1
+        except BaseException as e:  # reported below
+            errors.append(e)
+
+    th = threading.Thread(target=copy)
+    th.start()
+    try:
+        for k in range(60):
+            _same(I.gpu_propagate(inst, I.GPU_LOOP), exp, f"run {k}")
+        b = I.Batch([inst] * 3)
+        for k in range(20):
+            for got in b.propagate(sync_type=I.GPU_LOOP, max_rounds=100 - k):
+                np.testing.assert_array_equal(got.lbs, exp[0], err_msg=f"batch {k}")
+        b.close()
+    finally:
+        stop.set()
+        th.join()
+        array.free()
+    assert not errors, errors
+    assert copies[0] > 60
