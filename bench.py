@@ -574,7 +574,7 @@ def summarize_batch(d, out_md):
             for r in trace]
     wg = [int(r.get("Workgroup_Size_X") or r.get("Workgroup_Size") or 0) for r in trace]
     if len(dur) < 260:
-        raise SystemExit(f"{len(dur)} mega_kernel dispatches, expected at least 260")
+        raise SystemExit(f"{len(dur)} persistent launches, expected at least 260")
     batch, plain = dur[-260:-256], dur[-256:]
     line = None
     with open(f"{d}/bench.out") as fh:
@@ -592,7 +592,8 @@ def summarize_batch(d, out_md):
         fh.write(f"    rocprofv3 --kernel-trace --stats --output-format csv -d {d} -o batch -- python3 bench.py "
                  f"--no-serve --no-cpu --no-extra --no-tune > {d}/bench.out\n")
         fh.write(f"    python3 bench.py --summarize-batch {d} {out_md}\n\n")
-        fh.write(f"The kernel trace holds {len(dur)} `mega_kernel` dispatches in the bench's order (the 1M-row "
+        fh.write(f"The kernel trace holds {len(dur)} persistent launches (`mega_kernel`, and `rounds_kernel` of the plain "
+                 "launches, which run double-buffered rounds) in the bench's order (the 1M-row "
                  "problem, the drop-in call, the batch with the default layout, the autotuner's trials on a "
                  "sample of 32 instances, the batch with the tuned layout, the 256 plain launches); the figures "
                  "are the last 260 (end minus start timestamp).\n\n")

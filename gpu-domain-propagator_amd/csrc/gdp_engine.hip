@@ -1053,6 +1053,9 @@ void plan_rounds(Problem *P, const int *start, const int *count, const std::vect
     // 1.20 (1.80 / 1.65); 7.8M 1.65 / 1.69 (1.91 / 1.76); 9.0M with long rows 1.56
     // / 1.47 (1.60 / 1.47); 12.6M over 1M columns, 2 rounds 0.25 (0.17); 20.1M 3.4
     // / 3.3 (2.6 / 3.0).
+    // Of few rounds, us a call in the loop: 1.3M entries, one round 60 (73); 3.8M,
+    // two 87 (101); 7.0M over 110,000 columns, two 113 (114), over 550,000 127 (124);
+    // 7.6M over 1.2M columns, two 186 (133); 6.6M, two of many 201 (239).
     constexpr int kMaxRoundEntries = 8 << 20;
     // A batch leaves out the instances that are done, so its line lies higher:
     // 64 instances of 42,000 entries 0.98 / 1.01 (2.77 / 2.45), of 88,000 2.2 (4.05 /
@@ -1256,7 +1259,7 @@ Problem *build(const std::vector<InstanceView> &inst, bool replicas, const Tunin
         // ---- rows grouped by tree width: long rows first, then wide to
         // narrow; instance-major inside a bin so that items never mix units.
         // Ordered on the device; rows padded to multiples of kRowAlign entries
-        // (padding: column 0, coefficient 0), the padding count in the low
+        // (padding: column n, coefficient 0), the padding count in the low
         // bits of the row starts ----
         constexpr int kLongBin = 10;
         int *d_perm = dev_alloc<int>(device_columns ? P->n : C.n_ids, o);
